@@ -1,6 +1,7 @@
 // Entry of the persistent multi-batch trace (batch_kernel.h): argument checks and the
 // choice of the launcher for the scene's triangle test and the node layout.
 #include "batch_kernel.h"
+#include "wide_trace.h"
 
 namespace mh {
 
@@ -14,10 +15,10 @@ int launch_trace_batch(const DevScene& sc, const BatchLaunch& bl, void* stream) 
   if (sc.prim_kind == 1)
     return bl.layout == kLayoutRef   ? launch_batch_wald_ref(sc, bl, s)
            : bl.layout == kLayoutSoa ? launch_batch_wald_soa(sc, bl, s)
-                                     : launch_batch_wald_pair(sc, bl, s);
+                                     : launch_wide_table_wald(sc, bl, s);
   return bl.layout == kLayoutRef   ? launch_batch_ks_ref(sc, bl, s)
          : bl.layout == kLayoutSoa ? launch_batch_ks_soa(sc, bl, s)
-                                   : launch_batch_ks_pair(sc, bl, s);
+                                   : launch_wide_table_ks(sc, bl, s);
 }
 
 }  // namespace mh

@@ -1,6 +1,7 @@
-// Persistent multi-batch traversal for gfx950 (wave64). Included by the four
-// batch_<triangle>_<layout>.hip files, which instantiate the launchers of one triangle
-// test and node layout each, so that the kernel variants compile in parallel.
+// Persistent multi-batch traversal of the REF and SOA node layouts for gfx950 (wave64).
+// Included by the four batch_<triangle>_<layout>.hip files, which instantiate the launchers
+// of one triangle test and node layout each, so that the kernel variants compile in
+// parallel. (Frames in the default layout run k_trace_wide, wide_trace.h.)
 //
 // k_trace_batch consumes a table of ray batches (each its own SoA arrays, size and
 // closest-hit/any-hit flag) in one launch. Rays are numbered across batches by the
@@ -20,12 +21,10 @@
 // ends on short rays. The last wave to leave resets the counters, so consecutive launches
 // (and graph replays) need no clearing pass.
 //
-// Three node layouts, all giving the reference's one-ray results and visit order
+// Both layouts give the reference's one-ray results and visit order
 // (DynBVH::intersectNode on a one-ray packet, Model/Groups/DynBVH.cc:274-404; the
-// traversal loops are traverse.h's): PAIR (64-byte records with both child boxes), SOA
-// (the same records as four arrays of their 16-byte fields) and REF (the reference's
-// 32-byte records).
-// Triangle tests and arithmetic are those of trace.hip (shared header).
+// traversal loops are traverse.h's): SOA (64-byte records with both child boxes, as four
+// arrays of their 16-byte fields) and REF (the reference's 32-byte records).
 //
 // A table whose batches are all closest-hit (or all any-hit) runs a kernel specialised to
 // that kind, without the other traversal's code and registers; mixed tables branch per
@@ -118,7 +117,7 @@ __device__ __forceinline__ bool step_ref(const DevScene& sc, Lane& L, LaneStack<
   return true;
 }
 
-// Per-lane refill schedule, PAIR and SOA layouts: one round of traverse.h's trace_pair loop,
+// Per-lane refill schedule, SOA layout: one round of traverse.h's trace_pair loop,
 // resumed from the lane's state: the walk down inner nodes to a leaf (or to a miss), the leaf's
 // triangles and the pops to the next entry still worth visiting. The lanes of a wave walk
 // the inner nodes in lockstep (a lane that reached its leaf waits for the others), so the
@@ -131,7 +130,7 @@ __device__ __forceinline__ bool round_pair(const DevScene& sc, Lane& L, LaneStac
   while (L.cur >= 0) {
     float4 A, B, C;
     int4 M;
-    fetch_pair<LAYOUT>(sc, L.cur, A, B, C, M);
+    fetch_pair(sc, L.cur, A, B, C, M);
     float tn0, tn1;
     const bool h0 = slab_v<FAST>(A.x, A.y, A.z, A.w, B.x, B.y, L.r, L.h.minT, tn0);
     const bool h1 = slab_v<FAST>(B.z, B.w, C.x, C.y, C.z, C.w, L.r, L.h.minT, tn1);
@@ -222,7 +221,7 @@ __device__ __forceinline__ bool start_in(const DevScene& sc, const RefNode& root
       store_hit(B.hits, L.li, -1, L.h.minT, 0.f, 0.f, false);
       return false;
     }
-    L.cur = sc.root_ref;
+    L.cur = pair_root(sc);
   } else {
     L.cur = 0;
   }
@@ -481,9 +480,7 @@ int launch_b(const DevScene& sc, const BatchLaunch& bl, hipStream_t s) {
 }  // namespace
 
 // One launcher per triangle test and node layout (batch_<triangle>_<layout>.hip).
-int launch_batch_ks_pair(const DevScene& sc, const BatchLaunch& bl, hipStream_t s);
 int launch_batch_ks_ref(const DevScene& sc, const BatchLaunch& bl, hipStream_t s);
-int launch_batch_wald_pair(const DevScene& sc, const BatchLaunch& bl, hipStream_t s);
 int launch_batch_wald_ref(const DevScene& sc, const BatchLaunch& bl, hipStream_t s);
 int launch_batch_ks_soa(const DevScene& sc, const BatchLaunch& bl, hipStream_t s);
 int launch_batch_wald_soa(const DevScene& sc, const BatchLaunch& bl, hipStream_t s);

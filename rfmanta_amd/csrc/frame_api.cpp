@@ -171,6 +171,7 @@ int launch(mh_frame* f, void* stream) {
   bl.chunk = f->cfg.chunk;
   bl.xcd_remap = f->cfg.xcd_remap;
   bl.reverse = f->cfg.reverse;
+  bl.resident = mh_internal::resident_waves();
   bl.kinds = kinds_of(f->nb, f->n_any);
   HIP_OK((hipError_t)mh::launch_trace_batch(f->scene->dev(), bl, stream));
   return MH_OK;

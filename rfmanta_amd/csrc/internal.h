@@ -23,6 +23,8 @@ int ensure_init();
 // Compute units and architecture name of the library's device (valid after ensure_init()).
 int cu_count();
 const char* device_name();
+// Waves of the wide traversal kernel the device holds at once (five per SIMD).
+inline int resident_waves() { return 20 * cu_count(); }
 
 // The allocation-free trace's fixed scratch area (noalloc.hip). scratch_setup looks up
 // its device address on `device` (which must be current) once; ensure_init calls it. A
@@ -105,24 +107,27 @@ struct mh_scene {
   int workers = 1;
   uint32_t large_limit() const { return (uint32_t)(n_records / (20 * (uint32_t)workers)); }
 
-  DevBuf refs, pairs, tris, ids, big, d_verts, d_base, d_idx, leaves, levels;
+  DevBuf refs, wide, tris, ids, big, d_verts, d_base, d_idx, leaves, levels;
   // rotating update (mh_scene_update): costs, subtree sizes, parents, object boxes and
   // centroids, depth work arrays, the depth histogram and counters
   DevBuf costs, ssize, parent, obox, ocen, anc0, dep0, anc1, dep1, hist, counters;
   DevBuf split_list;  // rotating update: leaves whose parent's rotation may split them
   DevBuf levels_aux;  // rotating update: first child and word beside each level entry
-  // rotating update: per object slot, the record of the leaf whose first slot it is, else -1
-  // (filled from the leaf list after a build or load, kept by the update's level pass)
+  // Per object slot, the record of the leaf whose first slot it is, else -1.
   DevBuf leaf_at;
-  bool leaf_at_valid = false;
+  // The leaves partition the object slots (always, except in some loaded trees), so that a
+  // slot's leaf is the nearest one starting at or before it.
+  bool partition = false;
+  DevBuf irregular;  // int32[2]: mh::DevScene::irregular and the NaN mark of a pass
   DevBuf logtab;  // RTSAH table logarithm (device build)
   DevBuf normals, normal_idx, texcoords, tex_idx;  // shading attributes (mh_shade)
-  // The PairNodes as four arrays of their 16-byte fields (MH_LAYOUT_SOA launches):
-  // allocated on first use and copied from `pairs` again when pairs_gen (bumped by every
-  // call that writes the pair records) has moved past soa_gen.
-  DevBuf pairs_soa;
-  uint64_t pairs_gen = 0, soa_gen = ~0ull;
-  std::vector<int64_t> level_off;  // inner records of depth d: levels[level_off[d], level_off[d+1])
+  // The PairNodes and their copy as four arrays of their 16-byte fields (MH_LAYOUT_SOA
+  // launches): allocated on first use and made again when tree_gen (bumped by every call
+  // that writes the tree) has moved past soa_gen.
+  DevBuf pairs, pairs_soa;
+  uint64_t tree_gen = 0, soa_gen = ~0ull;
+  std::vector<mh::LevelList> lev;  // inner records of each depth, in `levels`
+  size_t list_cap = 0;             // entries of the leaf list and of each level list
 
   std::mutex spill_mu;  // guards the per-stream spill areas
   std::mutex stage_mu;  // serialises mh_trace_host calls on the staging buffers
@@ -144,22 +149,26 @@ struct mh_scene {
            parent.bytes + obox.bytes + ocen.bytes + anc0.bytes + dep0.bytes + anc1.bytes +
            dep1.bytes + hist.bytes + counters.bytes + logtab.bytes + normals.bytes +
            normal_idx.bytes + texcoords.bytes + tex_idx.bytes + pairs_soa.bytes +
-           split_list.bytes + levels_aux.bytes + leaf_at.bytes;
+           split_list.bytes + levels_aux.bytes + leaf_at.bytes + wide.bytes + irregular.bytes;
   }
-  // Traversal stack entries a single ray can hold at most (one push per level).
-  uint32_t stack_bound(int /*layout*/) const {
-    return depth;
+  // Traversal stack entries a single ray can hold at most: one push per level, or three per
+  // wide node of the deepest path.
+  uint32_t stack_bound(int layout) const {
+    return layout == MH_LAYOUT_PAIR ? 3 * ((depth + 1) / 2) : depth;
   }
   mh::DevScene dev() const {
     mh::DevScene d{};
-    d.pairs = pairs.as<const mh::PairNode>();
+    d.wide = wide.as<const mh::WideNode>();
+    d.n_wide = (uint32_t)(wide.bytes / sizeof(mh::WideNode));
+    d.leaf_at = leaf_at.as<const int32_t>();
+    d.irregular = irregular.as<const int32_t>();
     d.refs = refs.as<const mh::RefNode>();
     d.tris = tris.as<const float>();
     d.obj_ids = ids.as<const int32_t>();
     d.big_count = big.as<const int32_t>();
     d.root_ref = root_ref;
     d.prim_kind = prim_kind;
-    d.n_pairs = (uint32_t)(pairs.bytes / sizeof(mh::PairNode));
+    d.n_pairs = (uint32_t)(pairs_soa.bytes / sizeof(mh::PairNode));
     d.n_slots = (uint32_t)(tris.bytes / (12 * sizeof(float)));
     d.pairs_soa = pairs_soa.p;
     return d;

@@ -124,25 +124,157 @@ void rotation_state(const std::vector<mh::RefNode>& nodes, std::vector<float>& c
   }
 }
 
-// Lays the reference tree out for the device: PairNodes indexed by sibling pair, leaf
-// references, the leaf and per-depth lists for refits, the rotation state, then uploads.
-// With rtsah, isLeftCheaper is recomputed once the records are known to form a tree
-// (DynBVH::buildFromFile runs computeTraversalCost after reading, DynBVH.cc:2469-2472).
+// Room for the device tree of T objects and nrec records with n_inner inner records and
+// n_leaves leaves: level and leaf lists of T entries, which the rotating update needs (a
+// partition of T objects has at most T leaves and T - 1 inner records), and of every record
+// of a loaded tree whose leaves overlap (it can hold more leaves than objects). Of I inner
+// records at most (2 I + 1) / 3 lie at even depths: all but the root have an inner parent
+// at an odd depth, and that has at most two such children.
+int reserve_tree(mh_scene* s, size_t nrec, size_t n_inner, size_t n_leaves) {
+  const size_t T = s->nt;
+  s->list_cap = std::max<size_t>({1, T, n_inner, n_leaves});
+  const size_t n_wide = (2 * std::max(T, n_inner) + 1) / 3 + 1;
+  int rc;
+  if ((rc = s->refs.reserve(nrec * sizeof(mh::RefNode))) ||
+      (rc = s->wide.reserve(n_wide * sizeof(mh::WideNode))) ||
+      (rc = s->tris.reserve(T * 48)) || (rc = s->ids.reserve(T * 4)) ||
+      (rc = s->big.reserve(T * 4)) || (rc = s->leaf_at.reserve(T * 4)) ||
+      (rc = s->leaves.reserve(s->list_cap * 4)) || (rc = s->levels.reserve(2 * s->list_cap * 4)) ||
+      (rc = s->levels_aux.reserve(s->list_cap * 8)) || (rc = s->costs.reserve(nrec * 4)) ||
+      (rc = s->ssize.reserve(nrec * 4)) || (rc = s->hist.reserve(mh::kFrontierWords * 4)) ||
+      (rc = s->counters.reserve(16)) || (rc = s->irregular.reserve(8)))
+    return rc;
+  if (!s->host_ctr) {
+    void* h = nullptr;
+    if (hipHostMalloc(&h, (mh::kFrontierWords + 2) * 4, hipHostMallocDefault) != hipSuccess)
+      return fail(MH_E_NOMEM, "hipHostMalloc of the level counters' copy");
+    s->host_ctr = static_cast<unsigned*>(h);
+  }
+  return MH_OK;
+}
+
+mh::DevUpdate tree_view(mh_scene* s) {
+  mh::DevUpdate u{};
+  u.refs = s->refs.as<mh::RefNode>();
+  u.pairs = s->pairs.as<mh::PairNode>();
+  u.big_count = s->big.as<int32_t>();
+  u.costs = s->costs.as<float>();
+  u.ssize = s->ssize.as<uint32_t>();
+  u.parent = s->parent.as<int32_t>();
+  u.ids = s->ids.as<int32_t>();
+  u.verts = s->d_verts.as<float>();
+  u.idx = s->d_idx.as<uint32_t>();
+  u.leaf_at = s->leaf_at.as<int32_t>();
+  u.irregular = s->irregular.as<int32_t>();
+  u.n_objects = (int32_t)s->nt;
+  return u;
+}
+
+// The level lists, leaf list, leaf starts and wide nodes of the tree in `refs`, whose root
+// is an inner record, top down, one pass per even depth (the small depths at the top in one
+// launch). sizes: the expected inner records per depth, which set the grids. The first
+// batch of passes covers the expected depth with two levels to spare; a tree that turns out
+// deeper gets more passes after the counters are read back. MH_UPDATE_FRONTIER_LEVELS (1 or
+// more) sets the first batch's size instead, so that tests can reach the later batches.
+// Copies `extra` (two words) back along with the counters; synchronises the stream.
+// MH_OK, MH_E_UNSUPPORTED (deeper than the lists hold) or MH_E_STATE (not a binary tree).
+int wide_pass(mh_scene* s, const std::vector<mh::LevelList>& sizes, bool fixed_irregular,
+              const unsigned* extra, unsigned extra_out[2], hipStream_t st) {
+  const mh::DevUpdate u = tree_view(s);
+  mh::DevFrontier f{};
+  f.fr = s->hist.as<unsigned>();
+  f.even = s->levels.as<int32_t>();
+  f.odd = f.even + s->list_cap;
+  f.aux = s->levels_aux.as<int2>();
+  f.leaves = s->leaves.as<int32_t>();
+  f.wide = s->wide.as<mh::WideNode>();
+  f.irregular = s->irregular.as<int32_t>();
+  f.fixed = fixed_irregular;
+  f.cap = (unsigned)s->list_cap;
+  f.cap_wide = (unsigned)(s->wide.bytes / sizeof(mh::WideNode));
+  unsigned* hc = s->host_ctr;
+  const int n_sizes = (int)sizes.size();
+  constexpr int kEnd = mh::kMaxDepth;  // passes run at even depths below it
+  int d_end = n_sizes + 2;
+  if (const char* e = std::getenv("MH_UPDATE_FRONTIER_LEVELS"))
+    if (const int v = std::atoi(e); v >= 1) d_end = v;
+  d_end = std::min((d_end + 1) & ~1, kEnd);
+  mh::TopLevels t;
+  const int top = mh::top_levels(sizes.data(), n_sizes, 2, t);
+  int d = std::max(2, std::min({2 * top, d_end, mh::kTopLevels}));
+  HIP_OK((hipError_t)mh::launch_wide_top(u, f, d, st));
+  for (;;) {
+    for (; d < d_end; d += 2) {
+      // workgroups for the expected size (a grid-stride loop covers any other)
+      const int64_t n = d < n_sizes ? sizes[d].n : 256;
+      const unsigned blocks = (unsigned)std::min<int64_t>(2048, (n + n / 4 + 255) / 256);
+      HIP_OK((hipError_t)mh::launch_wide_level(u, f, d, blocks, st));
+    }
+    HIP_OK(hipMemcpyAsync(hc, f.fr, mh::kFrontierWords * 4, hipMemcpyDeviceToHost, st));
+    if (extra)
+      HIP_OK(hipMemcpyAsync(hc + mh::kFrontierWords, extra, 8, hipMemcpyDeviceToHost, st));
+    HIP_OK(hipStreamSynchronize(st));
+    if (hc[d_end] == 0 || d_end >= kEnd) break;
+    d_end = std::min(d_end + 16, kEnd);
+  }
+  if (extra) {
+    extra_out[0] = hc[mh::kFrontierWords];
+    extra_out[1] = hc[mh::kFrontierWords + 1];
+  }
+  unsigned deepest = 0;
+  while ((int)deepest < d_end && hc[deepest]) ++deepest;
+  if (hc[d_end] || deepest >= (unsigned)mh::kMaxDepth - 1)
+    return fail(MH_E_UNSUPPORTED, "tree deeper than %d levels", mh::kMaxDepth - 1);
+  s->lev.clear();
+  int64_t at[2] = {0, (int64_t)s->list_cap};
+  uint64_t n_inner = 0;
+  for (unsigned k = 0; k < deepest; ++k) {
+    s->lev.push_back(mh::LevelList{at[k & 1], (int64_t)hc[k]});
+    at[k & 1] += hc[k];
+    n_inner += hc[k];
+  }
+  const uint64_t n_leaves = hc[mh::kFrLeaves];
+  if (hc[mh::kFrOver] || n_leaves != n_inner + 1 || n_leaves > s->list_cap)
+    return fail(MH_E_STATE, "the records are not a binary tree (%llu inner, %llu leaves)",
+                (unsigned long long)n_inner, (unsigned long long)n_leaves);
+  s->n_inner = (uint32_t)n_inner;
+  s->n_leaves = (uint32_t)n_leaves;
+  s->depth = deepest;
+  return MH_OK;
+}
+
+// The state of a tree whose root is a leaf: no levels, one leaf at slot 0.
+int leaf_root(mh_scene* s, hipStream_t st) {
+  const int32_t zero[2] = {0, 0};
+  HIP_OK(hipMemcpyAsync(s->leaves.p, zero, 4, hipMemcpyHostToDevice, st));
+  HIP_OK(hipMemcpyAsync(s->irregular.p, zero, 8, hipMemcpyHostToDevice, st));
+  HIP_OK(hipStreamSynchronize(st));
+  s->lev.clear();
+  s->n_inner = 0;
+  s->n_leaves = 1;
+  s->depth = 0;
+  return MH_OK;
+}
+
+// Lays the reference tree out for the device: checks it, uploads its records and rotation
+// state, then has the device make the lists and wide nodes. With rtsah, isLeftCheaper is
+// recomputed once the records are known to form a tree (DynBVH::buildFromFile runs
+// computeTraversalCost after reading, DynBVH.cc:2469-2472).
 int upload(mh_scene* s, bool rtsah = false) {
   std::vector<mh::RefNode>& nodes = s->bvh.nodes;
   const uint32_t nrec = (uint32_t)nodes.size();
   const uint32_t T = s->nt;
   std::vector<int32_t> leaves;
-  std::vector<std::vector<int32_t>> by_depth;  // inner records per depth, preorder
-  std::vector<int32_t> big(T, 0);
+  std::vector<mh::LevelList> sizes;  // inner records per depth
   struct It {
     int32_t rec;
     uint32_t depth;
   };
   std::vector<It> st;
   st.push_back({0, 0});
-  uint32_t max_depth = 0, n_inner = 0, max_rec = 0, n_reached = 0;
+  uint32_t n_inner = 0, max_rec = 0, n_reached = 0;
   uint64_t leaf_objects = 0;
+  bool nested = true;  // every box holds its children's
   std::vector<uint8_t> seen(nrec, 0);
   while (!st.empty()) {
     It it = st.back();
@@ -151,7 +283,6 @@ int upload(mh_scene* s, bool rtsah = false) {
     if (seen[it.rec]) return fail(MH_E_INVALID, "record %d is reached twice: not a tree", it.rec);
     seen[it.rec] = 1;
     ++n_reached;
-    max_depth = std::max(max_depth, it.depth);
     max_rec = std::max(max_rec, (uint32_t)it.rec);
     if (n.leaf()) {
       if (n.children < 0) return fail(MH_E_INVALID, "record %d: negative leaf size", it.rec);
@@ -159,7 +290,6 @@ int upload(mh_scene* s, bool rtsah = false) {
         return fail(MH_E_INVALID, "record %d: leaf range outside object_ids", it.rec);
       leaves.push_back(it.rec);
       leaf_objects += (uint32_t)n.children;
-      if (n.children >= mh::kLeafCountInline) big[n.child] = n.children;
       continue;
     }
     if (n.child < 1 || (uint32_t)n.child + 1 >= nrec)
@@ -171,45 +301,16 @@ int upload(mh_scene* s, bool rtsah = false) {
     if (++n_inner > nrec) return fail(MH_E_INVALID, "node graph is not a tree");
     if (it.depth >= (uint32_t)mh::kMaxDepth - 1)
       return fail(MH_E_UNSUPPORTED, "tree deeper than %d levels", mh::kMaxDepth - 1);
-    if (by_depth.size() <= it.depth) by_depth.resize(it.depth + 1);
-    by_depth[it.depth].push_back(it.rec);
+    if (sizes.size() <= it.depth) sizes.resize(it.depth + 1, mh::LevelList{0, 0});
+    ++sizes[it.depth].n;
+    for (int side = 0; side < 2; ++side) {
+      const mh::Aabb &b = n.box, &c = nodes[n.child + side].box;
+      for (int k = 0; k < 3; ++k) nested = nested && c.lo[k] >= b.lo[k] && c.hi[k] <= b.hi[k];
+    }
     st.push_back({n.child + 1, it.depth + 1});
     st.push_back({n.child, it.depth + 1});
   }
   if (rtsah) mh::compute_rtsah(nodes, 0);
-  auto encode = [&](int32_t rec) -> int32_t {
-    const mh::RefNode& n = nodes[rec];
-    if (!n.leaf()) return (n.child - 1) >> 1;
-    const int c = std::min<int>(n.children, mh::kLeafCountInline);
-    return ~((n.child << mh::kLeafCountBits) | c);
-  };
-  const size_t n_pairs = std::max<size_t>(1, nrec / 2);
-  std::vector<mh::PairNode> pairs(n_pairs);
-  for (const auto& lv : by_depth)
-    for (int32_t r : lv) {
-      const mh::RefNode& n = nodes[r];
-      mh::PairNode& P = pairs[(n.child - 1) >> 1];
-      for (int side = 0; side < 2; ++side) {
-        const mh::RefNode& c = nodes[n.child + side];
-        float* b = P.b + 6 * side;
-        b[0] = c.box.lo[0];
-        b[1] = c.box.hi[0];
-        b[2] = c.box.lo[1];
-        b[3] = c.box.hi[1];
-        b[4] = c.box.lo[2];
-        b[5] = c.box.hi[2];
-        P.ref[side] = encode(n.child + side);
-      }
-      P.meta = (int32_t)(n.axis & 3) | ((n.bits & 1) << 2);
-      P.node = r;
-    }
-  s->root_ref = encode(0);
-  s->n_inner = n_inner;
-  s->n_leaves = (uint32_t)leaves.size();
-  s->leaf_at_valid = false;
-  s->depth = max_depth;
-  s->next_free = max_rec + 1;
-  s->n_records = nrec;
   // Leaf ranges lie inside [0, T); they partition it iff their sizes sum to T and no slot
   // is covered twice.
   bool partition = leaf_objects == T;
@@ -219,44 +320,35 @@ int upload(mh_scene* s, bool rtsah = false) {
       for (int k = 0; k < nodes[r].children && partition; ++k)
         partition = !cover[nodes[r].child + k]++;
   }
-  s->updatable = partition && n_reached == max_rec + 1;
-  std::vector<int32_t> levels;
-  s->level_off.assign(1, 0);
-  for (auto& v : by_depth) {
-    levels.insert(levels.end(), v.begin(), v.end());
-    s->level_off.push_back((int64_t)levels.size());
-  }
   std::vector<float> costs;
   std::vector<uint32_t> ssize;
   rotation_state(nodes, costs, ssize);
 
   int rc;
-  if ((rc = s->refs.reserve(nrec * sizeof(mh::RefNode)))) return rc;
-  if ((rc = s->pairs.reserve(n_pairs * sizeof(mh::PairNode)))) return rc;
-  if ((rc = s->tris.reserve((size_t)T * 12 * sizeof(float)))) return rc;
-  if ((rc = s->ids.reserve((size_t)T * sizeof(int32_t)))) return rc;
-  if ((rc = s->big.reserve((size_t)T * sizeof(int32_t)))) return rc;
-  // Leaf and level lists: room for T entries, which the rotating update needs (a
-  // partition of T objects has at most T leaves and T - 1 inner records), and for every
-  // record of a loaded tree whose leaves overlap (it can hold more leaves than objects).
-  const size_t list_cap = std::max<size_t>({(size_t)std::max(1u, T), leaves.size(), levels.size()});
-  if ((rc = s->leaves.reserve(list_cap * sizeof(int32_t)))) return rc;
-  if ((rc = s->levels.reserve(list_cap * sizeof(int32_t)))) return rc;
-  if ((rc = s->costs.reserve(nrec * sizeof(float)))) return rc;
-  if ((rc = s->ssize.reserve(nrec * sizeof(uint32_t)))) return rc;
+  if ((rc = reserve_tree(s, nrec, n_inner, leaves.size()))) return rc;
+  s->partition = partition;
+  s->updatable = partition && n_reached == max_rec + 1;
+  s->next_free = max_rec + 1;
+  s->n_records = nrec;
+  ++s->tree_gen;
   HIP_OK(hipMemcpy(s->refs.p, nodes.data(), nrec * sizeof(mh::RefNode), hipMemcpyHostToDevice));
-  ++s->pairs_gen;
-  HIP_OK(hipMemcpy(s->pairs.p, pairs.data(), n_pairs * sizeof(mh::PairNode),
-                   hipMemcpyHostToDevice));
   HIP_OK(hipMemcpy(s->ids.p, s->bvh.ids.data(), (size_t)T * 4, hipMemcpyHostToDevice));
-  HIP_OK(hipMemcpy(s->big.p, big.data(), (size_t)T * 4, hipMemcpyHostToDevice));
-  if (!leaves.empty())
-    HIP_OK(hipMemcpy(s->leaves.p, leaves.data(), leaves.size() * 4, hipMemcpyHostToDevice));
-  if (!levels.empty())
-    HIP_OK(hipMemcpy(s->levels.p, levels.data(), levels.size() * 4, hipMemcpyHostToDevice));
   HIP_OK(hipMemcpy(s->costs.p, costs.data(), nrec * sizeof(float), hipMemcpyHostToDevice));
   HIP_OK(hipMemcpy(s->ssize.p, ssize.data(), nrec * sizeof(uint32_t), hipMemcpyHostToDevice));
-
+  HIP_OK(hipMemset(s->leaf_at.p, 0xFF, (size_t)T * 4));
+  HIP_OK(hipMemset(s->irregular.p, 0, 8));
+  if (n_inner > 0) {
+    if ((rc = wide_pass(s, sizes, !partition || !nested, nullptr, nullptr, nullptr))) return rc;
+    s->root_ref = 0;
+  } else {
+    const mh::RefNode& n = nodes[0];
+    if ((rc = leaf_root(s, nullptr))) return rc;
+    const int32_t zero = 0, count = n.children;
+    HIP_OK(hipMemcpy(s->leaf_at.as<int32_t>() + n.child, &zero, 4, hipMemcpyHostToDevice));
+    HIP_OK(hipMemcpy(s->big.as<int32_t>() + n.child, &count, 4, hipMemcpyHostToDevice));
+    s->root_ref = ~((n.child << mh::kLeafCountBits) |
+                    std::min<int>(n.children, mh::kLeafCountInline));
+  }
   mh::DevRefit r{};
   r.tris = s->tris.as<float>();
   r.obj_ids = s->ids.as<int32_t>();
@@ -284,6 +376,23 @@ int validate_ids(const std::vector<int32_t>& ids, uint32_t T) {
 
 mh::DevScene dev_scene(const mh_scene* s) { return s->dev(); }
 
+// mh_trace. The wide kernel gets a wave of its own for every 64 rays, up to kTraceBlocksPerCu
+// times four waves per compute unit (the spill area has a column per lane), and takes them
+// by a static stride from the end of the set: the hardware then starts waves as others end.
+// 2M camera rays of the 1M-triangle heightfield: 161 us; 202 with half as many waves, 267
+// with the resident ones alone (a wave's share of the rays fixed up front), 504 with those
+// and a ray counter (its atomics come from all XCDs, about 15 ns each). From the end, since a
+// camera image's rays come bottom row first and the long ones, along the ground to the
+// horizon, would start late: 256 us in the other order.
+constexpr int kTraceBlocksPerCu = 32;
+// Sets too small to give every SIMD a wave are cut into waves of fewer rays, which wait for
+// fewer others: 4,096 rays in a 10,000-triangle soup 98 us at 64 rays a wave, 67 at 4.
+constexpr int64_t kMinWaveRays = 4;
+// Ring entries unless the caller says: 16 (five waves per SIMD fill the LDS) spill less than
+// 8 (786,432 camera and bounce rays in a 200,000-triangle soup 1274 against 1337 us).
+constexpr int kWideRing = 16;
+
+// The caller's ring, or the one the reference records' kernel takes.
 int choose_stack(const mh_trace_opts* o) {
   const int v = o ? o->stack_lds : 0;
   return (v == 8 || v == 16 || v == 32) ? v : 8;
@@ -319,27 +428,52 @@ int trace_impl(const mh_scene* cs, const mh_rays* rays, const mh_hits* hits, int
       return fail(MH_E_UNSUPPORTED, "tree depth %u exceeds the packet stack (126)", s->depth);
   } else {
     const int S = choose_stack(opts);
-    const int bpc = (opts && opts->blocks_per_cu > 0) ? opts->blocks_per_cu : 16;
-    const int64_t want = (n + 255) / 256;
-    const int64_t cap = (int64_t)g_lib.cu_count * bpc;
-    cfg.blocks = (int)std::max<int64_t>(1, std::min(want, cap));
-    cfg.stack_lds = S;
-    cfg.spill_stride = (int64_t)cfg.blocks * 256;
-    const int64_t need = std::max<int64_t>(0, (int64_t)s->stack_bound(MH_LAYOUT_PAIR) - S);
-    if (need > 0 && fixed_spill) {
+    const int wide_S = opts && opts->stack_lds == S ? S : kWideRing;
+    const int bpc = (opts && opts->blocks_per_cu > 0) ? opts->blocks_per_cu : kTraceBlocksPerCu;
+    const int64_t cus = g_lib.cu_count;
+    // The reference records' kernel: its stack is shorter, and the counters are kept there.
+    const int64_t ref_need = std::max<int64_t>(0, (int64_t)s->stack_bound(MH_LAYOUT_REF) - S);
+    const int64_t ref_want = (n + 255) / 256;
+    int64_t ref_blocks = std::min(ref_want, cus * 16);
+    if (ref_need > 0 && fixed_spill) {
       // Fewer workgroups (the kernel strides over the rays, results are unchanged) until
       // every lane's spill column fits the area; at least one workgroup per compute unit.
-      const int64_t per_block = need * 256 * 8;
+      const int64_t per_block = ref_need * 256 * 8;
       const int64_t fit = (int64_t)(fixed_bytes / (size_t)per_block);
-      const int64_t floor_blocks = std::min<int64_t>(want, g_lib.cu_count);
+      const int64_t floor_blocks = std::min<int64_t>(ref_want, cus);
       if (fit < floor_blocks)
         return fail(MH_E_UNSUPPORTED,
                     "tree depth %u needs %lld bytes of stack spill for %lld workgroups; the "
                     "fixed area holds %zu (use mh_trace, or a larger stack_lds)",
                     s->depth, (long long)(per_block * floor_blocks), (long long)floor_blocks,
                     fixed_bytes);
-      cfg.blocks = (int)std::min<int64_t>(cfg.blocks, fit);
-      cfg.spill_stride = (int64_t)cfg.blocks * 256;
+      ref_blocks = std::min(ref_blocks, fit);
+    }
+    const int64_t chunk =
+        std::min<int64_t>(64, std::max<int64_t>(kMinWaveRays, (n + 4 * cus - 1) / (4 * cus)));
+    const int64_t waves = (n + chunk - 1) / chunk;
+    int64_t blocks = std::min(waves, 4 * cus * bpc);
+    int64_t need = std::max<int64_t>(0, (int64_t)s->stack_bound(MH_LAYOUT_PAIR) - wide_S);
+    bool wide = !cfg.counters;
+    if (fixed_spill && need > 0) {  // the wide nodes' longer stack may not fit where a ref's does
+      const int64_t fit = (int64_t)(fixed_bytes / (size_t)(need * 64 * 8));
+      wide = wide && fit >= std::min(waves, 4 * cus);
+      blocks = std::min(blocks, fit);
+    }
+    if (wide) {
+      cfg.layout = MH_LAYOUT_PAIR;
+      cfg.stack_lds = wide_S;
+      cfg.chunk = (int)chunk;
+      cfg.blocks = (int)blocks;
+      cfg.spill_stride = blocks * 64;
+    } else {
+      need = ref_need;
+      cfg.layout = MH_LAYOUT_REF;
+      cfg.stack_lds = S;
+      cfg.blocks = (int)ref_blocks;
+      cfg.spill_stride = ref_blocks * 256;
+    }
+    if (need > 0 && fixed_spill) {
       cfg.spill = reinterpret_cast<int32_t*>(fixed_spill);
     } else if (need > 0) {
       std::lock_guard<std::mutex> lk(s->spill_mu);
@@ -360,19 +494,25 @@ int trace_impl(const mh_scene* cs, const mh_rays* rays, const mh_hits* hits, int
 }  // namespace
 
 int mh_internal::ensure_soa(mh_scene* s, void* stream) {
-  const size_t n = s->pairs.bytes / sizeof(mh::PairNode);
+  const size_t n = s->n_records / 2;
   if (n == 0) return fail(MH_E_STATE, "scene has no pair records");
-  if (s->pairs_soa.bytes < n * sizeof(mh::PairNode)) {
-    if (int rc = s->pairs_soa.reserve(n * sizeof(mh::PairNode))) return rc;
+  int rc;
+  if ((rc = s->pairs.reserve(n * sizeof(mh::PairNode)))) return rc;
+  if (s->pairs_soa.bytes != n * sizeof(mh::PairNode)) {
+    s->pairs_soa.release();
+    if ((rc = s->pairs_soa.reserve(n * sizeof(mh::PairNode)))) return rc;
     s->soa_gen = ~0ull;
   }
-  if (s->soa_gen == s->pairs_gen) return MH_OK;
+  if (s->soa_gen == s->tree_gen) return MH_OK;
+  const mh::DevUpdate u = tree_view(s);
+  for (const mh::LevelList& l : s->lev)
+    HIP_OK((hipError_t)mh::launch_list_pairs(u, s->levels.as<int32_t>() + l.first, l.n, stream));
   // field k (16 bytes at offset 16k of every 64-byte pair) into array k
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   for (size_t k = 0; k < 4; ++k)
     HIP_OK(hipMemcpy2DAsync(s->pairs_soa.as<char>() + k * n * 16, 16, s->pairs.as<char>() + 16 * k,
                             sizeof(mh::PairNode), 16, n, hipMemcpyDeviceToDevice, st));
-  s->soa_gen = s->pairs_gen;
+  s->soa_gen = s->tree_gen;
   return MH_OK;
 }
 
@@ -466,16 +606,11 @@ int build_device(mh_scene* s, int rtsah) {
   const int64_t cap = (int64_t)T / (mh::kBuildSerial + 1) + 2;
   const int64_t vcap = (int64_t)T / mh::kBuildVB + cap + 2;
   int rc;
-  if ((rc = s->refs.reserve(nrec * sizeof(mh::RefNode))) ||
-      (rc = s->pairs.reserve(std::max<size_t>(1, nrec / 2) * sizeof(mh::PairNode))) ||
-      (rc = s->tris.reserve((size_t)T * 48)) || (rc = s->ids.reserve((size_t)T * 4)) ||
-      (rc = s->big.reserve((size_t)T * 4)) || (rc = s->leaves.reserve((size_t)T * 4)) ||
-      (rc = s->levels.reserve((size_t)T * 4)) || (rc = s->costs.reserve(nrec * 4)) ||
-      (rc = s->ssize.reserve(nrec * 4)) || (rc = s->parent.reserve(nrec * 4)) ||
+  if ((rc = reserve_tree(s, nrec, 0, 0)) || (rc = s->parent.reserve(nrec * 4)) ||
       (rc = s->obox.reserve((size_t)T * 24)) || (rc = s->ocen.reserve((size_t)T * 12)) ||
       (rc = s->anc0.reserve(nrec * 4)) || (rc = s->dep0.reserve(nrec * 4)) ||
       (rc = s->anc1.reserve(nrec * 4)) || (rc = s->dep1.reserve(nrec * 4)) ||
-      (rc = s->hist.reserve(mh::kDepthHist * 4)) || (rc = s->counters.reserve(16)))
+      (rc = s->hist.reserve(mh::kDepthHist * 4)))
     return rc;
   if (!s->logtab.p) {
     std::vector<float> tab(mh::rtsah::kLogTable);
@@ -611,19 +746,9 @@ int build_device(mh_scene* s, int rtsah) {
   f.large = (uint32_t)(nrec / (20 * (size_t)s->workers));
   f.rtsah = rtsah;
   const int n_levels = (int)level_off.size() - 1;
-  ++s->pairs_gen;
+  ++s->tree_gen;
   HIP_OK((hipError_t)mh::build_launch_ranks(f, level_off.data(), n_levels, n_leaves, st));
   HIP_OK(hipMemcpyAsync(cnt, &n_final, 4, hipMemcpyHostToDevice, st));
-  mh::DevUpdate u = d.u;
-  u.refs = s->refs.as<mh::RefNode>();
-  u.pairs = s->pairs.as<mh::PairNode>();
-  u.big_count = s->big.as<int32_t>();
-  HIP_OK((hipError_t)mh::launch_rebuild_pairs(u, st));
-  const bool root_leaf = n_final == 1;
-  if (root_leaf && T >= (uint32_t)mh::kLeafCountInline) {
-    const int32_t n = (int32_t)T;
-    HIP_OK(hipMemcpyAsync(s->big.p, &n, 4, hipMemcpyHostToDevice, st));
-  }
   mh::DevRefit r{};
   r.tris = s->tris.as<float>();
   r.obj_ids = s->ids.as<int32_t>();
@@ -632,17 +757,25 @@ int build_device(mh_scene* s, int rtsah) {
   r.n_slots = (int32_t)T;
   r.prim_kind = s->prim_kind;
   HIP_OK((hipError_t)mh::launch_prim_setup(r, st));
-  HIP_OK(hipStreamSynchronize(st));
-  s->root_ref = root_leaf ? ~(int)std::min<uint32_t>(T, mh::kLeafCountInline) : 0;
+  HIP_OK(hipMemsetAsync(s->leaf_at.p, 0xFF, (size_t)T * 4, st));
+  HIP_OK(hipMemsetAsync(s->irregular.p, 0, 8, st));
+  if (n_final > 1) {
+    std::vector<mh::LevelList> sizes;
+    for (int k = 0; k < n_levels; ++k)
+      sizes.push_back(mh::LevelList{0, level_off[k + 1] - level_off[k]});
+    if ((rc = wide_pass(s, sizes, false, nullptr, nullptr, st))) return rc;
+    s->root_ref = 0;
+  } else {
+    if ((rc = leaf_root(s, st))) return rc;
+    const int32_t zero = 0, n = (int32_t)T;
+    HIP_OK(hipMemcpy(s->leaf_at.p, &zero, 4, hipMemcpyHostToDevice));
+    HIP_OK(hipMemcpy(s->big.p, &n, 4, hipMemcpyHostToDevice));
+    s->root_ref = ~(int)std::min<uint32_t>(T, mh::kLeafCountInline);
+  }
   s->next_free = n_final;
   s->n_records = (uint32_t)nrec;
-  s->n_inner = (uint32_t)level_off.back();
-  s->leaf_at_valid = false;
-  s->n_leaves = (uint32_t)n_leaves;
-  s->depth = deepest;
-  s->level_off = std::move(level_off);
   s->bvh = mh::DynBvh();
-  s->updatable = true;
+  s->partition = s->updatable = true;
   s->built = true;
   return MH_OK;
 }
@@ -886,7 +1019,9 @@ int mh_scene_refit(mh_scene* s, void* stream) {
   if (rc) return rc;
   mh::DevRefit r{};
   r.refs = s->refs.as<mh::RefNode>();
-  r.pairs = s->pairs.as<mh::PairNode>();
+  r.wide = s->wide.as<mh::WideNode>();
+  r.leaf_at = s->partition ? s->leaf_at.as<int32_t>() : nullptr;
+  r.irregular = s->irregular.as<int32_t>();
   r.tris = s->tris.as<float>();
   r.obj_ids = s->ids.as<int32_t>();
   r.verts = s->d_verts.as<float>();
@@ -896,9 +1031,8 @@ int mh_scene_refit(mh_scene* s, void* stream) {
   r.n_leaves = (int32_t)s->n_leaves;
   r.n_slots = (int32_t)s->nt;
   r.prim_kind = s->prim_kind;
-  ++s->pairs_gen;
-  HIP_OK((hipError_t)mh::launch_refit(r, s->level_off.data(), (int)s->level_off.size() - 1,
-                                      stream));
+  ++s->tree_gen;
+  HIP_OK((hipError_t)mh::launch_refit(r, s->lev.data(), (int)s->lev.size(), stream));
   return MH_OK;
 }
 
@@ -914,54 +1048,25 @@ int mh_scene_update(mh_scene* s, void* stream) {
   const uint32_t T = s->nt;
   const size_t nrec = s->refs.bytes / sizeof(mh::RefNode);
   // Work arrays, allocated at the first update.
-  if ((rc = s->parent.reserve(nrec * 4)) || (rc = s->hist.reserve(mh::kFrontierWords * 4)) ||
-      (rc = s->counters.reserve(16)) ||
-      (rc = s->split_list.reserve((size_t)std::max<uint32_t>(1u, T) * 4)) ||
-      (rc = s->levels_aux.reserve((size_t)std::max<uint32_t>(1u, T) * 8)) ||
-      (rc = s->leaf_at.reserve((size_t)std::max<uint32_t>(1u, T) * 4)))
+  if ((rc = s->parent.reserve(nrec * 4)) ||
+      (rc = s->split_list.reserve((size_t)std::max<uint32_t>(1u, T) * 4)))
     return rc;
-  if (!s->host_ctr) {
-    void* h = nullptr;
-    if (hipHostMalloc(&h, (mh::kFrontierWords + 2) * 4, hipHostMallocDefault) != hipSuccess)
-      return fail(MH_E_NOMEM, "hipHostMalloc of the update's counter copy");
-    s->host_ctr = static_cast<unsigned*>(h);
-  }
   unsigned* nfree = s->counters.as<unsigned>();
-  int* err = reinterpret_cast<int*>(nfree + 1);
   const unsigned init[3] = {s->next_free, 0u, 0u};  // next_free, err, split list entries
   HIP_OK(hipMemcpyAsync(nfree, init, sizeof(init), hipMemcpyHostToDevice, st));
-  mh::DevUpdate u{};
-  u.refs = s->refs.as<mh::RefNode>();
-  u.pairs = s->pairs.as<mh::PairNode>();
-  u.big_count = s->big.as<int32_t>();
-  u.costs = s->costs.as<float>();
-  u.ssize = s->ssize.as<uint32_t>();
-  u.parent = s->parent.as<int32_t>();
-  u.ids = s->ids.as<int32_t>();
-  u.obox = nullptr;  // object boxes and centroids from the vertices, where they are needed
-  u.ocen = nullptr;
-  u.verts = s->d_verts.as<float>();
-  u.idx = s->d_idx.as<uint32_t>();
+  mh::DevUpdate u = tree_view(s);  // (object boxes are formed from the vertices)
   u.next_free = nfree;
-  u.err = err;
+  u.err = reinterpret_cast<int*>(nfree + 1);
   u.split_list = s->split_list.as<int32_t>();
   u.split_count = nfree + 2;
-  u.leaf_at = s->leaf_at.as<int32_t>();
   u.n_records = (int32_t)nrec;
-  u.n_objects = (int32_t)T;
   // largeSubtreeSize = nodes.size() / (20 * numProcs) (DynBVH.cc:1776)
   u.large = (uint32_t)(nrec / (20 * (size_t)s->workers));
-  ++s->pairs_gen;
-  if (!s->leaf_at_valid) {  // after a build or load: the leaf starting at each slot
-    HIP_OK(hipMemsetAsync(s->leaf_at.p, 0xFF, (size_t)std::max<uint32_t>(1u, T) * 4, st));
-    HIP_OK((hipError_t)mh::launch_leaf_starts(u, s->leaves.as<int32_t>(), s->n_leaves, st));
-    s->leaf_at_valid = true;  // the level pass below keeps it for the next frame
-  }
+  ++s->tree_gen;
   // leaf pass (triangle records and leaf boxes from the current vertices), leaf splits,
   // rotations depth by depth
   HIP_OK((hipError_t)mh::launch_update_tree(u, s->n_leaves, s->levels.as<int32_t>(),
-                                            s->level_off.data(),
-                                            (int)s->level_off.size() - 1, st));
+                                            s->lev.data(), (int)s->lev.size(), st));
   mh::DevRefit r{};  // triangle records in slot order from the current vertices
   r.tris = s->tris.as<float>();
   r.obj_ids = s->ids.as<int32_t>();
@@ -970,79 +1075,28 @@ int mh_scene_update(mh_scene* s, void* stream) {
   r.n_slots = (int32_t)T;
   r.prim_kind = s->prim_kind;
   HIP_OK((hipError_t)mh::launch_prim_setup(r, st));
-  // Level lists, leaf list and PairNodes of the new topology, top down, one pass per depth
-  // (the small depths at the top in one launch). The first batch of passes covers the
-  // previous depth with two levels to spare; a tree
-  // that grew deeper than that gets more passes after the counters are read back.
-  // MH_UPDATE_FRONTIER_LEVELS (1 or more) sets the first batch's size instead, so that
-  // tests can reach the later batches.
-  const int prev_levels = (int)s->level_off.size() - 1;
-  const unsigned cap = (unsigned)std::max<uint32_t>(1u, T);
-  unsigned* fr = s->hist.as<unsigned>();
-  unsigned* hc = s->host_ctr;
-  const bool inner_root = s->n_inner > 0;  // rotations never turn a leaf root inner
-  int d = 0, d_end = 0;
-  if (inner_root) {
-    d_end = std::min(prev_levels + 2, mh::kMaxDepth - 1);
-    if (const char* e = std::getenv("MH_UPDATE_FRONTIER_LEVELS")) {
-      const int v = std::atoi(e);
-      if (v >= 1) d_end = std::min(v, mh::kMaxDepth - 1);
-    }
-    // the depths that were small in the previous frame run in one workgroup
-    mh::TopLevels t;
-    const int n_top = std::max(1, std::min(mh::top_levels(s->level_off.data(), prev_levels, t),
-                                           d_end));
-    HIP_OK((hipError_t)mh::launch_frontier_top(u, fr, s->levels.as<int32_t>(),
-                                               s->levels_aux.as<int2>(),
-                                               s->leaves.as<int32_t>(), cap, n_top, st));
-    d = n_top;
-  }
-  for (;;) {
-    for (; d < d_end; ++d) {
-      // workgroups for the depth's size in the previous frame (a grid-stride loop covers
-      // any other size)
-      const int64_t prev = d < prev_levels ? s->level_off[d + 1] - s->level_off[d] : 256;
-      const unsigned blocks = (unsigned)std::min<int64_t>(2048, (prev + prev / 4 + 255) / 256);
-      HIP_OK((hipError_t)mh::launch_frontier(u, fr, s->levels.as<int32_t>(),
-                                             s->levels_aux.as<int2>(),
-                                             s->leaves.as<int32_t>(), cap, d, blocks, st));
-    }
-    if (inner_root)
-      HIP_OK(hipMemcpyAsync(hc, fr, mh::kFrontierWords * 4, hipMemcpyDeviceToHost, st));
-    HIP_OK(hipMemcpyAsync(hc + mh::kFrontierWords, nfree, 8, hipMemcpyDeviceToHost, st));
+  // Lists and wide nodes of the new topology.
+  unsigned now[2] = {0, 0};  // records in use, error
+  rc = MH_OK;
+  if (s->n_inner > 0) {  // rotations never turn a leaf root inner
+    const std::vector<mh::LevelList> sizes = s->lev;
+    rc = wide_pass(s, sizes, false, nfree, now, st);
+  } else {
+    HIP_OK(hipMemcpyAsync(s->host_ctr, nfree, 8, hipMemcpyDeviceToHost, st));
     HIP_OK(hipStreamSynchronize(st));
-    if (!inner_root || hc[d_end] == 0 || d_end >= mh::kMaxDepth - 1) break;
-    d_end = std::min(d_end + 16, mh::kMaxDepth - 1);
+    now[0] = s->host_ctr[0];
+    now[1] = s->host_ctr[1];
   }
   // Either failure leaves a device tree that must not be traced: the scene needs a build.
-  if (hc[mh::kFrontierWords + 1]) {
+  if (now[1]) {
     s->built = s->updatable = false;
     return fail(MH_E_STATE, "leaf splits ran out of node records; build the scene again");
   }
-  s->next_free = hc[mh::kFrontierWords];
-  if (!inner_root) {
-    s->n_leaves = 1;
-    return MH_OK;
-  }
-  unsigned deepest = 0;
-  while ((int)deepest < d_end && hc[deepest]) ++deepest;
-  if (hc[d_end] || deepest >= (unsigned)mh::kMaxDepth - 1) {
+  if (rc) {
     s->built = s->updatable = false;
-    return fail(MH_E_UNSUPPORTED, "tree deeper than %d levels after rotations; build the "
-                "scene again", mh::kMaxDepth - 1);
+    return rc;
   }
-  s->level_off.assign(1, 0);
-  for (unsigned k = 0; k < deepest; ++k) s->level_off.push_back(s->level_off.back() + hc[k]);
-  const uint64_t n_inner = (uint64_t)s->level_off.back(), n_leaves = hc[mh::kMaxDepth];
-  if (hc[mh::kMaxDepth + 1] || n_leaves != n_inner + 1 || n_leaves > cap) {
-    s->built = s->updatable = false;
-    return fail(MH_E_STATE, "the updated records are not a binary tree (%llu inner, %llu "
-                "leaves); build the scene again", (unsigned long long)n_inner,
-                (unsigned long long)n_leaves);
-  }
-  s->n_inner = (uint32_t)n_inner;
-  s->n_leaves = (uint32_t)n_leaves;
-  s->depth = deepest;
+  s->next_free = now[0];
   return MH_OK;
 }
 

@@ -2,19 +2,23 @@
 //
 // HBM layout of one scene (all arrays 256-byte aligned, one allocation each):
 //   refs      RefNode[2T]      reference DynBVH records, 32 B (packet traversal, refit)
-//   pairs     PairNode[T]      one 64-B record per pair of sibling records (2p+1, 2p+2):
-//                              both boxes, so one fetch decides both children of a node
-//                              (single-ray traversal). Sibling records are allocated in
-//                              pairs (nextFree += 2 from 1), so record r sits in pair
-//                              (r - 1) / 2 on side (r - 1) & 1, and a node whose children
-//                              are (c, c + 1) refers to pair (c - 1) / 2.
+//   wide      WideNode[]       one 128-B record per inner record of even depth, with the
+//                              boxes of its grandchildren (single-ray traversal); record k
+//                              belongs to entry k of the even level list
+//   pairs     PairNode[T]      made for MH_LAYOUT_SOA launches only: one 64-B record per
+//                              pair of sibling records (2p+1, 2p+2). Sibling records are
+//                              allocated in pairs (nextFree += 2 from 1), so record r sits
+//                              in pair (r - 1) / 2 on side (r - 1) & 1, and a node whose
+//                              children are (c, c + 1) refers to pair (c - 1) / 2.
 //   tris      float4[3T]       per object slot (object_ids order), 48 B:
 //                              Kensler-Shirley: p0, e0 = p1-p0, e1 = p0-p2, n = e0 x e1
 //                              Wald: n_u n_v n_d k | b_nu b_nv b_d n_k | c_nu c_nv c_d 0
 //   obj_ids   int32[T]         object_ids
 //   big_count int32[T]         leaf size at a leaf's first slot when it is >= 15
 //   verts     float[3V], idx uint32[3T], base_verts float[3V]    mesh (refit, animation)
-//   leaves int32[L], levels int32[I]   leaf records; inner records grouped by depth
+//   leaves int32[L], levels int32[I]   leaf records; inner records grouped by depth, the
+//                              even depths in one list and the odd depths in another
+//   leaf_at int32[T]           per object slot, the leaf record that starts there, else -1
 //   costs float[2T], ssize uint32[2T], parent int32[2T], obj boxes/centroids   rotating
 //                              update state (allocated at the first mh_scene_update)
 #pragma once
@@ -42,16 +46,37 @@ struct alignas(16) PairNode {
 };
 static_assert(sizeof(PairNode) == 64, "pair node is 64 bytes");
 
+// Inner record of even depth with the boxes two levels below it. Slots 0 and 1 are the left
+// child's children, 2 and 3 the right child's; a child that is a leaf takes its side's
+// first slot itself and leaves the other empty. An empty slot's box is inverted, so that no
+// ray meets it, and its reference is a leaf of no objects. One cache line: the node is
+// fetched whole, and a lane takes the near and the far row of each axis by its own offsets.
+struct alignas(128) WideNode {
+  float plane[6][4];  // lo.x, hi.x, lo.y, hi.y, lo.z, hi.z of the four boxes
+  int32_t ref[4];     // wide node (>= 0) or leaf code
+  // Visit order: bit 3 o + j for direction octant o (bit k set iff d[k] > 0), bit 24 + j for
+  // any-hit rays: the second of the pair is visited first, for the pair of children (j = 0),
+  // the left child's pair (1) and the right child's (2).
+  uint32_t order;
+  int32_t pad[3];
+};
+static_assert(sizeof(WideNode) == 128, "wide node is one cache line");
+constexpr int32_t kWideEmpty = -1;  // ~((0 << kLeafCountBits) | 0)
 
 struct DevScene {
-  const PairNode* pairs;
+  const WideNode* wide;
+  uint32_t n_wide;         // the bound of the wide table's descriptor
+  const int32_t* leaf_at;
+  // Nonzero: the tree's boxes do not nest or its leaves overlap (a loaded tree), or a vertex
+  // is not a number; every ray then takes the reference's own traversal.
+  const int32_t* irregular;
   const RefNode* refs;
   const float* tris;  // 12 floats per slot
   const int32_t* obj_ids;
   const int32_t* big_count;
   int32_t root_ref;   // pair-encoded reference of record 0
   int32_t prim_kind;  // 0 KS, 1 Wald
-  uint32_t n_pairs;   // PairNodes allocated (the bound of the pair table's descriptor)
+  uint32_t n_pairs;   // PairNodes of the SOA copy
   const void* pairs_soa;  // kLayoutSoa: 16-byte field k of pair p at [k * n_pairs + p], or null
   uint32_t n_slots;   // triangle records allocated (the bound of the triangle table's)
 };
@@ -69,17 +94,19 @@ struct DevHits {
 
 struct LaunchCfg {
   int any_hit;
-  int packet_size;    // 1 = single-ray kernel
+  int packet_size;    // 1 = single-ray kernels
   int stack_lds;      // 8/16/32 (single-ray)
-  int blocks;         // grid size in blocks of 256
-  int64_t* counters;  // device int64[2] or null
+  int layout;         // kLayoutPair or kLayoutRef (single-ray)
+  int blocks;         // grid size: blocks of 64 lanes (kLayoutPair) or 256 (kLayoutRef)
+  int64_t* counters;  // device int64[2] or null: box and triangle tests (kLayoutRef)
   int32_t* spill;     // per-thread stack spill (single-ray)
   int64_t spill_stride;
+  int chunk;          // kLayoutPair: rays a wave takes at a time, 1..64
 };
 
 // Node layouts of the single-ray traversal (MH_LAYOUT_*). A non-root record r's box is
 // also held by PairNode (r - 1) / 2, side (r - 1) & 1.
-constexpr int kLayoutPair = 0;  // 64-byte PairNodes, both child boxes per fetch
+constexpr int kLayoutPair = 0;  // 128-byte WideNodes, four boxes per fetch
 constexpr int kLayoutRef = 1;   // 32-byte reference records, own box tested at visit
 constexpr int kLayoutSoa = 2;   // the PairNodes as four arrays of their 16-byte fields
 
@@ -120,6 +147,7 @@ struct BatchLaunch {
   int chunk;      // rays per counter grab (multiple of 64); 0 = static stride, no counter
   int xcd_remap;  // contiguous ray shares per XCD
   int reverse;    // hand chunks out from the end of the table
+  int resident;   // waves of the wide kernel the device holds at once (kLayoutPair)
   int kinds;      // 0 mixed table, 1 closest-hit batches only, 2 any-hit batches only
 };
 
@@ -129,15 +157,24 @@ int launch_trace_batch(const DevScene& sc, const BatchLaunch& bl, void* stream);
 int launch_trace(const DevScene& sc, const DevRays& rays, const DevHits& hits, int64_t n,
                  const LaunchCfg& cfg, void* stream);
 
+// The inner records of one depth: entries [first, first + n) of the level lists. The lists
+// of the even depths lie one after the other from entry 0, those of the odd depths from
+// entry list_cap.
+struct LevelList {
+  int64_t first, n;
+};
+
 struct DevRefit {
   RefNode* refs;
-  PairNode* pairs;
+  WideNode* wide;
   float* tris;
   const int32_t* obj_ids;
   const float* verts;
   const uint32_t* idx;
-  const int32_t* leaves;  // leaf record ids
-  const int32_t* levels;  // inner record ids grouped by depth (level_off gives the groups)
+  const int32_t* leaves;   // leaf record ids
+  const int32_t* leaf_at;  // null: the leaves do not partition the slots, take the leaf list
+  const int32_t* levels;
+  int32_t* irregular;      // [0] DevScene::irregular, [1] set by a pass that met a NaN box
   int32_t n_leaves;
   int32_t n_slots;        // T
   int32_t prim_kind;
@@ -147,19 +184,20 @@ struct DevRefit {
 constexpr int kMaxDepth = 256;  // deepest tree the level lists hold
 
 // The top depths of a tree that one workgroup runs in one launch, with a barrier between
-// depths (refit and update): depths [0, n), each of at most kTopNodes records, depth d at
-// [off[d], off[d + 1]) of the level list.
+// depths (refit and update): depths [0, n), each of at most kTopNodes records.
 constexpr int kTopLevels = 32;
 constexpr int kTopNodes = 512;
 struct TopLevels {
-  int32_t off[kTopLevels + 1];
+  int32_t first[kTopLevels], cnt[kTopLevels];
   int32_t n;
 };
-// The top depths of level_off (n_levels + 1 host offsets) that fit: fills t, returns t.n.
-inline int top_levels(const int64_t* level_off, int n_levels, TopLevels& t) {
+// The top depths (every `step`-th one) that fit: fills t, returns t.n.
+inline int top_levels(const LevelList* lev, int n_levels, int step, TopLevels& t) {
   int n = 0;
-  while (n < n_levels && n < kTopLevels && level_off[n + 1] - level_off[n] <= kTopNodes) ++n;
-  for (int d = 0; d <= n; ++d) t.off[d] = (int32_t)level_off[d];
+  for (int d = 0; d < n_levels && n < kTopLevels && lev[d].n <= kTopNodes; d += step, ++n) {
+    t.first[n] = (int32_t)lev[d].first;
+    t.cnt[n] = (int32_t)lev[d].n;
+  }
   t.n = n;
   return n;
 }
@@ -180,7 +218,8 @@ struct DevUpdate {
   int* err;              // set when the record array is full
   int32_t* split_list;   // update: leaves whose parent's rotation may split them
   unsigned* split_count; // update: entries of split_list (cleared by the host)
-  int32_t* leaf_at;      // update: per slot, the leaf whose first slot it is, else -1
+  int32_t* leaf_at;      // per slot, the leaf whose first slot it is, else -1
+  int32_t* irregular;    // update: [1] is set by the leaf pass for a NaN box
   int32_t n_records;     // capacity, 2T
   int32_t n_objects;     // T
   uint32_t large;        // largeSubtreeSize
@@ -192,9 +231,9 @@ int launch_leaf_starts(const DevUpdate& u, const int32_t* leaves, int64_t n_leav
 // Leaf pass over the object slots (u.leaf_at), leaf splits, then one launch per depth
 // (deepest first).
 int launch_update_tree(const DevUpdate& u, int64_t n_leaves, const int32_t* levels,
-                       const int64_t* level_off, int n_levels, void* stream);
-// PairNodes and big leaf counts of every record pair in use, from the reference records.
-int launch_rebuild_pairs(const DevUpdate& u, void* stream);
+                       const LevelList* lev, int n_levels, void* stream);
+// The PairNodes of the n inner records of a level list.
+int launch_list_pairs(const DevUpdate& u, const int32_t* levels, int64_t n, void* stream);
 // Depth of every record in use by `steps` pointer-jumping steps (even, at most 8; 8 covers
 // any depth below kMaxDepth); hist[d] inner records at depth d, hist[kMaxDepth] leaves,
 // hist[kMaxDepth + 1] the deepest depth, hist[kMaxDepth + 2] nonzero when the steps did
@@ -204,24 +243,37 @@ int launch_depths(const DevUpdate& u, int32_t* anc0, int32_t* dep0, int32_t* anc
                   unsigned* hist, int steps, void* stream);
 int launch_depth_scatter(const DevUpdate& u, const int32_t* dep, unsigned* cursor,
                          int32_t* levels, int32_t* leaves, void* stream);
-// Level lists and PairNodes of an updated tree, top down from an inner root: counters fr
-// (kFrontierWords: inner records per depth, leaves at [kMaxDepth], an overflow flag at
-// [kMaxDepth + 1], list offsets from [kMaxDepth + 2]). launch_frontier_top clears them and
-// runs depths [0, n_top) (1 <= n_top <= kTopLevels) in one workgroup; launch_frontier(d)
-// then lists depth d + 1 (d < kMaxDepth - 1) and the leaf children of depth d, in
-// `blocks` workgroups. Each list holds at most cap entries; aux (cap entries) holds each
-// level entry's first child and record word for the next depth.
-constexpr int kFrontierWords = 2 * kMaxDepth + 3;
-int launch_frontier_top(const DevUpdate& u, unsigned* fr, int32_t* levels, int2* aux,
-                        int32_t* leaves, unsigned cap, int n_top, void* stream);
-int launch_frontier(const DevUpdate& u, unsigned* fr, int32_t* levels, int2* aux,
-                    int32_t* leaves, unsigned cap, int d, unsigned blocks, void* stream);
+// wide.hip: level lists, leaf list, leaf starts and wide nodes of a tree, top down from an
+// inner root. Counters fr: [d] inner records at depth d, [kFrLeaves] leaves, [kFrOver] set
+// when a list would pass its capacity, [kFrOff + d] where depth d starts in its list.
+// launch_wide_top clears them and runs the even depths below n_top in one workgroup;
+// launch_wide_level(d) then runs an even depth d in `blocks` workgroups: it writes the wide
+// nodes of depth d and lists depths d + 1 and d + 2 and the leaves met on the way.
+constexpr int kFrLeaves = kMaxDepth + 2;
+constexpr int kFrOver = kMaxDepth + 3;
+constexpr int kFrOff = kMaxDepth + 4;
+constexpr int kFrontierWords = kFrOff + kMaxDepth + 4;
+struct DevFrontier {
+  unsigned* fr;
+  int32_t* even;    // even level list (a wide node's index is its place here)
+  int32_t* odd;
+  int2* aux;        // beside each even entry, its record's first child and word
+  int32_t* leaves;
+  WideNode* wide;
+  int32_t* irregular;  // [0] is set from `fixed` and the NaN mark [1], which is cleared
+  int32_t fixed;
+  unsigned cap;        // entries each list holds
+  unsigned cap_wide;   // wide nodes
+};
+int launch_wide_top(const DevUpdate& u, const DevFrontier& f, int n_top, void* stream);
+int launch_wide_level(const DevUpdate& u, const DevFrontier& f, int d, unsigned blocks,
+                      void* stream);
 
 // refit.hip
 int launch_prim_setup(const DevRefit& r, void* stream);  // tris from verts (all slots)
-// tris + leaf boxes, then one launch per level of inner records from the deepest up;
-// level_off (host, n_levels + 1 entries) delimits each depth's records in r.levels.
-int launch_refit(const DevRefit& r, const int64_t* level_off, int n_levels, void* stream);
+// tris + leaf boxes, then one launch per even depth from the deepest up: the boxes of its
+// records and of their children, and its wide nodes.
+int launch_refit(const DevRefit& r, const LevelList* lev, int n_levels, void* stream);
 int launch_displace_sine(float* verts, const float* base, int64_t n_verts, float amp, float freq,
                          float phase, void* stream);
 

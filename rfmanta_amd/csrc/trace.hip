@@ -1,8 +1,9 @@
 // Traversal kernels for gfx950 (wave64).
 //
-// k_trace_ray: one ray per lane, DynBVH::intersect on a one-ray packet
-//   (Model/Groups/DynBVH.cc:101-404) over 64-byte PairNodes with an LDS ring stack; the
-//   traversal itself is traverse.h's, shared with the batch kernel.
+// Single rays take k_trace_wide (wide_trace.h). k_trace_ray: one ray per lane,
+//   DynBVH::intersect on a one-ray packet (Model/Groups/DynBVH.cc:101-404) over the
+//   reference's 32-byte records, for callers that count box and triangle tests and for trees
+//   too deep for the wide nodes' stack in a fixed spill area; the traversal is traverse.h's.
 //
 // k_trace_packet: one RayPacket of up to 64 consecutive rays per wave, the reference's
 //   packet recursion (intersectNode/firstIntersects/lastIntersects, DynBVH.cc:274-905,
@@ -24,6 +25,13 @@
 #include "traverse.h"
 
 namespace mh {
+
+// wide_ks.hip, wide_wald.hip
+int launch_wide_one_ks(const DevScene& sc, const BatchDev& rays, const LaunchCfg& cfg,
+                       hipStream_t s);
+int launch_wide_one_wald(const DevScene& sc, const BatchDev& rays, const LaunchCfg& cfg,
+                         hipStream_t s);
+
 namespace {
 
 constexpr int kBlock = 256;
@@ -31,10 +39,9 @@ constexpr int kWaves = kBlock / 64;
 constexpr int kPacketStack = 128;
 
 // ---------------------------------------------------------------------------
-// Single-ray traversal (traverse.h), grid-stride over the rays. Eight waves per SIMD (the
-// scalar registers otherwise limit it to seven): more node fetches in flight per SIMD.
+// Single-ray traversal of the reference's records (traverse.h), grid-stride over the rays.
 // ---------------------------------------------------------------------------
-template <bool ANY, int PRIM, int LAYOUT, int S, bool STATS>
+template <bool ANY, int PRIM, int S, bool STATS>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_trace_ray(
     DevScene sc, DevRays rays, DevHits hits, int64_t n, int2* spill, int64_t spill_stride,
     unsigned long long* counters) {
@@ -49,7 +56,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) 
   const GRays gr = global_view(rays);
   const GHits gh = global_view(hits);
   for (int64_t ri = gtid; ri < n; ri += stride)
-    trace_store<ANY, PRIM, LAYOUT, S, kBlock, STATS>(sc, root, gr, gh, ri, st, nbox, ntri);
+    trace_store<ANY, PRIM, kLayoutRef, S, kBlock, STATS>(sc, root, gr, gh, ri, st, nbox, ntri);
   if (STATS && counters) {
     atomicAdd(counters + 0, nbox);
     atomicAdd(counters + 1, ntri);
@@ -252,7 +259,7 @@ __global__ __launch_bounds__(kBlock) void k_trace_packet(DevScene sc, DevRays ra
   }
 }
 
-template <bool ANY, int PRIM, int LAYOUT, bool STATS>
+template <bool ANY, int PRIM, bool STATS>
 int launch_ray_s(const DevScene& sc, const DevRays& rays, const DevHits& hits, int64_t n,
                  const LaunchCfg& cfg, hipStream_t s) {
   unsigned long long* c = reinterpret_cast<unsigned long long*>(cfg.counters);
@@ -260,15 +267,15 @@ int launch_ray_s(const DevScene& sc, const DevRays& rays, const DevHits& hits, i
   dim3 g(cfg.blocks), b(kBlock);
   switch (cfg.stack_lds) {
     case 8:
-      hipLaunchKernelGGL((k_trace_ray<ANY, PRIM, LAYOUT, 8, STATS>), g, b, 0, s, sc, rays, hits, n, sp,
+      hipLaunchKernelGGL((k_trace_ray<ANY, PRIM, 8, STATS>), g, b, 0, s, sc, rays, hits, n, sp,
                          cfg.spill_stride, c);
       break;
     case 32:
-      hipLaunchKernelGGL((k_trace_ray<ANY, PRIM, LAYOUT, 32, STATS>), g, b, 0, s, sc, rays, hits, n, sp,
+      hipLaunchKernelGGL((k_trace_ray<ANY, PRIM, 32, STATS>), g, b, 0, s, sc, rays, hits, n, sp,
                          cfg.spill_stride, c);
       break;
     default:
-      hipLaunchKernelGGL((k_trace_ray<ANY, PRIM, LAYOUT, 16, STATS>), g, b, 0, s, sc, rays, hits, n, sp,
+      hipLaunchKernelGGL((k_trace_ray<ANY, PRIM, 16, STATS>), g, b, 0, s, sc, rays, hits, n, sp,
                          cfg.spill_stride, c);
       break;
   }
@@ -291,8 +298,8 @@ int launch_any_prim(const DevScene& sc, const DevRays& rays, const DevHits& hits
                          dim3(kBlock), 0, s, sc, rays, hits, n, cfg.packet_size, c);
     return (int)hipGetLastError();
   }
-  return stats ? launch_ray_s<ANY, PRIM, kLayoutPair, true>(sc, rays, hits, n, cfg, s)
-               : launch_ray_s<ANY, PRIM, kLayoutPair, false>(sc, rays, hits, n, cfg, s);
+  return stats ? launch_ray_s<ANY, PRIM, true>(sc, rays, hits, n, cfg, s)
+               : launch_ray_s<ANY, PRIM, false>(sc, rays, hits, n, cfg, s);
 }
 
 }  // namespace
@@ -300,6 +307,11 @@ int launch_any_prim(const DevScene& sc, const DevRays& rays, const DevHits& hits
 int launch_trace(const DevScene& sc, const DevRays& rays, const DevHits& hits, int64_t n,
                  const LaunchCfg& cfg, void* stream) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  if (cfg.packet_size <= 1 && cfg.layout == kLayoutPair) {
+    if (cfg.counters) return (int)hipErrorInvalidValue;
+    const BatchDev b{rays, hits, n, 0, cfg.any_hit ? 1u : 0u, 0};
+    return sc.prim_kind == 1 ? launch_wide_one_wald(sc, b, cfg, s) : launch_wide_one_ks(sc, b, cfg, s);
+  }
   if (cfg.any_hit) {
     return sc.prim_kind == 1 ? launch_any_prim<true, 1>(sc, rays, hits, n, cfg, s)
                              : launch_any_prim<true, 0>(sc, rays, hits, n, cfg, s);

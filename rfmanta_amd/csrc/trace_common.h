@@ -41,6 +41,12 @@ __device__ __forceinline__ float4 fetch_record(const MhBufRsrc& t, int index, in
   const MhBufF4 v = mh_struct_buffer_load_v4f32(t, index, offset, 0, 0);
   return make_float4(v.x, v.y, v.z, v.w);
 }
+// The same at a byte offset that differs from lane to lane.
+__device__ __forceinline__ float4 fetch_record_at(const MhBufRsrc& t, int index, int lane_offset,
+                                                  int offset) {
+  const MhBufF4 v = mh_struct_buffer_load_v4f32(t, index, lane_offset + offset, 0, 0);
+  return make_float4(v.x, v.y, v.z, v.w);
+}
 constexpr float kMaxT = 1.e19f;  // MAXT
 
 // Explicit address spaces. Pointers read from memory (batch tables) are otherwise

@@ -1,12 +1,13 @@
-// Single-ray traversal shared by the plain kernel (trace.hip) and the batch kernel
-// (batch.hip): DynBVH::intersect on a one-ray packet (Model/Groups/DynBVH.cc:101-404).
+// Single-ray traversal of the REF and SOA node layouts (the plain kernel's statistics
+// variant, trace.hip, and the batch kernel, batch_kernel.h): DynBVH::intersect on a one-ray
+// packet (Model/Groups/DynBVH.cc:101-404). The default layout's is wide_trace.h's.
 //
-// PAIR layout: inner nodes are 64-byte PairNodes holding both child boxes, so one fetch
-//   tests both children. The child the reference visits first (direction sign on the
-//   split axis for closest-hit, isLeftCheaper for any-hit, DynBVH.cc:386-398) is entered
-//   and the other is pushed with its entry distance; a popped entry is entered only if
-//   that distance is still <= minT, which is exactly the reference's later slab test of
-//   that child with the updated minT.
+// SOA layout: inner nodes are 64-byte PairNodes holding both child boxes, kept as four
+//   arrays of their 16-byte fields, so one fetch tests both children. The child the
+//   reference visits first (direction sign on the split axis for closest-hit,
+//   isLeftCheaper for any-hit, DynBVH.cc:386-398) is entered and the other is pushed with
+//   its entry distance; a popped entry is entered only if that distance is still <= minT,
+//   which is exactly the reference's later slab test of that child with the updated minT.
 // REF layout: the reference's 32-byte records; each node's own box is tested when it is
 //   visited, as firstIntersects does.
 // The stack is a per-lane ring of S entries in LDS ([slot][lane], conflict free) whose
@@ -87,49 +88,41 @@ __device__ __forceinline__ bool leaf(const DevScene& sc, int first, int cnt, con
   return false;
 }
 
-// The four 16-byte words of PairNode `cur`: one record of the pair table (kLayoutPair), or
-// one entry of each of the four field arrays (kLayoutSoa).
-template <int LAYOUT>
+// The four 16-byte words of PairNode `cur`, one entry of each of the four field arrays.
 __device__ __forceinline__ void fetch_pair(const DevScene& sc, int cur, float4& A, float4& B,
                                            float4& C, int4& M) {
-  float4 Mf;
-  if (LAYOUT == kLayoutSoa) {
-    const unsigned n = sc.n_pairs;
-    const MhBufRsrc t = record_table(sc.pairs_soa, 16, 4 * n);
-    A = fetch_record(t, cur, 0);
-    B = fetch_record(t, (int)(cur + n), 0);
-    C = fetch_record(t, (int)(cur + 2 * n), 0);
-    Mf = fetch_record(t, (int)(cur + 3 * n), 0);
-  } else {
-    const MhBufRsrc pt = record_table(sc.pairs, sizeof(PairNode), sc.n_pairs);
-    A = fetch_record(pt, cur, 0);
-    B = fetch_record(pt, cur, 16);
-    C = fetch_record(pt, cur, 32);
-    Mf = fetch_record(pt, cur, 48);
-  }
+  const unsigned n = sc.n_pairs;
+  const MhBufRsrc t = record_table(sc.pairs_soa, 16, 4 * n);
+  A = fetch_record(t, cur, 0);
+  B = fetch_record(t, (int)(cur + n), 0);
+  C = fetch_record(t, (int)(cur + 2 * n), 0);
+  const float4 Mf = fetch_record(t, (int)(cur + 3 * n), 0);
   M = make_int4(__float_as_int(Mf.x), __float_as_int(Mf.y), __float_as_int(Mf.z),
                 __float_as_int(Mf.w));
 }
 
-template <bool ANY, int PRIM, int S, int BLOCK, bool STATS, bool FAST, int LAYOUT = kLayoutPair>
+// PairNodes are numbered as their inner record's pair of children: the root's is pair 0.
+__device__ __forceinline__ int pair_root(const DevScene& sc) {
+  return sc.root_ref < 0 ? sc.root_ref : 0;
+}
+
+template <bool ANY, int PRIM, int S, int BLOCK, bool FAST>
 __device__ __forceinline__ void trace_pair(const DevScene& sc, const RefNode& root, const Ray& r,
-                                           RayHit& h, LaneStack<S, BLOCK>& st,
-                                           unsigned long long& nbox, unsigned long long& ntri) {
+                                           RayHit& h, LaneStack<S, BLOCK>& st) {
+  unsigned long long ntri = 0;
   float tn;
   bool go = slab_v<FAST>(root.box.lo[0], root.box.hi[0], root.box.lo[1], root.box.hi[1],
                          root.box.lo[2], root.box.hi[2], r, h.minT, tn);
-  if (STATS) ++nbox;
-  int cur = sc.root_ref;
+  int cur = pair_root(sc);
   st.reset();
   while (go) {
     if (cur >= 0) {
       float4 A, B, C;
       int4 M;
-      fetch_pair<LAYOUT>(sc, cur, A, B, C, M);
+      fetch_pair(sc, cur, A, B, C, M);
       float tn0, tn1;
       const bool h0 = slab_v<FAST>(A.x, A.y, A.z, A.w, B.x, B.y, r, h.minT, tn0);
       const bool h1 = slab_v<FAST>(B.z, B.w, C.x, C.y, C.z, C.w, r, h.minT, tn1);
-      if (STATS) nbox += 2;
       // Front child: isLeftCheaper (any-hit) or the direction's sign on the split axis.
       const bool one_first = ANY ? ((M.z >> 2) & 1) == 0 : __builtin_amdgcn_ubfe(r.dpos, M.z, 1) == 0;
       // Both hit: enter the front child, push the other. One hits: enter it. Written on
@@ -144,7 +137,7 @@ __device__ __forceinline__ void trace_pair(const DevScene& sc, const RefNode& ro
       const int first = code >> kLeafCountBits;
       int cnt = code & kLeafCountInline;
       if (cnt == kLeafCountInline) cnt = sc.big_count[first];
-      if (leaf<ANY, PRIM, STATS>(sc, first, cnt, r, h, ntri)) return;
+      if (leaf<ANY, PRIM, false>(sc, first, cnt, r, h, ntri)) return;
     }
     go = false;
     while (!st.empty()) {
@@ -160,21 +153,23 @@ __device__ __forceinline__ void trace_pair(const DevScene& sc, const RefNode& ro
   }
 }
 
+// The box tests are counted as the two of an inner record's children when it is entered.
 template <bool ANY, int PRIM, int S, int BLOCK, bool STATS, bool FAST>
 __device__ __forceinline__ void trace_ref(const DevScene& sc, const Ray& r, RayHit& h,
                                           LaneStack<S, BLOCK>& st, unsigned long long& nbox,
                                           unsigned long long& ntri) {
   int cur = 0;
   st.reset();
+  if (STATS) ++nbox;
   for (;;) {
     const RefNode nd = sc.refs[cur];
     float tn;
-    if (STATS) ++nbox;
     if (slab_v<FAST>(nd.box.lo[0], nd.box.hi[0], nd.box.lo[1], nd.box.hi[1], nd.box.lo[2],
                      nd.box.hi[2], r, h.minT, tn)) {
       if (nd.children != 0) {
         if (leaf<ANY, PRIM, STATS>(sc, nd.child, nd.children, r, h, ntri)) return;
       } else {
+        if (STATS) nbox += 2;
         const int front = ANY ? ((nd.bits & 1) ? 0 : 1) : (((r.dpos >> (nd.axis & 3)) & 1) ? 0 : 1);
         st.push(nd.child + 1 - front, 0.f);
         cur = nd.child + front;
@@ -206,12 +201,12 @@ __device__ __forceinline__ void trace_store(const DevScene& sc, const RefNode& r
     if (LAYOUT == kLayoutRef)
       trace_ref<ANY, PRIM, S, BLOCK, STATS, true>(sc, r, h, st, nbox, ntri);
     else
-      trace_pair<ANY, PRIM, S, BLOCK, STATS, true, LAYOUT>(sc, root, r, h, st, nbox, ntri);
+      trace_pair<ANY, PRIM, S, BLOCK, true>(sc, root, r, h, st);
   } else {
     if (LAYOUT == kLayoutRef)
       trace_ref<ANY, PRIM, S, BLOCK, STATS, false>(sc, r, h, st, nbox, ntri);
     else
-      trace_pair<ANY, PRIM, S, BLOCK, STATS, false, LAYOUT>(sc, root, r, h, st, nbox, ntri);
+      trace_pair<ANY, PRIM, S, BLOCK, false>(sc, root, r, h, st);
   }
   const bool hit = h.best >= 0;
   store_hit(hits, i, hit ? sc.obj_ids[h.best] : -1, (ANY && hit) ? kEps : h.minT, h.u, h.v, hit);

@@ -1,0 +1,547 @@
+// Single-ray traversal over the four-wide nodes for gfx950 (wave64): DynBVH::intersect on
+// one-ray packets (Model/Groups/DynBVH.cc:101-404), with the reference's results bit for
+// bit. Included by wide_ks.hip and wide_wald.hip, one per triangle test.
+//
+// What has to match. The reference visits the leaves in an order fixed by the split axes
+// and the direction's signs (isLeftCheaper for any hit, DynBVH.cc:386-398), and enters a
+// leaf if its slab test and those of the inner records above it pass with the minT of that
+// moment. Boxes nest and every step of the slab test is monotone, so a leaf whose own test
+// passes passes it all the way up: which leaves are entered depends on the leaf boxes
+// alone, and inner boxes may be tested with any arithmetic that never rejects what the
+// reference accepts. So here an inner test is one fused multiply-add a plane, widened by
+// more than all rounding errors (WideRay), two tree levels are tested at a time, and the
+// exact test of a leaf is run only where it matters: once a ray, for the leaf that holds its
+// hit. Should that test fail, which takes a hit within rounding of its leaf's box, the ray
+// is traced again by the reference's own steps (wide_redo). An accepted hit that a later
+// one replaces can be skipped if the later one clears it by more than the acceptance band
+// (anything the first kept out lies in that band or beyond, where the second rejects or
+// replaces it too); inside the band it is tested at once. Rays outside the bounds below and
+// trees whose boxes do not nest take wide_redo from the start.
+//
+// How the wave works. A node visit costs about 110 vector instructions and a triangle test
+// about 95, and each waits about 850 cycles for its record (L2 and MALL; a 10,000-triangle
+// tree as well). Every step the wave votes: node visits for the lanes at a node, or
+// triangle tests for the lanes at a leaf, whichever more lanes wait for; the others keep
+// their place. Walking every lane to its leaf before any triangle is tested (two loops, as
+// in batch_kernel.h) took 84 node visits and 21 tests a wave on a 10,000-triangle soup's
+// camera rays against 61 and 10 by vote, 147 and 59 against 100 and 44 at 200,000. Then one
+// stack entry is taken off for every lane that needs it: a loop until each lane has one that
+// is still in front of its hit cost more (up to three LDS round trips a step) than the
+// steps that the lanes with a culled entry sit out.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cfloat>
+
+#include "batch_kernel.h"
+#include "mh_device.h"
+#include "trace_common.h"
+#include "traverse.h"
+
+namespace mh {
+
+// A plane at p of axis k is met at p * inv[k] + c, with c = cn[k] for a near plane and cf[k]
+// for a far one.
+struct WideRay {
+  float inv[3], cn[3], cf[3];
+  int on[3], of[3];  // byte offsets of the near and the far row among an axis's two rows
+};
+
+// Sets w up for a ray; false if the bounds do not hold for it. reach is the largest
+// |coordinate| of the root box. With R = reach + max|o| every product below is at most
+// R |inv|; its roundings and those of the reference's (p - o) * inv come to at most six
+// times 2^-24 R |inv|, and c is moved outward by eight. A reciprocal is cut at 2^40 times
+// the smallest one (a direction component of zero has an infinite one): the cut plane
+// distances keep their signs, and the widening of such an axis alone, 2^19 R m, is beyond
+// any distance inside the root box, so a ray between the planes still passes. The bounds on
+// R m keep every product finite. A ray with an infinite minT and a zero component is left to
+// the reference's steps, which let infinite distances through there.
+__device__ __forceinline__ bool wide_setup(float reach, const Ray& r, float minT, WideRay& w) {
+  const float m = fminf(fminf(fabsf(r.inv[0]), fabsf(r.inv[1])), fabsf(r.inv[2]));
+  const float big = fmaxf(fmaxf(fabsf(r.inv[0]), fabsf(r.inv[1])), fabsf(r.inv[2]));
+  const float R = reach + fmaxf(fmaxf(fabsf(r.o[0]), fabsf(r.o[1])), fabsf(r.o[2]));
+  const float q = R * m, lim = m * 0x1p40f;
+  bool ok = q >= 0x1p-60f && q <= 0x1p60f && m >= 0x1p-60f && m <= 0x1p60f && !(minT != minT) &&
+            (minT <= FLT_MAX || big <= FLT_MAX);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    ok = ok && !(r.o[k] != r.o[k]) && !(r.d[k] != r.d[k]);
+    const float a = fminf(fabsf(r.inv[k]), lim);
+    w.inv[k] = __builtin_copysignf(a, r.inv[k]);
+    const float p = R * 0x1p-21f * a;
+    const float c = -(r.o[k] * w.inv[k]);
+    w.cn[k] = c - p;
+    w.cf[k] = c + p;
+    w.on[k] = w.inv[k] < 0.f ? 16 : 0;
+    w.of[k] = 16 - w.on[k];
+  }
+  return ok;
+}
+
+// A condition as the mask of the wave's lanes, and back: logic on masks is scalar work.
+__device__ __forceinline__ unsigned long long wave_mask(bool b) {
+  return __builtin_amdgcn_ballot_w64(b);
+}
+__device__ __forceinline__ bool lane_bit(unsigned long long m) {
+  return __builtin_amdgcn_inverse_ballot_w64(m);
+}
+
+constexpr int kIdle = (int)0x80000000;  // no ray
+constexpr int kPop = (int)0x80000001;   // takes its next node from the stack
+
+// One lane's ray.
+struct WideLane {
+  Ray r;  // inv is only live while the ray is set up
+  WideRay w;
+  RayHit h;
+  float enter;   // minT when the hit in h was accepted
+  unsigned ord;  // where the ray's visit order lies in WideNode::order (kAnyOrder: any hit)
+  int cur;       // node (>= 0), leaf code, kPop or kIdle
+  bool bad;      // the reference's own steps have to trace it
+};
+constexpr unsigned kAnyOrder = 24;
+
+// The reference's slab test of the leaf that holds object slot `slot`.
+__device__ __forceinline__ bool leaf_entered(const DevScene& sc, const WideLane& L, int slot,
+                                             float minT) {
+  int rec = sc.leaf_at[slot];
+  while (rec < 0) rec = sc.leaf_at[--slot];
+  const RefNode& nd = sc.refs[rec];
+  Ray r = L.r;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) r.inv[k] = L.w.inv[k];
+  // (a reciprocal may have been cut where a component is this small beside the largest)
+  const float dmin = fminf(fminf(fabsf(r.d[0]), fabsf(r.d[1])), fabsf(r.d[2]));
+  const float dmax = fmaxf(fmaxf(fabsf(r.d[0]), fabsf(r.d[1])), fabsf(r.d[2]));
+  if (dmin * 0x1p39f < dmax) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) r.inv[k] = 1.0f / r.d[k];
+  }
+  float tn;
+  return slab(nd.box.lo[0], nd.box.hi[0], nd.box.lo[1], nd.box.hi[1], nd.box.lo[2], nd.box.hi[2],
+              r, minT, tn);
+}
+
+// The lanes that meet one box of a node.
+__device__ __forceinline__ unsigned long long wide_box(float nx, float fx, float ny, float fy,
+                                                       float nz, float fz, const WideRay& w,
+                                                       float minT, float& tn) {
+  const float ax = __builtin_fmaf(nx, w.inv[0], w.cn[0]), bx = __builtin_fmaf(fx, w.inv[0], w.cf[0]);
+  const float ay = __builtin_fmaf(ny, w.inv[1], w.cn[1]), by = __builtin_fmaf(fy, w.inv[1], w.cf[1]);
+  const float az = __builtin_fmaf(nz, w.inv[2], w.cn[2]), bz = __builtin_fmaf(fz, w.inv[2], w.cf[2]);
+  tn = fmaxf(fmaxf(fmaxf(ax, ay), az), kEps);
+  const float tf = fminf(fminf(bx, by), bz);
+  return wave_mask(tn <= tf) & wave_mask(tn <= minT);
+}
+
+// Per-lane stack, its newest S entries in LDS ([entry][lane], no bank conflicts), older ones
+// in the thread's spill column. sp and base count in steps of U bytes.
+template <int S, int BLOCK>
+struct WideStack {
+  static_assert((S & (S - 1)) == 0 && S > 4, "ring size is a power of two");
+  static constexpr int U = BLOCK * 8, RM = (S - 1) * U;
+  MH_LDS char* col;
+  MH_GLOBAL unsigned long long* spill;  // [depth][spill_stride], this thread's column
+  int64_t spill_stride;
+  int sp = 0, base = 0;  // entries [base, sp) are in the ring, [0, base) spilled
+
+  __device__ __forceinline__ WideStack(unsigned long long* lds, unsigned long long* area,
+                                       int64_t stride, int64_t gtid, int tid)
+      : col((MH_LDS char*)(MH_LDS unsigned long long*)lds + 8 * tid),
+        spill((MH_GLOBAL unsigned long long*)area + gtid), spill_stride(stride) {}
+
+  __device__ __forceinline__ MH_LDS unsigned long long* at(int p) const {
+    return (MH_LDS unsigned long long*)(col + (p & RM));
+  }
+  __device__ __forceinline__ MH_GLOBAL unsigned long long* spilled(int p) const {
+    return spill + (int64_t)(p / U) * spill_stride;
+  }
+  __device__ __forceinline__ void reset() { sp = base = 0; }
+  // Up to three entries, the deepest first; each is written, and kept for the lanes of its
+  // mask.
+  __device__ __forceinline__ void push3(unsigned long long ma, int ra, float ta,
+                                        unsigned long long mb, int rb, float tb,
+                                        unsigned long long mc, int rc, float tc) {
+    if (wave_mask(sp - base > (S - 3) * U)) {
+      while (sp - base > (S - 3) * U) {
+        *spilled(base) = *at(base);
+        base += U;
+      }
+    }
+    *at(sp) = stack_entry(ra, ta);
+    sp += lane_bit(ma) ? U : 0;
+    *at(sp) = stack_entry(rb, tb);
+    sp += lane_bit(mb) ? U : 0;
+    *at(sp) = stack_entry(rc, tc);
+    sp += lane_bit(mc) ? U : 0;
+  }
+  // The newest entry of the lanes that have one (`have`); the caller takes it off.
+  __device__ __forceinline__ unsigned long long top(bool have) {
+    unsigned long long e = *at(sp - U);
+    const unsigned long long low = wave_mask(have) & wave_mask(sp == base);
+    if (low) {
+      if (lane_bit(low)) {
+        base -= U;
+        e = *spilled(base);
+      }
+    }
+    return e;
+  }
+};
+
+// Visits node L.cur: the boxes two levels down, the nearest in visit order next, the others
+// on the stack.
+template <int S, int BLOCK>
+__device__ __forceinline__ void wide_node_step(const DevScene& sc, WideLane& L,
+                                               WideStack<S, BLOCK>& st) {
+  const MhBufRsrc wt = record_table(sc.wide, sizeof(WideNode), sc.n_wide);
+  const WideRay& w = L.w;
+  const float4 NX = fetch_record_at(wt, L.cur, w.on[0], 0), FX = fetch_record_at(wt, L.cur, w.of[0], 0);
+  const float4 NY = fetch_record_at(wt, L.cur, w.on[1], 32), FY = fetch_record_at(wt, L.cur, w.of[1], 32);
+  const float4 NZ = fetch_record_at(wt, L.cur, w.on[2], 64), FZ = fetch_record_at(wt, L.cur, w.of[2], 64);
+  const float4 D = fetch_record(wt, L.cur, 96);
+  const unsigned order = __float_as_uint(fetch_record(wt, L.cur, 112).x) >> L.ord;
+  float t0, t1, t2, t3;
+  const unsigned long long H0 = wide_box(NX.x, FX.x, NY.x, FY.x, NZ.x, FZ.x, w, L.h.minT, t0);
+  const unsigned long long H1 = wide_box(NX.y, FX.y, NY.y, FY.y, NZ.y, FZ.y, w, L.h.minT, t1);
+  const unsigned long long H2 = wide_box(NX.z, FX.z, NY.z, FY.z, NZ.z, FZ.z, w, L.h.minT, t2);
+  const unsigned long long H3 = wide_box(NX.w, FX.w, NY.w, FY.w, NZ.w, FZ.w, w, L.h.minT, t3);
+  const int r0 = __float_as_int(D.x), r1 = __float_as_int(D.y), r2 = __float_as_int(D.z),
+            r3 = __float_as_int(D.w);
+  // into visit order: swap inside the left pair, inside the right pair, and the pairs
+  const unsigned long long P = wave_mask((order & 1u) != 0), Lm = wave_mask((order & 2u) != 0),
+                           Rm = wave_mask((order & 4u) != 0);
+  const bool sp = lane_bit(P), sl = lane_bit(Lm), sr = lane_bit(Rm);
+  const float ta = sl ? t1 : t0, tb = sl ? t0 : t1, tc = sr ? t3 : t2, td = sr ? t2 : t3;
+  const int ra = sl ? r1 : r0, rb = sl ? r0 : r1, rc = sr ? r3 : r2, rd = sr ? r2 : r3;
+  const float u1 = sp ? td : tb, u2 = sp ? ta : tc, u3 = sp ? tb : td;
+  const int q0 = sp ? rc : ra, q1 = sp ? rd : rb, q2 = sp ? ra : rc, q3 = sp ? rb : rd;
+  const unsigned long long a = (Lm & H1) | (~Lm & H0), b = (Lm & H0) | (~Lm & H1),
+                           c = (Rm & H3) | (~Rm & H2), d = (Rm & H2) | (~Rm & H3);
+  const unsigned long long G0 = (P & c) | (~P & a), G1 = (P & d) | (~P & b),
+                           G2 = (P & a) | (~P & c), G3 = (P & b) | (~P & d);
+  st.push3(G3 & (G0 | G1 | G2), q3, u3, G2 & (G0 | G1), q2, u2, G1 & G0, q1, u1);
+  int cur = lane_bit(G3) ? q3 : kPop;
+  cur = lane_bit(G2) ? q2 : cur;
+  cur = lane_bit(G1) ? q1 : cur;
+  L.cur = lane_bit(G0) ? q0 : cur;
+}
+
+// Tests one triangle of leaf L.cur (every one where it holds kLeafCountInline or more).
+template <int PRIM>
+__device__ __forceinline__ void wide_leaf_step(const DevScene& sc, WideLane& L) {
+  const int code = ~L.cur;
+  int slot = code >> kLeafCountBits;
+  const int count = code & kLeafCountInline;  // left in the leaf; 0 in an empty slot's code
+  int left = count == 0 ? 0 : 1;
+  if (count == kLeafCountInline) left = sc.big_count[slot];
+  bool done = false;
+  for (; left > 0 && !done; --left, ++slot) {
+    float t, u, v;
+    if (!prim_test<PRIM>(sc, slot, L.r, L.h.minT, t, u, v)) continue;
+    if (L.h.best >= 0 && !(t < L.h.minT - 4 * kEps))
+      L.bad |= !leaf_entered(sc, L, L.h.best, L.enter);
+    L.enter = L.h.minT;
+    L.h = RayHit{t, slot, u, v};
+    done = L.ord == kAnyOrder;
+  }
+  if (done)
+    L.cur = kIdle;
+  else if (count > 1 && count < kLeafCountInline)
+    L.cur -= (1 << kLeafCountBits) - 1;  // code: the next slot, one triangle fewer
+  else
+    L.cur = kPop;
+}
+
+// One step of the wave; a lane at a leaf weighs `weight` quarters of one at a node.
+template <int PRIM, int S, int BLOCK>
+__device__ __forceinline__ void wide_step(const DevScene& sc, WideLane& L, int weight,
+                                          WideStack<S, BLOCK>& st) {
+  const unsigned long long at_node = wave_mask(L.cur >= 0);
+  const unsigned long long at_leaf = wave_mask(L.cur < 0) & wave_mask(L.cur > kPop);
+  if (weight * __popcll(at_leaf) >= 4 * __popcll(at_node)) {
+    if (lane_bit(at_leaf)) wide_leaf_step<PRIM>(sc, L);
+  } else {
+    if (lane_bit(at_node)) wide_node_step<S, BLOCK>(sc, L, st);
+  }
+  if (L.cur == kPop) {
+    const bool have = st.sp > 0;
+    const unsigned long long e = st.top(have);
+    st.sp -= have ? st.U : 0;
+    L.cur = !have ? kIdle
+                  : (__uint_as_float((unsigned)(e >> 32)) <= L.h.minT ? (int)(unsigned)e : kPop);
+  }
+}
+
+// The reference's own traversal of ray i, on its 32-byte records.
+template <int PRIM, int S, int BLOCK>
+__device__ __forceinline__ void wide_redo(const DevScene& sc, const GRays& rays, int64_t i,
+                                          WideLane& L, WideStack<S, BLOCK>& st) {
+  const bool any = L.ord == kAnyOrder;
+  Ray r;
+  load_ray(rays, i, r);
+  RayHit h{rays.tmax[i], -1, 0.f, 0.f};
+  int cur = 0;
+  st.reset();
+  for (;;) {
+    const RefNode nd = sc.refs[cur];
+    float tn;
+    if (slab(nd.box.lo[0], nd.box.hi[0], nd.box.lo[1], nd.box.hi[1], nd.box.lo[2], nd.box.hi[2], r,
+             h.minT, tn)) {
+      if (nd.children != 0) {
+        bool done = false;
+        for (int k = 0; k < nd.children && !done; ++k) {
+          float t, u, v;
+          if (prim_test<PRIM>(sc, nd.child + k, r, h.minT, t, u, v)) {
+            h = RayHit{t, nd.child + k, u, v};
+            done = any;
+          }
+        }
+        if (done) break;
+      } else {
+        const int front = any ? ((nd.bits & 1) ? 0 : 1) : (((r.dpos >> (nd.axis & 3)) & 1) ? 0 : 1);
+        st.push3(0, 0, 0.f, 0, 0, 0.f, ~0ull, nd.child + 1 - front, 0.f);
+        cur = nd.child + front;
+        continue;
+      }
+    }
+    if (st.sp == 0) break;
+    cur = (int)(unsigned)st.top(true);
+    st.sp -= st.U;
+  }
+  L.h = h;
+}
+
+// Starts ray i of `rays` in an idle lane.
+template <int S, int BLOCK>
+__device__ __forceinline__ void wide_start(const DevScene& sc, float reach, const GRays& rays,
+                                           int64_t i, bool any, bool nested, WideLane& L,
+                                           WideStack<S, BLOCK>& st) {
+  load_ray(rays, i, L.r);
+  L.h = RayHit{rays.tmax[i], -1, 0.f, 0.f};
+  L.enter = L.h.minT;
+  st.reset();
+  const bool ok = nested & wide_setup(reach, L.r, L.h.minT, L.w);
+  L.bad = !ok;
+  L.cur = ok ? sc.root_ref : kIdle;
+  L.ord = any ? kAnyOrder : 3u * (L.r.dpos & 7u);
+}
+
+// Stores the hit of a lane that has come to the end of ray i.
+template <int PRIM, int S, int BLOCK>
+__device__ __forceinline__ void wide_finish(const DevScene& sc, const GRays& rays,
+                                            const GHits& hits, int64_t i, WideLane& L,
+                                            WideStack<S, BLOCK>& st) {
+  if (!L.bad && L.h.best >= 0) L.bad = !leaf_entered(sc, L, L.h.best, L.enter);
+  if (L.bad) wide_redo<PRIM, S, BLOCK>(sc, rays, i, L, st);
+  const bool hit = L.h.best >= 0;
+  store_hit(hits, i, hit ? sc.obj_ids[L.h.best] : -1, (L.ord == kAnyOrder && hit) ? kEps : L.h.minT, L.h.u,
+            L.h.v, hit);
+}
+
+struct WideArgs {
+  const BatchTable* table;  // TABLE: the batches
+  BatchDev one;             // !TABLE: the only one
+  unsigned long long* ctr;  // u64[2], zero between launches; null with a static stride
+  unsigned long long* spill;
+  int64_t spill_stride;
+  int nb;       // TABLE: batches, as the host counted them
+  int refill;   // idle lanes of a wave that make it take rays
+  int chunk;    // rays a wave takes at a time, at most total / fair (> 0), at least 64
+  int fair;
+  int remap;    // give each XCD a contiguous share of the first chunks
+  int reverse;  // hand chunks out from the end of the table
+  int weight;   // wide_step
+};
+
+// Persistent waves over the rays of one batch or of a table of batches, numbered through.
+// A wave takes `chunk` ray numbers at a time: first those at its own place, then by a
+// shared counter (or the next static stride without one), the counter asked ahead of time.
+// Idle lanes take the wave's next rays as soon as `refill` of them are idle. The last wave
+// to leave clears the counter, so launches and graph replays need no clearing pass. Five
+// waves a SIMD (96 registers; 80 for six spill).
+template <int PRIM, int S, int BLOCK, bool TABLE>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_trace_wide(
+    DevScene sc, WideArgs a) {
+  __shared__ unsigned long long s_ring[S * BLOCK];
+  extern __shared__ int64_t s_start[];  // TABLE: nb entries (dynamic LDS)
+  int nb = 1;
+  int64_t total = a.one.count;
+  const BatchDev* batches = nullptr;
+  const int tid = threadIdx.x, lane = tid & 63;
+  if constexpr (TABLE) {
+    // The dynamic LDS holds a.nb offsets; a table with more entries is cut to that.
+    const BatchTable* table = a.table;
+    nb = table->nb < a.nb ? table->nb : a.nb;
+    batches = table->batches;
+    total = nb == table->nb ? table->total : batches[nb - 1].start + batches[nb - 1].count;
+    for (int i = tid; i < nb; i += BLOCK) s_start[i] = batches[i].start;
+    __syncthreads();
+  }
+  int blk = blockIdx.x;
+  if (a.remap && (gridDim.x & 7) == 0) blk = (blk & 7) * (gridDim.x >> 3) + (blk >> 3);
+  const int64_t n_waves = (int64_t)gridDim.x * (BLOCK / 64);
+  const int64_t wave_id = ((int64_t)blk * BLOCK + tid) >> 6;
+  WideStack<S, BLOCK> st(s_ring, a.spill, a.spill_stride, (int64_t)blockIdx.x * BLOCK + tid, tid);
+  const RefNode root = sc.refs[0];
+  float reach = 0.f;
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+    reach = fmaxf(reach, fmaxf(fabsf(root.box.lo[k]), fabsf(root.box.hi[k])));
+  const bool nested = *sc.irregular == 0;
+
+  int64_t C = a.chunk;
+  if (a.fair > 0) {  // no more than a quarter of a resident wave's share of the rays
+    const int64_t share = (total / a.fair) & ~(int64_t)63;
+    C = share < 64 ? 64 : (share < C ? share : C);
+  }
+  int64_t next = wave_id * C;      // hand-out number of the wave's next chunk
+  int64_t pos = 0, end = 0;        // rays in hand
+  unsigned long long ahead = 0;    // lane 0: the counter's answer, the chunk after this one
+  bool asked = false;              // `next` has to be taken from it
+  WideLane L;
+  L.cur = kIdle;
+  int64_t li = -1;  // ray in its batch, -1 none
+  int bi = 0;       // its batch
+  // Runs fn(rays, hits, flags, start) for the lanes of `who`, batch by batch (nearly always
+  // one), so that a batch's record is read by scalar loads.
+  auto by_batch = [&](bool who, auto fn) {
+    if constexpr (!TABLE) {
+      if (who) fn(global_view(a.one.rays), global_view(a.one.hits), a.one.flags);
+    } else {
+      for (unsigned long long todo = wave_mask(who); todo;) {
+        const int b = __builtin_amdgcn_readlane(bi, __builtin_ctzll(todo));
+        const unsigned long long m = wave_mask(bi == b) & todo;
+        const BatchDev& B = batches[b];
+        if (lane_bit(m)) fn(global_view(B.rays), global_view(B.hits), B.flags);
+        todo &= ~m;
+      }
+    }
+  };
+
+  for (;;) {
+    const unsigned long long idle = wave_mask(L.cur == kIdle);
+    const int n_idle = __popcll(idle);
+    bool take_rays = n_idle >= a.refill, more = true;
+    if (take_rays) {
+      if (pos >= end && asked) {
+        next = (int64_t)__shfl((long long)ahead, 0, 64) + n_waves * C;
+        asked = false;
+      }
+      more = pos < end || next < total;
+      take_rays = more || n_idle == 64;
+    }
+    if (take_rays) {
+      by_batch(lane_bit(idle) && li >= 0, [&](const GRays& rays, const GHits& hits, uint32_t) {
+        wide_finish<PRIM, S, BLOCK>(sc, rays, hits, li, L, st);
+      });
+      if (lane_bit(idle)) li = -1;
+      if (!more) break;  // every lane is idle
+      if (pos >= end) {
+        pos = a.reverse ? (total - next - C > 0 ? total - next - C : 0) : next;
+        end = a.reverse ? total - next : (next + C < total ? next + C : total);
+        if (a.ctr) {
+          if (lane == 0) ahead = atomicAdd(a.ctr, (unsigned long long)C);
+          asked = true;
+        } else {
+          next += n_waves * C;
+        }
+      }
+      const int64_t g = pos + __popcll(idle & ((1ull << lane) - 1ull));
+      const bool take = lane_bit(idle) && g < end;
+      int64_t i = g;
+      if constexpr (TABLE) {
+        if (take) {
+          bi = find_batch(s_start, nb, g);
+          i = g - s_start[bi];
+        }
+      }
+      by_batch(take, [&](const GRays& rays, const GHits& hits, uint32_t flags) {
+        if (rays.masked && rays.masked[i]) {
+          store_hit(hits, i, -2, -kMaxT, 0.f, 0.f, true);
+        } else {
+          li = i;
+          wide_start<S, BLOCK>(sc, reach, rays, i, (flags & 1u) != 0, nested, L, st);
+        }
+      });
+      pos = pos + n_idle < end ? pos + n_idle : end;
+    }
+    wide_step<PRIM, S, BLOCK>(sc, L, a.weight, st);
+  }
+  if (a.ctr && lane == 0) {
+    const unsigned long long left = atomicAdd(a.ctr + 1, 1ull);
+    if (left == (unsigned long long)n_waves - 1) {
+      atomicExch(a.ctr, 0ull);
+      atomicExch(a.ctr + 1, 0ull);
+    }
+  }
+}
+
+namespace {
+
+template <int PRIM, int BLOCK, bool TABLE>
+int launch_wide(const DevScene& sc, const WideArgs& a, int blocks, int stack_lds, hipStream_t s) {
+  const dim3 g(blocks), b(BLOCK);
+  const size_t lds = TABLE ? sizeof(int64_t) * (size_t)a.nb : 0;  // batch start offsets
+  if (stack_lds == 8)
+    hipLaunchKernelGGL((k_trace_wide<PRIM, 8, BLOCK, TABLE>), g, b, lds, s, sc, a);
+  else if (stack_lds == 32)
+    hipLaunchKernelGGL((k_trace_wide<PRIM, 32, BLOCK, TABLE>), g, b, lds, s, sc, a);
+  else
+    hipLaunchKernelGGL((k_trace_wide<PRIM, 16, BLOCK, TABLE>), g, b, lds, s, sc, a);
+  return (int)hipGetLastError();
+}
+
+// A lane at a leaf weighs as much as one at a node: a triangle test costs about what a node
+// visit does. (Half of that is 4% better on camera rays and 6% worse on a soup's.)
+constexpr int kLeafWeight = 4;
+// Whole-wave chunks of more than 64 rays: the wave takes its chunk's next rays when this many
+// lanes are idle, and no chunk is more than a quarter of a resident wave's share of the rays.
+// (12 uneven batches, 3M rays in a 300,000-triangle soup, the frames' default configuration,
+// 256-ray chunks: 1691 us; 2928 with 64 idle lanes and whole chunks.)
+constexpr int kChunkRefill = 40;
+
+template <int PRIM>
+int launch_wide_table(const DevScene& sc, const BatchLaunch& bl, hipStream_t s) {
+  WideArgs a{};
+  a.table = bl.table;
+  a.ctr = bl.chunk == 0 ? nullptr : bl.counters;
+  a.spill = reinterpret_cast<unsigned long long*>(bl.spill);
+  a.spill_stride = bl.spill_stride;
+  a.nb = bl.nb;
+  a.refill = bl.refill == 64 && bl.chunk > 64 ? kChunkRefill : bl.refill;
+  a.chunk = bl.chunk == 0 ? 64 : bl.chunk;
+  a.fair = bl.chunk > 64 ? 4 * bl.resident : 0;
+  a.remap = bl.xcd_remap;
+  a.reverse = bl.reverse;
+  a.weight = kLeafWeight;
+  if (bl.block == 64) return launch_wide<PRIM, 64, true>(sc, a, bl.blocks, bl.stack_lds, s);
+  if (bl.block == 128) return launch_wide<PRIM, 128, true>(sc, a, bl.blocks, bl.stack_lds, s);
+  return launch_wide<PRIM, 256, true>(sc, a, bl.blocks, bl.stack_lds, s);
+}
+
+template <int PRIM>
+int launch_wide_one(const DevScene& sc, const BatchDev& rays, const LaunchCfg& cfg, hipStream_t s) {
+  WideArgs a{};
+  a.one = rays;
+  a.spill = reinterpret_cast<unsigned long long*>(cfg.spill);
+  a.spill_stride = cfg.spill_stride;
+  a.refill = 64;
+  a.chunk = cfg.chunk;
+  a.reverse = 1;
+  a.weight = kLeafWeight;
+  return launch_wide<PRIM, 64, false>(sc, a, cfg.blocks, cfg.stack_lds, s);
+}
+
+}  // namespace
+
+// One launcher per triangle test (wide_ks.hip, wide_wald.hip).
+int launch_wide_table_ks(const DevScene& sc, const BatchLaunch& bl, hipStream_t s);
+int launch_wide_table_wald(const DevScene& sc, const BatchLaunch& bl, hipStream_t s);
+int launch_wide_one_ks(const DevScene& sc, const BatchDev& rays, const LaunchCfg& cfg,
+                       hipStream_t s);
+int launch_wide_one_wald(const DevScene& sc, const BatchDev& rays, const LaunchCfg& cfg,
+                         hipStream_t s);
+
+}  // namespace mh
