@@ -389,8 +389,12 @@ constexpr int kTraceBlocksPerCu = 32;
 // fewer others: 4,096 rays in a 10,000-triangle soup 98 us at 64 rays a wave, 67 at 4.
 constexpr int64_t kMinWaveRays = 4;
 // Ring entries unless the caller says: 16 (five waves per SIMD fill the LDS) spill less than
-// 8 (786,432 camera and bounce rays in a 200,000-triangle soup 1274 against 1337 us).
-constexpr int kWideRing = 16;
+// 8 (786,432 camera and bounce rays in a 200,000-triangle soup 1274 against 1337 us), and
+// where there are few waves 32 need no spill area up to a depth of 21 (allocating one takes
+// a first call about 300 us). 32 with waves to spare cost occupancy: 199,023 rays 68
+// against 57 us.
+constexpr int kWideRing = 16, kFewWavesRing = 32;
+constexpr int64_t kFewWaves = 8;  // per compute unit
 
 // The caller's ring, or the one the reference records' kernel takes.
 int choose_stack(const mh_trace_opts* o) {
@@ -428,7 +432,6 @@ int trace_impl(const mh_scene* cs, const mh_rays* rays, const mh_hits* hits, int
       return fail(MH_E_UNSUPPORTED, "tree depth %u exceeds the packet stack (126)", s->depth);
   } else {
     const int S = choose_stack(opts);
-    const int wide_S = opts && opts->stack_lds == S ? S : kWideRing;
     const int bpc = (opts && opts->blocks_per_cu > 0) ? opts->blocks_per_cu : kTraceBlocksPerCu;
     const int64_t cus = g_lib.cu_count;
     // The reference records' kernel: its stack is shorter, and the counters are kept there.
@@ -452,6 +455,9 @@ int trace_impl(const mh_scene* cs, const mh_rays* rays, const mh_hits* hits, int
     const int64_t chunk =
         std::min<int64_t>(64, std::max<int64_t>(kMinWaveRays, (n + 4 * cus - 1) / (4 * cus)));
     const int64_t waves = (n + chunk - 1) / chunk;
+    const int wide_S = opts && opts->stack_lds == S ? S
+                       : waves <= kFewWaves * cus   ? kFewWavesRing
+                                                    : kWideRing;
     int64_t blocks = std::min(waves, 4 * cus * bpc);
     int64_t need = std::max<int64_t>(0, (int64_t)s->stack_bound(MH_LAYOUT_PAIR) - wide_S);
     bool wide = !cfg.counters;

@@ -204,22 +204,40 @@ static __device__ __forceinline__ bool wald_test(const float4 A, const float4 B,
   return true;
 }
 
+// The 48-byte record of object slot `slot`.
+struct PrimRecord {
+  float4 A, B, C;
+};
+static __device__ __forceinline__ PrimRecord fetch_prim(const DevScene& sc, int slot) {
+  const MhBufRsrc tt = record_table(sc.tris, 12 * sizeof(float), sc.n_slots);
+  const PrimRecord p{fetch_record(tt, slot, 0), fetch_record(tt, slot, 16),
+                     fetch_record(tt, slot, 32)};
+  return p;
+}
+// All 48 bytes are fetched before the first rejection test (one round trip) instead of the
+// compiler deferring the edge loads past the distance test.
+// (Input operands only: the values stay in the registers they were loaded into.)
+static __device__ __forceinline__ void hold_prim(const PrimRecord& p) {
+  asm volatile("" ::"v"(p.A.x), "v"(p.A.y), "v"(p.A.z), "v"(p.A.w), "v"(p.B.x), "v"(p.B.y),
+               "v"(p.B.z), "v"(p.B.w), "v"(p.C.x), "v"(p.C.y), "v"(p.C.z), "v"(p.C.w));
+}
+template <int PRIM>
+static __device__ __forceinline__ bool record_test(const PrimRecord& p, const Ray& r, float minT,
+                                                   float& t, float& u, float& v) {
+  return PRIM == 0 ? ks_test(p.A, p.B, p.C, r, minT, t, u, v)
+                   : wald_test(p.A, p.B, p.C, r, minT, t, u, v);
+}
+
 template <int PRIM>
 static __device__ __forceinline__ bool prim_test(const DevScene& sc, int slot, const Ray& r,
                                                  float minT, float& t, float& u, float& v) {
-  const MhBufRsrc tt = record_table(sc.tris, 12 * sizeof(float), sc.n_slots);
-  float4 A = fetch_record(tt, slot, 0), B = fetch_record(tt, slot, 16),
-         C = fetch_record(tt, slot, 32);
-  // All 48 bytes are fetched before the first rejection test (one round trip) instead of
-  // the compiler deferring the edge loads past the distance test.
-  // (Input operands only: the values stay in the registers they were loaded into.)
-  asm volatile("" ::"v"(A.x), "v"(A.y), "v"(A.z), "v"(A.w), "v"(B.x), "v"(B.y), "v"(B.z),
-               "v"(B.w), "v"(C.x), "v"(C.y), "v"(C.z), "v"(C.w));
-  if (PRIM == 0) return ks_test(A, B, C, r, minT, t, u, v);
-  return wald_test(A, B, C, r, minT, t, u, v);
+  const PrimRecord p = fetch_prim(sc, slot);
+  hold_prim(p);
+  return record_test<PRIM>(p, r, minT, t, u, v);
 }
 
-static __device__ __forceinline__ void load_ray(const GRays& rays, int64_t i, Ray& r) {
+template <class Index>
+static __device__ __forceinline__ void load_ray(const GRays& rays, Index i, Ray& r) {
   r.o[0] = rays.ox[i];
   r.o[1] = rays.oy[i];
   r.o[2] = rays.oz[i];
@@ -235,7 +253,8 @@ static __device__ __forceinline__ void load_ray(const GRays& rays, int64_t i, Ra
   r.dpos |= r.dpos << 4;
 }
 
-static __device__ __forceinline__ void store_hit(const GHits& h, int64_t i, int32_t prim, float t,
+template <class Index>
+static __device__ __forceinline__ void store_hit(const GHits& h, Index i, int32_t prim, float t,
                                           float u, float v, bool occ) {
   if (h.prim) h.prim[i] = prim;
   if (h.t) h.t[i] = t;

@@ -228,28 +228,41 @@ __device__ __forceinline__ void wide_node_step(const DevScene& sc, WideLane& L,
   L.cur = lane_bit(G0) ? q0 : cur;
 }
 
-// Tests one triangle of leaf L.cur (every one where it holds kLeafCountInline or more).
+// Tests the triangle of `slot`; true when that ends an any-hit ray.
+template <int PRIM>
+__device__ __forceinline__ bool wide_tri(const DevScene& sc, WideLane& L, int slot,
+                                         const PrimRecord& p) {
+  float t, u, v;
+  if (!record_test<PRIM>(p, L.r, L.h.minT, t, u, v)) return false;
+  if (L.h.best >= 0 && !(t < L.h.minT - 4 * kEps)) L.bad |= !leaf_entered(sc, L, L.h.best, L.enter);
+  L.enter = L.h.minT;
+  L.h = RayHit{t, slot, u, v};
+  return L.ord == kAnyOrder;
+}
+
+// Tests two triangles of leaf L.cur (every one where it holds kLeafCountInline or more), both
+// fetched at once: a surface's leaves hold two as a rule, and a second step for the second
+// one would wait for its record again. (One a step: 1M incoherent rays over the 1M-triangle
+// heightfield 228 against 205 us, shadow rays 239 against 214. Past the last slot the
+// descriptor reads zeros.)
 template <int PRIM>
 __device__ __forceinline__ void wide_leaf_step(const DevScene& sc, WideLane& L) {
   const int code = ~L.cur;
-  int slot = code >> kLeafCountBits;
+  const int slot = code >> kLeafCountBits;
   const int count = code & kLeafCountInline;  // left in the leaf; 0 in an empty slot's code
-  int left = count == 0 ? 0 : 1;
-  if (count == kLeafCountInline) left = sc.big_count[slot];
-  bool done = false;
-  for (; left > 0 && !done; --left, ++slot) {
-    float t, u, v;
-    if (!prim_test<PRIM>(sc, slot, L.r, L.h.minT, t, u, v)) continue;
-    if (L.h.best >= 0 && !(t < L.h.minT - 4 * kEps))
-      L.bad |= !leaf_entered(sc, L, L.h.best, L.enter);
-    L.enter = L.h.minT;
-    L.h = RayHit{t, slot, u, v};
-    done = L.ord == kAnyOrder;
+  const PrimRecord p = fetch_prim(sc, slot), q = fetch_prim(sc, slot + 1);
+  hold_prim(p);
+  hold_prim(q);
+  bool done = count > 0 && wide_tri<PRIM>(sc, L, slot, p);
+  if (!done && count > 1) done = wide_tri<PRIM>(sc, L, slot + 1, q);
+  if (!done && count == kLeafCountInline) {
+    const int end = slot + sc.big_count[slot];
+    for (int k = slot + 2; k < end && !done; ++k) done = wide_tri<PRIM>(sc, L, k, fetch_prim(sc, k));
   }
   if (done)
     L.cur = kIdle;
-  else if (count > 1 && count < kLeafCountInline)
-    L.cur -= (1 << kLeafCountBits) - 1;  // code: the next slot, one triangle fewer
+  else if (count > 2 && count < kLeafCountInline)
+    L.cur -= 2 * ((1 << kLeafCountBits) - 1);  // code: two slots on, two triangles fewer
   else
     L.cur = kPop;
 }
@@ -275,8 +288,8 @@ __device__ __forceinline__ void wide_step(const DevScene& sc, WideLane& L, int w
 }
 
 // The reference's own traversal of ray i, on its 32-byte records.
-template <int PRIM, int S, int BLOCK>
-__device__ __forceinline__ void wide_redo(const DevScene& sc, const GRays& rays, int64_t i,
+template <int PRIM, int S, int BLOCK, class Index>
+__device__ __forceinline__ void wide_redo(const DevScene& sc, const GRays& rays, Index i,
                                           WideLane& L, WideStack<S, BLOCK>& st) {
   const bool any = L.ord == kAnyOrder;
   Ray r;
@@ -313,10 +326,11 @@ __device__ __forceinline__ void wide_redo(const DevScene& sc, const GRays& rays,
   L.h = h;
 }
 
-// Starts ray i of `rays` in an idle lane.
-template <int S, int BLOCK>
+// Starts ray i of `rays` in an idle lane (Index: 32 bits where the views were moved to the
+// wave's first ray, so that the addresses are a scalar base and a lane offset).
+template <int S, int BLOCK, class Index>
 __device__ __forceinline__ void wide_start(const DevScene& sc, float reach, const GRays& rays,
-                                           int64_t i, bool any, bool nested, WideLane& L,
+                                           Index i, bool any, bool nested, WideLane& L,
                                            WideStack<S, BLOCK>& st) {
   load_ray(rays, i, L.r);
   L.h = RayHit{rays.tmax[i], -1, 0.f, 0.f};
@@ -329,9 +343,9 @@ __device__ __forceinline__ void wide_start(const DevScene& sc, float reach, cons
 }
 
 // Stores the hit of a lane that has come to the end of ray i.
-template <int PRIM, int S, int BLOCK>
+template <int PRIM, int S, int BLOCK, class Index>
 __device__ __forceinline__ void wide_finish(const DevScene& sc, const GRays& rays,
-                                            const GHits& hits, int64_t i, WideLane& L,
+                                            const GHits& hits, Index i, WideLane& L,
                                             WideStack<S, BLOCK>& st) {
   if (!L.bad && L.h.best >= 0) L.bad = !leaf_entered(sc, L, L.h.best, L.enter);
   if (L.bad) wide_redo<PRIM, S, BLOCK>(sc, rays, i, L, st);
@@ -341,54 +355,146 @@ __device__ __forceinline__ void wide_finish(const DevScene& sc, const GRays& ray
 }
 
 struct WideArgs {
-  const BatchTable* table;  // TABLE: the batches
-  BatchDev one;             // !TABLE: the only one
+  DevScene sc;
+  const BatchTable* table;  // a table of batches, or null
+  BatchDev one;             // table null: the only batch
   unsigned long long* ctr;  // u64[2], zero between launches; null with a static stride
   unsigned long long* spill;
   int64_t spill_stride;
-  int nb;       // TABLE: batches, as the host counted them
-  int refill;   // idle lanes of a wave that make it take rays
-  int chunk;    // rays a wave takes at a time, at most total / fair (> 0), at least 64
-  int fair;
+  int nb;       // batches of the table, as the host counted them
+  int refill;   // k_wide_lanes: idle lanes of a wave that make it take rays
+  int chunk;    // rays a wave takes at a time ...
+  int fair;     // ... at most total / fair where fair > 0, at least 64
   int remap;    // give each XCD a contiguous share of the first chunks
   int reverse;  // hand chunks out from the end of the table
   int weight;   // wide_step
 };
 
-// Persistent waves over the rays of one batch or of a table of batches, numbered through.
-// A wave takes `chunk` ray numbers at a time: first those at its own place, then by a
-// shared counter (or the next static stride without one), the counter asked ahead of time.
-// Idle lanes take the wave's next rays as soon as `refill` of them are idle. The last wave
-// to leave clears the counter, so launches and graph replays need no clearing pass. Five
-// waves a SIMD (96 registers; 80 for six spill).
-template <int PRIM, int S, int BLOCK, bool TABLE>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_trace_wide(
-    DevScene sc, WideArgs a) {
-  __shared__ unsigned long long s_ring[S * BLOCK];
-  extern __shared__ int64_t s_start[];  // TABLE: nb entries (dynamic LDS)
-  int nb = 1;
-  int64_t total = a.one.count;
-  const BatchDev* batches = nullptr;
-  const int tid = threadIdx.x, lane = tid & 63;
-  if constexpr (TABLE) {
-    // The dynamic LDS holds a.nb offsets; a table with more entries is cut to that.
-    const BatchTable* table = a.table;
-    nb = table->nb < a.nb ? table->nb : a.nb;
-    batches = table->batches;
-    total = nb == table->nb ? table->total : batches[nb - 1].start + batches[nb - 1].count;
-    for (int i = tid; i < nb; i += BLOCK) s_start[i] = batches[i].start;
-    __syncthreads();
-  }
-  int blk = blockIdx.x;
-  if (a.remap && (gridDim.x & 7) == 0) blk = (blk & 7) * (gridDim.x >> 3) + (blk >> 3);
-  const int64_t n_waves = (int64_t)gridDim.x * (BLOCK / 64);
-  const int64_t wave_id = ((int64_t)blk * BLOCK + tid) >> 6;
-  WideStack<S, BLOCK> st(s_ring, a.spill, a.spill_stride, (int64_t)blockIdx.x * BLOCK + tid, tid);
-  const RefNode root = sc.refs[0];
+// The kernel's arguments, to be read again (by scalar loads) where they are used: held in
+// registers from the start they crowd out others, and filling them in costs a wave of one
+// chunk more than it saves.
+__device__ __forceinline__ const WideArgs& args_again() {
+  auto p = __builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const WideArgs*)p;
+}
+
+__device__ __forceinline__ float root_reach(const DevScene& sc) {
+  const RefNode& root = sc.refs[0];
   float reach = 0.f;
 #pragma unroll
   for (int k = 0; k < 3; ++k)
     reach = fmaxf(reach, fmaxf(fabsf(root.box.lo[k]), fabsf(root.box.hi[k])));
+  return reach;
+}
+
+__device__ __forceinline__ GRays moved(GRays r, int64_t n) {
+  return GRays{r.ox + n, r.oy + n, r.oz + n, r.dx + n, r.dy + n,
+               r.dz + n, r.tmax + n, r.masked ? r.masked + n : nullptr};
+}
+__device__ __forceinline__ GHits moved(GHits h, int64_t n) {
+  return GHits{h.prim ? h.prim + n : nullptr, h.t ? h.t + n : nullptr, h.u ? h.u + n : nullptr,
+               h.v ? h.v + n : nullptr, h.occluded ? h.occluded + n : nullptr};
+}
+
+// Waves that trace their rays 64 at a time, a ray to a lane: chunks of `chunk` consecutive
+// rays by a static stride, each cut where a batch ends. A wave lives for about ten steps
+// on camera rays, so what it does beside them is kept short: no lane hand-out, batch
+// arrays read where a group starts and where it ends. Five waves a SIMD.
+template <int PRIM, int S, int BLOCK, bool TABLE>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_wide_whole(
+    WideArgs a) {
+  __shared__ unsigned long long s_ring[S * BLOCK];
+  extern __shared__ int64_t s_start[];  // TABLE: nb entries (dynamic LDS)
+  const int tid = threadIdx.x, lane = tid & 63;
+  int nb = 1;
+  int64_t total = a.one.count;
+  if constexpr (TABLE) {
+    // The dynamic LDS holds a.nb offsets; a table with more entries is cut to that.
+    const BatchTable* table = a.table;
+    nb = table->nb < a.nb ? table->nb : a.nb;
+    total = nb == table->nb ? table->total
+                            : table->batches[nb - 1].start + table->batches[nb - 1].count;
+    for (int i = tid; i < nb; i += BLOCK) s_start[i] = table->batches[i].start;
+    __syncthreads();
+  }
+  int blk = blockIdx.x;
+  if (TABLE && a.remap && (gridDim.x & 7) == 0) blk = (blk & 7) * (gridDim.x >> 3) + (blk >> 3);
+  WideStack<S, BLOCK> st(s_ring, a.spill, a.spill_stride, (int64_t)blockIdx.x * BLOCK + tid, tid);
+  const float reach = root_reach(a.sc);
+  const bool nested = *a.sc.irregular == 0;
+  const int C = a.chunk;
+  const int64_t stride = (int64_t)gridDim.x * (BLOCK / 64) * C;
+  // (the wave's number is the same in all its lanes: kept in scalar registers)
+  int64_t next = ((int64_t)blk * (BLOCK / 64) + __builtin_amdgcn_readfirstlane(tid >> 6)) * C;
+  for (; next < total; next += stride) {
+    int64_t pos = a.reverse ? (total - next - C > 0 ? total - next - C : 0) : next;
+    const int64_t stop = a.reverse ? total - next : (next + C < total ? next + C : total);
+    while (pos < stop) {
+      const BatchDev* B;
+      int64_t first = 0, end = stop;
+      int bi = 0;
+      if constexpr (TABLE) {
+        bi = __builtin_amdgcn_readfirstlane(find_batch(s_start, nb, pos));
+        B = a.table->batches + bi;
+        first = B->start;
+        end = first + B->count < stop ? first + B->count : stop;
+      } else {
+        B = &args_again().one;
+      }
+      const int n = (int)(end - pos < 64 ? end - pos : 64);
+      WideLane L;
+      L.cur = kIdle;
+      bool live = lane < n;
+      if (live) {
+        const GRays rays = moved(global_view(B->rays), pos - first);
+        if (rays.masked && rays.masked[lane]) {
+          store_hit(moved(global_view(B->hits), pos - first), lane, -2, -kMaxT, 0.f, 0.f, true);
+          live = false;
+        } else {
+          wide_start<S, BLOCK>(a.sc, reach, rays, (unsigned)lane, (B->flags & 1u) != 0, nested, L,
+                               st);
+        }
+      }
+      while (wave_mask(L.cur != kIdle)) wide_step<PRIM, S, BLOCK>(a.sc, L, a.weight, st);
+      if (live) {
+        const WideArgs& again = args_again();
+        const BatchDev* E = TABLE ? again.table->batches + bi : &again.one;
+        wide_finish<PRIM, S, BLOCK>(again.sc, moved(global_view(E->rays), pos - first),
+                                    moved(global_view(E->hits), pos - first), (unsigned)lane, L,
+                                    st);
+      }
+      pos += n;
+    }
+  }
+}
+
+// Persistent waves over the rays of a table of batches, numbered through, whose idle lanes
+// take the wave's next rays as soon as `refill` of them are idle. A wave takes `chunk` ray
+// numbers at a time: first those at its own place, then by a shared counter, asked ahead of
+// time. The last wave to leave clears the counter, so launches and graph replays need no
+// clearing pass. Five waves a SIMD (80 registers, for six, spill).
+template <int PRIM, int S, int BLOCK>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_wide_lanes(
+    WideArgs a) {
+  __shared__ unsigned long long s_ring[S * BLOCK];
+  extern __shared__ int64_t s_start[];  // nb entries (dynamic LDS)
+  const int tid = threadIdx.x, lane = tid & 63;
+  // The dynamic LDS holds a.nb offsets; a table with more entries is cut to that.
+  const BatchTable* table = a.table;
+  const int nb = table->nb < a.nb ? table->nb : a.nb;
+  const BatchDev* batches = table->batches;
+  const int64_t total =
+      nb == table->nb ? table->total : batches[nb - 1].start + batches[nb - 1].count;
+  for (int i = tid; i < nb; i += BLOCK) s_start[i] = batches[i].start;
+  __syncthreads();
+  int blk = blockIdx.x;
+  if (a.remap && (gridDim.x & 7) == 0) blk = (blk & 7) * (gridDim.x >> 3) + (blk >> 3);
+  const int64_t n_waves = (int64_t)gridDim.x * (BLOCK / 64);
+  const int64_t wave_id = (int64_t)blk * (BLOCK / 64) + __builtin_amdgcn_readfirstlane(tid >> 6);
+  WideStack<S, BLOCK> st(s_ring, a.spill, a.spill_stride, (int64_t)blockIdx.x * BLOCK + tid, tid);
+  const DevScene& sc = a.sc;
+  const float reach = root_reach(sc);
   const bool nested = *sc.irregular == 0;
 
   int64_t C = a.chunk;
@@ -407,16 +513,12 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5, 8))) v
   // Runs fn(rays, hits, flags, start) for the lanes of `who`, batch by batch (nearly always
   // one), so that a batch's record is read by scalar loads.
   auto by_batch = [&](bool who, auto fn) {
-    if constexpr (!TABLE) {
-      if (who) fn(global_view(a.one.rays), global_view(a.one.hits), a.one.flags);
-    } else {
-      for (unsigned long long todo = wave_mask(who); todo;) {
-        const int b = __builtin_amdgcn_readlane(bi, __builtin_ctzll(todo));
-        const unsigned long long m = wave_mask(bi == b) & todo;
-        const BatchDev& B = batches[b];
-        if (lane_bit(m)) fn(global_view(B.rays), global_view(B.hits), B.flags);
-        todo &= ~m;
-      }
+    for (unsigned long long todo = wave_mask(who); todo;) {
+      const int b = __builtin_amdgcn_readlane(bi, __builtin_ctzll(todo));
+      const unsigned long long m = wave_mask(bi == b) & todo;
+      const BatchDev& B = batches[b];
+      if (lane_bit(m)) fn(global_view(B.rays), global_view(B.hits), B.flags);
+      todo &= ~m;
     }
   };
 
@@ -441,21 +543,15 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5, 8))) v
       if (pos >= end) {
         pos = a.reverse ? (total - next - C > 0 ? total - next - C : 0) : next;
         end = a.reverse ? total - next : (next + C < total ? next + C : total);
-        if (a.ctr) {
-          if (lane == 0) ahead = atomicAdd(a.ctr, (unsigned long long)C);
-          asked = true;
-        } else {
-          next += n_waves * C;
-        }
+        if (lane == 0) ahead = atomicAdd(a.ctr, (unsigned long long)C);
+        asked = true;
       }
       const int64_t g = pos + __popcll(idle & ((1ull << lane) - 1ull));
       const bool take = lane_bit(idle) && g < end;
-      int64_t i = g;
-      if constexpr (TABLE) {
-        if (take) {
-          bi = find_batch(s_start, nb, g);
-          i = g - s_start[bi];
-        }
+      int64_t i = 0;
+      if (take) {
+        bi = find_batch(s_start, nb, g);
+        i = g - s_start[bi];
       }
       by_batch(take, [&](const GRays& rays, const GHits& hits, uint32_t flags) {
         if (rays.masked && rays.masked[i]) {
@@ -469,7 +565,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5, 8))) v
     }
     wide_step<PRIM, S, BLOCK>(sc, L, a.weight, st);
   }
-  if (a.ctr && lane == 0) {
+  if (lane == 0) {
     const unsigned long long left = atomicAdd(a.ctr + 1, 1ull);
     if (left == (unsigned long long)n_waves - 1) {
       atomicExch(a.ctr, 0ull);
@@ -480,16 +576,22 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5, 8))) v
 
 namespace {
 
-template <int PRIM, int BLOCK, bool TABLE>
-int launch_wide(const DevScene& sc, const WideArgs& a, int blocks, int stack_lds, hipStream_t s) {
-  const dim3 g(blocks), b(BLOCK);
-  const size_t lds = TABLE ? sizeof(int64_t) * (size_t)a.nb : 0;  // batch start offsets
-  if (stack_lds == 8)
-    hipLaunchKernelGGL((k_trace_wide<PRIM, 8, BLOCK, TABLE>), g, b, lds, s, sc, a);
-  else if (stack_lds == 32)
-    hipLaunchKernelGGL((k_trace_wide<PRIM, 32, BLOCK, TABLE>), g, b, lds, s, sc, a);
+template <int PRIM, int S, int BLOCK>
+void launch_table(const WideArgs& a, dim3 g, hipStream_t s) {
+  const size_t lds = sizeof(int64_t) * (size_t)a.nb;  // batch start offsets
+  if (a.ctr)
+    hipLaunchKernelGGL((k_wide_lanes<PRIM, S, BLOCK>), g, dim3(BLOCK), lds, s, a);
   else
-    hipLaunchKernelGGL((k_trace_wide<PRIM, 16, BLOCK, TABLE>), g, b, lds, s, sc, a);
+    hipLaunchKernelGGL((k_wide_whole<PRIM, S, BLOCK, true>), g, dim3(BLOCK), lds, s, a);
+}
+template <int PRIM, int BLOCK>
+int launch_table(const WideArgs& a, dim3 g, int stack_lds, hipStream_t s) {
+  if (stack_lds == 8)
+    launch_table<PRIM, 8, BLOCK>(a, g, s);
+  else if (stack_lds == 32)
+    launch_table<PRIM, 32, BLOCK>(a, g, s);
+  else
+    launch_table<PRIM, 16, BLOCK>(a, g, s);
   return (int)hipGetLastError();
 }
 
@@ -505,6 +607,7 @@ constexpr int kChunkRefill = 40;
 template <int PRIM>
 int launch_wide_table(const DevScene& sc, const BatchLaunch& bl, hipStream_t s) {
   WideArgs a{};
+  a.sc = sc;
   a.table = bl.table;
   a.ctr = bl.chunk == 0 ? nullptr : bl.counters;
   a.spill = reinterpret_cast<unsigned long long*>(bl.spill);
@@ -516,22 +619,30 @@ int launch_wide_table(const DevScene& sc, const BatchLaunch& bl, hipStream_t s) 
   a.remap = bl.xcd_remap;
   a.reverse = bl.reverse;
   a.weight = kLeafWeight;
-  if (bl.block == 64) return launch_wide<PRIM, 64, true>(sc, a, bl.blocks, bl.stack_lds, s);
-  if (bl.block == 128) return launch_wide<PRIM, 128, true>(sc, a, bl.blocks, bl.stack_lds, s);
-  return launch_wide<PRIM, 256, true>(sc, a, bl.blocks, bl.stack_lds, s);
+  const dim3 g(bl.blocks);
+  if (bl.block == 64) return launch_table<PRIM, 64>(a, g, bl.stack_lds, s);
+  if (bl.block == 128) return launch_table<PRIM, 128>(a, g, bl.stack_lds, s);
+  return launch_table<PRIM, 256>(a, g, bl.stack_lds, s);
 }
 
 template <int PRIM>
 int launch_wide_one(const DevScene& sc, const BatchDev& rays, const LaunchCfg& cfg, hipStream_t s) {
   WideArgs a{};
+  a.sc = sc;
   a.one = rays;
   a.spill = reinterpret_cast<unsigned long long*>(cfg.spill);
   a.spill_stride = cfg.spill_stride;
-  a.refill = 64;
   a.chunk = cfg.chunk;
   a.reverse = 1;
   a.weight = kLeafWeight;
-  return launch_wide<PRIM, 64, false>(sc, a, cfg.blocks, cfg.stack_lds, s);
+  const dim3 g(cfg.blocks), b(64);
+  if (cfg.stack_lds == 8)
+    hipLaunchKernelGGL((k_wide_whole<PRIM, 8, 64, false>), g, b, 0, s, a);
+  else if (cfg.stack_lds == 32)
+    hipLaunchKernelGGL((k_wide_whole<PRIM, 32, 64, false>), g, b, 0, s, a);
+  else
+    hipLaunchKernelGGL((k_wide_whole<PRIM, 16, 64, false>), g, b, 0, s, a);
+  return (int)hipGetLastError();
 }
 
 }  // namespace
