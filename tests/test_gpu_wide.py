@@ -1,0 +1,186 @@
+"""The four-wide traversal against the oracle where it can go wrong: set sizes around the
+waves' chunks, direction components of zero, rays outside its bounds, leaf sizes around the
+two triangles of a step and the inline leaf count, trees whose boxes do not nest or whose
+leaves overlap, and refits that meet or leave a vertex that is not a number. Results equal
+the oracle's one-ray packets bit for bit (closest hit) or in flag and triangle (any hit)."""
+
+import numpy as np
+import pytest
+
+from rfmanta_amd import _lib as L
+from rfmanta_amd import api, scenes
+
+pytestmark = pytest.mark.gpu
+
+
+def _bits(a):
+    return np.asarray(a, np.float32).view(np.uint32)
+
+
+def _check(oracle, scene, v, i, nodes, ids, rays, what, **kw):
+    for any_hit in (False, True):
+        o = oracle.trace(v, i, nodes, ids, rays, packet_size=1, any_hit=any_hit, **kw)
+        g = scene.trace_host(rays, any_hit=any_hit, packet_size=1)
+        assert np.array_equal(g["prim"], o["prim"]), (what, any_hit)
+        if any_hit:
+            assert np.array_equal(g["occluded"], o["occluded"]), what
+        else:
+            for k in ("t", "u", "v"):
+                assert np.array_equal(_bits(g[k]), _bits(o[k])), (what, k)
+
+
+def _take(rays, n):
+    return {k: np.ascontiguousarray(rays[k][:n]) for k in api.RAY_FIELDS}
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 63, 64, 65, 1023, 4097, 65537])
+def test_set_sizes(oracle, n):
+    v, i = scenes.heightfield(60, 40, seed=9)
+    nodes, ids, _ = oracle.build_bvh(v, i)
+    rays = scenes.random_rays(n, 5, (-1, -0.3, -0.7), (1, 0.6, 0.7))
+    with api.Scene(v, i) as s:
+        s.load_dynbvh(ids, nodes)
+        _check(oracle, s, v, i, nodes, ids, rays, n)
+
+
+def _odd_rays(n=640):
+    """Rays with zero components of both signs, tiny and huge directions, origins on box
+    planes, infinite and absent tmax, and components that are not finite."""
+    r = scenes.random_rays(n, 11, (-1.2, -0.5, -1.2), (1.2, 0.5, 1.2))
+    k = np.arange(n)
+    f = np.float32
+    for a, c in enumerate(("dx", "dy", "dz")):
+        r[c][k % 16 == a] = f(0.0)
+        r[c][k % 16 == 3 + a] = f(-0.0)
+    for c in ("dx", "dy", "dz"):
+        r[c][k % 16 == 6] *= f(1e-30)
+        r[c][k % 16 == 7] *= f(1e25)
+    r["dx"][k % 16 == 8] *= f(1e-20)
+    two = k % 16 == 9
+    r["dx"][two], r["dz"][two] = f(0.0), f(0.0)
+    r["ox"][two] = np.round(r["ox"][two] * 8) / 8
+    r["tmax"][k % 16 == 10] = np.inf
+    r["dx"][k % 32 == 10] = f(0.0)
+    r["tmax"][k % 16 == 11] = f(0.3)
+    r["ox"][k % 16 == 12] = f(1e6)
+    bad = k % 16 == 13
+    r["oy"][bad] = np.where(k[bad] % 32 < 16, f(np.nan), f(np.inf))
+    r["dy"][k % 16 == 14] = f(np.inf)
+    r["tmax"][k % 16 == 15] = np.where(k[k % 16 == 15] % 32 < 16, f(np.nan), f(-1.0))
+    return r
+
+
+@pytest.mark.parametrize("mesh", ["soup", "heightfield", "grid"])
+def test_odd_rays(oracle, mesh):
+    if mesh == "soup":
+        v, i = scenes.soup(700, seed=2, sigma=0.1)
+    else:
+        v, i = scenes.heightfield(17, 17, seed=2)
+        if mesh == "grid":  # flat boxes, vertices on binary fractions
+            v[:, 1] = 0
+    nodes, ids, _ = oracle.build_bvh(v, i)
+    with api.Scene(v, i) as s:
+        s.load_dynbvh(ids, nodes)
+        _check(oracle, s, v, i, nodes, ids, _odd_rays(), mesh)
+
+
+def _chain_of_leaves(oracle, v, i, sizes):
+    """A tree whose inner records each hold one leaf of the next size and the rest."""
+    T = len(i)
+    ids = np.arange(T, dtype=np.int32)
+    tri = v[i.astype(np.int64)]
+    lo, hi = tri.min(1), tri.max(1)
+    off = np.concatenate([[0], np.cumsum(sizes)])
+    m = len(sizes)
+    nodes = np.zeros(2 * T, oracle.NODE_DTYPE)
+
+    def leaf(r, k):
+        a, b = off[k], off[k + 1]
+        nodes[r]["lo"], nodes[r]["hi"] = lo[a:b].min(0), hi[a:b].max(0)
+        nodes[r]["child"], nodes[r]["children"] = a, sizes[k]
+
+    for k in range(m - 1):
+        r = 2 * k
+        nodes[r]["lo"], nodes[r]["hi"] = lo[off[k]:].min(0), hi[off[k]:].max(0)
+        nodes[r]["child"], nodes[r]["axis"] = 2 * k + 1, k % 3
+        leaf(2 * k + 1, k)
+    leaf(2 * (m - 1), m - 1)
+    return nodes, ids
+
+
+def test_leaf_sizes(oracle):
+    sizes = [1, 2, 3, 4, 5, 13, 14, 15, 16, 17, 31, 1, 2]
+    v, i = scenes.soup(sum(sizes), seed=8, sigma=0.3)
+    nodes, ids = _chain_of_leaves(oracle, v, i, sizes)
+    rays = scenes.random_rays(3000, 4, (-1, -1, -1), (1, 1, 1))
+    with api.Scene(v, i) as s:
+        s.load_dynbvh(ids, nodes)
+        _check(oracle, s, v, i, nodes, ids, rays, "chain")
+
+
+@pytest.mark.parametrize("how", ["not nested", "overlapping"])
+def test_trees_that_take_the_reference_steps(oracle, how):
+    v, i = scenes.heightfield(24, 16, seed=6)
+    nodes, ids, nn = oracle.build_bvh(v, i)
+    nodes = nodes.copy()
+    if how == "not nested":  # inner boxes shrunk: what they cut off is never visited
+        inner = np.nonzero(nodes["children"][:nn] == 0)[0][1::3]
+        nodes["hi"][inner, 0] -= np.float32(0.02)
+    else:  # a leaf that also holds its neighbour's first triangle
+        leaves = [r for r in range(nn) if nodes[r]["children"] > 0]
+        a = next(r for r in leaves if nodes[r]["child"] + nodes[r]["children"] < len(i))
+        nodes["children"][a] += 1
+    rays = scenes.random_rays(4000, 3, (-1, 0.1, -0.7), (1, 0.6, 0.7))
+    with api.Scene(v, i) as s:
+        s.load_dynbvh(ids, nodes)
+        _check(oracle, s, v, i, nodes, ids, rays, how)
+
+
+def test_refit_with_a_vertex_that_is_not_a_number(oracle):
+    v, i = scenes.heightfield(40, 30, seed=3)
+    nodes, ids, _ = oracle.build_bvh(v, i)
+    rays = scenes.random_rays(5000, 7, (-1, -0.2, -0.7), (1, 0.6, 0.7))
+    with api.Scene(v, i) as s:
+        s.load_dynbvh(ids, nodes)
+        for value in (np.nan, 0.05):
+            vd = v.copy()
+            vd[600, 1] = value
+            s.set_vertices(vd)
+            s.refit()
+            api.sync()
+            gi, gn = s.export_dynbvh()
+            if not np.isnan(value):
+                ref = nodes.copy()
+                oracle.refit(vd, i, ref, ids)
+                assert gn.tobytes() == ref.tobytes()
+            # the tree as it stands on the device, box for box
+            _check(oracle, s, vd, i, gn, gi, rays, value)
+
+
+@pytest.mark.parametrize("batches", [1, 3])
+def test_frames_of_zero_components_and_short_chunks(oracle, batches):
+    v, i = scenes.heightfield(50, 30, seed=5)
+    nodes, ids, _ = oracle.build_bvh(v, i)
+    sets = [_odd_rays(640)] + [scenes.random_rays(n, n, (-1, -0.2, -0.7), (1, 0.5, 0.7))
+                               for n in (1, 777)]
+    kinds = [False, True, False]
+    with api.Scene(v, i) as s:
+        s.load_dynbvh(ids, nodes)
+        dev = [(api.DeviceRays.upload(r), api.DeviceHits.alloc(len(r["ox"]), any_hit=a), a)
+               for r, a in list(zip(sets, kinds))[:batches]]
+        f = api.Frame(s, dev)
+        for refill, chunk in ((64, 0), (64, 64), (64, 256), (24, 64)):
+            for rev in (0, 1):
+                f.set_config(dict(layout=L.MH_LAYOUT_PAIR, stack_lds=8, block=64, blocks_per_cu=1,
+                                  refill=refill, chunk=chunk, reverse=rev))
+                for _, dh, _ in dev:
+                    dh.arrays["prim"].upload(np.full(dh.n, 777, np.int32))
+                f.launch()
+                api.sync()
+                for (_, dh, a), r in zip(dev, sets):
+                    o = oracle.trace(v, i, nodes, ids, r, packet_size=1, any_hit=a)
+                    g = dh.download()
+                    assert np.array_equal(g["prim"], o["prim"]), (refill, chunk, rev)
+                    if not a:
+                        assert np.array_equal(_bits(g["t"]), _bits(o["t"])), (refill, chunk, rev)
+        f.close()
