@@ -65,18 +65,9 @@ __device__ __forceinline__ void set_box(RefNode& n, const Box& b) {
     n.box.hi[k] = b.hi[k];
   }
 }
-// Object box: from u.obox when the caller filled it (k_obj_bounds), else from the
-// triangle's vertices with the same arithmetic (Mesh::getBBox, Model/Groups/Mesh.cc:228-237).
+// Object box, from the triangle's vertices (Mesh::getBBox, Model/Groups/Mesh.cc:228-237).
 __device__ __forceinline__ Box obj_box(const DevUpdate& u, int obj) {
   Box b;
-  if (u.obox) {
-    const float* p = u.obox + 6 * (size_t)obj;
-    for (int k = 0; k < 3; ++k) {
-      b.lo[k] = p[k];
-      b.hi[k] = p[3 + k];
-    }
-    return b;
-  }
   const uint32_t* t = u.idx + 3 * (size_t)obj;
   const float* p0 = u.verts + 3 * (size_t)t[0];
   for (int k = 0; k < 3; ++k) b.lo[k] = b.hi[k] = p0[k];
@@ -88,9 +79,7 @@ __device__ __forceinline__ Box obj_box(const DevUpdate& u, int obj) {
 __device__ __forceinline__ float box_cen(const Box& b, int axis) {
   return b.hi[axis] * 0.5f + b.lo[axis] * (1 - 0.5f);
 }
-// Object centroid: from u.ocen when filled, else from the object box.
 __device__ __forceinline__ float obj_cen(const DevUpdate& u, int obj, int axis) {
-  if (u.ocen) return u.ocen[3 * (size_t)obj + axis];
   return box_cen(obj_box(u, obj), axis);
 }
 // Vector::indexOfMaxComponent (Core/Geometry/Vector.h:382-393)
@@ -181,12 +170,8 @@ __device__ inline SplitChoice approx_choice(const DevUpdate& u, const Box& node_
   reset(cb);
   for (int i = b; i < e; ++i) {
     float c[3];
-    if (u.ocen) {
-      for (int k = 0; k < 3; ++k) c[k] = u.ocen[3 * (size_t)ids[i] + k];
-    } else {
-      const Box ob = obj_box(u, ids[i]);
-      for (int k = 0; k < 3; ++k) c[k] = box_cen(ob, k);
-    }
+    const Box ob = obj_box(u, ids[i]);
+    for (int k = 0; k < 3; ++k) c[k] = box_cen(ob, k);
     extend_pt(cb, c);
   }
   const float inv_parent_area = (float)(1.0 / (double)area(node_box));
@@ -204,7 +189,7 @@ __device__ inline SplitChoice approx_choice(const DevUpdate& u, const Box& node_
   }
   for (int i = b; i < e; ++i) {
     const Box ob = obj_box(u, ids[i]);
-    const float cen = u.ocen ? u.ocen[3 * (size_t)ids[i] + axis] : box_cen(ob, axis);
+    const float cen = box_cen(ob, axis);
     const float f = (cen - cb.lo[axis]) * scale;
     // int(f) as the reference's x86 build converts it (cvttss2si): NaN and values outside
     // the int range give INT_MIN, i.e. bin 0 after the clamp.

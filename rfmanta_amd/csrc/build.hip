@@ -9,19 +9,21 @@
 // node are a contiguous range of slots; each slot carries its object's centroid, id and
 // box (48 bytes, moved with the id), so every pass streams. A level's nodes are cut into
 // virtual blocks of kVB slots; per level:
-//   k_cbounds      centroid box of each node          (block reduce, then global atomics)
-//   k_seg_axis     longest centroid axis, bin scale   (one lane per node)
+//   k_level_open   node of each virtual block, accumulators cleared
 //   k_bins         16 bins: counts and boxes
-//   k_seg_split    the binned SAH sweep: split position or leaf
-//   k_count_less   objects left of the position
-//   k_seg_mid      split slot, or the middle when everything fell on one side
+//   k_seg_split    the binned SAH sweep: split position or leaf (16 lanes per node)
+//   k_count_less   objects left of the position; from their number the split slot, or the
+//                  middle when everything fell on one side (seg_mid)
 //   k_mis_count, k_scan_mis, k_mis_scatter, k_swap   partitionObjects
-//   k_child_bounds boxes of the two sides
+//   k_child_bounds boxes and centroid boxes of the two sides
 //   k_seg_children new record pair, child nodes to the next level or to phase 2
+// The node count of a level stays on the device; the host only bounds it (2^level at most).
 // Reductions must give what the reference's serial loops give. Its min/max are select
 // forms (a < b ? a : b) applied in slot order, so of equal values (+0 and -0) the last one
-// wins; each value is reduced as a 64-bit key (order-preserving value bits, then the slot
-// number) with integer atomics, which makes the result exact and independent of order.
+// wins; the values that records keep are reduced as 64-bit keys (order-preserving value
+// bits, then the slot number) with integer atomics, which makes the result exact and
+// independent of order. Bin and centroid boxes only feed differences and comparisons, where
+// the sign of a zero makes no difference, and are reduced as 32-bit keys.
 // partitionObjects (Hoare's scheme) exchanges the k-th slot from the left whose key is on
 // the right side with the k-th slot from the right whose key is on the left side; the
 // ranks come from a scan, and the exchanges are independent.
@@ -33,6 +35,7 @@
 
 #include <cfloat>
 #include <climits>
+#include <vector>
 
 #include "approx_sah.h"
 #include "mh_device.h"
@@ -46,7 +49,7 @@ constexpr int kPer = kBuildVB / kBlock;
 constexpr int kVB = kBuildVB;
 constexpr int kBins = kSamples;
 static_assert(kBins == kBuildBins, "bins");
-constexpr unsigned long long kMinInit = ~0ull;
+constexpr int kSetupVB = 2048;  // objects or vertices a workgroup of the set-up passes
 
 // 32-bit key that orders floats as numbers, with -0 and +0 equal.
 __device__ __forceinline__ uint32_t ord(float f) {
@@ -58,17 +61,54 @@ __device__ __forceinline__ float unord(uint32_t e) {
   return __uint_as_float((e & 0x80000000u) ? (e & 0x7FFFFFFFu) : ~e);
 }
 constexpr uint32_t kOrdZero = 0x80000000u;
-// min: smallest value, then the largest slot; max: largest value, then the largest slot.
+// Smallest value, then the largest slot. Maxima are minima of the negated values.
 __device__ __forceinline__ unsigned long long kmin(float v, uint32_t slot) {
   return ((unsigned long long)ord(v) << 32) | (0xFFFFFFFFu - slot);
-}
-__device__ __forceinline__ unsigned long long kmax(float v, uint32_t slot) {
-  return ((unsigned long long)ord(v) << 32) | slot;
 }
 __device__ __forceinline__ uint32_t kmin_slot(unsigned long long k) {
   return 0xFFFFFFFFu - (uint32_t)k;
 }
-__device__ __forceinline__ uint32_t kmax_slot(unsigned long long k) { return (uint32_t)k; }
+
+template <int kCtrl>
+__device__ __forceinline__ float dpp_mov(float x) {
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_int(x), kCtrl, 0xF, 0xF, true));
+}
+template <int kCtrl, int kRows>
+__device__ __forceinline__ int dpp_or_own(int x) {
+  return __builtin_amdgcn_update_dpp(x, x, kCtrl, kRows, 0xF, false);
+}
+// Smallest of the wave's values, by row shifts and row broadcasts, in every lane.
+template <int kCtrl, int kRows>
+__device__ __forceinline__ uint32_t umin_step(uint32_t x) {
+  const uint32_t t = (uint32_t)dpp_or_own<kCtrl, kRows>((int)x);
+  return t < x ? t : x;
+}
+__device__ __forceinline__ uint32_t wave_umin(uint32_t x) {
+  x = umin_step<0x111, 0xF>(x);
+  x = umin_step<0x112, 0xF>(x);
+  x = umin_step<0x114, 0xF>(x);
+  x = umin_step<0x118, 0xF>(x);
+  x = umin_step<0x142, 0xA>(x);
+  x = umin_step<0x143, 0xC>(x);
+  return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+}
+// A lane's smallest value, the later of equal ones; slots come in ascending order.
+struct MinSlot {
+  float v = FLT_MAX;
+  uint32_t at = 0;
+  __device__ __forceinline__ void take(float x, uint32_t slot) {
+    at = x <= v ? slot : at;
+    v = x <= v ? x : v;
+  }
+};
+// The wave's key: the slot only matters where the value is a zero (key_value).
+__device__ __forceinline__ unsigned long long wave_kmin(const MinSlot& m) {
+  const uint32_t o = ord(m.v), least = wave_umin(o);
+  uint32_t inv = 0;
+  if (least == kOrdZero) inv = wave_umin(o == kOrdZero ? 0xFFFFFFFFu - m.at : 0xFFFFFFFFu);
+  return ((unsigned long long)least << 32) | inv;
+}
 
 // Slot record: centroid, object id, box.
 struct alignas(16) Slot {
@@ -104,25 +144,68 @@ __device__ __forceinline__ float slot_c(const Slot* s, int64_t i, int a) {
 // The level node that owns virtual block v.
 __device__ __forceinline__ int find_seg(const DevBuild& d, int64_t v) { return d.vbseg[v]; }
 
+// Boxes are held as six minima (lo, -hi); negating is exact.
+__device__ __forceinline__ Box min_box(const float* m) {
+  Box b;
+  for (int a = 0; a < 3; ++a) {
+    b.lo[a] = m[a];
+    b.hi[a] = -m[3 + a];
+  }
+  return b;
+}
+
 struct VRange {
   int s;
   int64_t first, end;  // slots of this virtual block
 };
 __device__ __forceinline__ bool vrange(const DevBuild& d, VRange& r) {
   const int64_t v = blockIdx.x;
-  if (v >= (int64_t)d.ctr[kCtrNvb]) return false;
-  r.s = find_seg(d, v);
+  if (v >= (int64_t)d.ctr[kCtrNvb + d.level]) return false;
+  r.s = d.vbseg[v];
   const BuildSeg sg = d.seg[r.s];
   r.first = sg.b + (v - sg.vb0) * (int64_t)kVB;
   r.end = r.first + kVB < sg.e ? r.first + kVB : sg.e;
   return true;
 }
+__device__ __forceinline__ int n_segs(const DevBuild& d) { return (int)d.ctr[kCtrSegs + d.level]; }
 
-__device__ __forceinline__ unsigned long long& K(const DevBuild& d, int f, int s) {
-  return d.acck[(int64_t)f * d.cap + s];
+// Accumulators of a level node (kAcc*).
+__device__ __forceinline__ unsigned* acc(const DevBuild& d, int s) {
+  return d.acc + (int64_t)s * kAccWords;
 }
-__device__ __forceinline__ unsigned& Cn(const DevBuild& d, int f, int s) {
-  return d.accc[(int64_t)f * d.cap + s];
+__device__ __forceinline__ unsigned long long* acc_box(const DevBuild& d, int s) {
+  return reinterpret_cast<unsigned long long*>(acc(d, s));
+}
+// Split slot of a node and whether slots move (not in the middle fallback): when 0 or all
+// objects lie left of the position, partitionObjects moves nothing and the reference
+// splits at the middle (DynBVH.cc:2250-2261).
+__device__ __forceinline__ int seg_mid(const DevBuild& d, int s, const BuildSeg& sg, bool& moves) {
+  const int n = sg.e - sg.b, m = (int)acc(d, s)[kAccLess];
+  moves = m != 0 && m != n;
+  return moves ? sg.b + m : sg.b + n / 2;
+}
+// Value of a reduced key; a zero is read back from the winning slot for its sign.
+__device__ __forceinline__ float key_value(unsigned long long k, const float* slots, int stride,
+                                           int field, bool negated) {
+  const uint32_t o = (uint32_t)(k >> 32);
+  if (o == kOrdZero) return slots[(int64_t)kmin_slot(k) * stride + field];
+  return negated ? -unord(o) : unord(o);
+}
+
+// The binning of a node with centroid box keys c (three minima, three negated maxima):
+// its longest axis (BBox::longestAxis), start, width and scale.
+__device__ __forceinline__ BuildPlan make_plan(const unsigned* c) {
+  BuildPlan p{};
+  float lo[3], w[3];
+  for (int a = 0; a < 3; ++a) {
+    lo[a] = unord(c[a]);
+    w[a] = -unord(c[3 + a]) - lo[a];
+  }
+  p.axis = index_of_max(w[0], w[1], w[2]);
+  p.width = p.axis == 0 ? w[0] : (p.axis == 1 ? w[1] : w[2]);
+  p.lo_c = p.axis == 0 ? lo[0] : (p.axis == 1 ? lo[1] : lo[2]);
+  p.scale = ((float)kBins / p.width) * .999f;
+  return p;
 }
 
 // ---------------------------------------------------------------------------------------
@@ -132,44 +215,69 @@ __device__ __forceinline__ unsigned& Cn(const DevBuild& d, int f, int s) {
 // coordinate sets err = 2.
 __global__ __launch_bounds__(kBlock) void k_root_box(DevBuild d) {
   __shared__ unsigned long long sk[6];
-  if (threadIdx.x < 6) sk[threadIdx.x] = threadIdx.x < 3 ? kMinInit : 0ull;
+  if (threadIdx.x < 6) sk[threadIdx.x] = ~0ull;
   __syncthreads();
-  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (i < d.n_verts) {
+  const int64_t first = (int64_t)blockIdx.x * kSetupVB;
+  MinSlot m[6];
+  bool bad = false;
+  for (int k = 0; k < kSetupVB / kBlock; ++k) {
+    int64_t i = first + k * kBlock + threadIdx.x;
+    i = i < d.n_verts ? i : d.n_verts - 1;
     for (int a = 0; a < 3; ++a) {
       const float x = d.verts[3 * i + a];
-      if (!(x >= -FLT_MAX && x <= FLT_MAX)) atomicExch(d.u.err, 2);
-      atomicMin(&sk[a], kmin(x, (uint32_t)i));
-      atomicMax(&sk[3 + a], kmax(x, (uint32_t)i));
+      bad |= !(x >= -FLT_MAX && x <= FLT_MAX);
+      m[a].take(x, (uint32_t)i);
+      m[3 + a].take(-x, (uint32_t)i);
     }
   }
+  if (__ballot(bad) && (threadIdx.x & 63) == 0) atomicExch(d.u.err, 2);
+  for (int k = 0; k < 6; ++k) {
+    const unsigned long long key = wave_kmin(m[k]);
+    if ((threadIdx.x & 63) == 0) atomicMin(&sk[k], key);
+  }
   __syncthreads();
-  if (threadIdx.x < 3) atomicMin(&d.rootk[threadIdx.x], sk[threadIdx.x]);
-  if (threadIdx.x >= 3 && threadIdx.x < 6) atomicMax(&d.rootk[threadIdx.x], sk[threadIdx.x]);
+  if (threadIdx.x < 6) atomicMin(&d.rootk[threadIdx.x], sk[threadIdx.x]);
 }
 
-// Slot records from the object boxes and centroids (in object order, as object_ids
-// starts out).
+// Slot records, in object order as object_ids starts out: object box (Mesh::getBBox,
+// Mesh.cc:228-237) and centroid (BBox::center, BBox.h:63-65), and the box of the centroids.
 __global__ __launch_bounds__(kBlock) void k_slots(DevBuild d) {
-  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (i >= d.u.n_objects) return;
-  const float* b = d.u.obox + 6 * i;
-  const float* c = d.u.ocen + 3 * i;
-  float4* p = reinterpret_cast<float4*>(SL(d) + i);
-  p[0] = make_float4(c[0], c[1], c[2], __int_as_float((int)i));
-  p[1] = make_float4(b[0], b[1], b[2], b[3]);
-  p[2] = make_float4(b[4], b[5], 0.f, 0.f);
+  __shared__ unsigned sc[6];
+  if (threadIdx.x < 6) sc[threadIdx.x] = ~0u;
+  __syncthreads();
+  const int64_t first = (int64_t)blockIdx.x * kSetupVB;
+  uint32_t least[6];
+  for (int k = 0; k < 6; ++k) least[k] = ~0u;
+  for (int k = 0; k < kSetupVB / kBlock; ++k) {
+    const int64_t i = first + k * kBlock + threadIdx.x;
+    if (i >= d.u.n_objects) break;
+    const Box b = obj_box(d.u, (int)i);
+    float c[3];
+    for (int a = 0; a < 3; ++a) {
+      c[a] = box_cen(b, a);
+      const uint32_t lo = ord(c[a]), hi = ord(-c[a]);
+      least[a] = lo < least[a] ? lo : least[a];
+      least[3 + a] = hi < least[3 + a] ? hi : least[3 + a];
+    }
+    float4* p = reinterpret_cast<float4*>(SL(d) + i);
+    p[0] = make_float4(c[0], c[1], c[2], __int_as_float((int)i));
+    p[1] = make_float4(b.lo[0], b.lo[1], b.lo[2], b.hi[0]);
+    p[2] = make_float4(b.hi[1], b.hi[2], 0.f, 0.f);
+  }
+  for (int k = 0; k < 6; ++k) {
+    const uint32_t x = wave_umin(least[k]);
+    if ((threadIdx.x & 63) == 0) atomicMin(&sc[k], x);
+  }
+  __syncthreads();
+  if (threadIdx.x < 6) atomicMin(&d.rootc[threadIdx.x], sc[threadIdx.x]);
 }
 
 // Record 0 gets the vertex box; the root becomes the first node of phase 1 or 2.
 __global__ void k_root_init(DevBuild d, int serial) {
   RefNode& r = d.u.refs[0];
   for (int a = 0; a < 3; ++a) {
-    const unsigned long long kl = d.rootk[a], kh = d.rootk[3 + a];
-    r.box.lo[a] = (uint32_t)(kl >> 32) == kOrdZero ? d.verts[3 * (int64_t)kmin_slot(kl) + a]
-                                                   : unord((uint32_t)(kl >> 32));
-    r.box.hi[a] = (uint32_t)(kh >> 32) == kOrdZero ? d.verts[3 * (int64_t)kmax_slot(kh) + a]
-                                                   : unord((uint32_t)(kh >> 32));
+    r.box.lo[a] = key_value(d.rootk[a], d.verts, 3, a, false);
+    r.box.hi[a] = key_value(d.rootk[3 + a], d.verts, 3, a, true);
   }
   r.child = 0;
   r.children = 0;
@@ -182,112 +290,28 @@ __global__ void k_root_init(DevBuild d, int serial) {
     d.ctr[kCtrSmall] = 1;
   } else {
     d.seg[0] = root;
+    d.plan[0] = make_plan(d.rootc);
+    d.ctr[kCtrSegs] = 1;
+    d.ctr[kCtrNvb] = (unsigned)((d.u.n_objects + kVB - 1) / kVB);
   }
 }
 
 // ---------------------------------------------------------------------------------------
 // Phase 1: one level
 
-__global__ __launch_bounds__(kBlock) void k_acc_clear(DevBuild d) {
-  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  const int64_t nk = (int64_t)kKeyFields * d.nseg;
-  if (i < nk) {
-    const int f = (int)(i / d.nseg), s = (int)(i % d.nseg);
-    const bool is_min = (f >= kFcMin && f < kFcMax) || (f >= kFbMin && f < kFbMax) ||
-                        (f >= kFlMin && f < kFlMax) || (f >= kFrMin && f < kFrMax);
-    K(d, f, s) = is_min ? kMinInit : 0ull;
-  } else if (i < nk + (int64_t)kCntFields * d.nseg) {
-    const int64_t j = i - nk;
-    Cn(d, (int)(j / d.nseg), (int)(j % d.nseg)) = 0u;
-  }
-}
-
-// Exclusive prefix of the nodes' virtual block counts (one workgroup).
-__global__ __launch_bounds__(1024) void k_scan_segments(DevBuild d) {
-  __shared__ unsigned part[1024];
-  __shared__ unsigned carry;
-  if (threadIdx.x == 0) carry = 0;
-  __syncthreads();
-  for (int64_t base = 0; base < d.nseg; base += 1024) {
-    const int64_t s = base + threadIdx.x;
-    const unsigned n = s < d.nseg ? (unsigned)((d.seg[s].e - d.seg[s].b + kVB - 1) / kVB) : 0u;
-    part[threadIdx.x] = n;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {  // inclusive scan (Hillis-Steele)
-      const unsigned x = threadIdx.x >= (unsigned)off ? part[threadIdx.x - off] : 0u;
-      __syncthreads();
-      part[threadIdx.x] += x;
-      __syncthreads();
-    }
-    if (s < d.nseg) d.seg[s].vb0 = (int32_t)(carry + part[threadIdx.x] - n);
-    __syncthreads();
-    if (threadIdx.x == 1023) carry += part[1023];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) d.ctr[kCtrNvb] = carry;
-}
-
-// vbseg[v] = the node of virtual block v, for every virtual block of the level.
-__global__ __launch_bounds__(kBlock) void k_vb_map(DevBuild d) {
-  const int s = blockIdx.x * kBlock + threadIdx.x;
-  if (s >= d.nseg) return;
+// vbseg[v] = the node of virtual block v, and cleared accumulators: 16 lanes per node.
+__global__ __launch_bounds__(kBlock) void k_level_open(DevBuild d) {
+  const int s = (int)(((int64_t)blockIdx.x * kBlock + threadIdx.x) >> 4);
+  const int j = threadIdx.x & 15;
+  if (s >= n_segs(d)) return;
   const BuildSeg sg = d.seg[s];
   const int nvb = (sg.e - sg.b + kVB - 1) / kVB;
-  for (int k = 0; k < nvb; ++k) d.vbseg[sg.vb0 + k] = s;
-}
-
-__global__ __launch_bounds__(kBlock) void k_cbounds(DevBuild d) {
-  __shared__ unsigned long long sk[6];
-  VRange r;
-  if (!vrange(d, r)) return;
-  if (threadIdx.x < 6) sk[threadIdx.x] = threadIdx.x < 3 ? kMinInit : 0ull;
-  __syncthreads();
-  unsigned long long mn_[3] = {kMinInit, kMinInit, kMinInit}, mx_[3] = {0ull, 0ull, 0ull};
-  for (int k = 0; k < kPer; ++k) {
-    const int64_t i = r.first + k * kBlock + threadIdx.x;
-    if (i >= r.end) break;
-    for (int a = 0; a < 3; ++a) {
-      const float c = slot_c(SL(d), i, a);
-      const unsigned long long x = kmin(c, (uint32_t)i), y = kmax(c, (uint32_t)i);
-      mn_[a] = x < mn_[a] ? x : mn_[a];
-      mx_[a] = y > mx_[a] ? y : mx_[a];
-    }
+  for (int k = j; k < nvb; k += 16) d.vbseg[sg.vb0 + k] = s;
+  uint4* p = reinterpret_cast<uint4*>(acc(d, s));
+  for (int k = j; k < kAccWords / 4; k += 16) {
+    const unsigned x = 4 * k < kAccCounts ? ~0u : 0u;
+    p[k] = make_uint4(x, x, x, x);
   }
-  for (int a = 0; a < 3; ++a) {
-    atomicMin(&sk[a], mn_[a]);
-    atomicMax(&sk[3 + a], mx_[a]);
-  }
-  __syncthreads();
-  if (threadIdx.x < 3) atomicMin(&K(d, kFcMin + threadIdx.x, r.s), sk[threadIdx.x]);
-  if (threadIdx.x >= 3 && threadIdx.x < 6)
-    atomicMax(&K(d, kFcMax + threadIdx.x - 3, r.s), sk[threadIdx.x]);
-}
-
-// Value of a reduced key; a zero is read back from the winning slot for its sign.
-__device__ __forceinline__ float key_value(unsigned long long k, bool is_min, const Slot* slots,
-                                           int field) {
-  const uint32_t o = (uint32_t)(k >> 32);
-  if (o != kOrdZero) return unord(o);
-  const uint32_t slot = is_min ? kmin_slot(k) : kmax_slot(k);
-  return reinterpret_cast<const float*>(slots + slot)[field];
-}
-
-__global__ __launch_bounds__(kBlock) void k_seg_axis(DevBuild d) {
-  const int s = blockIdx.x * kBlock + threadIdx.x;
-  if (s >= d.nseg) return;
-  float lo[3], hi[3];
-  for (int a = 0; a < 3; ++a) {
-    lo[a] = key_value(K(d, kFcMin + a, s), true, SL(d), a);
-    hi[a] = key_value(K(d, kFcMax + a, s), false, SL(d), a);
-  }
-  BuildPlan p{};
-  const float w0 = hi[0] - lo[0], w1 = hi[1] - lo[1], w2 = hi[2] - lo[2];
-  p.axis = index_of_max(w0, w1, w2);  // BBox::longestAxis
-  const float w = p.axis == 0 ? w0 : (p.axis == 1 ? w1 : w2);
-  p.width = w;
-  p.lo_c = lo[p.axis];
-  p.scale = ((float)kBins / w) * .999f;
-  d.plan[s] = p;
 }
 
 __device__ __forceinline__ int bin_of(float c, float lo_c, float scale) {
@@ -298,95 +322,113 @@ __device__ __forceinline__ int bin_of(float c, float lo_c, float scale) {
   return which < 0 ? 0 : (which > kBins - 1 ? kBins - 1 : which);
 }
 
+// Bins of a virtual block in LDS, four copies by lane (lanes of one bin spread over four
+// words), then one global atomic per value.
 __global__ __launch_bounds__(kBlock) void k_bins(DevBuild d) {
-  __shared__ unsigned cnt[kBins];
-  __shared__ unsigned long long bmn[kBins * 3], bmx[kBins * 3];
+  constexpr int kCopies = 4;
+  __shared__ unsigned least[6 * kBins * kCopies], cnt[kBins * kCopies];
   VRange r;
   if (!vrange(d, r)) return;
-  for (int k = threadIdx.x; k < kBins * 3; k += kBlock) {
-    bmn[k] = kMinInit;
-    bmx[k] = 0ull;
-  }
-  if (threadIdx.x < kBins) cnt[threadIdx.x] = 0;
+  for (int k = threadIdx.x; k < 6 * kBins * kCopies; k += kBlock) least[k] = ~0u;
+  if (threadIdx.x < kBins * kCopies) cnt[threadIdx.x] = 0;
   __syncthreads();
   const BuildPlan p = d.plan[r.s];
+  const int copy = threadIdx.x & (kCopies - 1);
+#pragma unroll
   for (int k = 0; k < kPer; ++k) {
     const int64_t i = r.first + k * kBlock + threadIdx.x;
     if (i >= r.end) break;
     Slot o;
     load_slot(SL(d), i, o);
-    const int w = bin_of(o.c[p.axis], p.lo_c, p.scale);
+    const float cen = p.axis == 0 ? o.c[0] : (p.axis == 1 ? o.c[1] : o.c[2]);
+    const int w = bin_of(cen, p.lo_c, p.scale) * kCopies + copy;
     atomicAdd(&cnt[w], 1u);
     for (int a = 0; a < 3; ++a) {
-      atomicMin(&bmn[3 * w + a], kmin(o.lo[a], (uint32_t)i));
-      atomicMax(&bmx[3 * w + a], kmax(o.hi[a], (uint32_t)i));
+      atomicMin(&least[a * kBins * kCopies + w], ord(o.lo[a]));
+      atomicMin(&least[(3 + a) * kBins * kCopies + w], ord(-o.hi[a]));
     }
   }
   __syncthreads();
-  if (threadIdx.x < kBins * 3) {
-    const int w = threadIdx.x / 3;
-    if (cnt[w]) {
-      atomicMin(&K(d, kFbMin + threadIdx.x, r.s), bmn[threadIdx.x]);
-      atomicMax(&K(d, kFbMax + threadIdx.x, r.s), bmx[threadIdx.x]);
-      if (threadIdx.x % 3 == 0) atomicAdd(&Cn(d, kFcnt + w, r.s), cnt[w]);
+  if (threadIdx.x < 7 * kBins) {
+    const int w = threadIdx.x & (kBins - 1), f = threadIdx.x / kBins;
+    unsigned n = 0;
+    for (int k = 0; k < kCopies; ++k) n += cnt[w * kCopies + k];
+    if (n) {
+      if (f == 6) {
+        atomicAdd(&acc(d, r.s)[kAccCounts + w], n);
+      } else {
+        unsigned x = ~0u;
+        for (int k = 0; k < kCopies; ++k) {
+          const unsigned y = least[threadIdx.x * kCopies + k];
+          x = y < x ? y : x;
+        }
+        atomicMin(&acc(d, r.s)[kAccBins + threadIdx.x], x);
+      }
     }
   }
 }
 
-// The sweep of partitionApproxSAH (DynBVH.cc:2196-2236) over the reduced bins.
+// The sweep of partitionApproxSAH (DynBVH.cc:2196-2236) over the reduced bins, one lane per
+// bin: a node's 16 lanes are a row, whose scans are row shifts. (One lane per node, with
+// its bins in private memory, took 35 to 50 us a level.)
+template <int kCtrl>
+__device__ __forceinline__ float row_min(float x, bool c) {
+  const float t = dpp_mov<kCtrl>(x);
+  return c && t < x ? t : x;
+}
 __global__ __launch_bounds__(kBlock) void k_seg_split(DevBuild d) {
-  const int s = blockIdx.x * kBlock + threadIdx.x;
-  if (s >= d.nseg) return;
-  BuildPlan p = d.plan[s];
-  const BuildSeg sg = d.seg[s];
+  const int s = (int)(((int64_t)blockIdx.x * kBlock + threadIdx.x) >> 4);
+  const int w = threadIdx.x & 15, lane = threadIdx.x & 63;
+  const bool in = s < n_segs(d);
+  if (!__ballot(in)) return;
+  const int at = in ? s : 0;
+  const BuildSeg sg = d.seg[at];
+  BuildPlan p = d.plan[at];
+  const unsigned* A = acc(d, at);
   const int n = sg.e - sg.b;
-  Box bins[kBins];
-  int counts[kBins];
-  for (int w = 0; w < kBins; ++w) {
-    counts[w] = (int)Cn(d, kFcnt + w, s);
-    if (counts[w] == 0) {
-      reset(bins[w]);
-      continue;
-    }
-    for (int a = 0; a < 3; ++a) {
-      bins[w].lo[a] = key_value(K(d, kFbMin + 3 * w + a, s), true, SL(d), 4 + a);
-      bins[w].hi[a] = key_value(K(d, kFbMax + 3 * w + a, s), false, SL(d), 7 + a);
-    }
+  int nl = (int)A[kAccCounts + w];
+  float l[6], r[6];
+  for (int f = 0; f < 6; ++f)
+    l[f] = r[f] = nl ? unord(A[kAccBins + f * kBins + w]) : FLT_MAX;
+  for (int f = 0; f < 6; ++f) {
+    l[f] = row_min<0x111>(l[f], w >= 1);
+    l[f] = row_min<0x112>(l[f], w >= 2);
+    l[f] = row_min<0x114>(l[f], w >= 4);
+    l[f] = row_min<0x118>(l[f], w >= 8);
+    r[f] = row_min<0x101>(r[f], w < 15);
+    r[f] = row_min<0x102>(r[f], w < 14);
+    r[f] = row_min<0x104>(r[f], w < 12);
+    r[f] = row_min<0x108>(r[f], w < 8);
+    r[f] = dpp_mov<0x101>(r[f]);  // bins behind this one
+  }
+  for (int off = 1; off < 16; off <<= 1) {
+    const int t = __shfl_up(nl, off, 16);
+    nl += w >= off ? t : 0;
   }
   const float inv_parent_area = (float)(1.0 / (double)area(rbox(d.u.refs[sg.rec])));
-  float best_cost = n * kCIsec;
-  int best_axis = -1;
-  float best_pos = FLT_MAX;
-  float left_areas[kBins], right_areas[kBins];
-  int left_counts[kBins], right_counts[kBins];
-  Box lb, rb;
-  reset(lb);
-  reset(rb);
-  int nl = 0, nr = n;
-  for (int i = 0; i < kBins; ++i) {
-    nl += counts[i];
-    nr -= counts[i];
-    extend(lb, bins[i]);
-    left_counts[i] = nl;
-    right_counts[i] = nr;
-    left_areas[i] = area(lb);
+  const float left_area = area(min_box(l)), right_area = area(min_box(r));
+  const float cost =
+      (left_area * nl + right_area * (n - nl)) * inv_parent_area * kCIsec + kCTrav;
+  float best = w < kBins - 1 && cost < n * kCIsec ? cost : FLT_MAX;
+  const float own = best;
+  for (int off = 8; off; off >>= 1) {
+    const float t = __shfl_xor(best, off, 16);
+    best = t < best ? t : best;
   }
-  for (int i = kBins - 1; i >= 0; --i) {
-    right_areas[i] = (i == kBins - 1) ? FLT_MAX : area(rb);
-    extend(rb, bins[i]);
-  }
-  for (int i = 0; i < kBins - 1; ++i) {
-    const float cost = (left_areas[i] * left_counts[i] + right_areas[i] * right_counts[i]) *
-                           inv_parent_area * kCIsec + kCTrav;
-    if (cost < best_cost) {
-      best_cost = cost;
-      best_axis = p.axis;
-      best_pos = p.lo_c + p.width * (static_cast<float>(i + 1) / kBins);
-    }
-  }
-  p.leaf = best_axis == -1;
-  p.pos = best_pos;
+  const unsigned long long first = __ballot(own == best && own < FLT_MAX);
+  const unsigned mine = (unsigned)(first >> (lane & 48)) & 0xFFFFu;
+  if (!in || w != 0) return;
+  p.leaf = mine == 0;
+  const int i = mine ? __ffs((int)mine) - 1 : 0;
+  p.pos = p.lo_c + p.width * (static_cast<float>(i + 1) / kBins);
   d.plan[s] = p;
+}
+
+// A wave takes kVB / 4 consecutive slots of a virtual block, 64 at a time.
+constexpr int kWaveSlots = kVB / (kBlock / 64);
+constexpr int kWaveSteps = kWaveSlots / 64;
+__device__ __forceinline__ int64_t wave_slot(const VRange& r, int k) {
+  return r.first + (int64_t)(threadIdx.x >> 6) * kWaveSlots + k * 64 + (threadIdx.x & 63);
 }
 
 __global__ __launch_bounds__(kBlock) void k_count_less(DevBuild d) {
@@ -398,34 +440,23 @@ __global__ __launch_bounds__(kBlock) void k_count_less(DevBuild d) {
   if (threadIdx.x == 0) tot = 0;
   __syncthreads();
   unsigned c = 0;
-  for (int k = 0; k < kPer; ++k) {
-    const int64_t i = r.first + k * kBlock + threadIdx.x;
-    if (i >= r.end) break;
-    c += slot_c(SL(d), i, p.axis) < p.pos ? 1u : 0u;
+#pragma unroll
+  for (int k = 0; k < kWaveSteps; ++k) {
+    const int64_t i = wave_slot(r, k), j = i < r.end ? i : r.end - 1;
+    c += __popcll(__ballot(slot_c(SL(d), j, p.axis) < p.pos && i < r.end));
   }
-  if (c) atomicAdd(&tot, c);
+  if (c && (threadIdx.x & 63) == 0) atomicAdd(&tot, c);
   __syncthreads();
-  if (threadIdx.x == 0 && tot) atomicAdd(&Cn(d, kFless, r.s), tot);
-}
-
-// partitionObjects returns the number of objects left of the position; when that is 0
-// or all of them the reference splits at the middle (DynBVH.cc:2250-2261).
-__global__ __launch_bounds__(kBlock) void k_seg_mid(DevBuild d) {
-  const int s = blockIdx.x * kBlock + threadIdx.x;
-  if (s >= d.nseg) return;
-  BuildPlan p = d.plan[s];
-  if (p.leaf) return;
-  const BuildSeg sg = d.seg[s];
-  const int n = sg.e - sg.b;
-  const int m = (int)Cn(d, kFless, s);
-  p.nless = m;
-  p.split = (m == 0 || m == n) ? sg.b + n / 2 : sg.b + m;
-  d.plan[s] = p;
+  if (threadIdx.x == 0) {
+    d.vcnt[2 * (int64_t)blockIdx.x] = tot;
+    if (tot) atomicAdd(&acc(d, r.s)[kAccLess], tot);
+  }
 }
 
 // A slot is misplaced on the left if it lies before the split with a key >= the position,
 // on the right if it lies at or after the split with a key < the position. No slot moves
-// in the middle fallback.
+// in the middle fallback. Only the virtual block that holds the split counts its slots
+// again; the others have all of theirs on one side.
 __global__ __launch_bounds__(kBlock) void k_mis_count(DevBuild d) {
   __shared__ unsigned tl, tr;
   VRange r;
@@ -433,19 +464,27 @@ __global__ __launch_bounds__(kBlock) void k_mis_count(DevBuild d) {
   const int64_t v = blockIdx.x;
   const BuildPlan p = d.plan[r.s];
   const BuildSeg sg = d.seg[r.s];
-  const int n = sg.e - sg.b;
-  const bool active = !p.leaf && p.nless != 0 && p.nless != n;
+  bool moves;
+  const int mid = seg_mid(d, r.s, sg, moves);
+  if (p.leaf || !moves || mid >= r.end || mid <= r.first) {
+    if (threadIdx.x == 0) {
+      const unsigned less = p.leaf || !moves ? 0u : d.vcnt[2 * v];
+      const bool before = mid >= r.end;
+      d.vcnt[2 * v] = p.leaf || !moves || !before ? 0u : (unsigned)(r.end - r.first) - less;
+      d.vcnt[2 * v + 1] = before ? 0u : less;
+    }
+    return;
+  }
   if (threadIdx.x == 0) tl = tr = 0;
   __syncthreads();
-  if (active) {
-    unsigned cl = 0, cr = 0;
-    for (int k = 0; k < kPer; ++k) {
-      const int64_t i = r.first + k * kBlock + threadIdx.x;
-      if (i >= r.end) break;
-      const float c = slot_c(SL(d), i, p.axis);
-      cl += (i < p.split && !(c < p.pos)) ? 1u : 0u;
-      cr += (i >= p.split && c < p.pos) ? 1u : 0u;
-    }
+  unsigned cl = 0, cr = 0;
+  for (int k = 0; k < kWaveSteps; ++k) {
+    const int64_t i = wave_slot(r, k);
+    const bool less = i < r.end && slot_c(SL(d), i, p.axis) < p.pos;
+    cl += __popcll(__ballot(i < mid && !less));
+    cr += __popcll(__ballot(i >= mid && less));
+  }
+  if ((threadIdx.x & 63) == 0) {
     if (cl) atomicAdd(&tl, cl);
     if (cr) atomicAdd(&tr, cr);
   }
@@ -456,38 +495,47 @@ __global__ __launch_bounds__(kBlock) void k_mis_count(DevBuild d) {
   }
 }
 
-// Exclusive scans over all virtual blocks of the left and right counts (one workgroup):
-// gscan[v] (left) and gscan[vcap + 1 + v] (right), v in [0, nvb].
+// Exclusive scans over all virtual blocks of the left and right counts (one workgroup, four
+// virtual blocks a thread): gscan[v] (left) and gscan[vcap + 1 + v] (right), v in [0, nvb].
 __global__ __launch_bounds__(1024) void k_scan_mis(DevBuild d) {
-  __shared__ unsigned pl[1024], pr[1024];
-  __shared__ unsigned cl, cr;
-  const int64_t nvb = d.ctr[kCtrNvb];
+  __shared__ unsigned wl[16], wr[16];
+  const int64_t nvb = d.ctr[kCtrNvb + d.level];
   unsigned* gl = d.gscan;
   unsigned* gr = d.gscan + d.vcap + 1;
-  if (threadIdx.x == 0) cl = cr = 0;
-  __syncthreads();
-  for (int64_t base = 0; base < nvb; base += 1024) {
-    const int64_t v = base + threadIdx.x;
-    const unsigned a = v < nvb ? d.vcnt[2 * v] : 0u, b = v < nvb ? d.vcnt[2 * v + 1] : 0u;
-    pl[threadIdx.x] = a;
-    pr[threadIdx.x] = b;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-      const unsigned x = threadIdx.x >= (unsigned)off ? pl[threadIdx.x - off] : 0u;
-      const unsigned y = threadIdx.x >= (unsigned)off ? pr[threadIdx.x - off] : 0u;
-      __syncthreads();
-      pl[threadIdx.x] += x;
-      pr[threadIdx.x] += y;
-      __syncthreads();
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  unsigned cl = 0, cr = 0;  // before this round
+  for (int64_t base = 0; base < nvb; base += 4096) {
+    const int64_t v0 = base + 4 * (int64_t)threadIdx.x;
+    unsigned a[4], b[4], sl = 0, sr = 0;
+    for (int k = 0; k < 4; ++k) {
+      a[k] = v0 + k < nvb ? d.vcnt[2 * (v0 + k)] : 0u;
+      b[k] = v0 + k < nvb ? d.vcnt[2 * (v0 + k) + 1] : 0u;
+      sl += a[k];
+      sr += b[k];
     }
-    if (v < nvb) {
-      gl[v] = cl + pl[threadIdx.x] - a;
-      gr[v] = cr + pr[threadIdx.x] - b;
+    unsigned il = sl, ir = sr;  // inclusive over the wave
+    for (int off = 1; off < 64; off <<= 1) {
+      const unsigned x = (unsigned)__shfl_up((int)il, off), y = (unsigned)__shfl_up((int)ir, off);
+      il += lane >= off ? x : 0u;
+      ir += lane >= off ? y : 0u;
+    }
+    if (lane == 63) {
+      wl[wave] = il;
+      wr[wave] = ir;
     }
     __syncthreads();
-    if (threadIdx.x == 1023) {
-      cl += pl[1023];
-      cr += pr[1023];
+    unsigned pl = cl + il - sl, pr = cr + ir - sr;
+    for (int w = 0; w < 16; ++w) {
+      pl += w < wave ? wl[w] : 0u;
+      pr += w < wave ? wr[w] : 0u;
+      cl += wl[w];
+      cr += wr[w];
+    }
+    for (int k = 0; k < 4 && v0 + k < nvb; ++k) {
+      gl[v0 + k] = pl;
+      gr[v0 + k] = pr;
+      pl += a[k];
+      pr += b[k];
     }
     __syncthreads();
   }
@@ -497,55 +545,51 @@ __global__ __launch_bounds__(1024) void k_scan_mis(DevBuild d) {
   }
 }
 
-// Block-wide exclusive scan of one value per thread in slot order (threads own kPer
-// consecutive slots here); returns the thread's offset.
-__device__ __forceinline__ unsigned block_exscan(unsigned x, unsigned* buf) {
-  buf[threadIdx.x] = x;
-  __syncthreads();
-  for (int off = 1; off < kBlock; off <<= 1) {
-    const unsigned y = threadIdx.x >= (unsigned)off ? buf[threadIdx.x - off] : 0u;
-    __syncthreads();
-    buf[threadIdx.x] += y;
-    __syncthreads();
-  }
-  const unsigned r = buf[threadIdx.x] - x;
-  __syncthreads();
-  return r;
-}
-
+// Slots of the misplaced objects by rank: from the left in lpos, from the right in rpos.
 __global__ __launch_bounds__(kBlock) void k_mis_scatter(DevBuild d) {
-  __shared__ unsigned buf[kBlock];
+  __shared__ unsigned wl[kBlock / 64], wr[kBlock / 64];
   VRange r;
   if (!vrange(d, r)) return;
   const int64_t v = blockIdx.x;
   const BuildPlan p = d.plan[r.s];
   const BuildSeg sg = d.seg[r.s];
-  const int n = sg.e - sg.b;
-  if (p.leaf || p.nless == 0 || p.nless == n) return;  // uniform over the block
+  bool moves;
+  const int mid = seg_mid(d, r.s, sg, moves);
+  if (p.leaf || !moves) return;  // uniform over the block
   const unsigned* gl = d.gscan;
   const unsigned* gr = d.gscan + d.vcap + 1;
-  const int nvb_s = (n + kVB - 1) / kVB;
-  const unsigned baseL = gl[v] - gl[sg.vb0];
-  const unsigned baseR = gr[v] - gr[sg.vb0];
+  const int nvb_s = (sg.e - sg.b + kVB - 1) / kVB;
   const unsigned totR = gr[sg.vb0 + nvb_s] - gr[sg.vb0];
-  // this thread's kPer consecutive slots
-  const int64_t t0 = r.first + (int64_t)threadIdx.x * kPer;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const unsigned long long below = (1ull << lane) - 1ull;
+  unsigned long long ml[kWaveSteps], mr[kWaveSteps];
   unsigned cl = 0, cr = 0;
-  for (int k = 0; k < kPer; ++k) {
-    const int64_t i = t0 + k;
-    if (i >= r.end) break;
-    const float c = slot_c(SL(d), i, p.axis);
-    cl += (i < p.split && !(c < p.pos)) ? 1u : 0u;
-    cr += (i >= p.split && c < p.pos) ? 1u : 0u;
+#pragma unroll
+  for (int k = 0; k < kWaveSteps; ++k) {
+    const int64_t i = wave_slot(r, k), j = i < r.end ? i : r.end - 1;
+    const bool less = slot_c(SL(d), j, p.axis) < p.pos;
+    ml[k] = __ballot(i < r.end && i < mid && !less);
+    mr[k] = __ballot(i < r.end && i >= mid && less);
+    cl += __popcll(ml[k]);
+    cr += __popcll(mr[k]);
   }
-  unsigned rl = baseL + block_exscan(cl, buf);
-  unsigned rr = baseR + block_exscan(cr, buf);
-  for (int k = 0; k < kPer; ++k) {
-    const int64_t i = t0 + k;
-    if (i >= r.end) break;
-    const float c = slot_c(SL(d), i, p.axis);
-    if (i < p.split && !(c < p.pos)) d.lpos[sg.b + rl++] = (int32_t)i;
-    if (i >= p.split && c < p.pos) d.rpos[sg.b + (totR - 1 - rr++)] = (int32_t)i;
+  if (lane == 0) {
+    wl[wave] = cl;
+    wr[wave] = cr;
+  }
+  __syncthreads();
+  unsigned rl = gl[v] - gl[sg.vb0], rr = gr[v] - gr[sg.vb0];
+  for (int w = 0; w < wave; ++w) {
+    rl += wl[w];
+    rr += wr[w];
+  }
+#pragma unroll
+  for (int k = 0; k < kWaveSteps; ++k) {
+    const int32_t i = (int32_t)wave_slot(r, k);
+    if ((ml[k] >> lane) & 1) d.lpos[sg.b + rl + __popcll(ml[k] & below)] = i;
+    if ((mr[k] >> lane) & 1) d.rpos[sg.b + (totR - 1 - (rr + __popcll(mr[k] & below)))] = i;
+    rl += __popcll(ml[k]);
+    rr += __popcll(mr[k]);
   }
 }
 
@@ -554,10 +598,11 @@ __global__ __launch_bounds__(kBlock) void k_swap(DevBuild d) {
   if (!vrange(d, r)) return;
   const BuildPlan p = d.plan[r.s];
   const BuildSeg sg = d.seg[r.s];
-  const int n = sg.e - sg.b;
-  if (p.leaf || p.nless == 0 || p.nless == n) return;
+  bool moves;
+  (void)seg_mid(d, r.s, sg, moves);
+  if (p.leaf || !moves) return;
   const unsigned* gl = d.gscan;
-  const int nvb_s = (n + kVB - 1) / kVB;
+  const int nvb_s = (sg.e - sg.b + kVB - 1) / kVB;
   const int64_t nswap = gl[sg.vb0 + nvb_s] - gl[sg.vb0];
   for (int k = 0; k < kPer; ++k) {
     const int64_t i = r.first + k * kBlock + threadIdx.x;
@@ -578,96 +623,146 @@ __global__ __launch_bounds__(kBlock) void k_swap(DevBuild d) {
   }
 }
 
+// Boxes and centroid boxes of the two sides: reduced in registers over the wave (by lanes
+// into one LDS word of 64 bits, as before, 50 to 130 us a level), then in LDS over the
+// workgroup, then one global atomic per value.
 __global__ __launch_bounds__(kBlock) void k_child_bounds(DevBuild d) {
-  __shared__ unsigned long long sk[12];  // left min 3, left max 3, right min 3, right max 3
+  __shared__ unsigned long long sk[12];
+  __shared__ unsigned sc[12];
   VRange r;
   if (!vrange(d, r)) return;
   const BuildPlan p = d.plan[r.s];
   if (p.leaf) return;
-  if (threadIdx.x < 12) sk[threadIdx.x] = (threadIdx.x % 6) < 3 ? kMinInit : 0ull;
-  __syncthreads();
-  unsigned long long m[12];
-  for (int k = 0; k < 12; ++k) m[k] = (k % 6) < 3 ? kMinInit : 0ull;
-  for (int k = 0; k < kPer; ++k) {
-    const int64_t i = r.first + k * kBlock + threadIdx.x;
-    if (i >= r.end) break;
-    Slot o;
-    load_slot(SL(d), i, o);
-    const int side = i < p.split ? 0 : 6;
-    for (int a = 0; a < 3; ++a) {
-      const unsigned long long x = kmin(o.lo[a], (uint32_t)i), y = kmax(o.hi[a], (uint32_t)i);
-      m[side + a] = x < m[side + a] ? x : m[side + a];
-      m[side + 3 + a] = y > m[side + 3 + a] ? y : m[side + 3 + a];
-    }
+  const BuildSeg sg = d.seg[r.s];
+  bool moves;
+  const int mid = seg_mid(d, r.s, sg, moves);
+  if (threadIdx.x < 12) {
+    sk[threadIdx.x] = ~0ull;
+    sc[threadIdx.x] = ~0u;
   }
-  for (int k = 0; k < 12; ++k) {
-    if ((k % 6) < 3) {
-      if (m[k] != kMinInit) atomicMin(&sk[k], m[k]);
-    } else if (m[k] != 0ull) {
-      atomicMax(&sk[k], m[k]);
+  __syncthreads();
+  for (int side = 0; side < 2; ++side) {
+    const int64_t lo = side && mid > r.first ? mid : r.first;
+    const int64_t hi = !side && mid < r.end ? mid : r.end;
+    if (lo + (threadIdx.x & ~63) >= hi) continue;  // nothing for this wave
+    MinSlot m[6];
+    uint32_t c[6];
+    for (int k = 0; k < 6; ++k) c[k] = ~0u;
+    for (int64_t first = lo; first < hi; first += kBlock) {
+      int64_t i = first + threadIdx.x;
+      i = i < hi ? i : hi - 1;  // the last slot again: changes no minimum
+      Slot o;
+      load_slot(SL(d), i, o);
+      for (int a = 0; a < 3; ++a) {
+        m[a].take(o.lo[a], (uint32_t)i);
+        m[3 + a].take(-o.hi[a], (uint32_t)i);
+        const uint32_t x = ord(o.c[a]), y = ord(-o.c[a]);
+        c[a] = x < c[a] ? x : c[a];
+        c[3 + a] = y < c[3 + a] ? y : c[3 + a];
+      }
+    }
+    for (int k = 0; k < 6; ++k) {
+      const unsigned long long key = wave_kmin(m[k]);
+      const uint32_t x = wave_umin(c[k]);
+      if ((threadIdx.x & 63) == 0) {
+        atomicMin(&sk[6 * side + k], key);
+        atomicMin(&sc[6 * side + k], x);
+      }
     }
   }
   __syncthreads();
   if (threadIdx.x < 12) {
-    const int k = threadIdx.x;
-    const int f = k < 3 ? kFlMin + k : k < 6 ? kFlMax + k - 3 : k < 9 ? kFrMin + k - 6 : kFrMax + k - 9;
-    if ((k % 6) < 3) {
-      if (sk[k] != kMinInit) atomicMin(&K(d, f, r.s), sk[k]);
-    } else if (sk[k] != 0ull) {
-      atomicMax(&K(d, f, r.s), sk[k]);
-    }
+    if (sk[threadIdx.x] != ~0ull) atomicMin(&acc_box(d, r.s)[threadIdx.x], sk[threadIdx.x]);
+  } else if (threadIdx.x < 24) {
+    const unsigned x = sc[threadIdx.x - 12];
+    if (x != ~0u) atomicMin(&acc(d, r.s)[kAccCen + threadIdx.x - 12], x);
   }
 }
 
-__device__ __forceinline__ void push_node(const DevBuild& d, int rec, int b, int e) {
-  const BuildSeg sg{rec, b, e, 0};
-  if (e - b > kBuildSerial) {
-    d.seg_next[atomicAdd(&d.ctr[kCtrNext], 1u)] = sg;
-  } else {
-    d.small[atomicAdd(&d.ctr[kCtrSmall], 1u)] = sg;
-  }
-}
-
+// One lane per node; a wave's nodes take their places from each counter with one atomic
+// (an atomic per node and counter took up to 137 us a level).
 __global__ __launch_bounds__(kBlock) void k_seg_children(DevBuild d) {
   const int s = blockIdx.x * kBlock + threadIdx.x;
-  if (s >= d.nseg) return;
-  const BuildPlan p = d.plan[s];
-  const BuildSeg sg = d.seg[s];
+  const int lane = threadIdx.x & 63;
+  const unsigned long long below = (1ull << lane) - 1ull;
+  const bool in = s < n_segs(d);
+  if (!__ballot(in)) return;
+  const int at = in ? s : 0;
+  const BuildPlan p = d.plan[at];
+  const BuildSeg sg = d.seg[at];
+  bool moves;
+  const int mid = seg_mid(d, at, sg, moves);
+  const bool inner = in && !p.leaf, leaf = in && p.leaf;
+  const int b[2] = {sg.b, mid}, e[2] = {mid, sg.e};
+  unsigned long long next[2], small[2];
+  int vbs = 0;  // virtual blocks of this node's children
+  for (int side = 0; side < 2; ++side) {
+    const bool large = e[side] - b[side] > kBuildSerial;
+    next[side] = __ballot(inner && large);
+    small[side] = __ballot(inner && !large);
+    if (inner && large) vbs += (e[side] - b[side] + kVB - 1) / kVB;
+  }
+  int vb_end = vbs;
+  for (int off = 1; off < 64; off <<= 1) {
+    const int t = __shfl_up(vb_end, off);
+    vb_end += lane >= off ? t : 0;
+  }
+  const unsigned long long inners = __ballot(inner), leaves = __ballot(leaf);
+  const unsigned amount[5] = {2u * (unsigned)__popcll(inners),
+                              (unsigned)(__popcll(next[0]) + __popcll(next[1])),
+                              (unsigned)(__popcll(small[0]) + __popcll(small[1])),
+                              (unsigned)__popcll(leaves), (unsigned)__shfl(vb_end, 63)};
+  unsigned* const counter[5] = {d.u.next_free, d.ctr + kCtrSegs + d.level + 1, d.ctr + kCtrSmall,
+                                d.ctr + kCtrBig, d.ctr + kCtrNvb + d.level + 1};
+  unsigned got = 0;
+  for (int k = 0; k < 5; ++k)
+    if (lane == k && amount[k]) got = atomicAdd(counter[k], amount[k]);
+  unsigned base[5];
+  for (int k = 0; k < 5; ++k) base[k] = (unsigned)__shfl((int)got, k);
+  if (!in) return;
   RefNode& nd = d.u.refs[sg.rec];
-  const int n = sg.e - sg.b;
-  if (p.leaf) {  // sorted later, with the other large leaves
-    if (n > 32767) {
-      atomicExch(d.u.err, 3);
-      return;
-    }
+  if (leaf) {  // sorted later, with the other large leaves
+    const int n = sg.e - sg.b;
+    if (n > 32767) atomicExch(d.u.err, 3);
     nd.child = sg.b;
     nd.children = (int16_t)n;
     nd.axis = 0;
-    d.big[atomicAdd(&d.ctr[kCtrBig], 1u)] = sg;
+    d.big[base[3] + __popcll(leaves & below)] = sg;
     return;
   }
-  const unsigned spot = atomicAdd(d.u.next_free, 2u);
-  if (spot + 1 >= (unsigned)d.u.n_records) {
+  unsigned spot = base[0] + 2u * (unsigned)__popcll(inners & below);
+  if (spot + 1 >= (unsigned)d.u.n_records) {  // cannot happen: N objects need < 2N records
     atomicExch(d.u.err, 1);
-    return;
+    spot = 0;
   }
   nd.child = (int32_t)spot;
   nd.children = 0;
   nd.axis = (uint8_t)p.axis;
+  int vb = (int)base[4] + vb_end - vbs;
+  unsigned q_next = base[1], q_small = base[2];
   for (int side = 0; side < 2; ++side) {
     RefNode& c = d.u.refs[spot + side];
-    const int fmin = side ? kFrMin : kFlMin, fmax = side ? kFrMax : kFlMax;
+    const unsigned long long* k = acc_box(d, s) + 6 * side;
     for (int a = 0; a < 3; ++a) {
-      c.box.lo[a] = key_value(K(d, fmin + a, s), true, SL(d), 4 + a);
-      c.box.hi[a] = key_value(K(d, fmax + a, s), false, SL(d), 7 + a);
+      c.box.lo[a] = key_value(k[a], d.slots, 12, 4 + a, false);
+      c.box.hi[a] = key_value(k[3 + a], d.slots, 12, 7 + a, true);
     }
     c.child = 0;
     c.children = 0;
     c.axis = 0;
     c.bits = 0;
+    const BuildSeg child{(int32_t)spot + side, b[side], e[side], vb};
+    if ((next[side] >> lane) & 1) {
+      const unsigned q = q_next + (unsigned)__popcll(next[side] & below);
+      d.seg_next[q] = child;
+      d.plan_next[q] = make_plan(acc(d, s) + kAccCen + 6 * side);
+      vb += (e[side] - b[side] + kVB - 1) / kVB;
+    } else {
+      d.small[q_small + (unsigned)__popcll(small[side] & below)] = child;
+    }
+    q_next += (unsigned)__popcll(next[side]);
+    q_small += (unsigned)__popcll(small[side]);
   }
-  push_node(d, spot, sg.b, p.split);
-  push_node(d, spot + 1, p.split, sg.e);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -682,11 +777,6 @@ __global__ __launch_bounds__(kBlock) void k_seg_children(DevBuild d) {
 // 28 thousand subtrees of a million triangles, and 3300 to 6900 us with 32 to 1 lanes of a
 // wave in use; this takes 193 us.
 
-template <int kCtrl>
-__device__ __forceinline__ float dpp_mov(float x) {
-  return __int_as_float(
-      __builtin_amdgcn_update_dpp(0, __float_as_int(x), kCtrl, 0xF, 0xF, true));
-}
 __device__ __forceinline__ float lane_get(float x, int src) {
   return __int_as_float(__builtin_amdgcn_ds_bpermute(src << 2, __float_as_int(x)));
 }
@@ -728,15 +818,6 @@ struct SegScan {
   }
 };
 
-// Boxes are held as six minima (lo, -hi); negating is exact.
-__device__ __forceinline__ Box min_box(const float* m) {
-  Box b;
-  for (int a = 0; a < 3; ++a) {
-    b.lo[a] = m[a];
-    b.hi[a] = -m[3 + a];
-  }
-  return b;
-}
 __device__ __forceinline__ void put_record(RefNode* r, const float* m, int child, int children,
                                            int axis) {
   float4* p = reinterpret_cast<float4*>(r);
@@ -968,33 +1049,55 @@ __global__ __launch_bounds__(1024) void k_sort_big(DevBuild d, int32_t* scratch)
 // ---------------------------------------------------------------------------------------
 // Phase 3: reference numbering and the bottom-up passes
 
-
 __global__ __launch_bounds__(kBlock) void k_ic_leaves(DevFinish f, int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (i < n) f.ic[f.leaves[i]] = 0;
 }
-__global__ __launch_bounds__(kBlock) void k_ic_level(DevFinish f, int64_t first, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  const int x = f.levels[first + i];
+// The small depths at the top run in one workgroup (k_*_top): the barrier between depths
+// orders them as separate launches would (the workgroup's waves share one compute unit and
+// its L1, so stores before the barrier are seen by loads after it).
+template <class F>
+__device__ __forceinline__ void top_up(const TopLevels& t, F node) {
+  for (int d = t.n - 1; d >= 0; --d) {
+    for (int i = (int)threadIdx.x; i < t.cnt[d]; i += kBlock) node((int64_t)t.first[d] + i);
+    __syncthreads();
+  }
+}
+__device__ __forceinline__ void ic_node(const DevFinish& f, int64_t i) {
+  const int x = f.levels[i];
   const int c = f.trefs[x].child;
   f.ic[x] = 1 + f.ic[c] + f.ic[c + 1];
 }
-__global__ void k_rank_root(DevFinish f) {
-  f.rank[0] = 0;
-  f.fin[0] = 0;
+__global__ __launch_bounds__(kBlock) void k_ic_level(DevFinish f, int64_t first, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (i < n) ic_node(f, first + i);
 }
 // Pairs are handed out in preorder of their parents (DynBVH::build recursion).
-__global__ __launch_bounds__(kBlock) void k_rank_level(DevFinish f, int64_t first, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  const int x = f.levels[first + i];
+__device__ __forceinline__ void rank_node(const DevFinish& f, int64_t i) {
+  const int x = f.levels[i];
   const int c = f.trefs[x].child;
   const int rk = f.rank[x];
   f.fin[c] = 2 * rk + 1;
   f.fin[c + 1] = 2 * rk + 2;
   f.rank[c] = rk + 1;
   f.rank[c + 1] = rk + 1 + f.ic[c];
+}
+__global__ __launch_bounds__(kBlock) void k_rank_level(DevFinish f, int64_t first, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (i < n) rank_node(f, first + i);
+}
+// Counts up and ranks down through the top depths.
+__global__ __launch_bounds__(kBlock) void k_ic_rank_top(DevFinish f, TopLevels t) {
+  top_up(t, [&](int64_t i) { ic_node(f, i); });
+  if (threadIdx.x == 0) {
+    f.rank[0] = 0;
+    f.fin[0] = 0;
+  }
+  __syncthreads();
+  for (int d = 0; d < t.n; ++d) {
+    for (int i = (int)threadIdx.x; i < t.cnt[d]; i += kBlock) rank_node(f, (int64_t)t.first[d] + i);
+    __syncthreads();
+  }
 }
 // Records in use move to their reference numbers; records from the node count on are
 // left as DynBVH::allocate leaves them after a reset. Holes (records the one-lane
@@ -1042,38 +1145,56 @@ __global__ __launch_bounds__(kBlock) void k_fin_leaves(DevFinish f, int64_t n) {
   f.rt[2 * r] = c.c0;
   f.rt[2 * r + 1] = c.c1;
 }
-__global__ __launch_bounds__(kBlock) void k_fin_level(DevFinish f, int64_t first, int64_t n) {
+__device__ __forceinline__ Aabb aabb(const RefNode& n) {
+  Aabb b;
+  for (int a = 0; a < 3; ++a) {
+    b.lo[a] = n.box.lo[a];
+    b.hi[a] = n.box.hi[a];
+  }
+  return b;
+}
+// The crossing probabilities of every inner node. They depend on the boxes alone, so all
+// depths go in one launch: some 30 us of dependent float work that each depth's launch
+// would otherwise wait for (12 to 87 us a depth, 1160 us of a million triangles' build).
+__global__ __launch_bounds__(kBlock) void k_fin_probs(DevFinish f, int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (i >= n) return;
-  const int r = f.levels[first + i];
+  const RefNode nd = f.refs[f.levels[i]];
+  const Aabb L = aabb(f.refs[nd.child]), R = aabb(f.refs[nd.child + 1]);
+  float lr, jl, jr;
+  rtsah::probabilities(f.logtab, aabb(nd), L, R, lr, jl, jr);
+  f.prob[0][i] = lr;
+  f.prob[1][i] = jl;
+  f.prob[2][i] = jr;
+}
+__device__ __forceinline__ void fin_node(const DevFinish& f, int64_t i) {
+  const int r = f.levels[i];
   RefNode& nd = f.refs[r];
   const int c = nd.child;
   const uint32_t size = 1 + f.ssize[c] + f.ssize[c + 1];
   f.ssize[r] = size;
   uint8_t bits = nd.bits & ~3;
   if (size > f.large) bits |= 2;
-  const RefNode L = f.refs[c], R = f.refs[c + 1];
-  const float ar = area(rbox(nd)), al = area(rbox(L)), arr = area(rbox(R));
+  const float ar = area(rbox(nd)), al = area(rbox(f.refs[c])), arr = area(rbox(f.refs[c + 1]));
   f.costs[r] = kCTrav + (al * f.costs[c] + arr * f.costs[c + 1]) / ar;
-  Aabb P, Lb, Rb;
-  for (int a = 0; a < 3; ++a) {
-    P.lo[a] = nd.box.lo[a];
-    P.hi[a] = nd.box.hi[a];
-    Lb.lo[a] = L.box.lo[a];
-    Lb.hi[a] = L.box.hi[a];
-    Rb.lo[a] = R.box.lo[a];
-    Rb.hi[a] = R.box.hi[a];
-  }
   if (f.rtsah) {
     bool left_cheaper = false;
     const rtsah::CostPair cl{f.rt[2 * c], f.rt[2 * c + 1]};
     const rtsah::CostPair cr{f.rt[2 * c + 2], f.rt[2 * c + 3]};
-    const rtsah::CostPair o = rtsah::combine(f.logtab, P, Lb, Rb, cl, cr, left_cheaper);
+    const rtsah::CostPair o =
+        rtsah::combine(f.prob[0][i], f.prob[1][i], f.prob[2][i], cl, cr, left_cheaper);
     if (left_cheaper) bits |= 1;
     f.rt[2 * r] = o.c0;
     f.rt[2 * r + 1] = o.c1;
   }
   nd.bits = bits;
+}
+__global__ __launch_bounds__(kBlock) void k_fin_level(DevFinish f, int64_t first, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (i < n) fin_node(f, first + i);
+}
+__global__ __launch_bounds__(kBlock) void k_fin_top(DevFinish f, TopLevels t) {
+  top_up(t, [&](int64_t i) { fin_node(f, i); });
 }
 
 unsigned grid(int64_t n, int block = kBlock) { return (unsigned)((n + block - 1) / block); }
@@ -1085,26 +1206,20 @@ unsigned grid(int64_t n, int block = kBlock) { return (unsigned)((n + block - 1)
 
 int build_launch_setup(const DevBuild& d, int serial, void* stream) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  hipLaunchKernelGGL(k_root_box, dim3(grid(d.n_verts)), dim3(kBlock), 0, s, d);
-  hipLaunchKernelGGL(k_slots, dim3(grid(d.u.n_objects)), dim3(kBlock), 0, s, d);
+  hipLaunchKernelGGL(k_root_box, dim3(grid(d.n_verts, kSetupVB)), dim3(kBlock), 0, s, d);
+  hipLaunchKernelGGL(k_slots, dim3(grid(d.u.n_objects, kSetupVB)), dim3(kBlock), 0, s, d);
   hipLaunchKernelGGL(k_root_init, dim3(1), dim3(1), 0, s, d, serial);
   return (int)hipGetLastError();
 }
 
-int build_launch_level(const DevBuild& d, int64_t nvb_bound, void* stream) {
+int build_launch_level(const DevBuild& d, int64_t nseg_bound, int64_t nvb_bound, void* stream) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const unsigned gs = grid(d.nseg);
+  const unsigned gs = grid(nseg_bound), g16 = grid(nseg_bound, kBlock / 16);
   const unsigned gv = (unsigned)nvb_bound;
-  hipLaunchKernelGGL(k_acc_clear, dim3(grid((int64_t)(kKeyFields + kCntFields) * d.nseg)),
-                     dim3(kBlock), 0, s, d);
-  hipLaunchKernelGGL(k_scan_segments, dim3(1), dim3(1024), 0, s, d);
-  hipLaunchKernelGGL(k_vb_map, dim3(gs), dim3(kBlock), 0, s, d);
-  hipLaunchKernelGGL(k_cbounds, dim3(gv), dim3(kBlock), 0, s, d);
-  hipLaunchKernelGGL(k_seg_axis, dim3(gs), dim3(kBlock), 0, s, d);
+  hipLaunchKernelGGL(k_level_open, dim3(g16), dim3(kBlock), 0, s, d);
   hipLaunchKernelGGL(k_bins, dim3(gv), dim3(kBlock), 0, s, d);
-  hipLaunchKernelGGL(k_seg_split, dim3(gs), dim3(kBlock), 0, s, d);
+  hipLaunchKernelGGL(k_seg_split, dim3(g16), dim3(kBlock), 0, s, d);
   hipLaunchKernelGGL(k_count_less, dim3(gv), dim3(kBlock), 0, s, d);
-  hipLaunchKernelGGL(k_seg_mid, dim3(gs), dim3(kBlock), 0, s, d);
   hipLaunchKernelGGL(k_mis_count, dim3(gv), dim3(kBlock), 0, s, d);
   hipLaunchKernelGGL(k_scan_mis, dim3(1), dim3(1024), 0, s, d);
   hipLaunchKernelGGL(k_mis_scatter, dim3(gv), dim3(kBlock), 0, s, d);
@@ -1127,17 +1242,22 @@ int build_launch_serial(const DevBuild& d, int64_t n_small, int64_t n_big, int32
 int build_launch_ranks(const DevFinish& f, const int64_t* level_off, int n_levels,
                        int64_t n_leaves, void* stream) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  std::vector<LevelList> lev;
+  for (int d = 0; d < n_levels; ++d)
+    lev.push_back(LevelList{level_off[d], level_off[d + 1] - level_off[d]});
+  TopLevels t;
+  const int top = top_levels(lev.data(), n_levels, 1, t);
   if (n_leaves > 0)
     hipLaunchKernelGGL(k_ic_leaves, dim3(grid(n_leaves)), dim3(kBlock), 0, s, f, n_leaves);
-  for (int d = n_levels - 1; d >= 0; --d) {
-    const int64_t first = level_off[d], n = level_off[d + 1] - first;
-    if (n > 0) hipLaunchKernelGGL(k_ic_level, dim3(grid(n)), dim3(kBlock), 0, s, f, first, n);
-  }
-  hipLaunchKernelGGL(k_rank_root, dim3(1), dim3(1), 0, s, f);
-  for (int d = 0; d < n_levels; ++d) {
-    const int64_t first = level_off[d], n = level_off[d + 1] - first;
-    if (n > 0) hipLaunchKernelGGL(k_rank_level, dim3(grid(n)), dim3(kBlock), 0, s, f, first, n);
-  }
+  for (int d = n_levels - 1; d >= top; --d)
+    if (lev[d].n > 0)
+      hipLaunchKernelGGL(k_ic_level, dim3(grid(lev[d].n)), dim3(kBlock), 0, s, f, lev[d].first,
+                         lev[d].n);
+  hipLaunchKernelGGL(k_ic_rank_top, dim3(1), dim3(kBlock), 0, s, f, t);
+  for (int d = top; d < n_levels; ++d)
+    if (lev[d].n > 0)
+      hipLaunchKernelGGL(k_rank_level, dim3(grid(lev[d].n)), dim3(kBlock), 0, s, f, lev[d].first,
+                         lev[d].n);
   hipLaunchKernelGGL(k_emit, dim3(grid(f.n_records)), dim3(kBlock), 0, s, f);
   const int64_t n_inner = level_off[n_levels];
   const int64_t m = n_inner > n_leaves ? n_inner : n_leaves;
@@ -1145,10 +1265,13 @@ int build_launch_ranks(const DevFinish& f, const int64_t* level_off, int n_level
     hipLaunchKernelGGL(k_map_lists, dim3(grid(m)), dim3(kBlock), 0, s, f, n_inner, n_leaves);
   if (n_leaves > 0)
     hipLaunchKernelGGL(k_fin_leaves, dim3(grid(n_leaves)), dim3(kBlock), 0, s, f, n_leaves);
-  for (int d = n_levels - 1; d >= 0; --d) {
-    const int64_t first = level_off[d], n = level_off[d + 1] - first;
-    if (n > 0) hipLaunchKernelGGL(k_fin_level, dim3(grid(n)), dim3(kBlock), 0, s, f, first, n);
-  }
+  if (f.rtsah && n_inner > 0)
+    hipLaunchKernelGGL(k_fin_probs, dim3(grid(n_inner)), dim3(kBlock), 0, s, f, n_inner);
+  for (int d = n_levels - 1; d >= top; --d)
+    if (lev[d].n > 0)
+      hipLaunchKernelGGL(k_fin_level, dim3(grid(lev[d].n)), dim3(kBlock), 0, s, f, lev[d].first,
+                         lev[d].n);
+  if (top > 0) hipLaunchKernelGGL(k_fin_top, dim3(1), dim3(kBlock), 0, s, f, t);
   return (int)hipGetLastError();
 }
 

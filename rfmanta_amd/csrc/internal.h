@@ -110,7 +110,7 @@ struct mh_scene {
   DevBuf refs, wide, tris, ids, big, d_verts, d_base, d_idx, leaves, levels;
   // rotating update (mh_scene_update): costs, subtree sizes, parents, object boxes and
   // centroids, depth work arrays, the depth histogram and counters
-  DevBuf costs, ssize, parent, obox, ocen, anc0, dep0, anc1, dep1, hist, counters;
+  DevBuf costs, ssize, parent, anc0, dep0, anc1, dep1, hist, counters;
   DevBuf split_list;  // rotating update: leaves whose parent's rotation may split them
   DevBuf levels_aux;  // rotating update: first child and word beside each level entry
   // Per object slot, the record of the leaf whose first slot it is, else -1.
@@ -146,7 +146,7 @@ struct mh_scene {
   size_t device_bytes() const {
     return refs.bytes + pairs.bytes + tris.bytes + ids.bytes + big.bytes + d_verts.bytes +
            d_base.bytes + d_idx.bytes + leaves.bytes + levels.bytes + costs.bytes + ssize.bytes +
-           parent.bytes + obox.bytes + ocen.bytes + anc0.bytes + dep0.bytes + anc1.bytes +
+           parent.bytes + anc0.bytes + dep0.bytes + anc1.bytes +
            dep1.bytes + hist.bytes + counters.bytes + logtab.bytes + normals.bytes +
            normal_idx.bytes + texcoords.bytes + tex_idx.bytes + pairs_soa.bytes +
            split_list.bytes + levels_aux.bytes + leaf_at.bytes + wide.bytes + irregular.bytes;

@@ -603,8 +603,7 @@ int mh_scene_destroy(mh_scene* scene) {
 }
 
 // DynBVH::rebuild with USE_APPROXIMATE_BUILD, on the device (build.hip): object boxes,
-// the level loop over nodes of many objects (one counter read-back per level), one lane
-// per small node, then the reference numbering and the bottom-up passes.
+// the level loop over nodes of many objects, one wave per small node, then the reference numbering and the bottom-up passes.
 int build_device(mh_scene* s, int rtsah) {
   using mh_internal::DevBuf;
   const uint32_t T = s->nt;
@@ -613,7 +612,6 @@ int build_device(mh_scene* s, int rtsah) {
   const int64_t vcap = (int64_t)T / mh::kBuildVB + cap + 2;
   int rc;
   if ((rc = reserve_tree(s, nrec, 0, 0)) || (rc = s->parent.reserve(nrec * 4)) ||
-      (rc = s->obox.reserve((size_t)T * 24)) || (rc = s->ocen.reserve((size_t)T * 12)) ||
       (rc = s->anc0.reserve(nrec * 4)) || (rc = s->dep0.reserve(nrec * 4)) ||
       (rc = s->anc1.reserve(nrec * 4)) || (rc = s->dep1.reserve(nrec * 4)) ||
       (rc = s->hist.reserve(mh::kDepthHist * 4)))
@@ -624,89 +622,92 @@ int build_device(mh_scene* s, int rtsah) {
     if ((rc = s->logtab.reserve(tab.size() * 4))) return rc;
     HIP_OK(hipMemcpy(s->logtab.p, tab.data(), tab.size() * 4, hipMemcpyHostToDevice));
   }
-  // Work arrays of this build only.
-  DevBuf slots, trefs, seg0, seg1, small, big, plan, acck, accc, ctr, vbseg, vcnt, gscan,
-      scratch, rootk, ic, rank, fin, rt;
-  if ((rc = slots.reserve((size_t)T * 48)) || (rc = trefs.reserve(nrec * 32)) ||
-      (rc = seg0.reserve(cap * 16)) || (rc = seg1.reserve(cap * 16)) ||
-      (rc = small.reserve((size_t)T * 16)) || (rc = big.reserve(cap * 16)) ||
-      (rc = plan.reserve(cap * 32)) || (rc = acck.reserve(cap * mh::kKeyFields * 8)) ||
-      (rc = accc.reserve(cap * mh::kCntFields * 4)) || (rc = ctr.reserve(16)) ||
-      (rc = vbseg.reserve(vcap * 4)) || (rc = vcnt.reserve(vcap * 8)) || (rc = gscan.reserve(2 * (vcap + 1) * 4)) ||
-      (rc = scratch.reserve(nrec * 4)) || (rc = rootk.reserve(48)) ||
-      (rc = ic.reserve(nrec * 4)) || (rc = rank.reserve(nrec * 4)) ||
-      (rc = fin.reserve(nrec * 4)) || (rc = rt.reserve(nrec * 8)))
-    return rc;
+  // Work arrays of this build only, in one allocation.
+  size_t held = 0;
+  auto place = [&](size_t bytes) {
+    const size_t at = held;
+    held += (bytes + 255) & ~(size_t)255;
+    return at;
+  };
+  const size_t o_slots = place((size_t)T * 48), o_trefs = place(nrec * 32),
+               o_seg0 = place(cap * sizeof(mh::BuildSeg)),
+               o_seg1 = place(cap * sizeof(mh::BuildSeg)),
+               o_small = place((size_t)T * sizeof(mh::BuildSeg)),
+               o_big = place(cap * sizeof(mh::BuildSeg)),
+               o_plan0 = place(cap * sizeof(mh::BuildPlan)),
+               o_plan1 = place(cap * sizeof(mh::BuildPlan)),
+               o_acc = place((size_t)cap * mh::kAccWords * 4), o_ctr = place(mh::kCtrCount * 4),
+               o_vbseg = place(vcap * 4), o_vcnt = place(vcap * 8),
+               o_gscan = place(2 * (vcap + 1) * 4), o_scratch = place(nrec * 4),
+               o_root = place(48 + 24), o_ic = place(nrec * 4), o_rank = place(nrec * 4),
+               o_fin = place(nrec * 4), o_rt = place(nrec * 8);
+  DevBuf work;
+  if ((rc = work.reserve(held))) return rc;
+  auto at = [&](size_t offset) { return static_cast<void*>(work.as<char>() + offset); };
   hipStream_t st = nullptr;
-  unsigned* cnt = s->counters.as<unsigned>();  // [0] records in use, [1] error
-  HIP_OK(hipMemsetAsync(cnt, 0, 16, st));
-  HIP_OK(hipMemsetAsync(ctr.p, 0, 16, st));
-  HIP_OK(hipMemsetAsync(rootk.p, 0xFF, 24, st));
-  HIP_OK(hipMemsetAsync(rootk.as<char>() + 24, 0, 24, st));
+  HIP_OK(hipMemsetAsync(at(o_ctr), 0, mh::kCtrCount * 4, st));
+  HIP_OK(hipMemsetAsync(at(o_root), 0xFF, 48 + 24, st));
 
   mh::DevBuild d{};
-  d.u.refs = trefs.as<mh::RefNode>();
-  d.u.costs = s->costs.as<float>();  // scratch until the bottom-up pass rewrites them
-  d.u.ssize = s->ssize.as<uint32_t>();
-  d.u.parent = s->parent.as<int32_t>();
+  unsigned* ctr = static_cast<unsigned*>(at(o_ctr));
+  d.u.refs = static_cast<mh::RefNode*>(at(o_trefs));
   d.u.ids = s->ids.as<int32_t>();
-  d.u.obox = s->obox.as<float>();
-  d.u.ocen = s->ocen.as<float>();
   d.u.verts = s->d_verts.as<float>();
   d.u.idx = s->d_idx.as<uint32_t>();
-  d.u.next_free = cnt;
-  d.u.err = reinterpret_cast<int*>(cnt + 1);
+  d.u.next_free = ctr + mh::kCtrRecords;
+  d.u.err = reinterpret_cast<int*>(ctr + mh::kCtrErr);
   d.u.n_records = (int32_t)nrec;
   d.u.n_objects = (int32_t)T;
-  d.u.large = (uint32_t)(nrec / (20 * (size_t)s->workers));
-  d.slots = slots.as<float>();
+  d.slots = static_cast<float*>(at(o_slots));
   d.verts = s->d_verts.as<float>();
   d.n_verts = s->nv;
-  d.small = small.as<mh::BuildSeg>();
-  d.big = big.as<mh::BuildSeg>();
-  d.plan = plan.as<mh::BuildPlan>();
-  d.acck = acck.as<unsigned long long>();
-  d.accc = accc.as<unsigned>();
-  d.cap = cap;
-  d.ctr = ctr.as<unsigned>();
-  d.vbseg = vbseg.as<int32_t>();
-  d.vcnt = vcnt.as<unsigned>();
-  d.gscan = gscan.as<unsigned>();
+  d.small = static_cast<mh::BuildSeg*>(at(o_small));
+  d.big = static_cast<mh::BuildSeg*>(at(o_big));
+  d.acc = static_cast<unsigned*>(at(o_acc));
+  d.ctr = ctr;
+  d.vbseg = static_cast<int32_t*>(at(o_vbseg));
+  d.vcnt = static_cast<unsigned*>(at(o_vcnt));
+  d.gscan = static_cast<unsigned*>(at(o_gscan));
   d.vcap = vcap;
-  d.lpos = scratch.as<int32_t>();
-  d.rpos = scratch.as<int32_t>() + T;
-  d.rootk = rootk.as<unsigned long long>();
-  HIP_OK((hipError_t)mh::launch_obj_bounds(d.u, st));
+  d.lpos = static_cast<int32_t*>(at(o_scratch));
+  d.rpos = d.lpos + T;
+  d.rootk = static_cast<unsigned long long*>(at(o_root));
+  d.rootc = reinterpret_cast<unsigned*>(d.rootk + 6);
   const bool serial_root = T <= (uint32_t)mh::kBuildSerial;
-  d.seg = seg0.as<mh::BuildSeg>();
+  d.seg = static_cast<mh::BuildSeg*>(at(o_seg0));
+  d.plan = static_cast<mh::BuildPlan*>(at(o_plan0));
   HIP_OK((hipError_t)mh::build_launch_setup(d, serial_root ? 1 : 0, st));
-  mh::BuildSeg* cur = seg0.as<mh::BuildSeg>();
-  mh::BuildSeg* nxt = seg1.as<mh::BuildSeg>();
-  int64_t nseg = serial_root ? 0 : 1;
-  unsigned back[mh::kCtrCount];
-  int err = 0;
-  while (nseg > 0) {
-    d.seg = cur;
-    d.seg_next = nxt;
-    d.nseg = (int32_t)nseg;
-    HIP_OK(hipMemsetAsync(d.ctr + mh::kCtrNext, 0, 4, st));
-    const int64_t nvb_bound = (int64_t)T / mh::kBuildVB + nseg + 1;
-    HIP_OK((hipError_t)mh::build_launch_level(d, nvb_bound, st));
-    HIP_OK(hipMemcpyAsync(back, d.ctr, sizeof(back), hipMemcpyDeviceToHost, st));
-    HIP_OK(hipMemcpyAsync(&err, cnt + 1, 4, hipMemcpyDeviceToHost, st));
+  d.seg_next = static_cast<mh::BuildSeg*>(at(o_seg1));
+  d.plan_next = static_cast<mh::BuildPlan*>(at(o_plan1));
+  // Level k holds at most 2^k nodes, which is a tight bound until nodes of few objects
+  // appear: those levels are launched one after the other, and only from then on does the
+  // host read the number of nodes back before it launches a level.
+  unsigned back[mh::kCtrCount] = {};
+  int64_t bound = serial_root ? 0 : 1;
+  bool counted = false;
+  for (int level = 0; bound > 0; ++level) {
+    if (level == mh::kMaxDepth)
+      return fail(MH_E_UNSUPPORTED, "tree deeper than %d levels", mh::kMaxDepth - 1);
+    d.level = level;
+    HIP_OK((hipError_t)mh::build_launch_level(d, bound, (int64_t)T / mh::kBuildVB + bound + 1, st));
+    std::swap(d.seg, d.seg_next);
+    std::swap(d.plan, d.plan_next);
+    bound = std::min(2 * bound, cap);
+    if (!counted && bound < cap) continue;
+    counted = true;
+    HIP_OK(hipMemcpyAsync(back, ctr, sizeof(back), hipMemcpyDeviceToHost, st));
     HIP_OK(hipStreamSynchronize(st));
-    if (err) break;
-    nseg = back[mh::kCtrNext];
-    std::swap(cur, nxt);
+    if (back[mh::kCtrErr]) break;
+    bound = back[mh::kCtrSegs + level + 1];
   }
-  HIP_OK(hipMemcpyAsync(back, d.ctr, sizeof(back), hipMemcpyDeviceToHost, st));
-  HIP_OK(hipMemcpyAsync(&err, cnt + 1, 4, hipMemcpyDeviceToHost, st));
+  HIP_OK(hipMemcpyAsync(back, ctr, sizeof(back), hipMemcpyDeviceToHost, st));
   HIP_OK(hipStreamSynchronize(st));
+  const unsigned err = back[mh::kCtrErr];
   if (err == 2) return fail(MH_E_INVALID, "non-finite vertex coordinate");
   if (err == 3) return fail(MH_E_UNSUPPORTED, "a leaf of more than 32767 objects");
   if (err) return fail(MH_E_STATE, "device build ran out of node records");
   HIP_OK((hipError_t)mh::build_launch_serial(d, back[mh::kCtrSmall], back[mh::kCtrBig],
-                                             scratch.as<int32_t>(), st));
+                                             static_cast<int32_t*>(at(o_scratch)), st));
   // Depths of the temporary tree, then its per-depth lists.
   HIP_OK(hipMemsetAsync(s->hist.p, 0, mh::kDepthHist * 4, st));
   HIP_OK((hipError_t)mh::launch_depths(d.u, s->anc0.as<int32_t>(), s->dep0.as<int32_t>(),
@@ -715,7 +716,7 @@ int build_device(mh_scene* s, int rtsah) {
   std::vector<unsigned> hist(mh::kDepthHist);
   unsigned used[2];
   HIP_OK(hipMemcpyAsync(hist.data(), s->hist.p, hist.size() * 4, hipMemcpyDeviceToHost, st));
-  HIP_OK(hipMemcpyAsync(used, cnt, 8, hipMemcpyDeviceToHost, st));
+  HIP_OK(hipMemcpyAsync(used, ctr, 8, hipMemcpyDeviceToHost, st));
   HIP_OK(hipStreamSynchronize(st));
   if (used[1]) return fail(MH_E_STATE, "device build ran out of node records");
   const unsigned deepest = hist[mh::kMaxDepth + 1];
@@ -732,19 +733,23 @@ int build_device(mh_scene* s, int rtsah) {
   HIP_OK((hipError_t)mh::launch_depth_scatter(d.u, s->dep0.as<int32_t>(), s->hist.as<unsigned>(),
                                               s->levels.as<int32_t>(), s->leaves.as<int32_t>(),
                                               st));
-  HIP_OK(hipMemsetAsync(fin.p, 0xFF, nrec * 4, st));
+  HIP_OK(hipMemsetAsync(at(o_fin), 0xFF, nrec * 4, st));
   mh::DevFinish f{};
-  f.trefs = trefs.as<mh::RefNode>();
+  f.trefs = d.u.refs;
   f.refs = s->refs.as<mh::RefNode>();
-  f.tcount = cnt;
-  f.ic = ic.as<int32_t>();
-  f.rank = rank.as<int32_t>();
-  f.fin = fin.as<int32_t>();
+  f.tcount = ctr;
+  f.ic = static_cast<int32_t*>(at(o_ic));
+  f.rank = static_cast<int32_t*>(at(o_rank));
+  f.fin = static_cast<int32_t*>(at(o_fin));
+  // written after the numbering, when these three are free
+  f.prob[0] = static_cast<float*>(at(o_ic));
+  f.prob[1] = static_cast<float*>(at(o_rank));
+  f.prob[2] = static_cast<float*>(at(o_scratch));
   f.levels = s->levels.as<int32_t>();
   f.leaves = s->leaves.as<int32_t>();
   f.costs = s->costs.as<float>();
   f.ssize = s->ssize.as<uint32_t>();
-  f.rt = rt.as<float>();
+  f.rt = static_cast<float*>(at(o_rt));
   f.logtab = s->logtab.as<float>();
   const uint32_t n_final = (uint32_t)(level_off.back() + n_leaves);
   f.n_records = (int32_t)nrec;
@@ -754,7 +759,7 @@ int build_device(mh_scene* s, int rtsah) {
   const int n_levels = (int)level_off.size() - 1;
   ++s->tree_gen;
   HIP_OK((hipError_t)mh::build_launch_ranks(f, level_off.data(), n_levels, n_leaves, st));
-  HIP_OK(hipMemcpyAsync(cnt, &n_final, 4, hipMemcpyHostToDevice, st));
+  HIP_OK(hipMemcpyAsync(s->counters.p, &n_final, 4, hipMemcpyHostToDevice, st));
   mh::DevRefit r{};
   r.tris = s->tris.as<float>();
   r.obj_ids = s->ids.as<int32_t>();

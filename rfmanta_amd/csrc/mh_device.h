@@ -210,8 +210,6 @@ struct DevUpdate {
   uint32_t* ssize;       // DynBVH::subtree_size, per record
   int32_t* parent;       // parent links of records built by leaf splits
   int32_t* ids;          // object_ids (leaf splits permute ranges)
-  float* obox;           // per object: lo xyz, hi xyz (null: formed from verts and idx)
-  float* ocen;           // per object: centroid xyz (null: formed from the object box)
   const float* verts;
   const uint32_t* idx;
   unsigned* next_free;   // records in use (nextFree)
@@ -224,7 +222,6 @@ struct DevUpdate {
   int32_t n_objects;     // T
   uint32_t large;        // largeSubtreeSize
 };
-int launch_obj_bounds(const DevUpdate& u, void* stream);
 // u.leaf_at from a leaf list (the caller sets every entry to -1 first).
 int launch_leaf_starts(const DevUpdate& u, const int32_t* leaves, int64_t n_leaves,
                        void* stream);
@@ -308,36 +305,43 @@ int launch_copy(void* dst, const void* src, size_t bytes, int cu_count, void* st
 // Device build (build.hip): DynBVH::rebuild with the approximate SAH at every node.
 constexpr int16_t kHole = -1;     // children of a temporary record no node uses
 constexpr int kBuildSerial = 64;  // nodes of at most this many objects: one wave each
-constexpr int kBuildVB = 2048;     // slots per virtual block of the level passes
+constexpr int kBuildVB = 1024;     // slots per virtual block of the level passes
 constexpr int kBuildBins = 16;     // BVH_num_samples (DynBVH.cc:34)
 
-// Accumulators of one level node, stored field-major ([field][node]) so the per-level
-// clear streams.
+// Accumulators of one level node, in 32-bit words: keys that reduce by minimum (maxima
+// negated), all cleared to ones, then counts, cleared to zero.
 enum : int {
-  kFcMin = 0,                    // 3 centroid min keys
-  kFcMax = 3,                    // 3 centroid max keys
-  kFbMin = 6,                    // 16 x 3 bin min keys
-  kFbMax = kFbMin + 3 * kBuildBins,   // 16 x 3 bin max keys
-  kFlMin = kFbMax + 3 * kBuildBins,   // 3 left-side min keys
-  kFlMax = kFlMin + 3,
-  kFrMin = kFlMax + 3,
-  kFrMax = kFrMin + 3,
-  kKeyFields = kFrMax + 3,
+  kAccBox = 0,                             // 64-bit keys: left and right box, 6 each
+  kAccCen = kAccBox + 2 * 12,              // left and right centroid box, 6 each
+  kAccBins = kAccCen + 12,                 // [6][bin] bin boxes
+  kAccCounts = kAccBins + 6 * kBuildBins,  // objects of each bin
+  kAccLess = kAccCounts + kBuildBins,      // objects left of the position
+  kAccWords = (kAccLess + 1 + 31) / 32 * 32,
 };
-enum : int { kFcnt = 0, kFless = kBuildBins, kCntFields = kBuildBins + 1 };
+static_assert(kAccCounts % 4 == 0, "cleared four words at a time");
 
 struct BuildSeg {  // a node of the current level: its temporary record and slot range
   int32_t rec, b, e, vb0;
 };
-struct BuildPlan {
-  int32_t axis, leaf, split, nless;
+struct BuildPlan {  // its binning and split
+  int32_t axis, leaf;
   float lo_c, scale, pos, width;
 };
 
-enum : int { kCtrNext = 0, kCtrSmall = 1, kCtrBig = 2, kCtrNvb = 3, kCtrCount = 4 };
+// Counters: records in use, error, small nodes, large leaves, then the nodes and the
+// virtual blocks of each level.
+enum : int {
+  kCtrRecords = 0,
+  kCtrErr = 1,
+  kCtrSmall = 2,
+  kCtrBig = 3,
+  kCtrSegs = 4,
+  kCtrNvb = kCtrSegs + kMaxDepth + 2,
+  kCtrCount = kCtrNvb + kMaxDepth + 2,
+};
 
 struct DevBuild {
-  DevUpdate u;                    // temporary records, ids, object boxes, counters
+  DevUpdate u;                    // temporary records, ids, mesh, counters
   float* slots;                   // 12 floats per slot: centroid, id, box
   const float* verts;
   int64_t n_verts;
@@ -346,20 +350,20 @@ struct DevBuild {
   BuildSeg* small;
   BuildSeg* big;
   BuildPlan* plan;
-  unsigned long long* acck;       // [kKeyFields][cap]
-  unsigned* accc;                 // [kCntFields][cap]
-  int64_t cap;                    // capacity of the node lists
+  BuildPlan* plan_next;
+  unsigned* acc;                  // [node][kAccWords]
   unsigned* ctr;                  // kCtr*
   int32_t* vbseg;                 // per virtual block: its node
-  unsigned* vcnt;                 // per virtual block: left, right misplaced counts
+  unsigned* vcnt;                 // per virtual block: objects left of the position (first
+                                  // word), then left, right misplaced counts
   unsigned* gscan;                // exclusive scans of vcnt (left at [0, nvb], right after)
   int64_t vcap;                   // capacity of the virtual block arrays
   int32_t* lpos;
   int32_t* rpos;
   unsigned long long* rootk;      // 6 keys: vertex box
-  int32_t nseg;
+  unsigned* rootc;                // 6 keys: box of the object centroids
+  int32_t level;
 };
-
 
 struct DevFinish {
   const RefNode* trefs;    // temporary records
@@ -373,6 +377,7 @@ struct DevFinish {
   float* costs;
   uint32_t* ssize;
   float* rt;               // RTSAH pairs (c0, c1) per final record
+  float* prob[3];          // crossing probabilities per entry of levels
   const float* logtab;
   int32_t n_records;
   int32_t n_final;         // records of the tree (inner + leaves)
@@ -381,7 +386,7 @@ struct DevFinish {
 };
 
 int build_launch_setup(const DevBuild& d, int serial, void* stream);
-int build_launch_level(const DevBuild& d, int64_t nvb_bound, void* stream);
+int build_launch_level(const DevBuild& d, int64_t nseg_bound, int64_t nvb_bound, void* stream);
 int build_launch_serial(const DevBuild& d, int64_t n_small, int64_t n_big, int32_t* scratch,
                         void* stream);
 int build_launch_ranks(const DevFinish& f, const int64_t* level_off, int n_levels,

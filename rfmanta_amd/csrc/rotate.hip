@@ -9,8 +9,6 @@
 // (DynBVH.cc:3051-3372). A node only touches records of its own subtree, so all nodes of
 // one depth (depth taken at the start of the frame) run in parallel, deepest first, one
 // thread per node:
-//   k_obj_bounds     per object: box and centroid (DynBVH.cc:2018-2030), for the device
-//                    build; the update forms them from the vertices where it needs them
 //   k_upd_leaves     one lane per object slot, the first slot of each leaf doing the leaf:
 //                    leaf boxes (DynBVH.cc:2091-2097), and a list of the leaves the
 //                    parent's rotation may split
@@ -229,23 +227,6 @@ __device__ void rotate_node(const DevUpdate& u, int node) {
       mark(RL);
       mark(RR);
     }
-  }
-}
-
-__global__ __launch_bounds__(kBlock) void k_obj_bounds(DevUpdate u) {
-  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (i >= u.n_objects) return;
-  Box b;
-  const float* p0 = u.verts + 3 * (size_t)u.idx[3 * i + 0];
-  for (int k = 0; k < 3; ++k) b.lo[k] = b.hi[k] = p0[k];  // Mesh::getBBox (Mesh.cc:228-237)
-  extend_pt(b, u.verts + 3 * (size_t)u.idx[3 * i + 1]);
-  extend_pt(b, u.verts + 3 * (size_t)u.idx[3 * i + 2]);
-  float* o = u.obox + 6 * (size_t)i;
-  for (int k = 0; k < 3; ++k) {
-    o[k] = b.lo[k];
-    o[3 + k] = b.hi[k];
-    // BBox::center = Interpolate(min, max, 0.5f) (BBox.h:63-65, MiscMath.h:136-139)
-    u.ocen[3 * (size_t)i + k] = b.hi[k] * 0.5f + b.lo[k] * (1 - 0.5f);
   }
 }
 
@@ -576,13 +557,6 @@ int64_t depth_chunk(int64_t n, unsigned& blocks) {
 }
 
 }  // namespace
-
-int launch_obj_bounds(const DevUpdate& u, void* stream) {
-  if (u.n_objects <= 0) return 0;
-  hipLaunchKernelGGL(k_obj_bounds, dim3(grid(u.n_objects)), dim3(kBlock), 0,
-                     reinterpret_cast<hipStream_t>(stream), u);
-  return (int)hipGetLastError();
-}
 
 int launch_leaf_starts(const DevUpdate& u, const int32_t* leaves, int64_t n_leaves,
                        void* stream) {

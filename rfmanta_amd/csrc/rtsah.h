@@ -191,11 +191,10 @@ struct CostPair {
 
 MH_HD inline CostPair leaf_cost(int children) { return CostPair{children * 3.0f + 1.0f, 0.0f}; }
 
-// An inner node's pair from its children's; left_cheaper receives isLeftCheaper.
-MH_HD inline CostPair combine(const float* tab, const Aabb& P, const Aabb& Lb, const Aabb& Rb,
-                              const CostPair& L, const CostPair& R, bool& left_cheaper) {
-  float Plr, Pjl, Pjr;
-  probabilities(tab, P, Lb, Rb, Plr, Pjl, Pjr);
+// An inner node's pair from its children's and the node's crossing probabilities;
+// left_cheaper receives isLeftCheaper.
+MH_HD inline CostPair combine(float Plr, float Pjl, float Pjr, const CostPair& L,
+                              const CostPair& R, bool& left_cheaper) {
   const float Pl = Pjl + Plr, Pr = Pjr + Plr;
   const float Pe = 1 - Pjr - Pjl - Plr;
   const float lc = Pl * L.c0 + (Pjr + Plr * L.c1) * R.c0 + (1 + Pl * L.c1 + (1 - Pl)) * 1.0f;
@@ -204,6 +203,12 @@ MH_HD inline CostPair combine(const float* tab, const Aabb& P, const Aabb& Lb, c
   c1 = c1 <= 0.0f ? 0.0f : (c1 >= 1.0f ? 1.0f : c1);
   left_cheaper = lc < rc;
   return CostPair{lo_of(lc, rc), c1};
+}
+MH_HD inline CostPair combine(const float* tab, const Aabb& P, const Aabb& Lb, const Aabb& Rb,
+                              const CostPair& L, const CostPair& R, bool& left_cheaper) {
+  float Plr, Pjl, Pjr;
+  probabilities(tab, P, Lb, Rb, Plr, Pjl, Pjr);
+  return combine(Plr, Pjl, Pjr, L, R, left_cheaper);
 }
 
 }  // namespace rtsah
