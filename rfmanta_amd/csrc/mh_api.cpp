@@ -1071,6 +1071,7 @@ int mh_scene_update(mh_scene* s, void* stream) {
   u.split_list = s->split_list.as<int32_t>();
   u.split_count = nfree + 2;
   u.n_records = (int32_t)nrec;
+  u.n_old = (int32_t)s->next_free;
   // largeSubtreeSize = nodes.size() / (20 * numProcs) (DynBVH.cc:1776)
   u.large = (uint32_t)(nrec / (20 * (size_t)s->workers));
   ++s->tree_gen;

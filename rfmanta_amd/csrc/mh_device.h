@@ -219,13 +219,14 @@ struct DevUpdate {
   int32_t* leaf_at;      // per slot, the leaf whose first slot it is, else -1
   int32_t* irregular;    // update: [1] is set by the leaf pass for a NaN box
   int32_t n_records;     // capacity, 2T
+  int32_t n_old;         // update: records in use before the frame's leaf splits
   int32_t n_objects;     // T
   uint32_t large;        // largeSubtreeSize
 };
 // u.leaf_at from a leaf list (the caller sets every entry to -1 first).
 int launch_leaf_starts(const DevUpdate& u, const int32_t* leaves, int64_t n_leaves,
                        void* stream);
-// Leaf pass over the object slots (u.leaf_at), leaf splits, then one launch per depth
+// Leaf pass over the object slots (u.leaf_at), leaf splits, then one launch per two depths
 // (deepest first).
 int launch_update_tree(const DevUpdate& u, int64_t n_leaves, const int32_t* levels,
                        const LevelList* lev, int n_levels, void* stream);

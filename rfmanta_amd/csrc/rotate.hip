@@ -13,7 +13,7 @@
 //                    leaf boxes (DynBVH.cc:2091-2097), and a list of the leaves the
 //                    parent's rotation may split
 //   k_split_leaves   those splits, ahead of the rotations (same subtrees)
-//   k_upd_level      one launch per depth: union of the child boxes, then rotateNode
+//   k_upd_level      one launch per two depths: union of the child boxes, then rotateNode
 //   k_upd_top        the same for the small depths at the top, in one workgroup
 // The next frame's level lists and the wide nodes of the new tree follow in wide.hip. (The
 // depth pass k_parents, k_jump, k_depth_hist, k_depth_scatter serves the device build, whose
@@ -35,6 +35,24 @@ namespace mh {
 namespace {
 
 constexpr int kBlock = 256;
+
+// A record as two 16-byte words: lo.x lo.y lo.z hi.x | hi.y hi.z child word, where word
+// holds axis (byte 0), bits (byte 1) and children (int16, bytes 2-3).
+struct RecWords {
+  float4 a, b;
+};
+__device__ __forceinline__ RecWords load_rec(const RefNode* refs, int64_t r) {
+  const float4* p = reinterpret_cast<const float4*>(refs + r);
+  return RecWords{p[0], p[1]};
+}
+__device__ __forceinline__ int rec_child(const RecWords& w) { return __float_as_int(w.b.z); }
+__device__ __forceinline__ int rec_children(const RecWords& w) {
+  return __float_as_int(w.b.w) >> 16;  // arithmetic shift: the int16 with its sign
+}
+__device__ __forceinline__ Box rec_box(const RecWords& w) {
+  return Box{{w.a.x, w.a.y, w.a.z}, {w.a.w, w.b.x, w.b.y}};
+}
+
 __device__ __forceinline__ void swap_rec(const DevUpdate& u, int a, int b) {
   int4* pa = reinterpret_cast<int4*>(u.refs + a);
   int4* pb = reinterpret_cast<int4*>(u.refs + b);
@@ -51,10 +69,9 @@ __device__ __forceinline__ void swap_rec(const DevUpdate& u, int a, int b) {
   u.ssize[b] = z;
 }
 
-__device__ __forceinline__ Box unite(const DevUpdate& u, int a, int b) {
-  Box x = rbox(u.refs[a]);
-  extend(x, rbox(u.refs[b]));
-  return x;
+__device__ __forceinline__ Box unite(Box a, const Box& b) {
+  extend(a, b);
+  return a;
 }
 
 // Step 3 of rotateNode: the axis of largest overlap and child order (DynBVH.cc:3305-3352).
@@ -69,31 +86,50 @@ __device__ void guess_axis(const DevUpdate& u, int parent, int a, int b) {
   if (ha > hb) swap_rec(u, a, b);
 }
 
-// DynBVH::rotateNode (DynBVH.cc:3051-3372)
-__device__ void rotate_node(const DevUpdate& u, int node) {
+// One inner node of the update: the union of its child boxes (DynBVH.cc:2110-2116), then
+// DynBVH::rotateNode (DynBVH.cc:3051-3372). `tail` is the second half of the node's record.
+// The children, and then the grandchildren of both sides with their costs, are loaded
+// together before anything is stored (of a leaf child, the children once more): a lane
+// waits for three loads in a row, and most nodes end with their own record and cost stored.
+__device__ void upd_node(const DevUpdate& u, int node, const float4& tail) {
   RefNode* refs = u.refs;
   float* costs = u.costs;
   uint32_t* ss = u.ssize;
-  const int L = refs[node].child, R = L + 1;
+  const int L = __float_as_int(tail.z), R = L + 1;
+  const RecWords wl = load_rec(refs, L), wr = load_rec(refs, R);
+  const float costL = costs[L], costR = costs[R];
   // rotateNode first splits leaf children of more than one object with the approximate SAH
   // (DynBVH.cc:3057-3069); k_split_leaves has done that for every leaf before the levels.
-  const int LL = refs[L].child, LR = LL + 1, RL = refs[R].child, RR = RL + 1;
-  const bool l_inner = refs[L].children == 0, r_inner = refs[R].children == 0;
-  const float nodeArea = area(rbox(refs[node]));
-  const float leftArea = area(rbox(refs[L]));
-  const float rightArea = area(rbox(refs[R]));
+  const bool l_inner = rec_children(wl) == 0, r_inner = rec_children(wr) == 0;
+  const int LL = l_inner ? rec_child(wl) : L, LR = LL + 1;
+  const int RL = r_inner ? rec_child(wr) : L, RR = RL + 1;
+  const RecWords wll = load_rec(refs, LL), wlr = load_rec(refs, LR);
+  const RecWords wrl = load_rec(refs, RL), wrr = load_rec(refs, RR);
+  const float costLL = costs[LL], costLR = costs[LR], costRL = costs[RL], costRR = costs[RR];
+  const Box bl = rec_box(wl), br = rec_box(wr);
+  const Box bll = rec_box(wll), blr = rec_box(wlr), brl = rec_box(wrl), brr = rec_box(wrr);
+  Box b;
+  reset(b);
+  extend(b, bl);
+  extend(b, br);
+  float4* self = reinterpret_cast<float4*>(refs + node);
+  self[0] = make_float4(b.lo[0], b.lo[1], b.lo[2], b.hi[0]);
+  self[1] = make_float4(b.hi[1], b.hi[2], tail.z, tail.w);
+  const float nodeArea = area(b);
+  const float leftArea = area(bl);
+  const float rightArea = area(br);
   float llA = 0.f, lrA = 0.f, rlA = 0.f, rrA = 0.f;
   Box boxA, boxB;
   reset(boxA);
   reset(boxB);
   float areaA = 0.f, areaB = 0.f;
   int best = 0;
-  float bestCost = nodeArea * kCTrav + leftArea * costs[L] + rightArea * costs[R];
+  float bestCost = nodeArea * kCTrav + leftArea * costL + rightArea * costR;
   if (l_inner) {
-    llA = area(rbox(refs[LL]));
-    lrA = area(rbox(refs[LR]));
-    const float partial = nodeArea * kCTrav + rightArea * costs[R] + lrA * costs[LR] + llA * costs[LL];
-    const Box b1 = unite(u, R, LR);
+    llA = area(bll);
+    lrA = area(blr);
+    const float partial = nodeArea * kCTrav + rightArea * costR + lrA * costLR + llA * costLL;
+    const Box b1 = unite(br, blr);
     const float a1 = area(b1);
     const float c1 = a1 * kCTrav + partial;
     if (c1 < bestCost) {
@@ -102,7 +138,7 @@ __device__ void rotate_node(const DevUpdate& u, int node) {
       boxA = b1;
       areaA = a1;
     }
-    const Box b2 = unite(u, R, LL);
+    const Box b2 = unite(br, bll);
     const float a2 = area(b2);
     const float c2 = a2 * kCTrav + partial;
     if (c2 < bestCost) {
@@ -113,10 +149,10 @@ __device__ void rotate_node(const DevUpdate& u, int node) {
     }
   }
   if (r_inner) {
-    rlA = area(rbox(refs[RL]));
-    rrA = area(rbox(refs[RR]));
-    const float partial = nodeArea * kCTrav + leftArea * costs[L] + rrA * costs[RR] + rlA * costs[RL];
-    const Box b3 = unite(u, L, RR);
+    rlA = area(brl);
+    rrA = area(brr);
+    const float partial = nodeArea * kCTrav + leftArea * costL + rrA * costRR + rlA * costRL;
+    const Box b3 = unite(bl, brr);
     const float a3 = area(b3);
     const float c3 = a3 * kCTrav + partial;
     if (c3 < bestCost) {
@@ -125,7 +161,7 @@ __device__ void rotate_node(const DevUpdate& u, int node) {
       boxA = b3;
       areaA = a3;
     }
-    const Box b4 = unite(u, L, RL);
+    const Box b4 = unite(bl, brl);
     const float a4 = area(b4);
     const float c4 = a4 * kCTrav + partial;
     if (c4 < bestCost) {
@@ -135,8 +171,8 @@ __device__ void rotate_node(const DevUpdate& u, int node) {
       areaA = a4;
     }
     if (l_inner) {
-      const float partial2 = nodeArea * kCTrav + llA * costs[LL] + lrA * costs[LR] + rlA * costs[RL] + rrA * costs[RR];
-      const Box b5l = unite(u, LL, RL), b5r = unite(u, LR, RR);
+      const float partial2 = nodeArea * kCTrav + llA * costLL + lrA * costLR + rlA * costRL + rrA * costRR;
+      const Box b5l = unite(bll, brl), b5r = unite(blr, brr);
       const float a5l = area(b5l), a5r = area(b5r);
       const float c5 = (a5l + a5r) * kCTrav + partial2;
       if (c5 < bestCost) {
@@ -147,7 +183,7 @@ __device__ void rotate_node(const DevUpdate& u, int node) {
         boxB = b5r;
         areaB = a5r;
       }
-      const Box b6l = unite(u, LL, RR), b6r = unite(u, RL, LR);
+      const Box b6l = unite(bll, brr), b6r = unite(brl, blr);
       const float a6l = area(b6l), a6r = area(b6r);
       const float c6 = (a6l + a6r) * kCTrav + partial2;
       if (c6 < bestCost) {
@@ -166,33 +202,33 @@ __device__ void rotate_node(const DevUpdate& u, int node) {
   switch (best) {
     case 1:
       set_box(refs[L], boxA);
-      costs[L] = kCTrav + ((lrA * costs[LR] + rightArea * costs[R]) * invA);
+      costs[L] = kCTrav + ((lrA * costLR + rightArea * costR) * invA);
       swap_rec(u, LL, R);
       ss[L] = ss[LL] + ss[LR] + 1;
       break;
     case 2:
       set_box(refs[L], boxA);
-      costs[L] = kCTrav + ((llA * costs[LL] + rightArea * costs[R]) * invA);
+      costs[L] = kCTrav + ((llA * costLL + rightArea * costR) * invA);
       swap_rec(u, LR, R);
       ss[L] = ss[LL] + ss[LR] + 1;
       break;
     case 3:
       set_box(refs[R], boxA);
-      costs[R] = kCTrav + ((rrA * costs[RR] + leftArea * costs[L]) * invA);
+      costs[R] = kCTrav + ((rrA * costRR + leftArea * costL) * invA);
       swap_rec(u, RL, L);
       ss[R] = ss[RL] + ss[RR] + 1;
       break;
     case 4:
       set_box(refs[R], boxA);
-      costs[R] = kCTrav + ((rlA * costs[RL] + leftArea * costs[L]) * invA);
+      costs[R] = kCTrav + ((rlA * costRL + leftArea * costL) * invA);
       swap_rec(u, RR, L);
       ss[R] = ss[RL] + ss[RR] + 1;
       break;
     case 5:
       set_box(refs[L], boxA);
       set_box(refs[R], boxB);
-      costs[L] = kCTrav + ((llA * costs[LL] + rlA * costs[RL]) * invA);
-      costs[R] = kCTrav + ((lrA * costs[LR] + rrA * costs[RR]) / areaB);
+      costs[L] = kCTrav + ((llA * costLL + rlA * costRL) * invA);
+      costs[R] = kCTrav + ((lrA * costLR + rrA * costRR) / areaB);
       swap_rec(u, LR, RL);
       ss[L] = ss[LL] + ss[LR] + 1;
       ss[R] = ss[RL] + ss[RR] + 1;
@@ -200,8 +236,8 @@ __device__ void rotate_node(const DevUpdate& u, int node) {
     default:  // 6
       set_box(refs[L], boxA);
       set_box(refs[R], boxB);
-      costs[L] = kCTrav + ((llA * costs[LL] + rrA * costs[RR]) * invA);
-      costs[R] = kCTrav + ((lrA * costs[LR] + rlA * costs[RL]) / areaB);
+      costs[L] = kCTrav + ((llA * costLL + rrA * costRR) * invA);
+      costs[R] = kCTrav + ((lrA * costLR + rlA * costRL) / areaB);
       swap_rec(u, LR, RR);
       ss[L] = ss[LL] + ss[LR] + 1;
       ss[R] = ss[RL] + ss[RR] + 1;
@@ -296,30 +332,51 @@ __global__ __launch_bounds__(kBlock) void k_split_leaves(DevUpdate u) {
     split_leaf(u, u.split_list[i]);
 }
 
-// One inner node of the update: the union of its child boxes, then rotateNode.
+__device__ __forceinline__ float4 rec_tail(const DevUpdate& u, int rec) {
+  return reinterpret_cast<const float4*>(u.refs + rec)[1];
+}
 __device__ __forceinline__ void upd_node(const DevUpdate& u, int node) {
-  const int c = u.refs[node].child;
-  Box b;
-  reset(b);
-  extend(b, rbox(u.refs[c]));
-  extend(b, rbox(u.refs[c + 1]));
-  set_box(u.refs[node], b);
-  rotate_node(u, node);
+  upd_node(u, node, rec_tail(u, node));
+}
+
+// Entry i of an even level list and its children, by a pair of lanes: each lane does the
+// child on its side if that was an inner record when the frame began (a leaf split this
+// frame leads to a record from n_old on and is not rotated), then the first lane the entry
+// itself. A depth reads each node's children and grandchildren, so a launch per depth reads
+// every record three times and is bound by those reads; two depths a launch read half of
+// them from the caches. Rotations of an 8M-triangle heightfield: 586 us a depth at a time,
+// 526 us by pairs of depths, 427 us with the loads of a node together (upd_node).
+__device__ __forceinline__ void upd_entry(const DevUpdate& u, const int32_t* recs, int64_t i,
+                                          bool live) {
+  const int side = threadIdx.x & 1;
+  int node = 0;
+  float4 tail = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (live) {
+    node = recs[i];
+    tail = rec_tail(u, node);
+    const int kid = __float_as_int(tail.z) + side;
+    const float4 kt = rec_tail(u, kid);
+    if ((__float_as_int(kt.w) >> 16) == 0 && __float_as_int(kt.z) < u.n_old) upd_node(u, kid, kt);
+  }
+  __syncthreads();
+  if (live && side == 0) upd_node(u, node, tail);
 }
 
 __global__ __launch_bounds__(kBlock) void k_upd_level(DevUpdate u, const int32_t* recs,
                                                       int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  upd_node(u, recs[i]);
+  const int64_t i = ((int64_t)blockIdx.x * kBlock + threadIdx.x) >> 1;
+  upd_entry(u, recs, i, i < n);
 }
 
-// The top depths [0, t.n), deepest first, in one workgroup: the barrier between depths
-// orders them as separate launches would (the workgroup's waves share one compute unit
-// and its L1, so stores before the barrier are seen by loads after it).
+// The top even depths, deepest first, in one workgroup: the barrier between depths orders
+// them as separate launches would (the workgroup's waves share one compute unit and its
+// L1, so stores before the barrier are seen by loads after it).
 __global__ __launch_bounds__(kBlock) void k_upd_top(DevUpdate u, const int32_t* recs, TopLevels t) {
   for (int d = t.n - 1; d >= 0; --d) {
-    for (int i = (int)threadIdx.x; i < t.cnt[d]; i += kBlock) upd_node(u, recs[t.first[d] + i]);
+    for (int i0 = 0; i0 < 2 * t.cnt[d]; i0 += kBlock) {
+      const int i = (i0 + (int)threadIdx.x) >> 1;
+      upd_entry(u, recs + t.first[d], i, i < t.cnt[d]);
+    }
     __syncthreads();
   }
 }
@@ -329,20 +386,6 @@ __global__ __launch_bounds__(kBlock) void k_upd_top(DevUpdate u, const int32_t* 
 __device__ __forceinline__ int64_t used(const unsigned* next_free, int32_t n_records) {
   const unsigned n = *next_free;
   return n < (unsigned)n_records ? (int64_t)n : (int64_t)n_records;
-}
-
-// A record as two 16-byte words: lo.x lo.y lo.z hi.x | hi.y hi.z child word, where word
-// holds axis (byte 0), bits (byte 1) and children (int16, bytes 2-3).
-struct RecWords {
-  float4 a, b;
-};
-__device__ __forceinline__ RecWords load_rec(const RefNode* refs, int64_t r) {
-  const float4* p = reinterpret_cast<const float4*>(refs + r);
-  return RecWords{p[0], p[1]};
-}
-__device__ __forceinline__ int rec_child(const RecWords& w) { return __float_as_int(w.b.z); }
-__device__ __forceinline__ int rec_children(const RecWords& w) {
-  return __float_as_int(w.b.w) >> 16;  // arithmetic shift: the int16 with its sign
 }
 
 // Child reference of a PairNode for a loaded record: its pair index (inner) or its leaf
@@ -576,10 +619,10 @@ int launch_update_tree(const DevUpdate& u, int64_t n_leaves, const int32_t* leve
     hipLaunchKernelGGL(k_split_leaves, dim3(g < 1024 ? g : 1024), dim3(kBlock), 0, s, u);
   }
   TopLevels t;
-  const int top = top_levels(lev, n_levels, 1, t);
-  for (int d = n_levels - 1; d >= top; --d)
+  const int top = 2 * top_levels(lev, n_levels, 2, t);
+  for (int d = (n_levels - 1) & ~1; d >= top; d -= 2)
     if (lev[d].n > 0)
-      hipLaunchKernelGGL(k_upd_level, dim3(grid(lev[d].n)), dim3(kBlock), 0, s, u,
+      hipLaunchKernelGGL(k_upd_level, dim3(grid(2 * lev[d].n)), dim3(kBlock), 0, s, u,
                          levels + lev[d].first, lev[d].n);
   if (top > 0) hipLaunchKernelGGL(k_upd_top, dim3(1), dim3(kBlock), 0, s, u, levels, t);
   return (int)hipGetLastError();
