@@ -7,10 +7,15 @@
 //
 // k_trace_packet: one RayPacket of up to 64 consecutive rays per wave, the reference's
 //   packet recursion (intersectNode/firstIntersects/lastIntersects, DynBVH.cc:274-905,
-//   scalar branch). Node records are read with uniform (scalar) loads, each lane tests
-//   its own ray, and ballots give firstActive/lastActive. The interval-arithmetic
-//   frustum test (DynBVH.cc:682-721) runs on wave-reduced ray bounds. The wave-uniform
-//   stack of (node, firstActive) lives in LDS.
+//   scalar branch). Node and triangle records are read with uniform (scalar) loads, each
+//   lane tests its own ray, and everything about the packet (rays still looking, rays that
+//   hit, firstActive/lastActive, child order) is kept as wave-uniform masks. The
+//   interval-arithmetic frustum test (DynBVH.cc:682-721) runs on wave-reduced ray bounds.
+//   Bound by vector issue, so what is uniform stays in scalar registers (vector loads of
+//   the records, vector masks and a stack in LDS took 1.16 times as long: 801 against
+//   706 us for 2.07M camera rays in packets of 64 over a 1M-triangle heightfield). Testing
+//   both children at their parent, so that the farther one need not be pushed, was slower
+//   (849 us): a child that is hit is then tested twice.
 //
 // Arithmetic follows the reference's scalar build operation for operation: no
 // contraction (the library is compiled with -ffp-contract=off), IEEE division for
@@ -36,7 +41,6 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr int kWaves = kBlock / 64;
-constexpr int kPacketStack = 128;
 
 // ---------------------------------------------------------------------------
 // Single-ray traversal of the reference's records (traverse.h), grid-stride over the rays.
@@ -67,6 +71,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) 
 // Packet traversal (one RayPacket per wave)
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
+__device__ __forceinline__ float uni(float x) { return __int_as_float(uni(__float_as_int(x))); }
+using Mask = unsigned long long;
+__device__ __forceinline__ Mask mask_of(bool x) { return __builtin_amdgcn_ballot_w64(x); }
 __device__ __forceinline__ int lowest(unsigned long long m) { return __builtin_ctzll(m); }
 __device__ __forceinline__ int highest(unsigned long long m) { return 63 - __builtin_clzll(m); }
 
@@ -112,13 +119,45 @@ struct IA {
   float min_rcp[3], max_rcp[3], min_org[3], max_org[3];
 };
 
+// Records at wave-uniform indices, through the scalar cache.
+typedef float Float4 __attribute__((ext_vector_type(4)));
+typedef const __attribute__((address_space(4))) Float4* UniformWords;
+__device__ __forceinline__ UniformWords uniform_words(const void* p) {
+  return (UniformWords)reinterpret_cast<unsigned long long>(p);
+}
+struct UniformNode {
+  float lo[3], hi[3];
+  int child, word;
+  __device__ __forceinline__ UniformNode(const RefNode* refs, int i) {
+    const UniformWords p = uniform_words(refs + i);
+    const Float4 a = p[0], b = p[1];
+    lo[0] = a.x;
+    lo[1] = a.y;
+    lo[2] = a.z;
+    hi[0] = a.w;
+    hi[1] = b.x;
+    hi[2] = b.y;
+    child = __float_as_int(b.z);
+    word = __float_as_int(b.w);
+  }
+  __device__ __forceinline__ int children() const { return word >> 16; }
+  __device__ __forceinline__ int axis() const { return word & 255; }
+  __device__ __forceinline__ int left_cheaper() const { return (word >> 8) & 1; }
+};
+__device__ __forceinline__ PrimRecord uniform_prim(const DevScene& sc, int slot) {
+  const UniformWords p = uniform_words(sc.tris + 12 * (int64_t)slot);
+  const Float4 a = p[0], b = p[1], c = p[2];
+  return PrimRecord{make_float4(a.x, a.y, a.z, a.w), make_float4(b.x, b.y, b.z, b.w),
+                    make_float4(c.x, c.y, c.z, c.w)};
+}
+
 // Interval-arithmetic frustum exit of the scalar firstIntersects (DynBVH.cc:682-721).
-__device__ __forceinline__ bool frustum_miss(const RefNode& nd, const IA& ia) {
+__device__ __forceinline__ bool frustum_miss(const UniformNode& nd, const IA& ia) {
   float tmin_f = 1e-5f, tmax_f = FLT_MAX;
 #pragma unroll
   for (int axis = 0; axis < 3; ++axis) {
-    float a = nd.box.lo[axis] - ia.max_org[axis];
-    float b = nd.box.hi[axis] - ia.min_org[axis];
+    float a = nd.lo[axis] - ia.max_org[axis];
+    float b = nd.hi[axis] - ia.min_org[axis];
     const float ar0 = a * ia.min_rcp[axis];
     const float ar1 = a * ia.max_rcp[axis];
     const float br0 = b * ia.min_rcp[axis];
@@ -139,7 +178,6 @@ template <bool ANY, int PRIM, bool STATS>
 __global__ __launch_bounds__(kBlock) void k_trace_packet(DevScene sc, DevRays rays,
                                                          DevHits hits, int64_t n, int psize,
                                                          unsigned long long* counters) {
-  __shared__ int2 stk[kWaves][kPacketStack];
   const int lane = threadIdx.x & 63;
   const int wv = threadIdx.x >> 6;
   const int64_t pk = (int64_t)blockIdx.x * kWaves + wv;
@@ -169,54 +207,85 @@ __global__ __launch_bounds__(kBlock) void k_trace_packet(DevScene sc, DevRays ra
   const bool contrib = st == 0;
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
-    ia.min_rcp[a] = fold_min(r.inv[a], contrib, lane);
-    ia.max_rcp[a] = fold_max(r.inv[a], contrib, lane);
-    ia.min_org[a] = fold_min(r.o[a], contrib, lane);
-    ia.max_org[a] = fold_max(r.o[a], contrib, lane);
+    ia.min_rcp[a] = uni(fold_min(r.inv[a], contrib, lane));
+    ia.max_rcp[a] = uni(fold_max(r.inv[a], contrib, lane));
+    ia.min_org[a] = uni(fold_min(r.o[a], contrib, lane));
+    ia.max_org[a] = uni(fold_max(r.o[a], contrib, lane));
   }
 
   int pos = -1;
   float hu = 0.f, hv = 0.f;
   unsigned long long nbox = 0, ntri = 0;
-  int sp = 0;
-  stk[wv][sp++] = make_int2(0, 0);
-  while (sp > 0) {
-    --sp;
-    const int2 e = stk[wv][sp];
-    const int nid = uni(e.x);
-    const int b = uni(e.y);
-    const RefNode nd = sc.refs[nid];
-    const bool elig = in && lane >= b && st != -1 && !(ANY && st == 1);
-    const unsigned long long E = __ballot(elig);
-    if (E == 0) continue;
-    const int rb = lowest(E);
+  // Rays and boxes for which the min/max form of the slab test is exact: no product is a
+  // NaN with finite origins, finite reciprocals other than zero and boxes without NaNs.
+  bool plain = regular_ray(r, minT) && r.inv[0] != 0.f && r.inv[1] != 0.f && r.inv[2] != 0.f;
+  plain = mask_of(in && !plain) == 0 && *sc.irregular == 0;
+  Mask alive = mask_of(st == 0);  // rays still looking
+  const Mask pos_x = mask_of(r.d[0] > 0.f), pos_y = mask_of(r.d[1] > 0.f),
+             pos_z = mask_of(r.d[2] > 0.f);
+  // The stack of (node, firstActive), at most 126 entries (the host refuses deeper trees):
+  // entry k in lane k % 64 of a register pair, written and read at a wave-uniform index.
+  int stk_node[2] = {0, 0}, stk_b[2] = {0, 0};
+  int sp = 0, nid = 0, b = 0;
+  for (;;) {
+    const UniformNode nd(sc.refs, nid);
+    const Mask E = alive & (~(Mask)0 << b);
     float tn;
-    const bool hb = elig && slab(nd.box.lo[0], nd.box.hi[0], nd.box.lo[1], nd.box.hi[1],
-                                 nd.box.lo[2], nd.box.hi[2], r, minT, tn);
-    const unsigned long long H = __ballot(hb);
-    if (!((H >> rb) & 1ull)) {
+    Mask H;
+    if (plain)
+      H = mask_of(slab_fast(nd.lo[0], nd.hi[0], nd.lo[1], nd.hi[1], nd.lo[2], nd.hi[2], r, minT,
+                            tn));
+    else
+      H = mask_of(slab(nd.lo[0], nd.hi[0], nd.lo[1], nd.hi[1], nd.lo[2], nd.hi[2], r, minT, tn));
+    H &= E;
+    // (a node that no ray hits is left either way; the frustum test only counts then)
+    if (E != 0 && !((H >> lowest(E)) & 1) && (STATS || H != 0)) {
       if (frustum_miss(nd, ia)) {
         if (STATS) nbox += 1;
-        continue;
+        H = 0;
+      } else if (STATS && H == 0) {
+        nbox += __popcll(E);
       }
     }
-    if (H == 0) {
-      if (STATS) nbox += __popcll(E);
-      continue;
-    }
-    const int fa = lowest(H);
-    if (STATS) nbox += __popcll(E & (fa >= 63 ? ~0ull : ((2ull << fa) - 1)));
-    if (nd.children != 0) {
-      const unsigned long long Lm = H & above(b);
+    if (H != 0) {
+      const int fa = lowest(H);
+      if (STATS) nbox += __popcll(E & (fa >= 63 ? ~0ull : ((2ull << fa) - 1)));
+      if (nd.children() == 0) {
+        int front;
+        if (ANY) {
+          front = nd.left_cheaper() ? 0 : 1;
+        } else {
+          const int axis = nd.axis();
+          const Mask ahead = axis == 0 ? pos_x : (axis == 1 ? pos_y : pos_z);
+          front = ((ahead >> fa) & 1) ? 0 : 1;
+        }
+        const int other = nd.child + 1 - front;
+        const bool here = lane == (sp & 63);
+        if (sp < 64) {
+          stk_node[0] = here ? other : stk_node[0];
+          stk_b[0] = here ? fa : stk_b[0];
+        } else {
+          stk_node[1] = here ? other : stk_node[1];
+          stk_b[1] = here ? fa : stk_b[1];
+        }
+        ++sp;
+        nid = nd.child + front;
+        b = fa;
+        continue;
+      }
+      const Mask Lm = H & above(b);
       const int la = Lm ? highest(Lm) : b;
       int sb = fa, se = la + 1;
-      for (int k = 0; k < nd.children; ++k) {
-        const int slot = nd.child + k;
+      const int end = nd.child + nd.children();
+      PrimRecord next = uniform_prim(sc, nd.child);
+      for (int slot = nd.child; slot < end; ++slot) {
+        const PrimRecord tri = next;
+        if (slot + 1 < end) next = uniform_prim(sc, slot + 1);
         if (STATS) ntri += (unsigned long long)(se - sb);
         const bool act = lane >= sb && lane < se;
         if (act) {
           float t, u, v;
-          if (prim_test<PRIM>(sc, slot, r, minT, t, u, v)) {
+          if (record_test<PRIM>(tri, r, minT, t, u, v)) {
             minT = t;
             st = 1;
             pos = slot;
@@ -229,24 +298,24 @@ __global__ __launch_bounds__(kBlock) void k_trace_packet(DevScene sc, DevRays ra
           // subpacket shrinks to the rays still unoccluded.
           const bool hit_here = act && st == 1;
           if (hit_here) minT = kEps;
-          if (__ballot(hit_here)) {
-            const unsigned long long alive = __ballot(act && st == 0);
-            if (!alive) break;
-            sb = lowest(alive);
-            se = highest(alive) + 1;
+          if (mask_of(hit_here)) {
+            alive &= ~mask_of(hit_here);
+            const Mask left = mask_of(act && st == 0);
+            if (!left) break;
+            sb = lowest(left);
+            se = highest(left) + 1;
           }
         }
       }
+    }
+    if (sp == 0) break;
+    --sp;
+    if (sp < 64) {
+      nid = __builtin_amdgcn_readlane(stk_node[0], sp);
+      b = __builtin_amdgcn_readlane(stk_b[0], sp);
     } else {
-      int front;
-      if (ANY) {
-        front = (nd.bits & 1) ? 0 : 1;
-      } else {
-        const float da = pick3(nd.axis, r.d[0], r.d[1], r.d[2]);
-        front = (__shfl(da, fa, 64) > 0.f) ? 0 : 1;
-      }
-      stk[wv][sp++] = make_int2(nd.child + 1 - front, fa);
-      stk[wv][sp++] = make_int2(nd.child + front, fa);
+      nid = __builtin_amdgcn_readlane(stk_node[1], sp & 63);
+      b = __builtin_amdgcn_readlane(stk_b[1], sp & 63);
     }
   }
   if (in) {
