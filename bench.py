@@ -67,8 +67,7 @@ PROFILE_JSON = "profiles/counters_trace_batch_heightfield1M.json"
 # full-size GPU tests check against the oracle): pinned so that the counter profile of the
 # kernel is taken on the very launch that is timed.
 C1_CONFIG = scenes_mod.C1_LAUNCH
-KERNEL_SOURCES = ("batch_kernel.h", "traverse.h", "trace_common.h", "mh_device.h",
-                  "batch_ks_pair.hip")
+KERNEL_SOURCES = ("wide_trace.h", "wide_ks.hip", "trace_common.h", "mh_device.h")
 
 
 def log(msg: str) -> None:
@@ -264,7 +263,7 @@ def main() -> int:
     roofline = {"bound": "valu", "achieved": round(achieved_tops, 3), "peak": VALU_PEAK_TOPS,
                 "unit": "Tops/s", "frac": round(achieved_tops / VALU_PEAK_TOPS, 4),
                 "traffic": None,
-                "kernel": "k_trace_batch (primary + bounce batches, closest-hit, KS)",
+                "kernel": "k_wide_lanes (primary + bounce batches, closest-hit, KS)",
                 "ops_per_test": {"box": BOX_OPS, "triangle": TRI_OPS},
                 "ops_per_launch": int(alg_ops), "rays_per_launch": n_prim + n_b,
                 "launch_ms": round(k_frame, 4),
@@ -649,10 +648,10 @@ def bench_c4(api, scenes, args) -> dict:
     sc.close()
     total_s = sum(frame_ms) * 1e-3
     # Algorithmic bytes of the timed refit (mh_scene_refit): per triangle its id, indices and
-    # vertices read (4 + 12 + 36) and its 48-byte record written; per leaf its list entry and
-    # record read (4 + 32) and its box stored in the record and in the PairNode (2 x 24);
-    # per inner record its list entry, child index and two child boxes read (4 + 4 + 48) and
-    # its box stored twice (2 x 24).
+    # vertices read (4 + 12 + 36) and its 48-byte record written; per leaf its first slot's
+    # entry and record read (4 + 32) and its box stored in the record and in a wide node
+    # (2 x 24); per inner record its list entry, child index and two child boxes read
+    # (4 + 4 + 48) and its box stored twice (2 x 24).
     n_leaf = st["nodes"] - st["inner"]
     refit_bytes = nt * (52 + 48) + n_leaf * (36 + 48) + st["inner"] * (56 + 48)
     res = {"frames": args.c4_frames, "tris": nt, "rays_per_frame": rays // args.c4_frames,

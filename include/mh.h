@@ -86,11 +86,11 @@ typedef struct mh_hits {
 
 /* Node layouts of the single-ray traversal. All give DynBVH::intersect's one-ray results
  * and visit order. */
-#define MH_LAYOUT_PAIR 0 /* 64-byte nodes holding both child boxes */
+#define MH_LAYOUT_PAIR 0 /* four-wide nodes: two levels of the tree in 128 bytes */
 #define MH_LAYOUT_REF 1  /* the reference's 32-byte BVHNode records (frames only) */
-#define MH_LAYOUT_SOA 2  /* the 64-byte nodes as four arrays of their 16-byte fields (frames
-                            only; the scene keeps the copy, refreshed after builds, refits
-                            and updates) */
+#define MH_LAYOUT_SOA 2  /* 64-byte nodes of both child boxes as four arrays of their 16-byte
+                            fields (frames only; made at the first use, refreshed after
+                            builds, refits and updates) */
 
 /* Trace options; NULL means the defaults given in brackets. */
 typedef struct mh_trace_opts {
