@@ -217,7 +217,7 @@ struct DevUpdate {
   int32_t* split_list;   // update: leaves whose parent's rotation may split them
   unsigned* split_count; // update: entries of split_list (cleared by the host)
   int32_t* leaf_at;      // per slot, the leaf whose first slot it is, else -1
-  int32_t* irregular;    // update: [1] is set by the leaf pass for a NaN box
+  int32_t* irregular;    // update: [1] is set by the leaf pass for an object with a NaN box
   int32_t n_records;     // capacity, 2T
   int32_t n_old;         // update: records in use before the frame's leaf splits
   int32_t n_objects;     // T

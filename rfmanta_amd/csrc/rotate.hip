@@ -287,7 +287,15 @@ __global__ __launch_bounds__(kBlock) void k_upd_leaves(DevUpdate u, int64_t n_sl
   const int first = nd.child, cnt = nd.children;
   Box b;
   reset(b);
-  auto object = [&](int slot) { return obj_box(u, u.ids[slot]); };
+  // A NaN in an object's box marks the frame. It is looked for here and not in the folded
+  // box: the fold's select forms drop a NaN, and the objects before it, at the next object,
+  // and the children of such a leaf, once it is split, stick out of its box.
+  bool nan = false;
+  auto object = [&](int slot) {
+    const Box o = obj_box(u, u.ids[slot]);
+    for (int k = 0; k < 3; ++k) nan = nan || o.lo[k] != o.lo[k];  // (hi is NaN when lo is)
+    return o;
+  };
   // The parent's rotation tries to split this leaf with the approximate SAH. Two objects:
   // decide it now, from the same object boxes (partition2Objs); more: leave the binned
   // decision to the split pass, whose registers it needs. A root leaf has no parent, a
@@ -304,8 +312,6 @@ __global__ __launch_bounds__(kBlock) void k_upd_leaves(DevUpdate u, int64_t n_sl
   }
   set_box(nd, b);
   nd.axis = 0;
-  bool nan = false;
-  for (int k = 0; k < 3; ++k) nan = nan || b.lo[k] != b.lo[k] || b.hi[k] != b.hi[k];
   if (nan && u.irregular) u.irregular[1] = 1;
   // the candidates go to the split list, one atomic per wave
   const bool cand = rec != 0 && maybe;

@@ -9,6 +9,7 @@ import pytest
 
 from rfmanta_amd import _lib as L
 from rfmanta_amd import api, scenes
+from test_gpu_update import _tree_of_leaf_sizes
 
 pytestmark = pytest.mark.gpu
 
@@ -155,6 +156,32 @@ def test_refit_with_a_vertex_that_is_not_a_number(oracle):
                 assert gn.tobytes() == ref.tobytes()
             # the tree as it stands on the device, box for box
             _check(oracle, s, vd, i, gn, gi, rays, value)
+
+
+@pytest.mark.parametrize("seed", range(4))
+def test_update_with_a_vertex_that_is_not_a_number(oracle, seed):
+    rng = np.random.default_rng(seed)
+    sizes = [int(x) for x in rng.integers(3, 9, 60)]
+    v, i = scenes.soup(sum(sizes), seed=seed, sigma=0.3)
+    ids = rng.permutation(sum(sizes)).astype(np.int32)
+    nodes, _ = _tree_of_leaf_sizes(oracle, v, i, sizes, ids)
+    starts = np.cumsum([0] + sizes[:-1])
+    rays = scenes.random_rays(4000, 7 + seed, (-1, -1, -1), (1, 1, 1))
+    with api.Scene(v, i) as s:
+        s.load_dynbvh(ids, nodes)
+        for bad in (True, False):
+            vd = v.copy()
+            if bad:  # the last corner of a leaf's first object, dropped from the leaf's box
+                vd[i[ids[starts[::3]], 2], seed % 3] = np.nan
+            s.set_vertices(vd)
+            s.update()
+            api.sync()
+            gi, gn = s.export_dynbvh()
+            _check(oracle, s, vd, i, gn, gi, rays, bad)
+            g = s.trace_host(rays, packet_size=64)
+            o = oracle.trace(vd, i, gn, gi, rays, packet_size=64)
+            assert np.array_equal(g["prim"], o["prim"]), bad
+            assert np.array_equal(_bits(g["t"]), _bits(o["t"])), bad
 
 
 @pytest.mark.parametrize("batches", [1, 3])

@@ -1,0 +1,171 @@
+"""Loads, refits and rotating updates of a scene through the C ABI on the host: mh_api.cpp
+and the kernels of refit.hip, rotate.hip and wide.hip as they are, over the host's HIP
+runtime of tests/hostrun/simt (whole workgroups with their barriers, ballots and shuffles,
+buffers of exact size), with AddressSanitizer. Trees equal the oracle's, and every structure
+that the traversal reads beside them (wide nodes, big leaf counts, leaf starts, triangle
+records) agrees with the records (scene_host.cpp)."""
+
+import os
+import shutil
+import subprocess
+from concurrent.futures import ThreadPoolExecutor
+from pathlib import Path
+
+import numpy as np
+import pytest
+
+from rfmanta_amd import scenes
+from test_gpu_update import _tree_of_leaf_sizes, canonical_equal
+
+REPO = Path(__file__).resolve().parents[1]
+SIMT = REPO / "tests" / "hostrun" / "simt"
+CSRC = REPO / "rfmanta_amd" / "csrc"
+
+
+@pytest.fixture(scope="module")
+def scene_host(tmp_path_factory):
+    cxx = shutil.which("g++")
+    if cxx is None:
+        pytest.skip("no C++ compiler")
+    d = tmp_path_factory.mktemp("scene_host")
+    sources = [SIMT / "simt.cpp", SIMT / "scene_host.cpp", CSRC / "mh_api.cpp",
+               CSRC / "sah_builder.cpp", CSRC / "refit.hip", CSRC / "rotate.hip", CSRC / "wide.hip"]
+
+    def compile_one(src):
+        subprocess.run([cxx, "-x", "c++", "-std=c++17", "-g", "-O1", "-fsanitize=address",
+                        "-fno-omit-frame-pointer", "-ffp-contract=off", f"-I{SIMT}", f"-I{CSRC}",
+                        f"-I{REPO / 'include'}", "-c", str(src), "-o", str(d / (src.name + ".o"))],
+                       check=True, capture_output=True)
+
+    with ThreadPoolExecutor(4) as ex:
+        list(ex.map(compile_one, sources))
+    exe = d / "scene_host"
+    subprocess.run([cxx, "-fsanitize=address", *[str(d / (s.name + ".o")) for s in sources], "-o",
+                    str(exe), "-lpthread"], check=True, capture_output=True)
+    return exe
+
+
+class _Scene:
+    """A directory of inputs for scene_host, and what it saved."""
+
+    def __init__(self, exe, d, oracle, v, i):
+        self.exe, self.d, self.oracle = exe, d, oracle
+        self.ops = []
+        np.ascontiguousarray(v, np.float32).tofile(d / "verts.bin")
+        np.ascontiguousarray(i, np.uint32).tofile(d / "idx.bin")
+
+    def load(self, name, nodes, ids):
+        nodes.tofile(self.d / f"{name}.nodes")
+        np.ascontiguousarray(ids, np.int32).tofile(self.d / f"{name}.ids")
+        self.ops.append(f"load:{name}")
+
+    def vertices(self, name, v):
+        np.ascontiguousarray(v, np.float32).tofile(self.d / name)
+        self.ops.append(f"verts:{name}")
+
+    def run(self, **env):
+        r = subprocess.run([str(self.exe), str(self.d), *self.ops], capture_output=True, text=True,
+                           env=dict(os.environ, ASAN_OPTIONS="detect_leaks=0", **env))
+        assert r.returncode == 0, r.stderr[-3000:]
+        return [dict(zip(l.split()[::2], map(int, l.split()[1::2]))) for l in r.stdout.splitlines()]
+
+    def saved(self, name):
+        return (np.fromfile(self.d / f"{name}.nodes", self.oracle.NODE_DTYPE),
+                np.fromfile(self.d / f"{name}.ids", np.int32))
+
+
+def _big_leaves(oracle, seed=7):
+    rng = np.random.default_rng(seed)
+    sizes = [int(x) for x in rng.integers(1, 9, 300)] + [64, 65, 130, 1, 63, 127, 2, 128]
+    rng.shuffle(sizes)
+    T = sum(sizes)
+    v, i = scenes.soup(T, seed=17)
+    ids = rng.permutation(T).astype(np.int32)
+    nodes, nn = _tree_of_leaf_sizes(oracle, v, i, sizes, ids)
+    return v, i, nodes, ids, nn
+
+
+def _trees(oracle, kind):
+    if kind == "leaves of 1 to 130":
+        return _big_leaves(oracle)
+    if kind == "soup":
+        v, i = scenes.soup(1500, seed=3, sigma=0.05)
+    elif kind == "heightfield":
+        v, i = scenes.heightfield(40, 30, seed=4)
+    else:
+        v, i = scenes.soup(int(kind), seed=5)
+    nodes, ids, nn = oracle.build_bvh(v, i)
+    return v, i, nodes, ids, nn
+
+
+@pytest.mark.parametrize("kind", ["leaves of 1 to 130", "soup", "heightfield", "1", "2", "3", "5"])
+def test_refits_and_updates(scene_host, oracle, tmp_path, kind):
+    """Two refits of a loaded tree, then updates (which split large leaves) and a refit after
+    each."""
+    v, i, nodes, ids, nn = _trees(oracle, kind)
+    s = _Scene(scene_host, tmp_path, oracle, v, i)
+    s.load("tree", nodes, ids)
+    s.ops.append("save:s0")
+    st = oracle.RotState(nodes, ids, nn)
+    want = [(st.nodes.copy(), st.ids.copy())]
+    for f in range(1, 7):
+        vd = v.copy()
+        vd[:, 1] += (0.2 * np.sin(3 * v[:, 0] + 0.9 * f)).astype(np.float32)
+        s.vertices(f"v{f}", vd)
+        if f in (3, 5):
+            s.ops.append("update")
+            st.update(vd, i)
+        else:
+            s.ops.append("refit")
+            oracle.refit(vd, i, st.nodes, st.ids)
+        s.ops.append(f"save:s{f}")
+        want.append((st.nodes.copy(), st.ids.copy()))
+    seen = s.run()
+    if kind == "leaves of 1 to 130":
+        assert st.next_free.value > nn  # the large leaves were split
+    for f, (wn, wi) in enumerate(want):
+        gn, gi = s.saved(f"s{f}")
+        ok, msg, n = canonical_equal(gn, gi, wn, wi)
+        assert ok, (f, msg)
+        assert seen[f]["inner"] + seen[f]["leaves"] == n
+        assert seen[f]["nested"] == 1 and seen[f]["irregular"] == 0
+
+
+@pytest.mark.parametrize("levels", ["1", "2", "3", "8"])
+def test_update_in_several_batches_of_levels(scene_host, oracle, tmp_path, levels):
+    v, i, nodes, ids, nn = _trees(oracle, "soup")
+    s = _Scene(scene_host, tmp_path, oracle, v, i)
+    s.load("tree", nodes, ids)
+    vd = (v + np.random.default_rng(1).normal(0, 0.2, v.shape)).astype(np.float32)
+    s.vertices("v1", vd)
+    s.ops += ["update", "save:s1"]
+    s.run(MH_UPDATE_FRONTIER_LEVELS=levels)
+    st = oracle.RotState(nodes, ids, nn)
+    st.update(vd, i)
+    ok, msg, _ = canonical_equal(*s.saved("s1"), st.nodes, st.ids)
+    assert ok, msg
+
+
+@pytest.mark.parametrize("seed", range(6))
+def test_update_with_a_vertex_that_is_not_a_number(scene_host, oracle, tmp_path, seed):
+    """A leaf's box is folded object by object, and a NaN and what came before it is dropped
+    by the object after it; split leaves then stick out of it. Either the tree's boxes nest or
+    it is marked, and a later frame without the NaN clears the mark."""
+    rng = np.random.default_rng(seed)
+    sizes = [int(x) for x in rng.integers(3, 9, 12)]
+    v, i = scenes.soup(sum(sizes), seed=seed)
+    ids = rng.permutation(sum(sizes)).astype(np.int32)
+    nodes, _ = _tree_of_leaf_sizes(oracle, v, i, sizes, ids)
+    s = _Scene(scene_host, tmp_path, oracle, v, i)
+    s.load("tree", nodes, ids)
+    starts = np.cumsum([0] + sizes[:-1])
+    vd = v.copy()
+    for leaf in range(0, 12, 3):  # the last corner of a leaf's first objects
+        vd[i[ids[starts[leaf]], 2], leaf // 3 % 3] = np.nan
+    s.vertices("nan", vd)
+    s.ops += ["update", "save:a"]
+    s.vertices("v", v)
+    s.ops += ["update", "save:b"]
+    a, b = s.run()
+    assert a["irregular"] == 1 or a["nested"] == 1
+    assert b["irregular"] == 0 and b["nested"] == 1
