@@ -244,10 +244,10 @@ int wide_pass(mh_scene* s, const std::vector<mh::LevelList>& sizes, bool fixed_i
 }
 
 // The state of a tree whose root is a leaf: no levels, one leaf at slot 0.
-int leaf_root(mh_scene* s, hipStream_t st) {
-  const int32_t zero[2] = {0, 0};
-  HIP_OK(hipMemcpyAsync(s->leaves.p, zero, 4, hipMemcpyHostToDevice, st));
-  HIP_OK(hipMemcpyAsync(s->irregular.p, zero, 8, hipMemcpyHostToDevice, st));
+int leaf_root(mh_scene* s, bool irregular, hipStream_t st) {
+  const int32_t zero = 0, mark[2] = {irregular, 0};
+  HIP_OK(hipMemcpyAsync(s->leaves.p, &zero, 4, hipMemcpyHostToDevice, st));
+  HIP_OK(hipMemcpyAsync(s->irregular.p, mark, 8, hipMemcpyHostToDevice, st));
   HIP_OK(hipStreamSynchronize(st));
   s->lev.clear();
   s->n_inner = 0;
@@ -342,7 +342,10 @@ int upload(mh_scene* s, bool rtsah = false) {
     s->root_ref = 0;
   } else {
     const mh::RefNode& n = nodes[0];
-    if ((rc = leaf_root(s, nullptr))) return rc;
+    bool nan = false;
+    for (int k = 0; k < 3; ++k)
+      nan = nan || n.box.lo[k] != n.box.lo[k] || n.box.hi[k] != n.box.hi[k];
+    if ((rc = leaf_root(s, nan, nullptr))) return rc;
     const int32_t zero = 0, count = n.children;
     HIP_OK(hipMemcpy(s->leaf_at.as<int32_t>() + n.child, &zero, 4, hipMemcpyHostToDevice));
     HIP_OK(hipMemcpy(s->big.as<int32_t>() + n.child, &count, 4, hipMemcpyHostToDevice));
@@ -777,7 +780,7 @@ int build_device(mh_scene* s, int rtsah) {
     if ((rc = wide_pass(s, sizes, false, nullptr, nullptr, st))) return rc;
     s->root_ref = 0;
   } else {
-    if ((rc = leaf_root(s, st))) return rc;
+    if ((rc = leaf_root(s, false, st))) return rc;
     const int32_t zero = 0, n = (int32_t)T;
     HIP_OK(hipMemcpy(s->leaf_at.p, &zero, 4, hipMemcpyHostToDevice));
     HIP_OK(hipMemcpy(s->big.p, &n, 4, hipMemcpyHostToDevice));
@@ -1094,10 +1097,16 @@ int mh_scene_update(mh_scene* s, void* stream) {
     const std::vector<mh::LevelList> sizes = s->lev;
     rc = wide_pass(s, sizes, false, nfree, now, st);
   } else {
+    int32_t mark[2];  // the leaf pass's NaN mark, which wide_pass takes over otherwise
     HIP_OK(hipMemcpyAsync(s->host_ctr, nfree, 8, hipMemcpyDeviceToHost, st));
+    HIP_OK(hipMemcpyAsync(mark, s->irregular.p, 8, hipMemcpyDeviceToHost, st));
     HIP_OK(hipStreamSynchronize(st));
     now[0] = s->host_ctr[0];
     now[1] = s->host_ctr[1];
+    mark[0] = mark[1];
+    mark[1] = 0;
+    HIP_OK(hipMemcpyAsync(s->irregular.p, mark, 8, hipMemcpyHostToDevice, st));
+    HIP_OK(hipStreamSynchronize(st));
   }
   // Either failure leaves a device tree that must not be traced: the scene needs a build.
   if (now[1]) {

@@ -198,7 +198,8 @@ int launch_refit(const DevRefit& r, const LevelList* lev, int n_levels, void* st
     if (lev[d].n > 0)
       hipLaunchKernelGGL(k_refit_level, grid(lev[d].n), dim3(kBlock), 0, s, r, lev[d].first,
                          lev[d].n);
-  if (t.n > 0) hipLaunchKernelGGL(k_refit_top, dim3(1), dim3(kBlock), 0, s, r, t);
+  // (also where the root is a leaf and there is no level: the NaN mark)
+  hipLaunchKernelGGL(k_refit_top, dim3(1), dim3(kBlock), 0, s, r, t);
   return (int)hipGetLastError();
 }
 

@@ -184,6 +184,32 @@ def test_update_with_a_vertex_that_is_not_a_number(oracle, seed):
             assert np.array_equal(_bits(g["t"]), _bits(o["t"])), bad
 
 
+@pytest.mark.parametrize("n", [2, 4])
+def test_single_leaf_with_a_vertex_that_is_not_a_number(oracle, n):
+    v, i = scenes.soup(n, seed=n, sigma=0.5)
+    bad = v.copy()
+    bad[i[-1, 2], 1] = np.nan
+    nodes = np.zeros(2 * n, oracle.NODE_DTYPE)
+    nodes["children"][0] = n
+    ids = np.arange(n, dtype=np.int32)
+    oracle.refit(bad, i, nodes, ids)
+    rays = scenes.random_rays(2000, n, (-1.5, -1.5, -1.5), (1.5, 1.5, 1.5))
+    with api.Scene(bad, i) as s:
+        s.load_dynbvh(ids, nodes)
+        for k, step in enumerate([None, s.refit, s.update]):
+            for vd in (bad, v) if step else (bad,):
+                if step:
+                    s.set_vertices(vd)
+                    step()
+                    api.sync()
+                gi, gn = s.export_dynbvh()
+                _check(oracle, s, vd, i, gn, gi, rays, k)
+                g = s.trace_host(rays, packet_size=64)
+                o = oracle.trace(vd, i, gn, gi, rays, packet_size=64)
+                assert np.array_equal(g["prim"], o["prim"]), k
+                assert np.array_equal(_bits(g["t"]), _bits(o["t"])), k
+
+
 @pytest.mark.parametrize("batches", [1, 3])
 def test_frames_of_zero_components_and_short_chunks(oracle, batches):
     v, i = scenes.heightfield(50, 30, seed=5)

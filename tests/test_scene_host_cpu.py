@@ -169,3 +169,28 @@ def test_update_with_a_vertex_that_is_not_a_number(scene_host, oracle, tmp_path,
     a, b = s.run()
     assert a["irregular"] == 1 or a["nested"] == 1
     assert b["irregular"] == 0 and b["nested"] == 1
+
+
+def _leaf_root(oracle, v, i):
+    nodes = np.zeros(2 * len(i), oracle.NODE_DTYPE)
+    nodes["children"][0] = len(i)
+    ids = np.arange(len(i), dtype=np.int32)
+    oracle.refit(v, i, nodes, ids)
+    return nodes, ids
+
+
+@pytest.mark.parametrize("n", [1, 2, 4, 70])
+def test_single_leaf_with_a_vertex_that_is_not_a_number(scene_host, oracle, tmp_path, n):
+    """A tree of one leaf has no inner records to carry the mark through: loads, refits and
+    updates set it from the leaf's box all the same, and clear it."""
+    v, i = scenes.soup(n, seed=n)
+    bad = v.copy()
+    bad[i[-1, 2], 1] = np.nan
+    s = _Scene(scene_host, tmp_path, oracle, bad, i)
+    s.load("bad", *_leaf_root(oracle, bad, i))
+    s.ops.append("save:s0")
+    for k, (vd, op) in enumerate([(v, "refit"), (bad, "refit"), (v, "update"), (bad, "update"),
+                                  (v, "refit")]):
+        s.vertices(f"v{k}", vd)
+        s.ops += [op, f"save:s{k + 1}"]
+    assert [a["irregular"] for a in s.run()] == [1, 0, 1, 0, 1, 0]
