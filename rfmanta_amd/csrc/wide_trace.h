@@ -10,13 +10,17 @@
 // alone, and inner boxes may be tested with any arithmetic that never rejects what the
 // reference accepts. So here an inner test is one fused multiply-add a plane, widened by
 // more than all rounding errors (WideRay), two tree levels are tested at a time, and the
-// exact test of a leaf is run only where it matters: once a ray, for the leaf that holds its
-// hit. Should that test fail, which takes a hit within rounding of its leaf's box, the ray
-// is traced again by the reference's own steps (wide_redo). An accepted hit that a later
-// one replaces can be skipped if the later one clears it by more than the acceptance band
-// (anything the first kept out lies in that band or beyond, where the second rejects or
-// replaces it too); inside the band it is tested at once. Rays outside the bounds below and
-// trees whose boxes do not nest take wide_redo from the start.
+// exact test of a leaf is run only for leaves that gave a hit: when a later hit replaces it
+// or the ray ends, with the minT of the hit's acceptance (a leaf that passes with that one
+// passes with the larger one of its visit). While every such leaf passes, minT is the
+// reference's at every leaf, and the leaves visited here are its leaves and others that
+// accepted nothing. Should one fail, which takes a hit within rounding of its leaf's box,
+// the ray is traced again by the reference's own steps (wide_redo). Nothing is assumed of
+// where triangles lie in their boxes: a grazing ray's computed distance may lie before the
+// box, and a loaded tree's boxes may be those of another pose. (Leaving out the test of a
+// hit replaced by one that is clearly nearer gained up to 0.8%: 1,593 against 1,606 us for
+// 12 uneven batches in a 300,000-triangle soup, nothing on a heightfield.) Rays outside the
+// bounds below and trees whose boxes do not nest take wide_redo from the start.
 //
 // How the wave works. A node visit costs about 110 vector instructions and a triangle test
 // about 95, and each waits about 850 cycles for its record (L2 and MALL; a 10,000-triangle
@@ -235,7 +239,7 @@ __device__ __forceinline__ bool wide_tri(const DevScene& sc, WideLane& L, int sl
                                          const PrimRecord& p) {
   float t, u, v;
   if (!record_test<PRIM>(p, L.r, L.h.minT, t, u, v)) return false;
-  if (L.h.best >= 0 && !(t < L.h.minT - 4 * kEps)) L.bad |= !leaf_entered(sc, L, L.h.best, L.enter);
+  if (L.h.best >= 0) L.bad |= !leaf_entered(sc, L, L.h.best, L.enter);
   L.enter = L.h.minT;
   L.h = RayHit{t, slot, u, v};
   return L.ord == kAnyOrder;

@@ -137,6 +137,36 @@ def test_trees_that_take_the_reference_steps(oracle, how):
         _check(oracle, s, v, i, nodes, ids, rays, how)
 
 
+def test_leaf_boxes_that_do_not_hold_their_triangles(oracle):
+    """A loaded tree may hold boxes of another pose. Along the ray: a leaf whose box the ray
+    misses by less than the inner boxes are widened, with a triangle on the ray at 10; a leaf
+    whose box starts at 11, with a triangle at 3; a leaf with its triangle at 5. The reference
+    never enters the first leaf, so it enters the second."""
+    def wall(x):
+        return [[x, -1, -1], [x, 1, -1], [x, 0, 2]]
+
+    v = np.array(wall(10) + wall(3) + wall(5), np.float32)
+    i = np.arange(9, dtype=np.uint32).reshape(3, 3)
+    nodes = np.zeros(6, oracle.NODE_DTYPE)
+    box = [((3, -1, -1), (12, 1, 2)), ((3, -1, -1), (12, 1, 2)), ((5, -1, -1), (5, 1, 2)),
+           ((10, -1, -1), (10, -5e-6, 2)), ((11, -1, -1), (12, 1, 2))]
+    for r, (lo, hi) in enumerate(box):
+        nodes["lo"][r], nodes["hi"][r] = lo, hi
+    nodes["child"][0], nodes["child"][1] = 1, 3
+    for r, slot in ((2, 2), (3, 0), (4, 1)):
+        nodes["child"][r], nodes["children"][r] = slot, 1
+    ids = np.arange(3, dtype=np.int32)
+    n = 70
+    rays = {k: np.zeros(n, np.float32) for k in api.RAY_FIELDS}
+    rays["dx"][:] = 1
+    rays["tmax"][:] = 1e19
+    rays["oz"][:] = np.linspace(-0.3, 0.3, n)
+    with api.Scene(v, i) as s:
+        s.load_dynbvh(ids, nodes)
+        assert (oracle.trace(v, i, nodes, ids, rays, packet_size=1)["prim"] == 1).all()
+        _check(oracle, s, v, i, nodes, ids, rays, "stale boxes")
+
+
 def test_refit_with_a_vertex_that_is_not_a_number(oracle):
     v, i = scenes.heightfield(40, 30, seed=3)
     nodes, ids, _ = oracle.build_bvh(v, i)
