@@ -5,8 +5,9 @@
 // What has to match. The reference visits the leaves in an order fixed by the split axes
 // and the direction's signs (isLeftCheaper for any hit, DynBVH.cc:386-398), and enters a
 // leaf if its slab test and those of the inner records above it pass with the minT of that
-// moment. Boxes nest and every step of the slab test is monotone, so a leaf whose own test
-// passes passes it all the way up: which leaves are entered depends on the leaf boxes
+// moment. Boxes nest and every step of the slab test is monotone (products that are not
+// numbers aside, see leaf_entered), so a leaf whose own test passes passes it all the way
+// up: which leaves are entered depends on the leaf boxes
 // alone, and inner boxes may be tested with any arithmetic that never rejects what the
 // reference accepts. So here an inner test is one fused multiply-add a plane, widened by
 // more than all rounding errors (WideRay), two tree levels are tested at a time, and the
@@ -107,7 +108,10 @@ struct WideLane {
 };
 constexpr unsigned kAnyOrder = 24;
 
-// The reference's slab test of the leaf that holds object slot `slot`.
+// The reference's slab test of the leaf that holds object slot `slot`. False as well for a
+// ray without a component along an axis whose origin lies on a plane of the leaf: products
+// that are not numbers drop out of the reference's test there, and a box around one that
+// passes need not pass.
 __device__ __forceinline__ bool leaf_entered(const DevScene& sc, const WideLane& L, int slot,
                                              float minT) {
   int rec = sc.leaf_at[slot];
@@ -120,8 +124,13 @@ __device__ __forceinline__ bool leaf_entered(const DevScene& sc, const WideLane&
   const float dmin = fminf(fminf(fabsf(r.d[0]), fabsf(r.d[1])), fabsf(r.d[2]));
   const float dmax = fmaxf(fmaxf(fabsf(r.d[0]), fabsf(r.d[1])), fabsf(r.d[2]));
   if (dmin * 0x1p39f < dmax) {
+    bool plane = false;
 #pragma unroll
-    for (int k = 0; k < 3; ++k) r.inv[k] = 1.0f / r.d[k];
+    for (int k = 0; k < 3; ++k) {
+      r.inv[k] = 1.0f / r.d[k];
+      plane |= fabsf(r.inv[k]) > FLT_MAX && (nd.box.lo[k] == r.o[k] || nd.box.hi[k] == r.o[k]);
+    }
+    if (plane) return false;
   }
   float tn;
   return slab(nd.box.lo[0], nd.box.hi[0], nd.box.lo[1], nd.box.hi[1], nd.box.lo[2], nd.box.hi[2],

@@ -137,6 +137,31 @@ def test_trees_that_take_the_reference_steps(oracle, how):
         _check(oracle, s, v, i, nodes, ids, rays, how)
 
 
+def test_origin_in_the_plane_of_a_flat_leaf(oracle):
+    """Rays without an x component in the plane of a leaf's flat box, which passes the
+    reference's slab test while its parent's fails (a loaded tree whose leaf holds its
+    triangle's box of another pose)."""
+    v = np.array([[0.5, -1, 1], [0.5, 2, 1], [-1, 0, 1], [3, -1, 2], [3, 2, 2], [2, 0, 2]], np.float32)
+    i = np.arange(6, dtype=np.uint32).reshape(2, 3)
+    nodes = np.zeros(4, oracle.NODE_DTYPE)
+    for r, (lo, hi) in enumerate([((0.25, -2, 0), (3, 2, 2)), ((0.25, -2, 0), (0.25, 2, 2)),
+                                  ((2, -1, 2), (3, 2, 2))]):
+        nodes["lo"][r], nodes["hi"][r] = lo, hi
+    nodes["child"][0] = 1
+    nodes["child"][1], nodes["children"][1] = 0, 1
+    nodes["child"][2], nodes["children"][2] = 1, 1
+    rays = {k: np.zeros(256, np.float32) for k in api.RAY_FIELDS}
+    rays["ox"][:] = 0.25
+    rays["dx"][1::2] = -0.0
+    rays["oy"][:] = np.linspace(-0.9, 1.9, 256)
+    rays["dz"][:] = 1
+    rays["tmax"][:] = np.where(np.arange(256) % 4 < 2, 1e19, np.inf)
+    ids = np.arange(2, dtype=np.int32)
+    with api.Scene(v, i) as s:
+        s.load_dynbvh(ids, nodes)
+        _check(oracle, s, v, i, nodes, ids, rays, "flat")
+
+
 def test_leaf_boxes_that_do_not_hold_their_triangles(oracle):
     """A loaded tree may hold boxes of another pose. Along the ray: a leaf whose box the ray
     misses by less than the inner boxes are widened, with a triangle on the ray at 10; a leaf
