@@ -61,15 +61,13 @@ struct WideRay {
 // the smallest one (a direction component of zero has an infinite one): the cut plane
 // distances keep their signs, and the widening of such an axis alone, 2^19 R m, is beyond
 // any distance inside the root box, so a ray between the planes still passes. The bounds on
-// R m keep every product finite. A ray with an infinite minT and a zero component is left to
-// the reference's steps, which let infinite distances through there.
+// R m keep every product along the longest component finite, so every box the reference
+// enters is left at a finite distance, also for a ray with an infinite minT.
 __device__ __forceinline__ bool wide_setup(float reach, const Ray& r, float minT, WideRay& w) {
   const float m = fminf(fminf(fabsf(r.inv[0]), fabsf(r.inv[1])), fabsf(r.inv[2]));
-  const float big = fmaxf(fmaxf(fabsf(r.inv[0]), fabsf(r.inv[1])), fabsf(r.inv[2]));
   const float R = reach + fmaxf(fmaxf(fabsf(r.o[0]), fabsf(r.o[1])), fabsf(r.o[2]));
   const float q = R * m, lim = m * 0x1p40f;
-  bool ok = q >= 0x1p-60f && q <= 0x1p60f && m >= 0x1p-60f && m <= 0x1p60f && !(minT != minT) &&
-            (minT <= FLT_MAX || big <= FLT_MAX);
+  bool ok = q >= 0x1p-60f && q <= 0x1p60f && m >= 0x1p-60f && m <= 0x1p60f && !(minT != minT);
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     ok = ok && !(r.o[k] != r.o[k]) && !(r.d[k] != r.d[k]);

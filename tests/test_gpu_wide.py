@@ -137,6 +137,33 @@ def test_trees_that_take_the_reference_steps(oracle, how):
         _check(oracle, s, v, i, nodes, ids, rays, how)
 
 
+@pytest.mark.parametrize("mesh", ["heightfield", "grid", "soup"])
+@pytest.mark.parametrize("axis", [0, 1, 2])
+def test_axis_parallel_rays_without_end(oracle, mesh, axis):
+    """Infinite tmax and one or two zero components, origins on and off box planes."""
+    if mesh == "soup":
+        v, i = scenes.soup(700, seed=2, sigma=0.1)
+    else:
+        v, i = scenes.heightfield(17, 17, seed=2)
+        if mesh == "grid":
+            v[:, 1] = 0
+    nodes, ids, _ = oracle.build_bvh(v, i)
+    n = 1200
+    rays = scenes.random_rays(n, 13 + axis, (-1.2, -1.2, -1.2), (1.2, 1.2, 1.2))
+    k = np.arange(n)
+    d = ["dx", "dy", "dz"]
+    rays[d[axis]][:] = np.where(k % 2, 1, -1) * np.float32(1)
+    rays[d[(axis + 1) % 3]][:] = np.where(k % 4 < 2, 0.0, -0.0)
+    rays[d[(axis + 2) % 3]][k % 3 == 0] = 0.0
+    for o in ("ox", "oy", "oz"):
+        on = k % 5 < 2
+        rays[o][on] = np.round(rays[o][on] * 8) / 8
+    rays["tmax"][:] = np.inf
+    with api.Scene(v, i) as s:
+        s.load_dynbvh(ids, nodes)
+        _check(oracle, s, v, i, nodes, ids, rays, mesh)
+
+
 def test_origin_in_the_plane_of_a_flat_leaf(oracle):
     """Rays without an x component in the plane of a leaf's flat box, which passes the
     reference's slab test while its parent's fails (a loaded tree whose leaf holds its
