@@ -119,6 +119,8 @@ struct mh_scene {
   // slot's leaf is the nearest one starting at or before it.
   bool partition = false;
   DevBuf irregular;  // int32[2]: mh::DevScene::irregular and the NaN mark of a pass
+  // What a refit leaves in it without NaN boxes: overlapping leaves.
+  int fixed_irregular = 0;
   DevBuf logtab;  // RTSAH table logarithm (device build)
   DevBuf normals, normal_idx, texcoords, tex_idx;  // shading attributes (mh_shade)
   // The PairNodes and their copy as four arrays of their 16-byte fields (MH_LAYOUT_SOA

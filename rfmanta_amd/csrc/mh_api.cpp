@@ -178,7 +178,7 @@ mh::DevUpdate tree_view(mh_scene* s) {
 // more) sets the first batch's size instead, so that tests can reach the later batches.
 // Copies `extra` (two words) back along with the counters; synchronises the stream.
 // MH_OK, MH_E_UNSUPPORTED (deeper than the lists hold) or MH_E_STATE (not a binary tree).
-int wide_pass(mh_scene* s, const std::vector<mh::LevelList>& sizes, bool fixed_irregular,
+int wide_pass(mh_scene* s, const std::vector<mh::LevelList>& sizes, int irregular,
               const unsigned* extra, unsigned extra_out[2], hipStream_t st) {
   const mh::DevUpdate u = tree_view(s);
   mh::DevFrontier f{};
@@ -189,7 +189,7 @@ int wide_pass(mh_scene* s, const std::vector<mh::LevelList>& sizes, bool fixed_i
   f.leaves = s->leaves.as<int32_t>();
   f.wide = s->wide.as<mh::WideNode>();
   f.irregular = s->irregular.as<int32_t>();
-  f.fixed = fixed_irregular;
+  f.fixed = irregular;
   f.cap = (unsigned)s->list_cap;
   f.cap_wide = (unsigned)(s->wide.bytes / sizeof(mh::WideNode));
   unsigned* hc = s->host_ctr;
@@ -244,7 +244,7 @@ int wide_pass(mh_scene* s, const std::vector<mh::LevelList>& sizes, bool fixed_i
 }
 
 // The state of a tree whose root is a leaf: no levels, one leaf at slot 0.
-int leaf_root(mh_scene* s, bool irregular, hipStream_t st) {
+int leaf_root(mh_scene* s, int irregular, hipStream_t st) {
   const int32_t zero = 0, mark[2] = {irregular, 0};
   HIP_OK(hipMemcpyAsync(s->leaves.p, &zero, 4, hipMemcpyHostToDevice, st));
   HIP_OK(hipMemcpyAsync(s->irregular.p, mark, 8, hipMemcpyHostToDevice, st));
@@ -327,6 +327,17 @@ int upload(mh_scene* s, bool rtsah = false) {
   int rc;
   if ((rc = reserve_tree(s, nrec, n_inner, leaves.size()))) return rc;
   s->partition = partition;
+  s->fixed_irregular = partition ? 0 : 1;
+  if (!partition) {  // one big_count entry for two large leaves that start at one slot?
+    std::vector<int32_t> big(T, 0);
+    for (int32_t r : leaves) {
+      const int n = nodes[r].children;
+      if (n < mh::kLeafCountInline) continue;
+      int32_t& b = big[nodes[r].child];
+      if (b && b != n) s->fixed_irregular = 2;
+      b = n;
+    }
+  }
   s->updatable = partition && n_reached == max_rec + 1;
   s->next_free = max_rec + 1;
   s->n_records = nrec;
@@ -338,14 +349,14 @@ int upload(mh_scene* s, bool rtsah = false) {
   HIP_OK(hipMemset(s->leaf_at.p, 0xFF, (size_t)T * 4));
   HIP_OK(hipMemset(s->irregular.p, 0, 8));
   if (n_inner > 0) {
-    if ((rc = wide_pass(s, sizes, !partition || !nested, nullptr, nullptr, nullptr))) return rc;
+    if ((rc = wide_pass(s, sizes, s->fixed_irregular | !nested, nullptr, nullptr, nullptr))) return rc;
     s->root_ref = 0;
   } else {
     const mh::RefNode& n = nodes[0];
     bool nan = false;
     for (int k = 0; k < 3; ++k)
       nan = nan || n.box.lo[k] != n.box.lo[k] || n.box.hi[k] != n.box.hi[k];
-    if ((rc = leaf_root(s, nan, nullptr))) return rc;
+    if ((rc = leaf_root(s, s->fixed_irregular | nan, nullptr))) return rc;
     const int32_t zero = 0, count = n.children;
     HIP_OK(hipMemcpy(s->leaf_at.as<int32_t>() + n.child, &zero, 4, hipMemcpyHostToDevice));
     HIP_OK(hipMemcpy(s->big.as<int32_t>() + n.child, &count, 4, hipMemcpyHostToDevice));
@@ -773,14 +784,15 @@ int build_device(mh_scene* s, int rtsah) {
   HIP_OK((hipError_t)mh::launch_prim_setup(r, st));
   HIP_OK(hipMemsetAsync(s->leaf_at.p, 0xFF, (size_t)T * 4, st));
   HIP_OK(hipMemsetAsync(s->irregular.p, 0, 8, st));
+  s->fixed_irregular = 0;
   if (n_final > 1) {
     std::vector<mh::LevelList> sizes;
     for (int k = 0; k < n_levels; ++k)
       sizes.push_back(mh::LevelList{0, level_off[k + 1] - level_off[k]});
-    if ((rc = wide_pass(s, sizes, false, nullptr, nullptr, st))) return rc;
+    if ((rc = wide_pass(s, sizes, 0, nullptr, nullptr, st))) return rc;
     s->root_ref = 0;
   } else {
-    if ((rc = leaf_root(s, false, st))) return rc;
+    if ((rc = leaf_root(s, 0, st))) return rc;
     const int32_t zero = 0, n = (int32_t)T;
     HIP_OK(hipMemcpy(s->leaf_at.p, &zero, 4, hipMemcpyHostToDevice));
     HIP_OK(hipMemcpy(s->big.p, &n, 4, hipMemcpyHostToDevice));
@@ -1036,6 +1048,7 @@ int mh_scene_refit(mh_scene* s, void* stream) {
   r.wide = s->wide.as<mh::WideNode>();
   r.leaf_at = s->partition ? s->leaf_at.as<int32_t>() : nullptr;
   r.irregular = s->irregular.as<int32_t>();
+  r.fixed = s->fixed_irregular;
   r.tris = s->tris.as<float>();
   r.obj_ids = s->ids.as<int32_t>();
   r.verts = s->d_verts.as<float>();
@@ -1095,7 +1108,8 @@ int mh_scene_update(mh_scene* s, void* stream) {
   rc = MH_OK;
   if (s->n_inner > 0) {  // rotations never turn a leaf root inner
     const std::vector<mh::LevelList> sizes = s->lev;
-    rc = wide_pass(s, sizes, false, nfree, now, st);
+    s->fixed_irregular = 0;
+    rc = wide_pass(s, sizes, 0, nfree, now, st);
   } else {
     int32_t mark[2];  // the leaf pass's NaN mark, which wide_pass takes over otherwise
     HIP_OK(hipMemcpyAsync(s->host_ctr, nfree, 8, hipMemcpyDeviceToHost, st));

@@ -67,8 +67,10 @@ struct DevScene {
   const WideNode* wide;
   uint32_t n_wide;         // the bound of the wide table's descriptor
   const int32_t* leaf_at;
-  // Nonzero: the tree's boxes do not nest or its leaves overlap (a loaded tree), or a vertex
-  // is not a number; every ray then takes the reference's own traversal.
+  // 1: single rays traverse the records instead of the wide nodes. The tree's boxes do not
+  // nest or its leaves overlap (a loaded tree), or a box is not a number. Beyond 1: big_count does not hold either (leaves of
+  // kLeafCountInline or more objects that start at one slot), every ray takes the
+  // reference's own steps.
   const int32_t* irregular;
   const RefNode* refs;
   const float* tris;  // 12 floats per slot
@@ -175,6 +177,7 @@ struct DevRefit {
   const int32_t* leaf_at;  // null: the leaves do not partition the slots, take the leaf list
   const int32_t* levels;
   int32_t* irregular;      // [0] DevScene::irregular, [1] set by a pass that met a NaN box
+  int32_t fixed;           // DevScene::irregular without NaN boxes
   int32_t n_leaves;
   int32_t n_slots;        // T
   int32_t prim_kind;

@@ -158,7 +158,7 @@ __global__ __launch_bounds__(kBlock) void k_refit_top(DevRefit r, TopLevels t) {
     __syncthreads();
   }
   if (threadIdx.x == 0) {
-    r.irregular[0] = r.leaf_at == nullptr || r.irregular[1] != 0;
+    r.irregular[0] = r.fixed | (r.irregular[1] != 0);
     r.irregular[1] = 0;
   }
 }

@@ -21,7 +21,9 @@
 // box, and a loaded tree's boxes may be those of another pose. (Leaving out the test of a
 // hit replaced by one that is clearly nearer gained up to 0.8%: 1,593 against 1,606 us for
 // 12 uneven batches in a 300,000-triangle soup, nothing on a heightfield.) Rays outside the
-// bounds below and trees whose boxes do not nest take wide_redo from the start.
+// bounds below take wide_redo from the start. Trees whose boxes do not nest are traversed on
+// their 32-byte records, the two children of a record a step, every box tested exactly
+// (wide_pair_step).
 //
 // How the wave works. A node visit costs about 110 vector instructions and a triangle test
 // about 95, and each waits about 850 cycles for its record (L2 and MALL; a 10,000-triangle
@@ -258,12 +260,13 @@ __device__ __forceinline__ bool wide_tri(const DevScene& sc, WideLane& L, int sl
 // one would wait for its record again. (One a step: 1M incoherent rays over the 1M-triangle
 // heightfield 228 against 205 us, shadow rays 239 against 214. Past the last slot the
 // descriptor reads zeros.)
-template <int PRIM>
+// PAIRS: the leaf's own box has been tested.
+template <int PRIM, bool PAIRS>
 __device__ __forceinline__ void wide_leaf_step(const DevScene& sc, WideLane& L) {
   const int code = ~L.cur;
   const int slot = code >> kLeafCountBits;
   const int count = code & kLeafCountInline;  // left in the leaf; 0 in an empty slot's code
-  const int old = L.h.best;
+  const int old = PAIRS ? -1 : L.h.best;
   const float entered = L.enter;
   const PrimRecord p = fetch_prim(sc, slot), q = fetch_prim(sc, slot + 1);
   hold_prim(p);
@@ -284,16 +287,50 @@ __device__ __forceinline__ void wide_leaf_step(const DevScene& sc, WideLane& L) 
     L.cur = kPop;
 }
 
+// wide_pair_step's reference of a record: twice its first child, plus one if the ray visits
+// the second child first, or the leaf code.
+__device__ __forceinline__ int pair_ref(const WideLane& L, int child, int word) {
+  const int n = word >> 16;
+  if (n != 0) return ~((child << kLeafCountBits) | (n < kLeafCountInline ? n : kLeafCountInline));
+  const int first = L.ord == kAnyOrder ? (word >> 8) & 1 : (L.r.dpos >> (word & 3)) & 1;
+  return 2 * child + 1 - first;
+}
+
+// Visits the children L.cur of an inner record: the boxes of both are tested as the reference
+// tests them (the farther one's distance again when it is taken off the stack, which is its
+// later test with the minT of that moment).
+template <int S, int BLOCK>
+__device__ __forceinline__ void wide_pair_step(const DevScene& sc, WideLane& L,
+                                               WideStack<S, BLOCK>& st) {
+  const float4* p = reinterpret_cast<const float4*>(sc.refs + (L.cur >> 1));
+  const float4 A = p[0], B = p[1], C = p[2], D = p[3];
+  Ray r = L.r;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) r.inv[k] = L.w.inv[k];
+  float t0, t1;
+  const unsigned long long H0 = wave_mask(slab(A.x, A.w, A.y, B.x, A.z, B.y, r, L.h.minT, t0)),
+                           H1 = wave_mask(slab(C.x, C.w, C.y, D.x, C.z, D.y, r, L.h.minT, t1)),
+                           F = wave_mask((L.cur & 1) != 0);
+  const int r0 = pair_ref(L, __float_as_int(B.z), __float_as_int(B.w)),
+            r1 = pair_ref(L, __float_as_int(D.z), __float_as_int(D.w));
+  const bool f = lane_bit(F);
+  st.push3(H0 & H1, f ? r0 : r1, f ? t0 : t1, 0, 0, 0.f, 0, 0, 0.f);
+  L.cur = lane_bit(H0 & H1) ? (f ? r1 : r0) : (lane_bit(H0) ? r0 : (lane_bit(H1) ? r1 : kPop));
+}
+
 // One step of the wave; a lane at a leaf weighs `weight` quarters of one at a node.
-template <int PRIM, int S, int BLOCK>
+template <int PRIM, bool PAIRS, int S, int BLOCK>
 __device__ __forceinline__ void wide_step(const DevScene& sc, WideLane& L, int weight,
                                           WideStack<S, BLOCK>& st) {
   const unsigned long long at_node = wave_mask(L.cur >= 0);
   const unsigned long long at_leaf = wave_mask(L.cur < 0) & wave_mask(L.cur > kPop);
   if (weight * __popcll(at_leaf) >= 4 * __popcll(at_node)) {
-    if (lane_bit(at_leaf)) wide_leaf_step<PRIM>(sc, L);
-  } else {
-    if (lane_bit(at_node)) wide_node_step<S, BLOCK>(sc, L, st);
+    if (lane_bit(at_leaf)) wide_leaf_step<PRIM, PAIRS>(sc, L);
+  } else if (lane_bit(at_node)) {
+    if constexpr (PAIRS)
+      wide_pair_step<S, BLOCK>(sc, L, st);
+    else
+      wide_node_step<S, BLOCK>(sc, L, st);
   }
   if (L.cur == kPop) {
     const bool have = st.sp > 0;
@@ -347,24 +384,35 @@ __device__ __forceinline__ void wide_redo(const DevScene& sc, const GRays& rays,
 // wave's first ray, so that the addresses are a scalar base and a lane offset).
 template <int S, int BLOCK, class Index>
 __device__ __forceinline__ void wide_start(const DevScene& sc, float reach, const GRays& rays,
-                                           Index i, bool any, bool nested, WideLane& L,
+                                           Index i, bool any, int irregular, WideLane& L,
                                            WideStack<S, BLOCK>& st) {
   load_ray(rays, i, L.r);
   L.h = RayHit{rays.tmax[i], -1, 0.f, 0.f};
   L.enter = L.h.minT;
   st.reset();
-  const bool ok = nested & wide_setup(reach, L.r, L.h.minT, L.w);
+  L.ord = any ? kAnyOrder : 3u * (L.r.dpos & 7u);
+  if (irregular == 1) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) L.w.inv[k] = L.r.inv[k];
+    const RefNode& nd = sc.refs[0];
+    float tn;
+    const bool in = slab(nd.box.lo[0], nd.box.hi[0], nd.box.lo[1], nd.box.hi[1], nd.box.lo[2],
+                         nd.box.hi[2], L.r, L.h.minT, tn);
+    L.bad = false;
+    L.cur = in ? pair_ref(L, nd.child, (nd.children << 16) | (nd.bits << 8) | nd.axis) : kIdle;
+    return;
+  }
+  const bool ok = (irregular == 0) & wide_setup(reach, L.r, L.h.minT, L.w);
   L.bad = !ok;
   L.cur = ok ? sc.root_ref : kIdle;
-  L.ord = any ? kAnyOrder : 3u * (L.r.dpos & 7u);
 }
 
 // Stores the hit of a lane that has come to the end of ray i.
 template <int PRIM, int S, int BLOCK, class Index>
 __device__ __forceinline__ void wide_finish(const DevScene& sc, const GRays& rays,
-                                            const GHits& hits, Index i, WideLane& L,
-                                            WideStack<S, BLOCK>& st) {
-  if (!L.bad && L.h.best >= 0) L.bad = !leaf_entered(sc, L, L.h.best, L.enter);
+                                            const GHits& hits, Index i, int irregular,
+                                            WideLane& L, WideStack<S, BLOCK>& st) {
+  if (irregular == 0 && !L.bad && L.h.best >= 0) L.bad = !leaf_entered(sc, L, L.h.best, L.enter);
   if (L.bad) wide_redo<PRIM, S, BLOCK>(sc, rays, i, L, st);
   const bool hit = L.h.best >= 0;
   store_hit(hits, i, hit ? sc.obj_ids[L.h.best] : -1, (L.ord == kAnyOrder && hit) ? kEps : L.h.minT, L.h.u,
@@ -439,7 +487,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5, 8))) v
   if (TABLE && a.remap && (gridDim.x & 7) == 0) blk = (blk & 7) * (gridDim.x >> 3) + (blk >> 3);
   WideStack<S, BLOCK> st(s_ring, a.spill, a.spill_stride, (int64_t)blockIdx.x * BLOCK + tid, tid);
   const float reach = root_reach(a.sc);
-  const bool nested = *a.sc.irregular == 0;
+  const int irregular = *a.sc.irregular;
   const int C = a.chunk;
   const int64_t stride = (int64_t)gridDim.x * (BLOCK / 64) * C;
   // (the wave's number is the same in all its lanes: kept in scalar registers)
@@ -469,17 +517,20 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5, 8))) v
           store_hit(moved(global_view(B->hits), pos - first), lane, -2, -kMaxT, 0.f, 0.f, true);
           live = false;
         } else {
-          wide_start<S, BLOCK>(a.sc, reach, rays, (unsigned)lane, (B->flags & 1u) != 0, nested, L,
-                               st);
+          wide_start<S, BLOCK>(a.sc, reach, rays, (unsigned)lane, (B->flags & 1u) != 0, irregular,
+                               L, st);
         }
       }
-      while (wave_mask(L.cur != kIdle)) wide_step<PRIM, S, BLOCK>(a.sc, L, a.weight, st);
+      if (irregular == 0)
+        while (wave_mask(L.cur != kIdle)) wide_step<PRIM, false, S, BLOCK>(a.sc, L, a.weight, st);
+      else
+        while (wave_mask(L.cur != kIdle)) wide_step<PRIM, true, S, BLOCK>(a.sc, L, a.weight, st);
       if (live) {
         const WideArgs& again = args_again();
         const BatchDev* E = TABLE ? again.table->batches + bi : &again.one;
         wide_finish<PRIM, S, BLOCK>(again.sc, moved(global_view(E->rays), pos - first),
-                                    moved(global_view(E->hits), pos - first), (unsigned)lane, L,
-                                    st);
+                                    moved(global_view(E->hits), pos - first), (unsigned)lane,
+                                    irregular, L, st);
       }
       pos += n;
     }
@@ -490,12 +541,11 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5, 8))) v
 // take the wave's next rays as soon as `refill` of them are idle. A wave takes `chunk` ray
 // numbers at a time: first those at its own place, then by a shared counter, asked ahead of
 // time. The last wave to leave clears the counter, so launches and graph replays need no
-// clearing pass. Five waves a SIMD (80 registers, for six, spill).
-template <int PRIM, int S, int BLOCK>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_wide_lanes(
-    WideArgs a) {
-  __shared__ unsigned long long s_ring[S * BLOCK];
-  extern __shared__ int64_t s_start[];  // nb entries (dynamic LDS)
+// clearing pass. Five waves a SIMD (80 registers, for six, spill). PAIRS as a whole loop of
+// its own: both kinds of step in one loop cost the wide ones 5% (scalar registers).
+template <int PRIM, bool PAIRS, int S, int BLOCK>
+__device__ __forceinline__ void wide_lanes(const WideArgs& a, unsigned long long* s_ring,
+                                           int64_t* s_start) {
   const int tid = threadIdx.x, lane = tid & 63;
   // The dynamic LDS holds a.nb offsets; a table with more entries is cut to that.
   const BatchTable* table = a.table;
@@ -512,7 +562,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5, 8))) v
   WideStack<S, BLOCK> st(s_ring, a.spill, a.spill_stride, (int64_t)blockIdx.x * BLOCK + tid, tid);
   const DevScene& sc = a.sc;
   const float reach = root_reach(sc);
-  const bool nested = *sc.irregular == 0;
+  const int irregular = PAIRS ? 1 : *sc.irregular;
 
   int64_t C = a.chunk;
   if (a.fair > 0) {  // no more than a quarter of a resident wave's share of the rays
@@ -553,7 +603,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5, 8))) v
     }
     if (take_rays) {
       by_batch(lane_bit(idle) && li >= 0, [&](const GRays& rays, const GHits& hits, uint32_t) {
-        wide_finish<PRIM, S, BLOCK>(sc, rays, hits, li, L, st);
+        wide_finish<PRIM, S, BLOCK>(sc, rays, hits, li, irregular, L, st);
       });
       if (lane_bit(idle)) li = -1;
       if (!more) break;  // every lane is idle
@@ -575,12 +625,12 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5, 8))) v
           store_hit(hits, i, -2, -kMaxT, 0.f, 0.f, true);
         } else {
           li = i;
-          wide_start<S, BLOCK>(sc, reach, rays, i, (flags & 1u) != 0, nested, L, st);
+          wide_start<S, BLOCK>(sc, reach, rays, i, (flags & 1u) != 0, irregular, L, st);
         }
       });
       pos = pos + n_idle < end ? pos + n_idle : end;
     }
-    wide_step<PRIM, S, BLOCK>(sc, L, a.weight, st);
+    wide_step<PRIM, PAIRS, S, BLOCK>(sc, L, a.weight, st);
   }
   if (lane == 0) {
     const unsigned long long left = atomicAdd(a.ctr + 1, 1ull);
@@ -589,6 +639,17 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5, 8))) v
       atomicExch(a.ctr + 1, 0ull);
     }
   }
+}
+
+template <int PRIM, int S, int BLOCK>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_wide_lanes(
+    WideArgs a) {
+  __shared__ unsigned long long s_ring[S * BLOCK];
+  extern __shared__ int64_t s_start[];  // nb entries (dynamic LDS)
+  if (*a.sc.irregular == 1)
+    wide_lanes<PRIM, true, S, BLOCK>(a, s_ring, s_start);
+  else
+    wide_lanes<PRIM, false, S, BLOCK>(a, s_ring, s_start);
 }
 
 namespace {

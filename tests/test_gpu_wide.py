@@ -219,6 +219,48 @@ def test_leaf_boxes_that_do_not_hold_their_triangles(oracle):
         _check(oracle, s, v, i, nodes, ids, rays, "stale boxes")
 
 
+def _check_frames(oracle, scene, v, i, nodes, ids, rays, what):
+    sets = [(rays, False), (_take(rays, 777), True)]
+    dev = [(api.DeviceRays.upload(r), api.DeviceHits.alloc(len(r["ox"]), any_hit=a), a)
+           for r, a in sets]
+    f = api.Frame(scene, dev)
+    for refill, chunk in ((64, 0), (24, 64)):
+        f.set_config(dict(layout=L.MH_LAYOUT_PAIR, stack_lds=8, block=64, blocks_per_cu=1,
+                          refill=refill, chunk=chunk, reverse=0))
+        f.launch()
+        api.sync()
+        for (_, dh, a), (r, _) in zip(dev, sets):
+            o = oracle.trace(v, i, nodes, ids, r, packet_size=1, any_hit=a)
+            g = dh.download()
+            assert np.array_equal(g["prim"], o["prim"]), (what, refill, a)
+            if not a:
+                assert np.array_equal(_bits(g["t"]), _bits(o["t"])), (what, refill)
+    f.close()
+
+
+@pytest.mark.parametrize("how", ["not nested", "overlapping", "two large leaves at one slot"])
+def test_trees_traversed_on_their_records(oracle, how):
+    """Leaves around the inline leaf count in trees that the wide nodes do not serve, with odd
+    rays among the others."""
+    sizes = [1, 2, 3, 14, 15, 16, 17, 31, 1, 2, 5, 20]
+    v, i = scenes.soup(sum(sizes), seed=8, sigma=0.3)
+    nodes, ids = _chain_of_leaves(oracle, v, i, sizes)
+    if how == "not nested":
+        nodes["hi"][2:20:4, 0] -= np.float32(0.1)
+    elif how == "overlapping":
+        nodes["children"][3] += 1
+    else:  # the leaf before starts with the next one's objects, four fewer
+        r = 2 * sizes.index(20) - 1
+        nodes["child"][r], nodes["children"][r] = sum(sizes) - 20, 16
+    rays = scenes.random_rays(3000, 4, (-1, -1, -1), (1, 1, 1))
+    odd = _odd_rays()
+    rays = {k: np.concatenate([rays[k], odd[k]]) for k in api.RAY_FIELDS}
+    with api.Scene(v, i) as s:
+        s.load_dynbvh(ids, nodes)
+        _check(oracle, s, v, i, nodes, ids, rays, how)
+        _check_frames(oracle, s, v, i, nodes, ids, rays, how)
+
+
 def test_refit_with_a_vertex_that_is_not_a_number(oracle):
     v, i = scenes.heightfield(40, 30, seed=3)
     nodes, ids, _ = oracle.build_bvh(v, i)
