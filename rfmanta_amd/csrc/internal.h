@@ -119,8 +119,9 @@ struct mh_scene {
   // slot's leaf is the nearest one starting at or before it.
   bool partition = false;
   DevBuf irregular;  // int32[2]: mh::DevScene::irregular and the NaN mark of a pass
-  // What a refit leaves in it without NaN boxes: overlapping leaves.
+  // What a refit leaves in it without NaN boxes: overlapping leaves, too many wide nodes.
   int fixed_irregular = 0;
+  uint32_t max_wide = mh::kMaxWide;
   DevBuf logtab;  // RTSAH table logarithm (device build)
   DevBuf normals, normal_idx, texcoords, tex_idx;  // shading attributes (mh_shade)
   // The PairNodes and their copy as four arrays of their 16-byte fields (MH_LAYOUT_SOA

@@ -233,6 +233,12 @@ int wide_pass(mh_scene* s, const std::vector<mh::LevelList>& sizes, int irregula
     at[k & 1] += hc[k];
     n_inner += hc[k];
   }
+  if (at[0] > (int64_t)s->max_wide) {
+    s->fixed_irregular |= 1;
+    const int32_t word = irregular | 1;
+    HIP_OK(hipMemcpyAsync(s->irregular.p, &word, 4, hipMemcpyHostToDevice, st));
+    HIP_OK(hipStreamSynchronize(st));
+  }
   const uint64_t n_leaves = hc[mh::kFrLeaves];
   if (hc[mh::kFrOver] || n_leaves != n_inner + 1 || n_leaves > s->list_cap)
     return fail(MH_E_STATE, "the records are not a binary tree (%llu inner, %llu leaves)",

@@ -33,8 +33,9 @@ namespace mh {
 // ~((first_slot << 4) | c) with c = min(count, 15); c == 15 means "read big_count".
 constexpr int kLeafCountBits = 4;
 constexpr int kLeafCountInline = 15;
-// Fewer than 2^26 objects: leaf codes hold first_slot << 4 in an int, and the pair table
-// (64 B per object) stays within the 4 GiB that a buffer descriptor's byte offsets reach.
+// Fewer than 2^26 objects: leaf codes hold first_slot << 4 in an int, and the triangle and
+// pair tables (48 and 64 B per object) stay within the 4 GiB that a buffer descriptor's byte
+// offsets reach.
 constexpr uint32_t kMaxObjects = 1u << 26;
 
 struct alignas(16) PairNode {
@@ -61,6 +62,9 @@ struct alignas(128) WideNode {
   int32_t pad[3];
 };
 static_assert(sizeof(WideNode) == 128, "wide node is one cache line");
+// Wide nodes within the 4 GiB that a buffer descriptor's byte offsets reach. Trees of more
+// (from about 50M triangles on) are traversed on their records.
+constexpr uint32_t kMaxWide = 1u << 25;
 constexpr int32_t kWideEmpty = -1;  // ~((0 << kLeafCountBits) | 0)
 
 struct DevScene {
@@ -68,7 +72,8 @@ struct DevScene {
   uint32_t n_wide;         // the bound of the wide table's descriptor
   const int32_t* leaf_at;
   // 1: single rays traverse the records instead of the wide nodes. The tree's boxes do not
-  // nest or its leaves overlap (a loaded tree), or a box is not a number. Beyond 1: big_count does not hold either (leaves of
+  // nest or its leaves overlap (a loaded tree), a box is not a number, or there are more
+  // than kMaxWide wide nodes. Beyond 1: big_count does not hold either (leaves of
   // kLeafCountInline or more objects that start at one slot), every ray takes the
   // reference's own steps.
   const int32_t* irregular;

@@ -6,6 +6,7 @@
 //   DIR holds verts.bin and idx.bin; OP is one of
 //   load:NAME    NAME.ids and NAME.nodes into the scene
 //   verts:FILE   the vertices of FILE
+//   limit:N      trees of more than N wide nodes are traversed on their records
 //   refit, update
 //   save:NAME    the tree to NAME.ids and NAME.nodes, after checking what the traversal
 //                reads beside it: prints "irregular I nested N inner X leaves L depth D"
@@ -167,6 +168,8 @@ int main(int argc, char** argv) {
                                  (uint32_t)nodes.size(), MH_PRIM_KENSLER_SHIRLEY), op);
     } else if (what == "verts") {
       check(mh_scene_set_vertices(s, read<float>(name).data(), 0, nullptr), op);
+    } else if (what == "limit") {
+      s->max_wide = (uint32_t)std::atol(op.c_str() + colon + 1);
     } else if (what == "refit") {
       check(mh_scene_refit(s, nullptr), op);
     } else if (what == "update") {

@@ -194,3 +194,14 @@ def test_single_leaf_with_a_vertex_that_is_not_a_number(scene_host, oracle, tmp_
         s.vertices(f"v{k}", vd)
         s.ops += [op, f"save:s{k + 1}"]
     assert [a["irregular"] for a in s.run()] == [1, 0, 1, 0, 1, 0]
+
+
+def test_more_wide_nodes_than_a_descriptor_reaches(scene_host, oracle, tmp_path):
+    """Such a tree is marked, after a load, a refit and an update alike."""
+    v, i, nodes, ids, _ = _trees(oracle, "soup")
+    s = _Scene(scene_host, tmp_path, oracle, v, i)
+    s.ops.append("limit:100")
+    s.load("tree", nodes, ids)
+    s.ops += ["save:a", "refit", "save:b", "update", "save:c", "refit", "save:d", "limit:33554432",
+              "refit", "save:e", "update", "save:f", "refit", "save:g"]
+    assert [a["irregular"] for a in s.run()] == [1, 1, 1, 1, 1, 0, 0]
