@@ -177,9 +177,10 @@ mh::DevUpdate tree_view(mh_scene* s) {
 // deeper gets more passes after the counters are read back. MH_UPDATE_FRONTIER_LEVELS (1 or
 // more) sets the first batch's size instead, so that tests can reach the later batches.
 // Copies `extra` (two words) back along with the counters; synchronises the stream.
-// MH_OK, MH_E_UNSUPPORTED (deeper than the lists hold) or MH_E_STATE (not a binary tree).
-int wide_pass(mh_scene* s, const std::vector<mh::LevelList>& sizes, int irregular,
-              const unsigned* extra, unsigned extra_out[2], hipStream_t st) {
+// MH_OK, MH_E_UNSUPPORTED (inner records at more than max_levels depths) or MH_E_STATE (not
+// a binary tree).
+int wide_pass(mh_scene* s, const std::vector<mh::LevelList>& sizes, unsigned max_levels,
+              int irregular, const unsigned* extra, unsigned extra_out[2], hipStream_t st) {
   const mh::DevUpdate u = tree_view(s);
   mh::DevFrontier f{};
   f.fr = s->hist.as<unsigned>();
@@ -223,7 +224,7 @@ int wide_pass(mh_scene* s, const std::vector<mh::LevelList>& sizes, int irregula
   }
   unsigned deepest = 0;
   while ((int)deepest < d_end && hc[deepest]) ++deepest;
-  if (hc[d_end] || deepest >= (unsigned)mh::kMaxDepth - 1)
+  if (hc[d_end] || deepest > max_levels)
     return fail(MH_E_UNSUPPORTED, "tree deeper than %d levels", mh::kMaxDepth - 1);
   s->lev.clear();
   int64_t at[2] = {0, (int64_t)s->list_cap};
@@ -355,7 +356,9 @@ int upload(mh_scene* s, bool rtsah = false) {
   HIP_OK(hipMemset(s->leaf_at.p, 0xFF, (size_t)T * 4));
   HIP_OK(hipMemset(s->irregular.p, 0, 8));
   if (n_inner > 0) {
-    if ((rc = wide_pass(s, sizes, s->fixed_irregular | !nested, nullptr, nullptr, nullptr))) return rc;
+    if ((rc = wide_pass(s, sizes, mh::kMaxDepth - 1, s->fixed_irregular | !nested, nullptr, nullptr,
+                        nullptr)))
+      return rc;
     s->root_ref = 0;
   } else {
     const mh::RefNode& n = nodes[0];
@@ -795,7 +798,7 @@ int build_device(mh_scene* s, int rtsah) {
     std::vector<mh::LevelList> sizes;
     for (int k = 0; k < n_levels; ++k)
       sizes.push_back(mh::LevelList{0, level_off[k + 1] - level_off[k]});
-    if ((rc = wide_pass(s, sizes, 0, nullptr, nullptr, st))) return rc;
+    if ((rc = wide_pass(s, sizes, mh::kMaxDepth - 2, 0, nullptr, nullptr, st))) return rc;
     s->root_ref = 0;
   } else {
     if ((rc = leaf_root(s, 0, st))) return rc;
@@ -1115,7 +1118,7 @@ int mh_scene_update(mh_scene* s, void* stream) {
   if (s->n_inner > 0) {  // rotations never turn a leaf root inner
     const std::vector<mh::LevelList> sizes = s->lev;
     s->fixed_irregular = 0;
-    rc = wide_pass(s, sizes, 0, nfree, now, st);
+    rc = wide_pass(s, sizes, mh::kMaxDepth - 2, 0, nfree, now, st);
   } else {
     int32_t mark[2];  // the leaf pass's NaN mark, which wide_pass takes over otherwise
     HIP_OK(hipMemcpyAsync(s->host_ctr, nfree, 8, hipMemcpyDeviceToHost, st));

@@ -205,3 +205,35 @@ def test_more_wide_nodes_than_a_descriptor_reaches(scene_host, oracle, tmp_path)
     s.ops += ["save:a", "refit", "save:b", "update", "save:c", "refit", "save:d", "limit:33554432",
               "refit", "save:e", "update", "save:f", "refit", "save:g"]
     assert [a["irregular"] for a in s.run()] == [1, 1, 1, 1, 1, 0, 0]
+
+
+def _one_sided(oracle, v, i):
+    """A leaf of one triangle at every depth."""
+    T = len(i)
+    nodes = np.zeros(2 * T, oracle.NODE_DTYPE)
+    for k in range(T - 1):
+        nodes["child"][2 * k] = 2 * k + 1
+        nodes["child"][2 * k + 1], nodes["children"][2 * k + 1] = k, 1
+    nodes["child"][2 * T - 2], nodes["children"][2 * T - 2] = T - 1, 1
+    ids = np.arange(T, dtype=np.int32)
+    oracle.refit(v, i, nodes, ids)
+    return nodes, ids
+
+
+@pytest.mark.parametrize("n", [255, 256, 257])
+def test_deepest_trees(scene_host, oracle, tmp_path, n):
+    """Inner records down to depth 254 load and refit; one deeper is refused."""
+    v, i = scenes.soup(n, seed=n)
+    nodes, ids = _one_sided(oracle, v, i)
+    s = _Scene(scene_host, tmp_path, oracle, v, i)
+    s.load("tree", nodes, ids)
+    vd = (v * np.float32(1.5)).astype(np.float32)
+    s.vertices("v1", vd)
+    s.ops += ["refit", "save:s"]
+    if n > 256:
+        with pytest.raises(AssertionError, match="deeper than 255"):
+            s.run()
+        return
+    assert s.run()[0]["depth"] == n - 1
+    oracle.refit(vd, i, nodes, ids)
+    assert s.saved("s")[0].tobytes() == nodes.tobytes()
