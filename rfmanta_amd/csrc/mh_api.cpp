@@ -460,7 +460,8 @@ int trace_impl(const mh_scene* cs, const mh_rays* rays, const mh_hits* hits, int
     // The reference records' kernel: its stack is shorter, and the counters are kept there.
     const int64_t ref_need = std::max<int64_t>(0, (int64_t)s->stack_bound(MH_LAYOUT_REF) - S);
     const int64_t ref_want = (n + 255) / 256;
-    int64_t ref_blocks = std::min(ref_want, cus * 16);
+    int64_t ref_blocks =
+        std::min(ref_want, cus * (opts && opts->blocks_per_cu > 0 ? opts->blocks_per_cu : 16));
     if (ref_need > 0 && fixed_spill) {
       // Fewer workgroups (the kernel strides over the rays, results are unchanged) until
       // every lane's spill column fits the area; at least one workgroup per compute unit.

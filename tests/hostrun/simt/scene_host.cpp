@@ -6,6 +6,9 @@
 //   DIR holds verts.bin and idx.bin; OP is one of
 //   load:NAME    NAME.ids and NAME.nodes into the scene
 //   verts:FILE   the vertices of FILE
+//   trace:N,BLOCKS,RING,COUNT  mh_trace of N rays with blocks_per_cu, stack_lds and, if COUNT,
+//                counters: prints "blocks B layout L ring R spill BYTES" of its launch
+//   room:BYTES   no device allocation beyond BYTES succeeds from here on
 //   limit:N      trees of more than N wide nodes are traversed on their records
 //   refit, update
 //   save:NAME    the tree to NAME.ids and NAME.nodes, after checking what the traversal
@@ -18,9 +21,12 @@
 #include "internal.h"
 #include "prim_setup.h"
 
+mh::LaunchCfg g_launch;
+
 namespace mh {
-int launch_trace(const DevScene&, const DevRays&, const DevHits&, int64_t, const LaunchCfg&, void*) {
-  return 1;
+int launch_trace(const DevScene&, const DevRays&, const DevHits&, int64_t, const LaunchCfg& c, void*) {
+  g_launch = c;
+  return 0;
 }
 int launch_shade(const DevShade&, void*) { return 1; }
 int launch_copy(void*, const void*, size_t, int, void*) { return 1; }
@@ -168,6 +174,30 @@ int main(int argc, char** argv) {
                                  (uint32_t)nodes.size(), MH_PRIM_KENSLER_SHIRLEY), op);
     } else if (what == "verts") {
       check(mh_scene_set_vertices(s, read<float>(name).data(), 0, nullptr), op);
+    } else if (what == "trace") {
+      long n = 0;
+      mh_trace_opts o{};
+      int count = 0;
+      if (std::sscanf(op.c_str() + colon + 1, "%ld,%d,%d,%d", &n, &o.blocks_per_cu, &o.stack_lds,
+                      &count) != 4)
+        return 2;
+      int64_t counters[2];
+      if (count) o.counters = counters;
+      float f = 0.f;  // never read: the launch is only recorded
+      int32_t prim = 0;
+      const mh_rays rays{&f, &f, &f, &f, &f, &f, &f, nullptr};
+      const mh_hits hits{&prim, nullptr, nullptr, nullptr, nullptr};
+      check(mh_trace(s, &rays, &hits, n, 0, &o, nullptr), op);
+      const mh::LaunchCfg& c = g_launch;
+      const int lanes = c.layout == mh::kLayoutPair ? 64 : 256;
+      const int64_t stack = (int64_t)s->stack_bound(c.layout) - c.stack_lds;
+      need(c.spill_stride == (int64_t)c.blocks * lanes, "spill columns", c.spill_stride);
+      if (stack > 0)
+        need((size_t)stack * c.spill_stride * 8 <= s->spill[nullptr]->bytes, "spill area", stack);
+      std::printf("blocks %d layout %d ring %d spill %zu\n", c.blocks, c.layout, c.stack_lds,
+                  stack > 0 ? s->spill[nullptr]->bytes : (size_t)0);
+    } else if (what == "room") {
+      simt::room = (size_t)std::atoll(op.c_str() + colon + 1);
     } else if (what == "limit") {
       s->max_wide = (uint32_t)std::atol(op.c_str() + colon + 1);
     } else if (what == "refit") {

@@ -14,6 +14,9 @@
 dim3 threadIdx, blockIdx, gridDim, blockDim;
 
 namespace simt {
+
+size_t room = ~(size_t)0;
+
 namespace {
 
 constexpr size_t kStack = 256 << 10;
@@ -162,8 +165,8 @@ void launch(dim3 grid, dim3 block, const std::function<void()>& lane) {
 }  // namespace simt
 
 hipError_t hipMalloc(void** p, size_t n) {
-  *p = std::malloc(n);
-  if (*p) std::memset(*p, 0xA5, n);  // whatever was there before
+  *p = n <= simt::room ? std::malloc(n) : nullptr;
+  if (*p && n < (64 << 20)) std::memset(*p, 0xA5, n);  // whatever was there before
   return *p ? hipSuccess : hipErrorOutOfMemory;
 }
 hipError_t hipFree(void* p) {

@@ -54,6 +54,7 @@ enum class Op { kBarrier, kBallot, kShfl };
 // lane `src`; a shuffle from a lane that is not there ends the program.
 unsigned long long wait(Op op, unsigned long long value, int src, int site);
 void launch(dim3 grid, dim3 block, const std::function<void()>& lane);
+extern size_t room;  // the largest device allocation that succeeds
 }  // namespace simt
 
 inline void __syncthreads(int site = __builtin_LINE()) { simt::wait(simt::Op::kBarrier, 0, 0, site); }

@@ -237,3 +237,20 @@ def test_deepest_trees(scene_host, oracle, tmp_path, n):
     assert s.run()[0]["depth"] == n - 1
     oracle.refit(vd, i, nodes, ids)
     assert s.saved("s")[0].tobytes() == nodes.tobytes()
+
+
+def _launches(scene_host, oracle, tmp_path, n_tris, *ops):
+    v, i = scenes.soup(n_tris, seed=1)
+    s = _Scene(scene_host, tmp_path, oracle, v, i)
+    s.load("tree", *_one_sided(oracle, v, i))
+    s.ops += ops
+    return s.run()
+
+
+def test_blocks_per_cu_with_counters(scene_host, oracle, tmp_path):
+    """The caller's workgroups per compute unit hold for the counting kernel as for the other
+    (256 lanes each, of 256 compute units)."""
+    a, b, c, d = _launches(scene_host, oracle, tmp_path, 4, "trace:4000000,2,8,1", "trace:4000000,0,8,1",
+                           "trace:4000000,2,8,0", "trace:100,2,8,1")
+    assert (a["layout"], a["blocks"]) == (1, 512) and b["blocks"] == 4096
+    assert (c["layout"], c["blocks"]) == (0, 4 * 512) and d["blocks"] == 1
