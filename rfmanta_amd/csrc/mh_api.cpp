@@ -413,11 +413,15 @@ constexpr int kTraceBlocksPerCu = 32;
 constexpr int64_t kMinWaveRays = 4;
 // Ring entries unless the caller says: 16 (five waves per SIMD fill the LDS) spill less than
 // 8 (786,432 camera and bounce rays in a 200,000-triangle soup 1274 against 1337 us), and
-// where there are few waves 32 need no spill area up to a depth of 21 (allocating one takes
+// where there are few waves 32 need no spill area up to a depth of 20 (allocating one takes
 // a first call about 300 us). 32 with waves to spare cost occupancy: 199,023 rays 68
 // against 57 us.
 constexpr int kWideRing = 16, kFewWavesRing = 32;
 constexpr int64_t kFewWaves = 8;  // per compute unit
+// A stream's spill area, unless the resident waves alone need more: trees of up to 32 levels
+// (a heightfield of 8M triangles has 25) get all the waves below this, a tree of 60 levels
+// 2.8 times the resident ones, and no tree more than 965 MB.
+constexpr int64_t kSpillBytes = int64_t(512) << 20;
 
 // The caller's ring, or the one the reference records' kernel takes.
 int choose_stack(const mh_trace_opts* o) {
@@ -489,6 +493,9 @@ int trace_impl(const mh_scene* cs, const mh_rays* rays, const mh_hits* hits, int
       const int64_t fit = (int64_t)(fixed_bytes / (size_t)(need * 64 * 8));
       wide = wide && fit >= std::min(waves, 4 * cus);
       blocks = std::min(blocks, fit);
+    } else if (need > 0) {
+      blocks = std::min(blocks, std::max<int64_t>(mh_internal::resident_waves(),
+                                                  kSpillBytes / (need * 64 * 8)));
     }
     if (wide) {
       cfg.layout = MH_LAYOUT_PAIR;
@@ -510,7 +517,13 @@ int trace_impl(const mh_scene* cs, const mh_rays* rays, const mh_hits* hits, int
       DevBuf*& b = s->spill[stream];
       if (!b) b = new (std::nothrow) DevBuf();
       if (!b) return fail(MH_E_NOMEM, "spill descriptor");
-      if ((rc = b->reserve((size_t)need * cfg.spill_stride * 8))) return rc;
+      rc = b->reserve((size_t)need * cfg.spill_stride * 8);
+      if (rc == MH_E_NOMEM && wide && cfg.blocks > mh_internal::resident_waves()) {
+        cfg.blocks = mh_internal::resident_waves();
+        cfg.spill_stride = (int64_t)cfg.blocks * 64;
+        rc = b->reserve((size_t)need * cfg.spill_stride * 8);
+      }
+      if (rc) return rc;
       cfg.spill = b->as<int32_t>();
     }
   }

@@ -254,3 +254,23 @@ def test_blocks_per_cu_with_counters(scene_host, oracle, tmp_path):
                            "trace:4000000,2,8,0", "trace:100,2,8,1")
     assert (a["layout"], a["blocks"]) == (1, 512) and b["blocks"] == 4096
     assert (c["layout"], c["blocks"]) == (0, 4 * 512) and d["blocks"] == 1
+
+
+def test_spill_area_is_bounded(scene_host, oracle, tmp_path):
+    """Rays of a deep tree take fewer waves, at least the resident ones (20 per compute unit),
+    once the spill area passes 512 MiB; where that much is not to be had either, the resident
+    ones alone."""
+    mib = 1 << 20
+    deep = ["trace:4000000,0,0,0", f"room:{300 * mib}", "trace:4000000,16,16,0"]
+    a, b = _launches(scene_host, oracle, tmp_path, 61, *deep)
+    need = 3 * 30 - 16  # depth 60
+    assert a["ring"] == 16 and a["blocks"] == 512 * mib // (need * 512)
+    assert a["spill"] <= 512 * mib
+    # the area that is there already serves the second trace
+    assert b["blocks"] * 64 * need * 8 <= a["spill"]
+    c, = _launches(scene_host, oracle, tmp_path, 61, *deep[1:])
+    assert c["blocks"] == 5120 and c["spill"] == 5120 * 64 * need * 8
+    d, = _launches(scene_host, oracle, tmp_path, 256, deep[0])
+    assert d["blocks"] == 5120
+    e, = _launches(scene_host, oracle, tmp_path, 23, deep[0])
+    assert e["blocks"] == 32768  # depth 22: every wave of its own up to the cap
