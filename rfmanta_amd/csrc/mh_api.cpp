@@ -537,8 +537,7 @@ int trace_impl(const mh_scene* cs, const mh_rays* rays, const mh_hits* hits, int
 }  // namespace
 
 int mh_internal::ensure_soa(mh_scene* s, void* stream) {
-  const size_t n = s->n_records / 2;
-  if (n == 0) return fail(MH_E_STATE, "scene has no pair records");
+  const size_t n = std::max<size_t>(1, s->n_records / 2);  // (a single record has no pair)
   int rc;
   if ((rc = s->pairs.reserve(n * sizeof(mh::PairNode)))) return rc;
   if (s->pairs_soa.bytes != n * sizeof(mh::PairNode)) {

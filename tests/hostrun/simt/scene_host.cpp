@@ -8,6 +8,7 @@
 //   verts:FILE   the vertices of FILE
 //   trace:N,BLOCKS,RING,COUNT  mh_trace of N rays with blocks_per_cu, stack_lds and, if COUNT,
 //                counters: prints "blocks B layout L ring R spill BYTES" of its launch
+//   soa          the node arrays of the SOA layout
 //   room:BYTES   no device allocation beyond BYTES succeeds from here on
 //   limit:N      trees of more than N wide nodes are traversed on their records
 //   refit, update
@@ -196,6 +197,8 @@ int main(int argc, char** argv) {
         need((size_t)stack * c.spill_stride * 8 <= s->spill[nullptr]->bytes, "spill area", stack);
       std::printf("blocks %d layout %d ring %d spill %zu\n", c.blocks, c.layout, c.stack_lds,
                   stack > 0 ? s->spill[nullptr]->bytes : (size_t)0);
+    } else if (what == "soa") {
+      check(mh_internal::ensure_soa(s, nullptr), op);
     } else if (what == "room") {
       simt::room = (size_t)std::atoll(op.c_str() + colon + 1);
     } else if (what == "limit") {

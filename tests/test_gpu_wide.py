@@ -334,6 +334,28 @@ def test_single_leaf_with_a_vertex_that_is_not_a_number(oracle, n):
                 assert np.array_equal(_bits(g["t"]), _bits(o["t"])), k
 
 
+def test_frames_of_a_single_record(oracle):
+    v, i = scenes.soup(3, seed=1, sigma=0.5)
+    nodes = np.zeros(1, oracle.NODE_DTYPE)
+    nodes["children"] = 3
+    nodes["lo"], nodes["hi"] = v.min(0), v.max(0)
+    ids = np.arange(3, dtype=np.int32)
+    rays = scenes.random_rays(500, 2, (-1.5, -1.5, -1.5), (1.5, 1.5, 1.5))
+    o = oracle.trace(v, i, nodes, ids, rays, packet_size=1)
+    with api.Scene(v, i) as s:
+        s.load_dynbvh(ids, nodes)
+        dh = api.DeviceHits.alloc(500)
+        f = api.Frame(s, [(api.DeviceRays.upload(rays), dh, False)])
+        for layout in (L.MH_LAYOUT_PAIR, L.MH_LAYOUT_REF, L.MH_LAYOUT_SOA):
+            f.set_config(dict(layout=layout, stack_lds=8, block=64, blocks_per_cu=1, refill=64,
+                              chunk=64, reverse=0))
+            dh.arrays["prim"].upload(np.full(500, 777, np.int32))
+            f.launch()
+            api.sync()
+            assert np.array_equal(dh.download()["prim"], o["prim"]), layout
+        f.close()
+
+
 @pytest.mark.parametrize("batches", [1, 3])
 def test_frames_of_zero_components_and_short_chunks(oracle, batches):
     v, i = scenes.heightfield(50, 30, seed=5)

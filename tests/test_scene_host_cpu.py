@@ -274,3 +274,13 @@ def test_spill_area_is_bounded(scene_host, oracle, tmp_path):
     assert d["blocks"] == 5120
     e, = _launches(scene_host, oracle, tmp_path, 23, deep[0])
     assert e["blocks"] == 32768  # depth 22: every wave of its own up to the cap
+
+
+def test_soa_nodes_of_a_single_record(scene_host, oracle, tmp_path):
+    """A loaded tree may hold its root alone."""
+    v, i = scenes.soup(3, seed=1)
+    nodes, ids = _leaf_root(oracle, v, i)
+    s = _Scene(scene_host, tmp_path, oracle, v, i)
+    s.load("tree", nodes[:1], ids)
+    s.ops += ["soa", "refit", "soa"]
+    s.run()
