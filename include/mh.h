@@ -303,10 +303,13 @@ typedef struct mh_launch_config {
   int block;         /* lanes per workgroup: 64, 128 or 256 */
   int blocks_per_cu; /* persistent workgroups per compute unit */
   int refill;        /* idle lanes of a wave that trigger a refill, 1..63; 64 = whole-wave
-                        chunks (a wave traces `chunk` consecutive rays 64 at a time) */
+                        chunks (a wave traces `chunk` consecutive rays 64 at a time; in the
+                        PAIR layout a wave with a chunk of more than 64 takes the chunk's
+                        next rays when 40 lanes are idle) */
   int chunk;         /* rays a wave takes per grab from the shared counter, a multiple of 64
-                        (its first grab is assigned statically); 0 = static stride over the
-                        rays with no counter (whole-wave mode only) */
+                        (its first grab is assigned statically; in the PAIR layout at most a
+                        quarter of a resident wave's share of the rays); 0 = static stride
+                        over the rays with no counter (whole-wave mode only) */
   int xcd_remap;     /* 1 = give each XCD (every 8th workgroup) a contiguous share of the
                         rays so that neighbouring rays share an L2 */
   int reverse;       /* 1 = hand rays out from the end of the table (last batch first, in

@@ -74,7 +74,7 @@ int check_launch_config(const mh_launch_config& c) {
 namespace {
 
 const mh_launch_config kDefault = {MH_LAYOUT_PAIR, 8, 256, 16, 64, 256, 1, 0};
-
+constexpr int kTunedKernels = 2;  // 2: four-wide nodes, refill as given
 
 // Kernel specialisation for a table: closest-hit only, any-hit only, or mixed.
 int kinds_of(int nb, int n_any) { return n_any == 0 ? 1 : (n_any == nb ? 2 : 0); }
@@ -392,12 +392,13 @@ int mh_frame_autotune(mh_frame* f, int iters, const char* cache_path, int force,
   if (cache_path) cache = read_cache(cache_path);
   if (cache_path && !force && cache.count(key)) {
     const std::string& obj = cache[key];
-    double v[9];
-    const char* names[9] = {"layout", "stack_lds", "block", "blocks_per_cu",
-                            "refill", "chunk", "xcd_remap", "reverse", "ms"};
+    double v[10];
+    const char* names[10] = {"layout", "stack_lds", "block",     "blocks_per_cu", "refill",
+                             "chunk",  "xcd_remap", "reverse",   "ms",            "kernels"};
     bool ok = true;
-    for (int i = 0; i < 9; ++i) ok = ok && field(obj, names[i], v[i]);
-    if (ok) {  // entries written before the reverse field was added are tuned again
+    for (int i = 0; i < 10; ++i) ok = ok && field(obj, names[i], v[i]);
+    // entries tuned for other kernels, or written before a field was added, are tuned again
+    if (ok && (int)v[9] == kTunedKernels) {
       mh_launch_config c{(int)v[0], (int)v[1], (int)v[2], (int)v[3],
                          (int)v[4], (int)v[5], (int)v[6], (int)v[7]};
       if (mh_internal::check_launch_config(c) == MH_OK) {
@@ -454,7 +455,7 @@ int mh_frame_autotune(mh_frame* f, int iters, const char* cache_path, int force,
   // both hand-out orders (the order moves the best shape).
   base = best;
   for (int rev = 0; rev < 2; ++rev)
-    for (int r : {16, 32, 48})
+    for (int r : {32, 40, 48})
       for (int c : {64, 128, 256})
         for (const auto& bp : {std::pair<int, int>{256, 5}, {256, 6}, {256, 7}, {128, 10},
                                {128, 12}, {128, 14}}) {
@@ -480,9 +481,9 @@ int mh_frame_autotune(mh_frame* f, int iters, const char* cache_path, int force,
     std::snprintf(buf, sizeof(buf),
                   "{\"layout\": %d, \"stack_lds\": %d, \"block\": %d, \"blocks_per_cu\": %d, "
                   "\"refill\": %d, \"chunk\": %d, \"xcd_remap\": %d, \"reverse\": %d, "
-                  "\"ms\": %.5f}",
+                  "\"ms\": %.5f, \"kernels\": %d}",
                   best.layout, best.stack_lds, best.block, best.blocks_per_cu, best.refill,
-                  best.chunk, best.xcd_remap, best.reverse, best_ms);
+                  best.chunk, best.xcd_remap, best.reverse, best_ms, kTunedKernels);
     cache[key] = buf;
     write_cache(cache_path, cache);
   }

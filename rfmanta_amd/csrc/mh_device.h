@@ -158,6 +158,18 @@ struct BatchLaunch {
   int kinds;      // 0 mixed table, 1 closest-hit batches only, 2 any-hit batches only
 };
 
+// Idle lanes that make a wave of the wide kernel take rays (kLayoutPair): the caller's, but
+// whole-wave chunks of more than 64 rays go by this many instead of waiting for the last lane,
+// and no chunk is more than a quarter of a resident wave's share of the rays. (12 uneven
+// batches, 3M rays in a 300,000-triangle soup, 256-ray chunks: 1,691 us; 2,928 with 64 idle
+// lanes and whole chunks. At 8, 16, 24, 32, 40, 48 and 56 idle lanes that frame takes 1634,
+// 1546, 1525, 1482, 1513, 1571 and 1658 us, and 4.1M primary and bounce rays over a
+// 1M-triangle heightfield 793, 747, 715, 701, 700, 702 and 748; five to eight batches of 0.5
+// to 1.5M rays in 20,000 to 1M triangles differ by 1% from 24 to 48.)
+constexpr int kChunkRefill = 40;
+inline int wide_refill(int refill, int chunk) {
+  return refill == 64 && chunk > 64 ? kChunkRefill : refill;
+}
 int launch_trace_batch(const DevScene& sc, const BatchLaunch& bl, void* stream);
 
 // Launchers (trace.hip). Return hipError_t as int.

@@ -676,16 +676,6 @@ int launch_table(const WideArgs& a, dim3 g, int stack_lds, hipStream_t s) {
 // A lane at a leaf weighs as much as one at a node: a triangle test costs about what a node
 // visit does. (Half of that is 4% better on camera rays and 6% worse on a soup's.)
 constexpr int kLeafWeight = 4;
-// Whole-wave chunks of more than 64 rays: the wave takes its chunk's next rays when this many
-// lanes are idle, and no chunk is more than a quarter of a resident wave's share of the rays.
-// (12 uneven batches, 3M rays in a 300,000-triangle soup, the frames' default configuration,
-// 256-ray chunks: 1691 us; 2928 with 64 idle lanes and whole chunks.) It is also the least
-// number of idle lanes a wave waits for: a step covers two levels of the tree, so taking rays
-// is dear beside it. (2.07M primary and 1.73M bounce rays over a 1M-triangle heightfield, 10
-// workgroups of 128 lanes per compute unit: 638 us at 32 idle lanes, 614 at 40 and 48, 637 at
-// 56, 673 at 60.)
-constexpr int kChunkRefill = 40;
-
 template <int PRIM>
 int launch_wide_table(const DevScene& sc, const BatchLaunch& bl, hipStream_t s) {
   WideArgs a{};
@@ -695,7 +685,7 @@ int launch_wide_table(const DevScene& sc, const BatchLaunch& bl, hipStream_t s) 
   a.spill = reinterpret_cast<unsigned long long*>(bl.spill);
   a.spill_stride = bl.spill_stride;
   a.nb = bl.nb;
-  a.refill = bl.refill == 64 && bl.chunk > 64 ? kChunkRefill : std::max(bl.refill, kChunkRefill);
+  a.refill = wide_refill(bl.refill, bl.chunk);
   a.chunk = bl.chunk == 0 ? 64 : bl.chunk;
   a.fair = bl.chunk > 64 ? 4 * bl.resident : 0;
   a.remap = bl.xcd_remap;

@@ -255,13 +255,12 @@ def config1_scene(nx: int = 1000, nz: int = 500, seed: int = 0):
 
 
 # Launch configuration of the C1 frame (primary + bounce batches in one launch):
-# the round refill (a lane takes a new ray when 32 of its wave's lanes are idle, rays
-# handed out 256 at a time) from the end of the table, so the incoherent bounce rays go
-# first and the frame ends on short primary rays; 10 workgroups of 128 lanes per CU (five
-# waves per SIMD), LDS ring of 8, the wide nodes. In table order the same schedule at 12
-# workgroups per CU was 1.5-1.7% ahead of the static stride; handed out in reverse it is
-# 6-7% faster, and 2% more at 10 workgroups per CU.
-C1_LAUNCH = {"layout": 0, "stack_lds": 8, "block": 128, "blocks_per_cu": 10, "refill": 32,
+# the per-lane refill (lanes take new rays when 40 of their wave's are idle, rays handed out
+# 256 at a time) from the end of the table, so the incoherent bounce rays go first and the
+# frame ends on short primary rays; 10 workgroups of 128 lanes per CU (five waves per SIMD),
+# LDS ring of 8, the wide nodes. A step covers two levels of the tree, so taking rays is dear
+# beside it: 638 us a frame at 32 idle lanes, 614 at 40 and 48, 637 at 56, 673 at 60.
+C1_LAUNCH = {"layout": 0, "stack_lds": 8, "block": 128, "blocks_per_cu": 10, "refill": 40,
              "chunk": 256, "xcd_remap": 0, "reverse": 1}
 # The static stride (24 workgroups of 256 lanes per CU), in table order.
 C1_LAUNCH_STATIC = {"layout": 0, "stack_lds": 8, "block": 256, "blocks_per_cu": 24,

@@ -8,6 +8,8 @@
 //   verts:FILE   the vertices of FILE
 //   trace:N,BLOCKS,RING,COUNT  mh_trace of N rays with blocks_per_cu, stack_lds and, if COUNT,
 //                counters: prints "blocks B layout L ring R spill BYTES" of its launch
+//   refill:R,C   prints "refill N", the idle lanes that a launch configuration's refill and
+//                chunk come to in the default layout
 //   soa          the node arrays of the SOA layout
 //   room:BYTES   no device allocation beyond BYTES succeeds from here on
 //   limit:N      trees of more than N wide nodes are traversed on their records
@@ -197,6 +199,10 @@ int main(int argc, char** argv) {
         need((size_t)stack * c.spill_stride * 8 <= s->spill[nullptr]->bytes, "spill area", stack);
       std::printf("blocks %d layout %d ring %d spill %zu\n", c.blocks, c.layout, c.stack_lds,
                   stack > 0 ? s->spill[nullptr]->bytes : (size_t)0);
+    } else if (what == "refill") {
+      int r = 0, c = 0;
+      if (std::sscanf(op.c_str() + colon + 1, "%d,%d", &r, &c) != 2) return 2;
+      std::printf("refill %d\n", mh::wide_refill(r, c));
     } else if (what == "soa") {
       check(mh_internal::ensure_soa(s, nullptr), op);
     } else if (what == "room") {

@@ -284,3 +284,9 @@ def test_soa_nodes_of_a_single_record(scene_host, oracle, tmp_path):
     s.load("tree", nodes[:1], ids)
     s.ops += ["soa", "refit", "soa"]
     s.run()
+
+
+def test_refill_is_the_callers(scene_host, oracle, tmp_path):
+    ops = [(1, 64), (16, 256), (32, 128), (63, 1024), (64, 64), (64, 0), (64, 256)]
+    got = _launches(scene_host, oracle, tmp_path, 2, *[f"refill:{r},{c}" for r, c in ops])
+    assert [g["refill"] for g in got] == [1, 16, 32, 63, 64, 64, 40]
