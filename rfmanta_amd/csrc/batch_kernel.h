@@ -1,7 +1,7 @@
 // Persistent multi-batch traversal of the REF and SOA node layouts for gfx950 (wave64).
 // Included by the four batch_<triangle>_<layout>.hip files, which instantiate the launchers
 // of one triangle test and node layout each, so that the kernel variants compile in
-// parallel. (Frames in the default layout run k_trace_wide, wide_trace.h.)
+// parallel. (Frames in the default layout run wide_trace.h's kernels.)
 //
 // k_trace_batch consumes a table of ray batches (each its own SoA arrays, size and
 // closest-hit/any-hit flag) in one launch. Rays are numbered across batches by the

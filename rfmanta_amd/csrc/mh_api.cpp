@@ -461,7 +461,7 @@ int trace_impl(const mh_scene* cs, const mh_rays* rays, const mh_hits* hits, int
     const int S = choose_stack(opts);
     const int bpc = (opts && opts->blocks_per_cu > 0) ? opts->blocks_per_cu : kTraceBlocksPerCu;
     const int64_t cus = g_lib.cu_count;
-    // The reference records' kernel: its stack is shorter, and the counters are kept there.
+    // The reference records' kernel, which keeps the counters.
     const int64_t ref_need = std::max<int64_t>(0, (int64_t)s->stack_bound(MH_LAYOUT_REF) - S);
     const int64_t ref_want = (n + 255) / 256;
     int64_t ref_blocks =
@@ -488,11 +488,17 @@ int trace_impl(const mh_scene* cs, const mh_rays* rays, const mh_hits* hits, int
                                                     : kWideRing;
     int64_t blocks = std::min(waves, 4 * cus * bpc);
     int64_t need = std::max<int64_t>(0, (int64_t)s->stack_bound(MH_LAYOUT_PAIR) - wide_S);
-    bool wide = !cfg.counters;
-    if (fixed_spill && need > 0) {  // the wide nodes' longer stack may not fit where a ref's does
-      const int64_t fit = (int64_t)(fixed_bytes / (size_t)(need * 64 * 8));
-      wide = wide && fit >= std::min(waves, 4 * cus);
-      blocks = std::min(blocks, fit);
+    const bool wide = !cfg.counters;
+    auto fit = [&] { return (int64_t)(fixed_bytes / (size_t)(need * 64 * 8)); };
+    if (fixed_spill && need > 0 && fit() < std::min(waves, 4 * cus)) {
+      // Four waves per compute unit do not fit: on the records a ray's stack takes one entry
+      // a level (and the ring, which makes room for three at a time, spills two early), which
+      // the check above leaves room for.
+      cfg.pairs = 1;
+      need = std::max<int64_t>(0, (int64_t)s->depth + 2 - wide_S);
+    }
+    if (fixed_spill && need > 0) {
+      blocks = std::min(blocks, fit());
     } else if (need > 0) {
       blocks = std::min(blocks, std::max<int64_t>(mh_internal::resident_waves(),
                                                   kSpillBytes / (need * 64 * 8)));

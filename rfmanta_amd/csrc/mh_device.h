@@ -109,6 +109,7 @@ struct LaunchCfg {
   int32_t* spill;     // per-thread stack spill (single-ray)
   int64_t spill_stride;
   int chunk;          // kLayoutPair: rays a wave takes at a time, 1..64
+  int pairs;          // kLayoutPair: traverse the records, on a stack of one entry a level
 };
 
 // Node layouts of the single-ray traversal (MH_LAYOUT_*). A non-root record r's box is

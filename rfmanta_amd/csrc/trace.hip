@@ -1,9 +1,9 @@
 // Traversal kernels for gfx950 (wave64).
 //
-// Single rays take k_trace_wide (wide_trace.h). k_trace_ray: one ray per lane,
+// Single rays take k_wide_whole (wide_trace.h). k_trace_ray: one ray per lane,
 //   DynBVH::intersect on a one-ray packet (Model/Groups/DynBVH.cc:101-404) over the
-//   reference's 32-byte records, for callers that count box and triangle tests and for trees
-//   too deep for the wide nodes' stack in a fixed spill area; the traversal is traverse.h's.
+//   reference's 32-byte records, for callers that count box and triangle tests; the
+//   traversal is traverse.h's.
 //
 // k_trace_packet: one RayPacket of up to 64 consecutive rays per wave, the reference's
 //   packet recursion (intersectNode/firstIntersects/lastIntersects, DynBVH.cc:274-905,
@@ -45,7 +45,7 @@ constexpr int kWaves = kBlock / 64;
 // ---------------------------------------------------------------------------
 // Single-ray traversal of the reference's records (traverse.h), grid-stride over the rays.
 // ---------------------------------------------------------------------------
-template <bool ANY, int PRIM, int S, bool STATS>
+template <bool ANY, int PRIM, int S>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_trace_ray(
     DevScene sc, DevRays rays, DevHits hits, int64_t n, int2* spill, int64_t spill_stride,
     unsigned long long* counters) {
@@ -60,11 +60,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) 
   const GRays gr = global_view(rays);
   const GHits gh = global_view(hits);
   for (int64_t ri = gtid; ri < n; ri += stride)
-    trace_store<ANY, PRIM, kLayoutRef, S, kBlock, STATS>(sc, root, gr, gh, ri, st, nbox, ntri);
-  if (STATS && counters) {
-    atomicAdd(counters + 0, nbox);
-    atomicAdd(counters + 1, ntri);
-  }
+    trace_store<ANY, PRIM, kLayoutRef, S, kBlock, true>(sc, root, gr, gh, ri, st, nbox, ntri);
+  atomicAdd(counters + 0, nbox);
+  atomicAdd(counters + 1, ntri);
 }
 
 // ---------------------------------------------------------------------------
@@ -328,7 +326,7 @@ __global__ __launch_bounds__(kBlock) void k_trace_packet(DevScene sc, DevRays ra
   }
 }
 
-template <bool ANY, int PRIM, bool STATS>
+template <bool ANY, int PRIM>
 int launch_ray_s(const DevScene& sc, const DevRays& rays, const DevHits& hits, int64_t n,
                  const LaunchCfg& cfg, hipStream_t s) {
   unsigned long long* c = reinterpret_cast<unsigned long long*>(cfg.counters);
@@ -336,15 +334,15 @@ int launch_ray_s(const DevScene& sc, const DevRays& rays, const DevHits& hits, i
   dim3 g(cfg.blocks), b(kBlock);
   switch (cfg.stack_lds) {
     case 8:
-      hipLaunchKernelGGL((k_trace_ray<ANY, PRIM, 8, STATS>), g, b, 0, s, sc, rays, hits, n, sp,
+      hipLaunchKernelGGL((k_trace_ray<ANY, PRIM, 8>), g, b, 0, s, sc, rays, hits, n, sp,
                          cfg.spill_stride, c);
       break;
     case 32:
-      hipLaunchKernelGGL((k_trace_ray<ANY, PRIM, 32, STATS>), g, b, 0, s, sc, rays, hits, n, sp,
+      hipLaunchKernelGGL((k_trace_ray<ANY, PRIM, 32>), g, b, 0, s, sc, rays, hits, n, sp,
                          cfg.spill_stride, c);
       break;
     default:
-      hipLaunchKernelGGL((k_trace_ray<ANY, PRIM, 16, STATS>), g, b, 0, s, sc, rays, hits, n, sp,
+      hipLaunchKernelGGL((k_trace_ray<ANY, PRIM, 16>), g, b, 0, s, sc, rays, hits, n, sp,
                          cfg.spill_stride, c);
       break;
   }
@@ -367,8 +365,7 @@ int launch_any_prim(const DevScene& sc, const DevRays& rays, const DevHits& hits
                          dim3(kBlock), 0, s, sc, rays, hits, n, cfg.packet_size, c);
     return (int)hipGetLastError();
   }
-  return stats ? launch_ray_s<ANY, PRIM, true>(sc, rays, hits, n, cfg, s)
-               : launch_ray_s<ANY, PRIM, false>(sc, rays, hits, n, cfg, s);
+  return stats ? launch_ray_s<ANY, PRIM>(sc, rays, hits, n, cfg, s) : (int)hipErrorInvalidValue;
 }
 
 }  // namespace

@@ -152,7 +152,10 @@ __device__ __forceinline__ unsigned long long wide_box(float nx, float fx, float
 }
 
 // Per-lane stack, its newest S entries in LDS ([entry][lane], no bank conflicts), older ones
-// in the thread's spill column. sp and base count in steps of U bytes.
+// in the thread's spill column. sp and base count in steps of U bytes. A push makes room for
+// three entries whatever it keeps, so a column holds up to n - S of the wide nodes' at most n
+// entries (three a node), and up to n + 2 - S of n that come one at a time (wide_pair_step,
+// wide_redo: a tree of depth n; a column made for the wide nodes is longer than that).
 template <int S, int BLOCK>
 struct WideStack {
   static_assert((S & (S - 1)) == 0 && S > 4, "ring size is a power of two");
@@ -433,6 +436,7 @@ struct WideArgs {
   int remap;    // give each XCD a contiguous share of the first chunks
   int reverse;  // hand chunks out from the end of the table
   int weight;   // wide_step
+  int pairs;    // table null: traverse the records whatever the tree
 };
 
 // The kernel's arguments, to be read again (by scalar loads) where they are used: held in
@@ -487,7 +491,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5, 8))) v
   if (TABLE && a.remap && (gridDim.x & 7) == 0) blk = (blk & 7) * (gridDim.x >> 3) + (blk >> 3);
   WideStack<S, BLOCK> st(s_ring, a.spill, a.spill_stride, (int64_t)blockIdx.x * BLOCK + tid, tid);
   const float reach = root_reach(a.sc);
-  const int irregular = *a.sc.irregular;
+  int irregular = *a.sc.irregular;
+  if (!TABLE && a.pairs && irregular == 0) irregular = 1;
   const int C = a.chunk;
   const int64_t stride = (int64_t)gridDim.x * (BLOCK / 64) * C;
   // (the wave's number is the same in all its lanes: kept in scalar registers)
@@ -705,6 +710,7 @@ int launch_wide_one(const DevScene& sc, const BatchDev& rays, const LaunchCfg& c
   a.spill = reinterpret_cast<unsigned long long*>(cfg.spill);
   a.spill_stride = cfg.spill_stride;
   a.chunk = cfg.chunk;
+  a.pairs = cfg.pairs;
   a.reverse = 1;
   a.weight = kLeafWeight;
   const dim3 g(cfg.blocks), b(64);

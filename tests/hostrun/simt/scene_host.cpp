@@ -7,10 +7,11 @@
 //   load:NAME    NAME.ids and NAME.nodes into the scene
 //   verts:FILE   the vertices of FILE
 //   trace:N,BLOCKS,RING,COUNT  mh_trace of N rays with blocks_per_cu, stack_lds and, if COUNT,
-//                counters: prints "blocks B layout L ring R spill BYTES" of its launch
+//                counters: prints "blocks B layout L ring R spill BYTES pairs P" of its launch
 //   refill:R,C   prints "refill N", the idle lanes that a launch configuration's refill and
 //                chunk come to in the default layout
 //   soa          the node arrays of the SOA layout
+//   fixed:BYTES  later traces use a spill area of the caller's, as mh_trace_noalloc does
 //   room:BYTES   no device allocation beyond BYTES succeeds from here on
 //   limit:N      trees of more than N wide nodes are traversed on their records
 //   refit, update
@@ -25,6 +26,7 @@
 #include "prim_setup.h"
 
 mh::LaunchCfg g_launch;
+size_t g_fixed = 0;
 
 namespace mh {
 int launch_trace(const DevScene&, const DevRays&, const DevHits&, int64_t, const LaunchCfg& c, void*) {
@@ -190,15 +192,20 @@ int main(int argc, char** argv) {
       int32_t prim = 0;
       const mh_rays rays{&f, &f, &f, &f, &f, &f, &f, nullptr};
       const mh_hits hits{&prim, nullptr, nullptr, nullptr, nullptr};
-      check(mh_trace(s, &rays, &hits, n, 0, &o, nullptr), op);
+      static char fixed;
+      check(g_fixed ? mh_internal::trace_fixed_spill(s, &rays, &hits, n, 0, &o, nullptr, &fixed, g_fixed)
+                    : mh_trace(s, &rays, &hits, n, 0, &o, nullptr), op);
       const mh::LaunchCfg& c = g_launch;
       const int lanes = c.layout == mh::kLayoutPair ? 64 : 256;
-      const int64_t stack = (int64_t)s->stack_bound(c.layout) - c.stack_lds;
-      need(c.spill_stride == (int64_t)c.blocks * lanes, "spill columns", c.spill_stride);
-      if (stack > 0)
-        need((size_t)stack * c.spill_stride * 8 <= s->spill[nullptr]->bytes, "spill area", stack);
-      std::printf("blocks %d layout %d ring %d spill %zu\n", c.blocks, c.layout, c.stack_lds,
-                  stack > 0 ? s->spill[nullptr]->bytes : (size_t)0);
+      const int64_t stack =
+          (c.pairs ? (int64_t)s->depth + 2 : (int64_t)s->stack_bound(c.layout)) - c.stack_lds;
+      need(c.blocks > 0 && c.spill_stride == (int64_t)c.blocks * lanes, "spill columns", c.blocks);
+      const size_t area = stack <= 0 ? 0 : g_fixed ? g_fixed : s->spill[nullptr]->bytes;
+      if (stack > 0) need((size_t)stack * c.spill_stride * 8 <= area, "spill area", stack);
+      std::printf("blocks %d layout %d ring %d spill %zu pairs %d\n", c.blocks, c.layout,
+                  c.stack_lds, area, c.pairs);
+    } else if (what == "fixed") {
+      g_fixed = (size_t)std::atoll(op.c_str() + colon + 1);
     } else if (what == "refill") {
       int r = 0, c = 0;
       if (std::sscanf(op.c_str() + colon + 1, "%d,%d", &r, &c) != 2) return 2;

@@ -383,3 +383,64 @@ def test_frames_of_zero_components_and_short_chunks(oracle, batches):
                     if not a:
                         assert np.array_equal(_bits(g["t"]), _bits(o["t"])), (refill, chunk, rev)
         f.close()
+
+def _one_sided(oracle, v, i, deep_left=False):
+    """A leaf of one triangle at every depth."""
+    T = len(i)
+    nodes = np.zeros(2 * T, oracle.NODE_DTYPE)
+    rec = 0
+    for k in range(T - 1):
+        c = 2 * k + 1
+        nodes["child"][rec], nodes["axis"][rec], nodes["bits"][rec] = c, k % 3, k % 2
+        leaf, rec = (c + 1, c) if deep_left else (c, c + 1)
+        nodes["child"][leaf], nodes["children"][leaf] = k, 1
+    nodes["child"][rec], nodes["children"][rec] = T - 1, 1
+    ids = np.arange(T, dtype=np.int32)
+    oracle.refit(v, i, nodes, ids)
+    return nodes, ids
+
+
+@pytest.mark.parametrize("deep_left", [False, True])
+@pytest.mark.parametrize("n", [20, 65, 130, 256])
+def test_deep_trees_spill(oracle, n, deep_left):
+    """One-sided trees: the stack beyond each ring size, of the wide nodes, of the records (a
+    tree that does not nest) and of the reference's own steps (odd rays)."""
+    v, i = scenes.soup(n, seed=n, sigma=0.4)
+    nodes, ids = _one_sided(oracle, v, i, deep_left)
+    rays = scenes.random_rays(1500, 5, (-1.3, -1.3, -1.3), (1.3, 1.3, 1.3))
+    odd = _odd_rays()
+    rays = {k: np.concatenate([rays[k], odd[k]]) for k in api.RAY_FIELDS}
+    bad = nodes.copy()
+    bad["hi"][1:2 * n - 1:5, 0] -= np.float32(0.05)
+    with api.Scene(v, i) as s:
+        for tree in (nodes, bad):
+            s.load_dynbvh(ids, tree)
+            dr, dh = api.DeviceRays.upload(rays), api.DeviceHits.alloc(len(rays["ox"]))
+            o = oracle.trace(v, i, tree, ids, rays, packet_size=1)
+            for ring in (8, 16, 32):
+                dh.arrays["prim"].upload(np.full(dh.n, 777, np.int32))
+                s.trace(dr, dh, False, api.trace_opts(stack_lds=ring))
+                api.sync()
+                g = dh.download()
+                assert np.array_equal(g["prim"], o["prim"]), ring
+                assert np.array_equal(_bits(g["t"]), _bits(o["t"])), ring
+            _check_frames(oracle, s, v, i, tree, ids, rays, n)
+
+
+@pytest.mark.parametrize("ring", [0, 8, 16])
+def test_noalloc_on_deep_trees(oracle, ring):
+    """Depths where the fixed area holds the records' stack but not the wide nodes'."""
+    v, i = scenes.soup(72, seed=3, sigma=0.4)
+    nodes, ids = _one_sided(oracle, v, i)
+    n = 70_001
+    rays = scenes.random_rays(n, 6, (-1.3, -1.3, -1.3), (1.3, 1.3, 1.3))
+    with api.Scene(v, i) as s:
+        s.load_dynbvh(ids, nodes)
+        dr, dh = api.DeviceRays.upload(rays), api.DeviceHits.alloc(n)
+        opts = api.trace_opts(stack_lds=ring)
+        L.check(L.load().mh_trace_noalloc(s.h, dr.struct(), dh.struct(), n, 0, opts, None))
+        api.sync()
+        o = oracle.trace(v, i, nodes, ids, rays, packet_size=1)
+        g = dh.download()
+        assert np.array_equal(g["prim"], o["prim"])
+        assert np.array_equal(_bits(g["t"]), _bits(o["t"]))

@@ -290,3 +290,22 @@ def test_refill_is_the_callers(scene_host, oracle, tmp_path):
     ops = [(1, 64), (16, 256), (32, 128), (63, 1024), (64, 64), (64, 0), (64, 256)]
     got = _launches(scene_host, oracle, tmp_path, 2, *[f"refill:{r},{c}" for r, c in ops])
     assert [g["refill"] for g in got] == [1, 16, 32, 63, 64, 64, 40]
+
+
+@pytest.mark.parametrize("ring", [0, 8, 16, 32])
+@pytest.mark.parametrize("rays", [1, 64, 4097, 4000000])
+def test_fixed_spill_area_of_deep_trees(scene_host, oracle, tmp_path, ring, rays):
+    """Every launch fits the area (scene_host.cpp checks it), with the wide nodes while four
+    waves per compute unit do, then on the records, up to the depth that is refused."""
+    for n in (20, 50, 60, 73):
+        d = tmp_path / str(n)
+        d.mkdir()
+        got, = _launches(scene_host, oracle, d, n, f"fixed:{32 << 20}", f"trace:{rays},0,{ring},0")
+        assert got["layout"] == 0
+        if n in (20, 73) and rays > 4097:
+            assert got["pairs"] == (n == 73)
+    d = tmp_path / "refused"
+    d.mkdir()
+    if ring in (0, 8) and rays > 4097:
+        with pytest.raises(AssertionError, match="of stack spill for 256 workgroups"):
+            _launches(scene_host, oracle, d, 75, f"fixed:{32 << 20}", f"trace:{rays},0,{ring},0")
