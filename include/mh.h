@@ -98,9 +98,10 @@ typedef struct mh_trace_opts {
    * 2..64 = consecutive groups of packet_size rays traverse as one RayPacket on
    * one 64-lane wave (DynBVH::intersectNode packet semantics). */
   int packet_size;
-  /* [0] per-lane traversal stack entries held in LDS (8,16,32; 0 = autotuned). */
+  /* [0] per-lane traversal stack entries held in LDS (8, 16, 32; 0 = by the ray count). */
   int stack_lds;
-  /* [0] persistent blocks per CU (0 = autotuned). */
+  /* [0] at most this many times four waves per CU, which stride over the rays (0 = 32; 16
+   * with counters). */
   int blocks_per_cu;
   /* [NULL] optional device int64[2]: box tests, triangle tests (accumulated). */
   int64_t* counters;

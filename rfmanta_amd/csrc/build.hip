@@ -1100,8 +1100,8 @@ __global__ __launch_bounds__(kBlock) void k_ic_rank_top(DevFinish f, TopLevels t
   }
 }
 // Records in use move to their reference numbers; records from the node count on are
-// left as DynBVH::allocate leaves them after a reset. Holes (records the one-lane
-// subtrees reserved but did not use) have no number and vanish.
+// left as DynBVH::allocate leaves them after a reset. Holes (records that the
+// small nodes' subtrees reserved but did not use) have no number and vanish.
 __global__ __launch_bounds__(kBlock) void k_emit(DevFinish f) {
   const int64_t x = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (x >= f.n_records) return;
@@ -1202,7 +1202,7 @@ unsigned grid(int64_t n, int block = kBlock) { return (unsigned)((n + block - 1)
 }  // namespace
 
 // ---------------------------------------------------------------------------------------
-// Launchers (the host drives the level loop; see mh_scene_build_device)
+// Launchers (the host drives the level loop; see build_device in mh_api.cpp)
 
 int build_launch_setup(const DevBuild& d, int serial, void* stream) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);

@@ -108,8 +108,8 @@ struct mh_scene {
   uint32_t large_limit() const { return (uint32_t)(n_records / (20 * (uint32_t)workers)); }
 
   DevBuf refs, wide, tris, ids, big, d_verts, d_base, d_idx, leaves, levels;
-  // rotating update (mh_scene_update): costs, subtree sizes, parents, object boxes and
-  // centroids, depth work arrays, the depth histogram and counters
+  // rotating update (mh_scene_update): costs, subtree sizes, parents; device build: depth
+  // work arrays and the depth histogram (the level counters otherwise); counters
   DevBuf costs, ssize, parent, anc0, dep0, anc1, dep1, hist, counters;
   DevBuf split_list;  // rotating update: leaves whose parent's rotation may split them
   DevBuf levels_aux;  // rotating update: first child and word beside each level entry

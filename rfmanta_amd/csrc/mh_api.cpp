@@ -645,7 +645,8 @@ int mh_scene_destroy(mh_scene* scene) {
 }
 
 // DynBVH::rebuild with USE_APPROXIMATE_BUILD, on the device (build.hip): object boxes,
-// the level loop over nodes of many objects, one wave per small node, then the reference numbering and the bottom-up passes.
+// the level loop over nodes of many objects, one wave per small node, then the reference
+// numbering and the bottom-up passes.
 int build_device(mh_scene* s, int rtsah) {
   using mh_internal::DevBuf;
   const uint32_t T = s->nt;
@@ -754,7 +755,7 @@ int build_device(mh_scene* s, int rtsah) {
   HIP_OK(hipMemsetAsync(s->hist.p, 0, mh::kDepthHist * 4, st));
   HIP_OK((hipError_t)mh::launch_depths(d.u, s->anc0.as<int32_t>(), s->dep0.as<int32_t>(),
                                        s->anc1.as<int32_t>(), s->dep1.as<int32_t>(),
-                                       s->hist.as<unsigned>(), 8, st));
+                                       s->hist.as<unsigned>(), st));
   std::vector<unsigned> hist(mh::kDepthHist);
   unsigned used[2];
   HIP_OK(hipMemcpyAsync(hist.data(), s->hist.p, hist.size() * 4, hipMemcpyDeviceToHost, st));

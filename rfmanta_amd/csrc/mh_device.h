@@ -19,8 +19,8 @@
 //   leaves int32[L], levels int32[I]   leaf records; inner records grouped by depth, the
 //                              even depths in one list and the odd depths in another
 //   leaf_at int32[T]           per object slot, the leaf record that starts there, else -1
-//   costs float[2T], ssize uint32[2T], parent int32[2T], obj boxes/centroids   rotating
-//                              update state (allocated at the first mh_scene_update)
+//   costs float[2T], ssize uint32[2T], parent int32[2T]   rotating update state (parent:
+//                              allocated at the first mh_scene_update)
 #pragma once
 
 #include <cstdint>
@@ -81,7 +81,7 @@ struct DevScene {
   const float* tris;  // 12 floats per slot
   const int32_t* obj_ids;
   const int32_t* big_count;
-  int32_t root_ref;   // pair-encoded reference of record 0
+  int32_t root_ref;   // record 0: its wide node (0), or its leaf code
   int32_t prim_kind;  // 0 KS, 1 Wald
   uint32_t n_pairs;   // PairNodes of the SOA copy
   const void* pairs_soa;  // kLayoutSoa: 16-byte field k of pair p at [k * n_pairs + p], or null
@@ -244,22 +244,18 @@ struct DevUpdate {
   int32_t n_objects;     // T
   uint32_t large;        // largeSubtreeSize
 };
-// u.leaf_at from a leaf list (the caller sets every entry to -1 first).
-int launch_leaf_starts(const DevUpdate& u, const int32_t* leaves, int64_t n_leaves,
-                       void* stream);
 // Leaf pass over the object slots (u.leaf_at), leaf splits, then one launch per two depths
 // (deepest first).
 int launch_update_tree(const DevUpdate& u, int64_t n_leaves, const int32_t* levels,
                        const LevelList* lev, int n_levels, void* stream);
 // The PairNodes of the n inner records of a level list.
 int launch_list_pairs(const DevUpdate& u, const int32_t* levels, int64_t n, void* stream);
-// Depth of every record in use by `steps` pointer-jumping steps (even, at most 8; 8 covers
-// any depth below kMaxDepth); hist[d] inner records at depth d, hist[kMaxDepth] leaves,
-// hist[kMaxDepth + 1] the deepest depth, hist[kMaxDepth + 2] nonzero when the steps did
-// not reach the root (hist, kDepthHist entries, cleared by the caller). Depths in dep0.
-constexpr int kDepthHist = kMaxDepth + 3;
+// Depth of every record in use by pointer jumping; hist[d] inner records at depth d,
+// hist[kMaxDepth] leaves, hist[kMaxDepth + 1] the deepest depth (hist, kDepthHist entries,
+// cleared by the caller). Depths in dep0.
+constexpr int kDepthHist = kMaxDepth + 2;
 int launch_depths(const DevUpdate& u, int32_t* anc0, int32_t* dep0, int32_t* anc1, int32_t* dep1,
-                  unsigned* hist, int steps, void* stream);
+                  unsigned* hist, void* stream);
 int launch_depth_scatter(const DevUpdate& u, const int32_t* dep, unsigned* cursor,
                          int32_t* levels, int32_t* leaves, void* stream);
 // wide.hip: level lists, leaf list, leaf starts and wide nodes of a tree, top down from an

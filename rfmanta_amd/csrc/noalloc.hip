@@ -17,9 +17,9 @@
 
 namespace {
 
-// 32 MiB: the spill of a tree 64 levels deeper than the LDS ring at one 256-lane
-// workgroup per compute unit of a 256-CU device, or of the 1M-triangle heightfield's
-// tree (depth 22, ring 8) at more than four workgroups per compute unit.
+// 32 MiB: the spill of a tree 64 levels deeper than the LDS ring at four waves per compute
+// unit of a 256-CU device (one stack entry a level, the tree traversed on its records), or of
+// the 1M-triangle heightfield's tree (depth 22: 33 entries of the wide nodes, ring 16) at 15.
 constexpr size_t kScratchBytes = size_t(32) << 20;
 static_assert(kScratchBytes == MH_NOALLOC_SCRATCH_BYTES, "header and source disagree");
 

@@ -266,15 +266,6 @@ __device__ void upd_node(const DevUpdate& u, int node, const float4& tail) {
   }
 }
 
-// The leaf that starts at each object slot, from a leaf list.
-__global__ __launch_bounds__(kBlock) void k_leaf_starts(DevUpdate u, const int32_t* leaves,
-                                                        int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  const int rec = leaves[i];
-  u.leaf_at[u.refs[rec].child] = rec;
-}
-
 // One lane per object slot; the lane at a leaf's first slot does the leaf, so neighbouring
 // lanes take neighbouring leaves and gather neighbouring vertices. Object boxes come from
 // the vertices (Mesh::getBBox).
@@ -340,9 +331,6 @@ __global__ __launch_bounds__(kBlock) void k_split_leaves(DevUpdate u) {
 
 __device__ __forceinline__ float4 rec_tail(const DevUpdate& u, int rec) {
   return reinterpret_cast<const float4*>(u.refs + rec)[1];
-}
-__device__ __forceinline__ void upd_node(const DevUpdate& u, int node) {
-  upd_node(u, node, rec_tail(u, node));
 }
 
 // Entry i of an even level list and its children, by a pair of lanes: each lane does the
@@ -502,9 +490,8 @@ __device__ __forceinline__ void depth_range(const DevUpdate& u, int64_t chunk, i
 // Inner records per depth. Each workgroup counts a range of records in LDS and adds its
 // counts to the global histogram once per depth, so the few shared counters see one
 // atomic per workgroup and depth.
-__global__ __launch_bounds__(kBlock) void k_depth_hist(DevUpdate u, const int32_t* anc,
-                                                       const int32_t* dep, unsigned* hist,
-                                                       int64_t chunk) {
+__global__ __launch_bounds__(kBlock) void k_depth_hist(DevUpdate u, const int32_t* dep,
+                                                       unsigned* hist, int64_t chunk) {
   __shared__ unsigned lh[kMaxDepth];
   for (int i = threadIdx.x; i < kMaxDepth; i += kBlock) lh[i] = 0;
   __syncthreads();
@@ -513,7 +500,6 @@ __global__ __launch_bounds__(kBlock) void k_depth_hist(DevUpdate u, const int32_
   for (int64_t r0 = lo; r0 < hi; r0 += kBlock) {
     const int64_t r = r0 + threadIdx.x;
     int b = -1;
-    if (r < hi && anc[r] != -1) hist[kMaxDepth + 2] = 1u;  // the jumps did not reach the root
     if (r < hi && u.refs[r].children == 0) {
       const int d = dep[r];
       if (d < kMaxDepth)
@@ -607,14 +593,6 @@ int64_t depth_chunk(int64_t n, unsigned& blocks) {
 
 }  // namespace
 
-int launch_leaf_starts(const DevUpdate& u, const int32_t* leaves, int64_t n_leaves,
-                       void* stream) {
-  if (n_leaves > 0)
-    hipLaunchKernelGGL(k_leaf_starts, dim3(grid(n_leaves)), dim3(kBlock), 0,
-                       reinterpret_cast<hipStream_t>(stream), u, leaves, n_leaves);
-  return (int)hipGetLastError();
-}
-
 int launch_update_tree(const DevUpdate& u, int64_t n_leaves, const int32_t* levels,
                        const LevelList* lev, int n_levels, void* stream) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
@@ -642,15 +620,13 @@ int launch_list_pairs(const DevUpdate& u, const int32_t* levels, int64_t n, void
 }
 
 int launch_depths(const DevUpdate& u, int32_t* anc0, int32_t* dep0, int32_t* anc1, int32_t* dep1,
-                  unsigned* hist, int steps, void* stream) {
+                  unsigned* hist, void* stream) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const unsigned g = grid(u.n_records);
   hipLaunchKernelGGL(k_parents, dim3(g), dim3(kBlock), 0, s, u, anc0, dep0);
-  // 2^8 > kMaxDepth: eight doublings reach the root from any record; fewer (an even count,
-  // so that the results end in anc0/dep0) do for shallower trees, and the histogram pass
-  // flags a record they left short of the root.
-  if (steps < 2 || steps > 8 || (steps & 1)) steps = 8;
-  for (int it = 0; it < steps; ++it) {
+  // 2^8 = kMaxDepth: eight doublings reach the root from any record above that depth, and
+  // leave a deeper one at kMaxDepth. An even count, so that the results end in anc0/dep0.
+  for (int it = 0; it < 8; ++it) {
     const bool even = (it & 1) == 0;
     hipLaunchKernelGGL(k_jump, dim3(g), dim3(kBlock), 0, s, u.next_free, u.n_records,
                        even ? anc0 : anc1,
@@ -658,7 +634,7 @@ int launch_depths(const DevUpdate& u, int32_t* anc0, int32_t* dep0, int32_t* anc
   }
   unsigned blocks;
   const int64_t chunk = depth_chunk(u.n_records, blocks);
-  hipLaunchKernelGGL(k_depth_hist, dim3(blocks), dim3(kBlock), 0, s, u, anc0, dep0, hist, chunk);
+  hipLaunchKernelGGL(k_depth_hist, dim3(blocks), dim3(kBlock), 0, s, u, dep0, hist, chunk);
   hipLaunchKernelGGL(k_depth_finish, dim3(1), dim3(kBlock), 0, s, hist);
   return (int)hipGetLastError();
 }

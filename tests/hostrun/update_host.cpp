@@ -101,7 +101,7 @@ int main(int argc, char** argv) {
   }
   if (ctr[1]) return 4;
   for (int dep = (int)levels.size() - 1; dep >= 0; --dep)  // k_upd_level / k_upd_top
-    for (int r : levels[dep]) upd_node(u, r);
+    for (int r : levels[dep]) upd_node(u, r, rec_tail(u, r));
   // the new tree: PairNodes and leaf starts, as the level pass stores them
   std::vector<std::pair<int, int>> q{{0, 0}};
   int depth = 0;
