@@ -100,8 +100,7 @@ typedef struct mh_trace_opts {
   int packet_size;
   /* [0] per-lane traversal stack entries held in LDS (8, 16, 32; 0 = by the ray count). */
   int stack_lds;
-  /* [0] at most this many times four waves per CU, which stride over the rays (0 = 32; 16
-   * with counters). */
+  /* [0] at most this many times four waves per CU, which stride over the rays (0 = 32). */
   int blocks_per_cu;
   /* [NULL] optional device int64[2]: box tests, triangle tests (accumulated). */
   int64_t* counters;

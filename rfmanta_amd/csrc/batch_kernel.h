@@ -71,12 +71,10 @@ __device__ __forceinline__ void trace_span(const DevScene& sc, const RefNode& ro
                                            const GRays& rays, const GHits& hits,
                                            int64_t bstart, int64_t pos, int64_t gend, int lane,
                                            LaneStack<S, BLOCK>& st) {
-  unsigned long long nbox = 0, ntri = 0;
   for (int64_t b = pos; b < gend; b += 64) {
     const int64_t g = b + lane;
     if (g < gend)
-      trace_store<ANY, PRIM, LAYOUT, S, BLOCK, false>(sc, root, rays, hits, g - bstart, st, nbox,
-                                                      ntri);
+      trace_store<ANY, PRIM, LAYOUT, S, BLOCK>(sc, root, rays, hits, g - bstart, st);
   }
 }
 
@@ -95,14 +93,13 @@ struct Lane {
 // a run-time closest/any-hit flag; returns false when the ray is finished.
 template <int PRIM, int S, int BLOCK>
 __device__ __forceinline__ bool step_ref(const DevScene& sc, Lane& L, LaneStack<S, BLOCK>& st) {
-  unsigned long long ntri = 0;
   const RefNode nd = sc.refs[L.cur];
   float tn;
   if (slab(nd.box.lo[0], nd.box.hi[0], nd.box.lo[1], nd.box.hi[1], nd.box.lo[2], nd.box.hi[2],
            L.r, L.h.minT, tn)) {
     if (nd.children != 0) {
-      const bool done = L.any ? leaf<true, PRIM, false>(sc, nd.child, nd.children, L.r, L.h, ntri)
-                              : leaf<false, PRIM, false>(sc, nd.child, nd.children, L.r, L.h, ntri);
+      const bool done = L.any ? leaf<true, PRIM>(sc, nd.child, nd.children, L.r, L.h)
+                              : leaf<false, PRIM>(sc, nd.child, nd.children, L.r, L.h);
       if (done) return false;
     } else {
       const int front = L.any ? ((nd.bits & 1) ? 0 : 1)
@@ -125,7 +122,6 @@ __device__ __forceinline__ bool step_ref(const DevScene& sc, Lane& L, LaneStack<
 // finished lane is refilled between rounds. Returns false when the ray is finished.
 template <bool ANY, int PRIM, int S, int BLOCK, bool FAST, int LAYOUT>
 __device__ __forceinline__ bool round_pair(const DevScene& sc, Lane& L, LaneStack<S, BLOCK>& st) {
-  unsigned long long ntri = 0;
   bool missed = false;
   while (L.cur >= 0) {
     float4 A, B, C;
@@ -147,7 +143,7 @@ __device__ __forceinline__ bool round_pair(const DevScene& sc, Lane& L, LaneStac
     const int first = code >> kLeafCountBits;
     int cnt = code & kLeafCountInline;
     if (cnt == kLeafCountInline) cnt = sc.big_count[first];
-    if (leaf<ANY, PRIM, false>(sc, first, cnt, L.r, L.h, ntri)) return false;
+    if (leaf<ANY, PRIM>(sc, first, cnt, L.r, L.h)) return false;
   }
   while (!st.empty()) {
     int ref;

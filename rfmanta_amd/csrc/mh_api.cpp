@@ -423,12 +423,6 @@ constexpr int64_t kFewWaves = 8;  // per compute unit
 // 2.8 times the resident ones, and no tree more than 965 MB.
 constexpr int64_t kSpillBytes = int64_t(512) << 20;
 
-// The caller's ring, or the one the reference records' kernel takes.
-int choose_stack(const mh_trace_opts* o) {
-  const int v = o ? o->stack_lds : 0;
-  return (v == 8 || v == 16 || v == 32) ? v : 8;
-}
-
 // fixed_spill / fixed_bytes: a stack spill area the caller provides (mh_trace_noalloc);
 // null = the scene's per-stream spill buffer, grown here as needed.
 int trace_impl(const mh_scene* cs, const mh_rays* rays, const mh_hits* hits, int64_t n,
@@ -458,64 +452,47 @@ int trace_impl(const mh_scene* cs, const mh_rays* rays, const mh_hits* hits, int
     if (s->depth + 2 > 128)
       return fail(MH_E_UNSUPPORTED, "tree depth %u exceeds the packet stack (126)", s->depth);
   } else {
-    const int S = choose_stack(opts);
     const int bpc = (opts && opts->blocks_per_cu > 0) ? opts->blocks_per_cu : kTraceBlocksPerCu;
     const int64_t cus = g_lib.cu_count;
-    // The reference records' kernel, which keeps the counters.
-    const int64_t ref_need = std::max<int64_t>(0, (int64_t)s->stack_bound(MH_LAYOUT_REF) - S);
-    const int64_t ref_want = (n + 255) / 256;
-    int64_t ref_blocks =
-        std::min(ref_want, cus * (opts && opts->blocks_per_cu > 0 ? opts->blocks_per_cu : 16));
-    if (ref_need > 0 && fixed_spill) {
-      // Fewer workgroups (the kernel strides over the rays, results are unchanged) until
-      // every lane's spill column fits the area; at least one workgroup per compute unit.
-      const int64_t per_block = ref_need * 256 * 8;
-      const int64_t fit = (int64_t)(fixed_bytes / (size_t)per_block);
-      const int64_t floor_blocks = std::min<int64_t>(ref_want, cus);
-      if (fit < floor_blocks)
-        return fail(MH_E_UNSUPPORTED,
-                    "tree depth %u needs %lld bytes of stack spill for %lld workgroups; the "
-                    "fixed area holds %zu (use mh_trace, or a larger stack_lds)",
-                    s->depth, (long long)(per_block * floor_blocks), (long long)floor_blocks,
-                    fixed_bytes);
-      ref_blocks = std::min(ref_blocks, fit);
-    }
     const int64_t chunk =
         std::min<int64_t>(64, std::max<int64_t>(kMinWaveRays, (n + 4 * cus - 1) / (4 * cus)));
     const int64_t waves = (n + chunk - 1) / chunk;
-    const int wide_S = opts && opts->stack_lds == S ? S
-                       : waves <= kFewWaves * cus   ? kFewWavesRing
-                                                    : kWideRing;
+    const int own = opts ? opts->stack_lds : 0;  // the caller's ring
+    const int S = own == 8 || own == 16 || own == 32 ? own
+                  : waves <= kFewWaves * cus         ? kFewWavesRing
+                                                     : kWideRing;
+    // Entries of a spill column: the wide nodes' stack, or the records' one entry a level (and
+    // the ring, which makes room for three at a time, spills two early).
+    const int64_t wide_need = std::max<int64_t>(0, (int64_t)s->stack_bound(MH_LAYOUT_PAIR) - S);
+    const int64_t pairs_need = std::max<int64_t>(0, (int64_t)s->depth + 2 - S);
+    cfg.pairs = cfg.counters != nullptr;  // (the tests counted are those of the records' boxes)
+    int64_t need = cfg.pairs ? pairs_need : wide_need;
     int64_t blocks = std::min(waves, 4 * cus * bpc);
-    int64_t need = std::max<int64_t>(0, (int64_t)s->stack_bound(MH_LAYOUT_PAIR) - wide_S);
-    const bool wide = !cfg.counters;
     auto fit = [&] { return (int64_t)(fixed_bytes / (size_t)(need * 64 * 8)); };
-    if (fixed_spill && need > 0 && fit() < std::min(waves, 4 * cus)) {
-      // Four waves per compute unit do not fit: on the records a ray's stack takes one entry
-      // a level (and the ring, which makes room for three at a time, spills two early), which
-      // the check above leaves room for.
-      cfg.pairs = 1;
-      need = std::max<int64_t>(0, (int64_t)s->depth + 2 - wide_S);
-    }
-    if (fixed_spill && need > 0) {
-      blocks = std::min(blocks, fit());
+    if (fixed_spill) {
+      // Refused where columns of an entry a level beyond the ring (8 entries unless the caller
+      // says) do not fit for every 256 rays, up to 256 lanes per compute unit.
+      const int64_t deep = std::max<int64_t>(0, (int64_t)s->depth - (own == S ? S : 8));
+      const int64_t per_block = deep * 256 * 8, least = std::min<int64_t>((n + 255) / 256, cus);
+      if (per_block * least > (int64_t)fixed_bytes)
+        return fail(MH_E_UNSUPPORTED,
+                    "tree depth %u needs %lld bytes of stack spill for %lld workgroups; the "
+                    "fixed area holds %zu (use mh_trace, or a larger stack_lds)",
+                    s->depth, (long long)(per_block * least), (long long)least, fixed_bytes);
+      // Where four waves per compute unit do not fit with the wide nodes, the records do.
+      if (need > 0 && fit() < std::min(waves, 4 * cus)) {
+        cfg.pairs = 1;
+        need = pairs_need;
+      }
+      if (need > 0) blocks = std::min(blocks, fit());
     } else if (need > 0) {
       blocks = std::min(blocks, std::max<int64_t>(mh_internal::resident_waves(),
                                                   kSpillBytes / (need * 64 * 8)));
     }
-    if (wide) {
-      cfg.layout = MH_LAYOUT_PAIR;
-      cfg.stack_lds = wide_S;
-      cfg.chunk = (int)chunk;
-      cfg.blocks = (int)blocks;
-      cfg.spill_stride = blocks * 64;
-    } else {
-      need = ref_need;
-      cfg.layout = MH_LAYOUT_REF;
-      cfg.stack_lds = S;
-      cfg.blocks = (int)ref_blocks;
-      cfg.spill_stride = ref_blocks * 256;
-    }
+    cfg.stack_lds = S;
+    cfg.chunk = (int)chunk;
+    cfg.blocks = (int)blocks;
+    cfg.spill_stride = blocks * 64;
     if (need > 0 && fixed_spill) {
       cfg.spill = reinterpret_cast<int32_t*>(fixed_spill);
     } else if (need > 0) {
@@ -524,7 +501,7 @@ int trace_impl(const mh_scene* cs, const mh_rays* rays, const mh_hits* hits, int
       if (!b) b = new (std::nothrow) DevBuf();
       if (!b) return fail(MH_E_NOMEM, "spill descriptor");
       rc = b->reserve((size_t)need * cfg.spill_stride * 8);
-      if (rc == MH_E_NOMEM && wide && cfg.blocks > mh_internal::resident_waves()) {
+      if (rc == MH_E_NOMEM && cfg.blocks > mh_internal::resident_waves()) {
         cfg.blocks = mh_internal::resident_waves();
         cfg.spill_stride = (int64_t)cfg.blocks * 64;
         rc = b->reserve((size_t)need * cfg.spill_stride * 8);

@@ -103,13 +103,12 @@ struct LaunchCfg {
   int any_hit;
   int packet_size;    // 1 = single-ray kernels
   int stack_lds;      // 8/16/32 (single-ray)
-  int layout;         // kLayoutPair or kLayoutRef (single-ray)
-  int blocks;         // grid size: blocks of 64 lanes (kLayoutPair) or 256 (kLayoutRef)
-  int64_t* counters;  // device int64[2] or null: box and triangle tests (kLayoutRef)
+  int blocks;         // grid size in blocks of 64 lanes (single-ray)
+  int64_t* counters;  // device int64[2] or null: box and triangle tests
   int32_t* spill;     // per-thread stack spill (single-ray)
   int64_t spill_stride;
-  int chunk;          // kLayoutPair: rays a wave takes at a time, 1..64
-  int pairs;          // kLayoutPair: traverse the records, on a stack of one entry a level
+  int chunk;          // rays a wave takes at a time, 1..64 (single-ray)
+  int pairs;          // traverse the records, on a stack of one entry a level (single-ray)
 };
 
 // Node layouts of the single-ray traversal (MH_LAYOUT_*). A non-root record r's box is

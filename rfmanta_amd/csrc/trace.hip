@@ -1,9 +1,5 @@
-// Traversal kernels for gfx950 (wave64).
-//
-// Single rays take k_wide_whole (wide_trace.h). k_trace_ray: one ray per lane,
-//   DynBVH::intersect on a one-ray packet (Model/Groups/DynBVH.cc:101-404) over the
-//   reference's 32-byte records, for callers that count box and triangle tests; the
-//   traversal is traverse.h's.
+// Packet traversal for gfx950 (wave64), and the entry of plain traces: single rays take
+// k_wide_whole (wide_trace.h).
 //
 // k_trace_packet: one RayPacket of up to 64 consecutive rays per wave, the reference's
 //   packet recursion (intersectNode/firstIntersects/lastIntersects, DynBVH.cc:274-905,
@@ -41,29 +37,6 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr int kWaves = kBlock / 64;
-
-// ---------------------------------------------------------------------------
-// Single-ray traversal of the reference's records (traverse.h), grid-stride over the rays.
-// ---------------------------------------------------------------------------
-template <bool ANY, int PRIM, int S>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_trace_ray(
-    DevScene sc, DevRays rays, DevHits hits, int64_t n, int2* spill, int64_t spill_stride,
-    unsigned long long* counters) {
-  __shared__ unsigned long long s_ring[S * kBlock];
-  const int tid = threadIdx.x;
-  const int64_t gtid = (int64_t)blockIdx.x * kBlock + tid;
-  const int64_t stride = (int64_t)gridDim.x * kBlock;
-  unsigned long long nbox = 0, ntri = 0;
-  const RefNode root = sc.refs[0];
-  LaneStack<S, kBlock> st(s_ring, reinterpret_cast<unsigned long long*>(spill), spill_stride,
-                          gtid, tid);
-  const GRays gr = global_view(rays);
-  const GHits gh = global_view(hits);
-  for (int64_t ri = gtid; ri < n; ri += stride)
-    trace_store<ANY, PRIM, kLayoutRef, S, kBlock, true>(sc, root, gr, gh, ri, st, nbox, ntri);
-  atomicAdd(counters + 0, nbox);
-  atomicAdd(counters + 1, ntri);
-}
 
 // ---------------------------------------------------------------------------
 // Packet traversal (one RayPacket per wave)
@@ -327,45 +300,18 @@ __global__ __launch_bounds__(kBlock) void k_trace_packet(DevScene sc, DevRays ra
 }
 
 template <bool ANY, int PRIM>
-int launch_ray_s(const DevScene& sc, const DevRays& rays, const DevHits& hits, int64_t n,
-                 const LaunchCfg& cfg, hipStream_t s) {
+int launch_packets(const DevScene& sc, const DevRays& rays, const DevHits& hits, int64_t n,
+                   const LaunchCfg& cfg, hipStream_t s) {
+  const int64_t packets = (n + cfg.packet_size - 1) / cfg.packet_size;
+  const int64_t blocks = (packets + kWaves - 1) / kWaves;
   unsigned long long* c = reinterpret_cast<unsigned long long*>(cfg.counters);
-  int2* sp = reinterpret_cast<int2*>(cfg.spill);
-  dim3 g(cfg.blocks), b(kBlock);
-  switch (cfg.stack_lds) {
-    case 8:
-      hipLaunchKernelGGL((k_trace_ray<ANY, PRIM, 8>), g, b, 0, s, sc, rays, hits, n, sp,
-                         cfg.spill_stride, c);
-      break;
-    case 32:
-      hipLaunchKernelGGL((k_trace_ray<ANY, PRIM, 32>), g, b, 0, s, sc, rays, hits, n, sp,
-                         cfg.spill_stride, c);
-      break;
-    default:
-      hipLaunchKernelGGL((k_trace_ray<ANY, PRIM, 16>), g, b, 0, s, sc, rays, hits, n, sp,
-                         cfg.spill_stride, c);
-      break;
-  }
+  if (c)
+    hipLaunchKernelGGL((k_trace_packet<ANY, PRIM, true>), dim3((unsigned)blocks), dim3(kBlock), 0,
+                       s, sc, rays, hits, n, cfg.packet_size, c);
+  else
+    hipLaunchKernelGGL((k_trace_packet<ANY, PRIM, false>), dim3((unsigned)blocks), dim3(kBlock), 0,
+                       s, sc, rays, hits, n, cfg.packet_size, c);
   return (int)hipGetLastError();
-}
-
-template <bool ANY, int PRIM>
-int launch_any_prim(const DevScene& sc, const DevRays& rays, const DevHits& hits, int64_t n,
-                    const LaunchCfg& cfg, hipStream_t s) {
-  const bool stats = cfg.counters != nullptr;
-  if (cfg.packet_size > 1) {
-    const int64_t packets = (n + cfg.packet_size - 1) / cfg.packet_size;
-    const int64_t blocks = (packets + kWaves - 1) / kWaves;
-    unsigned long long* c = reinterpret_cast<unsigned long long*>(cfg.counters);
-    if (stats)
-      hipLaunchKernelGGL((k_trace_packet<ANY, PRIM, true>), dim3((unsigned)blocks), dim3(kBlock),
-                         0, s, sc, rays, hits, n, cfg.packet_size, c);
-    else
-      hipLaunchKernelGGL((k_trace_packet<ANY, PRIM, false>), dim3((unsigned)blocks),
-                         dim3(kBlock), 0, s, sc, rays, hits, n, cfg.packet_size, c);
-    return (int)hipGetLastError();
-  }
-  return stats ? launch_ray_s<ANY, PRIM>(sc, rays, hits, n, cfg, s) : (int)hipErrorInvalidValue;
 }
 
 }  // namespace
@@ -373,17 +319,16 @@ int launch_any_prim(const DevScene& sc, const DevRays& rays, const DevHits& hits
 int launch_trace(const DevScene& sc, const DevRays& rays, const DevHits& hits, int64_t n,
                  const LaunchCfg& cfg, void* stream) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (cfg.packet_size <= 1 && cfg.layout == kLayoutPair) {
-    if (cfg.counters) return (int)hipErrorInvalidValue;
+  if (cfg.packet_size <= 1) {
     const BatchDev b{rays, hits, n, 0, cfg.any_hit ? 1u : 0u, 0};
     return sc.prim_kind == 1 ? launch_wide_one_wald(sc, b, cfg, s) : launch_wide_one_ks(sc, b, cfg, s);
   }
   if (cfg.any_hit) {
-    return sc.prim_kind == 1 ? launch_any_prim<true, 1>(sc, rays, hits, n, cfg, s)
-                             : launch_any_prim<true, 0>(sc, rays, hits, n, cfg, s);
+    return sc.prim_kind == 1 ? launch_packets<true, 1>(sc, rays, hits, n, cfg, s)
+                             : launch_packets<true, 0>(sc, rays, hits, n, cfg, s);
   }
-  return sc.prim_kind == 1 ? launch_any_prim<false, 1>(sc, rays, hits, n, cfg, s)
-                           : launch_any_prim<false, 0>(sc, rays, hits, n, cfg, s);
+  return sc.prim_kind == 1 ? launch_packets<false, 1>(sc, rays, hits, n, cfg, s)
+                           : launch_packets<false, 0>(sc, rays, hits, n, cfg, s);
 }
 
 }  // namespace mh

@@ -1,6 +1,5 @@
-// Single-ray traversal of the REF and SOA node layouts (the plain kernel's statistics
-// variant, trace.hip, and the batch kernel, batch_kernel.h): DynBVH::intersect on a one-ray
-// packet (Model/Groups/DynBVH.cc:101-404). The default layout's is wide_trace.h's.
+// Single-ray traversal of the REF and SOA node layouts (batch_kernel.h): DynBVH::intersect
+// on a one-ray packet (Model/Groups/DynBVH.cc:101-404). The default layout's is wide_trace.h's.
 //
 // SOA layout: inner nodes are 64-byte PairNodes holding both child boxes, kept as four
 //   arrays of their 16-byte fields, so one fetch tests both children. The child the
@@ -71,11 +70,10 @@ struct RayHit {
 
 // Leaf: the triangles of slots [first, first+cnt) in order; returns true when an any-hit
 // ray is done.
-template <bool ANY, int PRIM, bool STATS>
+template <bool ANY, int PRIM>
 __device__ __forceinline__ bool leaf(const DevScene& sc, int first, int cnt, const Ray& r,
-                                     RayHit& h, unsigned long long& ntri) {
+                                     RayHit& h) {
   for (int k = 0; k < cnt; ++k) {
-    if (STATS) ++ntri;
     float t, u, v;
     if (prim_test<PRIM>(sc, first + k, r, h.minT, t, u, v)) {
       h.minT = t;
@@ -109,7 +107,6 @@ __device__ __forceinline__ int pair_root(const DevScene& sc) {
 template <bool ANY, int PRIM, int S, int BLOCK, bool FAST>
 __device__ __forceinline__ void trace_pair(const DevScene& sc, const RefNode& root, const Ray& r,
                                            RayHit& h, LaneStack<S, BLOCK>& st) {
-  unsigned long long ntri = 0;
   float tn;
   bool go = slab_v<FAST>(root.box.lo[0], root.box.hi[0], root.box.lo[1], root.box.hi[1],
                          root.box.lo[2], root.box.hi[2], r, h.minT, tn);
@@ -137,7 +134,7 @@ __device__ __forceinline__ void trace_pair(const DevScene& sc, const RefNode& ro
       const int first = code >> kLeafCountBits;
       int cnt = code & kLeafCountInline;
       if (cnt == kLeafCountInline) cnt = sc.big_count[first];
-      if (leaf<ANY, PRIM, false>(sc, first, cnt, r, h, ntri)) return;
+      if (leaf<ANY, PRIM>(sc, first, cnt, r, h)) return;
     }
     go = false;
     while (!st.empty()) {
@@ -153,23 +150,19 @@ __device__ __forceinline__ void trace_pair(const DevScene& sc, const RefNode& ro
   }
 }
 
-// The box tests are counted as the two of an inner record's children when it is entered.
-template <bool ANY, int PRIM, int S, int BLOCK, bool STATS, bool FAST>
+template <bool ANY, int PRIM, int S, int BLOCK, bool FAST>
 __device__ __forceinline__ void trace_ref(const DevScene& sc, const Ray& r, RayHit& h,
-                                          LaneStack<S, BLOCK>& st, unsigned long long& nbox,
-                                          unsigned long long& ntri) {
+                                          LaneStack<S, BLOCK>& st) {
   int cur = 0;
   st.reset();
-  if (STATS) ++nbox;
   for (;;) {
     const RefNode nd = sc.refs[cur];
     float tn;
     if (slab_v<FAST>(nd.box.lo[0], nd.box.hi[0], nd.box.lo[1], nd.box.hi[1], nd.box.lo[2],
                      nd.box.hi[2], r, h.minT, tn)) {
       if (nd.children != 0) {
-        if (leaf<ANY, PRIM, STATS>(sc, nd.child, nd.children, r, h, ntri)) return;
+        if (leaf<ANY, PRIM>(sc, nd.child, nd.children, r, h)) return;
       } else {
-        if (STATS) nbox += 2;
         const int front = ANY ? ((nd.bits & 1) ? 0 : 1) : (((r.dpos >> (nd.axis & 3)) & 1) ? 0 : 1);
         st.push(nd.child + 1 - front, 0.f);
         cur = nd.child + front;
@@ -184,11 +177,10 @@ __device__ __forceinline__ void trace_ref(const DevScene& sc, const Ray& r, RayH
 
 // One ray of `rays`/`hits` at index i, traced and stored (masked rays are stored as the
 // reference leaves them: prim MH_MASKED, t = -MAXT, occluded).
-template <bool ANY, int PRIM, int LAYOUT, int S, int BLOCK, bool STATS>
+template <bool ANY, int PRIM, int LAYOUT, int S, int BLOCK>
 __device__ __forceinline__ void trace_store(const DevScene& sc, const RefNode& root,
                                             const GRays& rays, const GHits& hits, int64_t i,
-                                            LaneStack<S, BLOCK>& st, unsigned long long& nbox,
-                                            unsigned long long& ntri) {
+                                            LaneStack<S, BLOCK>& st) {
   if (rays.masked && rays.masked[i]) {
     store_hit(hits, i, -2, -kMaxT, 0.f, 0.f, true);
     return;
@@ -199,12 +191,12 @@ __device__ __forceinline__ void trace_store(const DevScene& sc, const RefNode& r
   // The min/max slab test when every ray of the wave allows it (wave-uniform choice).
   if (__ballot(!regular_ray(r, h.minT)) == 0ull) {
     if (LAYOUT == kLayoutRef)
-      trace_ref<ANY, PRIM, S, BLOCK, STATS, true>(sc, r, h, st, nbox, ntri);
+      trace_ref<ANY, PRIM, S, BLOCK, true>(sc, r, h, st);
     else
       trace_pair<ANY, PRIM, S, BLOCK, true>(sc, root, r, h, st);
   } else {
     if (LAYOUT == kLayoutRef)
-      trace_ref<ANY, PRIM, S, BLOCK, STATS, false>(sc, r, h, st, nbox, ntri);
+      trace_ref<ANY, PRIM, S, BLOCK, false>(sc, r, h, st);
     else
       trace_pair<ANY, PRIM, S, BLOCK, false>(sc, root, r, h, st);
   }

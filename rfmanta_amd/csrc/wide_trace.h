@@ -105,6 +105,7 @@ struct WideLane {
   unsigned ord;  // where the ray's visit order lies in WideNode::order (kAnyOrder: any hit)
   int cur;       // node (>= 0), leaf code, kPop or kIdle
   bool bad;      // the reference's own steps have to trace it
+  unsigned nbox, ntri;  // COUNT: box and triangle tests
 };
 constexpr unsigned kAnyOrder = 24;
 
@@ -263,8 +264,8 @@ __device__ __forceinline__ bool wide_tri(const DevScene& sc, WideLane& L, int sl
 // one would wait for its record again. (One a step: 1M incoherent rays over the 1M-triangle
 // heightfield 228 against 205 us, shadow rays 239 against 214. Past the last slot the
 // descriptor reads zeros.)
-// PAIRS: the leaf's own box has been tested.
-template <int PRIM, bool PAIRS>
+// PAIRS: the leaf's own box has been tested. COUNT: the tests are counted.
+template <int PRIM, bool PAIRS, bool COUNT>
 __device__ __forceinline__ void wide_leaf_step(const DevScene& sc, WideLane& L) {
   const int code = ~L.cur;
   const int slot = code >> kLeafCountBits;
@@ -275,10 +276,14 @@ __device__ __forceinline__ void wide_leaf_step(const DevScene& sc, WideLane& L) 
   hold_prim(p);
   hold_prim(q);
   bool done = count > 0 && wide_tri<PRIM>(sc, L, slot, p);
+  if (COUNT) L.ntri += count > 1 && !done ? 2 : 1;
   if (!done && count > 1) done = wide_tri<PRIM>(sc, L, slot + 1, q);
   if (!done && count == kLeafCountInline) {
     const int end = slot + sc.big_count[slot];
-    for (int k = slot + 2; k < end && !done; ++k) done = wide_tri<PRIM>(sc, L, k, fetch_prim(sc, k));
+    for (int k = slot + 2; k < end && !done; ++k) {
+      if (COUNT) ++L.ntri;
+      done = wide_tri<PRIM>(sc, L, k, fetch_prim(sc, k));
+    }
   }
   // (of two hits in this leaf the later one's test covers both: its minT is the smaller one)
   if (old >= 0 && L.h.best != old) L.bad |= !leaf_entered(sc, L, old, entered);
@@ -302,9 +307,10 @@ __device__ __forceinline__ int pair_ref(const WideLane& L, int child, int word) 
 // Visits the children L.cur of an inner record: the boxes of both are tested as the reference
 // tests them (the farther one's distance again when it is taken off the stack, which is its
 // later test with the minT of that moment).
-template <int S, int BLOCK>
+template <bool COUNT, int S, int BLOCK>
 __device__ __forceinline__ void wide_pair_step(const DevScene& sc, WideLane& L,
                                                WideStack<S, BLOCK>& st) {
+  if (COUNT) L.nbox += 2;
   const float4* p = reinterpret_cast<const float4*>(sc.refs + (L.cur >> 1));
   const float4 A = p[0], B = p[1], C = p[2], D = p[3];
   Ray r = L.r;
@@ -322,16 +328,16 @@ __device__ __forceinline__ void wide_pair_step(const DevScene& sc, WideLane& L,
 }
 
 // One step of the wave; a lane at a leaf weighs `weight` quarters of one at a node.
-template <int PRIM, bool PAIRS, int S, int BLOCK>
+template <int PRIM, bool PAIRS, bool COUNT, int S, int BLOCK>
 __device__ __forceinline__ void wide_step(const DevScene& sc, WideLane& L, int weight,
                                           WideStack<S, BLOCK>& st) {
   const unsigned long long at_node = wave_mask(L.cur >= 0);
   const unsigned long long at_leaf = wave_mask(L.cur < 0) & wave_mask(L.cur > kPop);
   if (weight * __popcll(at_leaf) >= 4 * __popcll(at_node)) {
-    if (lane_bit(at_leaf)) wide_leaf_step<PRIM, PAIRS>(sc, L);
+    if (lane_bit(at_leaf)) wide_leaf_step<PRIM, PAIRS, COUNT>(sc, L);
   } else if (lane_bit(at_node)) {
     if constexpr (PAIRS)
-      wide_pair_step<S, BLOCK>(sc, L, st);
+      wide_pair_step<COUNT, S, BLOCK>(sc, L, st);
     else
       wide_node_step<S, BLOCK>(sc, L, st);
   }
@@ -345,7 +351,7 @@ __device__ __forceinline__ void wide_step(const DevScene& sc, WideLane& L, int w
 }
 
 // The reference's own traversal of ray i, on its 32-byte records.
-template <int PRIM, int S, int BLOCK, class Index>
+template <int PRIM, bool COUNT, int S, int BLOCK, class Index>
 __device__ __forceinline__ void wide_redo(const DevScene& sc, const GRays& rays, Index i,
                                           WideLane& L, WideStack<S, BLOCK>& st) {
   const bool any = L.ord == kAnyOrder;
@@ -363,6 +369,7 @@ __device__ __forceinline__ void wide_redo(const DevScene& sc, const GRays& rays,
         bool done = false;
         for (int k = 0; k < nd.children && !done; ++k) {
           float t, u, v;
+          if (COUNT) ++L.ntri;
           if (prim_test<PRIM>(sc, nd.child + k, r, h.minT, t, u, v)) {
             h = RayHit{t, nd.child + k, u, v};
             done = any;
@@ -370,6 +377,7 @@ __device__ __forceinline__ void wide_redo(const DevScene& sc, const GRays& rays,
         }
         if (done) break;
       } else {
+        if (COUNT) L.nbox += 2;
         const int front = any ? ((nd.bits & 1) ? 0 : 1) : (((r.dpos >> (nd.axis & 3)) & 1) ? 0 : 1);
         st.push3(0, 0, 0.f, 0, 0, 0.f, ~0ull, nd.child + 1 - front, 0.f);
         cur = nd.child + front;
@@ -394,6 +402,8 @@ __device__ __forceinline__ void wide_start(const DevScene& sc, float reach, cons
   L.enter = L.h.minT;
   st.reset();
   L.ord = any ? kAnyOrder : 3u * (L.r.dpos & 7u);
+  L.nbox = 1;  // the root's
+  L.ntri = 0;
   if (irregular == 1) {
 #pragma unroll
     for (int k = 0; k < 3; ++k) L.w.inv[k] = L.r.inv[k];
@@ -411,12 +421,12 @@ __device__ __forceinline__ void wide_start(const DevScene& sc, float reach, cons
 }
 
 // Stores the hit of a lane that has come to the end of ray i.
-template <int PRIM, int S, int BLOCK, class Index>
+template <int PRIM, bool COUNT, int S, int BLOCK, class Index>
 __device__ __forceinline__ void wide_finish(const DevScene& sc, const GRays& rays,
                                             const GHits& hits, Index i, int irregular,
                                             WideLane& L, WideStack<S, BLOCK>& st) {
   if (irregular == 0 && !L.bad && L.h.best >= 0) L.bad = !leaf_entered(sc, L, L.h.best, L.enter);
-  if (L.bad) wide_redo<PRIM, S, BLOCK>(sc, rays, i, L, st);
+  if (L.bad) wide_redo<PRIM, COUNT, S, BLOCK>(sc, rays, i, L, st);
   const bool hit = L.h.best >= 0;
   store_hit(hits, i, hit ? sc.obj_ids[L.h.best] : -1, (L.ord == kAnyOrder && hit) ? kEps : L.h.minT, L.h.u,
             L.h.v, hit);
@@ -427,6 +437,7 @@ struct WideArgs {
   const BatchTable* table;  // a table of batches, or null
   BatchDev one;             // table null: the only batch
   unsigned long long* ctr;  // u64[2], zero between launches; null with a static stride
+  unsigned long long* counters;  // COUNT: box and triangle tests
   unsigned long long* spill;
   int64_t spill_stride;
   int nb;       // batches of the table, as the host counted them
@@ -469,8 +480,9 @@ __device__ __forceinline__ GHits moved(GHits h, int64_t n) {
 // Waves that trace their rays 64 at a time, a ray to a lane: chunks of `chunk` consecutive
 // rays by a static stride, each cut where a batch ends. A wave lives for about ten steps
 // on camera rays, so what it does beside them is kept short: no lane hand-out, batch
-// arrays read where a group starts and where it ends. Five waves a SIMD.
-template <int PRIM, int S, int BLOCK, bool TABLE>
+// arrays read where a group starts and where it ends. Five waves a SIMD. COUNT: on the
+// records, whose tests are the reference's, adding up box and triangle tests.
+template <int PRIM, int S, int BLOCK, bool TABLE, bool COUNT>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_wide_whole(
     WideArgs a) {
   __shared__ unsigned long long s_ring[S * BLOCK];
@@ -493,6 +505,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5, 8))) v
   const float reach = root_reach(a.sc);
   int irregular = *a.sc.irregular;
   if (!TABLE && a.pairs && irregular == 0) irregular = 1;
+  unsigned long long nbox = 0, ntri = 0;
   const int C = a.chunk;
   const int64_t stride = (int64_t)gridDim.x * (BLOCK / 64) * C;
   // (the wave's number is the same in all its lanes: kept in scalar registers)
@@ -526,18 +539,34 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5, 8))) v
                                L, st);
         }
       }
-      if (irregular == 0)
-        while (wave_mask(L.cur != kIdle)) wide_step<PRIM, false, S, BLOCK>(a.sc, L, a.weight, st);
+      if (!COUNT && irregular == 0)
+        while (wave_mask(L.cur != kIdle))
+          wide_step<PRIM, false, COUNT, S, BLOCK>(a.sc, L, a.weight, st);
       else
-        while (wave_mask(L.cur != kIdle)) wide_step<PRIM, true, S, BLOCK>(a.sc, L, a.weight, st);
+        while (wave_mask(L.cur != kIdle))
+          wide_step<PRIM, true, COUNT, S, BLOCK>(a.sc, L, a.weight, st);
       if (live) {
         const WideArgs& again = args_again();
         const BatchDev* E = TABLE ? again.table->batches + bi : &again.one;
-        wide_finish<PRIM, S, BLOCK>(again.sc, moved(global_view(E->rays), pos - first),
-                                    moved(global_view(E->hits), pos - first), (unsigned)lane,
-                                    irregular, L, st);
+        wide_finish<PRIM, COUNT, S, BLOCK>(again.sc, moved(global_view(E->rays), pos - first),
+                                           moved(global_view(E->hits), pos - first),
+                                           (unsigned)lane, irregular, L, st);
+        if (COUNT) {
+          nbox += L.nbox;
+          ntri += L.ntri;
+        }
       }
       pos += n;
+    }
+  }
+  if (COUNT) {
+    for (int m = 1; m < 64; m <<= 1) {
+      nbox += __shfl_xor(nbox, m, 64);
+      ntri += __shfl_xor(ntri, m, 64);
+    }
+    if (lane == 0) {
+      atomicAdd(a.counters + 0, nbox);
+      atomicAdd(a.counters + 1, ntri);
     }
   }
 }
@@ -608,7 +637,7 @@ __device__ __forceinline__ void wide_lanes(const WideArgs& a, unsigned long long
     }
     if (take_rays) {
       by_batch(lane_bit(idle) && li >= 0, [&](const GRays& rays, const GHits& hits, uint32_t) {
-        wide_finish<PRIM, S, BLOCK>(sc, rays, hits, li, irregular, L, st);
+        wide_finish<PRIM, false, S, BLOCK>(sc, rays, hits, li, irregular, L, st);
       });
       if (lane_bit(idle)) li = -1;
       if (!more) break;  // every lane is idle
@@ -635,7 +664,7 @@ __device__ __forceinline__ void wide_lanes(const WideArgs& a, unsigned long long
       });
       pos = pos + n_idle < end ? pos + n_idle : end;
     }
-    wide_step<PRIM, PAIRS, S, BLOCK>(sc, L, a.weight, st);
+    wide_step<PRIM, PAIRS, false, S, BLOCK>(sc, L, a.weight, st);
   }
   if (lane == 0) {
     const unsigned long long left = atomicAdd(a.ctr + 1, 1ull);
@@ -665,7 +694,7 @@ void launch_table(const WideArgs& a, dim3 g, hipStream_t s) {
   if (a.ctr)
     hipLaunchKernelGGL((k_wide_lanes<PRIM, S, BLOCK>), g, dim3(BLOCK), lds, s, a);
   else
-    hipLaunchKernelGGL((k_wide_whole<PRIM, S, BLOCK, true>), g, dim3(BLOCK), lds, s, a);
+    hipLaunchKernelGGL((k_wide_whole<PRIM, S, BLOCK, true, false>), g, dim3(BLOCK), lds, s, a);
 }
 template <int PRIM, int BLOCK>
 int launch_table(const WideArgs& a, dim3 g, int stack_lds, hipStream_t s) {
@@ -702,25 +731,31 @@ int launch_wide_table(const DevScene& sc, const BatchLaunch& bl, hipStream_t s) 
   return launch_table<PRIM, 256>(a, g, bl.stack_lds, s);
 }
 
+template <int PRIM, bool COUNT>
+int launch_one(const WideArgs& a, const LaunchCfg& cfg, hipStream_t s) {
+  const dim3 g(cfg.blocks), b(64);
+  if (cfg.stack_lds == 8)
+    hipLaunchKernelGGL((k_wide_whole<PRIM, 8, 64, false, COUNT>), g, b, 0, s, a);
+  else if (cfg.stack_lds == 32)
+    hipLaunchKernelGGL((k_wide_whole<PRIM, 32, 64, false, COUNT>), g, b, 0, s, a);
+  else
+    hipLaunchKernelGGL((k_wide_whole<PRIM, 16, 64, false, COUNT>), g, b, 0, s, a);
+  return (int)hipGetLastError();
+}
+
 template <int PRIM>
 int launch_wide_one(const DevScene& sc, const BatchDev& rays, const LaunchCfg& cfg, hipStream_t s) {
   WideArgs a{};
   a.sc = sc;
   a.one = rays;
+  a.counters = reinterpret_cast<unsigned long long*>(cfg.counters);
   a.spill = reinterpret_cast<unsigned long long*>(cfg.spill);
   a.spill_stride = cfg.spill_stride;
   a.chunk = cfg.chunk;
   a.pairs = cfg.pairs;
   a.reverse = 1;
   a.weight = kLeafWeight;
-  const dim3 g(cfg.blocks), b(64);
-  if (cfg.stack_lds == 8)
-    hipLaunchKernelGGL((k_wide_whole<PRIM, 8, 64, false>), g, b, 0, s, a);
-  else if (cfg.stack_lds == 32)
-    hipLaunchKernelGGL((k_wide_whole<PRIM, 32, 64, false>), g, b, 0, s, a);
-  else
-    hipLaunchKernelGGL((k_wide_whole<PRIM, 16, 64, false>), g, b, 0, s, a);
-  return (int)hipGetLastError();
+  return a.counters ? launch_one<PRIM, true>(a, cfg, s) : launch_one<PRIM, false>(a, cfg, s);
 }
 
 }  // namespace

@@ -7,7 +7,7 @@
 //   load:NAME    NAME.ids and NAME.nodes into the scene
 //   verts:FILE   the vertices of FILE
 //   trace:N,BLOCKS,RING,COUNT  mh_trace of N rays with blocks_per_cu, stack_lds and, if COUNT,
-//                counters: prints "blocks B layout L ring R spill BYTES pairs P" of its launch
+//                counters: prints "blocks B ring R spill BYTES pairs P" of its launch
 //   refill:R,C   prints "refill N", the idle lanes that a launch configuration's refill and
 //                chunk come to in the default layout
 //   soa          the node arrays of the SOA layout
@@ -196,14 +196,12 @@ int main(int argc, char** argv) {
       check(g_fixed ? mh_internal::trace_fixed_spill(s, &rays, &hits, n, 0, &o, nullptr, &fixed, g_fixed)
                     : mh_trace(s, &rays, &hits, n, 0, &o, nullptr), op);
       const mh::LaunchCfg& c = g_launch;
-      const int lanes = c.layout == mh::kLayoutPair ? 64 : 256;
       const int64_t stack =
-          (c.pairs ? (int64_t)s->depth + 2 : (int64_t)s->stack_bound(c.layout)) - c.stack_lds;
-      need(c.blocks > 0 && c.spill_stride == (int64_t)c.blocks * lanes, "spill columns", c.blocks);
+          (c.pairs ? (int64_t)s->depth + 2 : (int64_t)s->stack_bound(MH_LAYOUT_PAIR)) - c.stack_lds;
+      need(c.blocks > 0 && c.spill_stride == (int64_t)c.blocks * 64, "spill columns", c.blocks);
       const size_t area = stack <= 0 ? 0 : g_fixed ? g_fixed : s->spill[nullptr]->bytes;
       if (stack > 0) need((size_t)stack * c.spill_stride * 8 <= area, "spill area", stack);
-      std::printf("blocks %d layout %d ring %d spill %zu pairs %d\n", c.blocks, c.layout,
-                  c.stack_lds, area, c.pairs);
+      std::printf("blocks %d ring %d spill %zu pairs %d\n", c.blocks, c.stack_lds, area, c.pairs);
     } else if (what == "fixed") {
       g_fixed = (size_t)std::atoll(op.c_str() + colon + 1);
     } else if (what == "refill") {

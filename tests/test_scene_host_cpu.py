@@ -248,12 +248,12 @@ def _launches(scene_host, oracle, tmp_path, n_tris, *ops):
 
 
 def test_blocks_per_cu_with_counters(scene_host, oracle, tmp_path):
-    """The caller's workgroups per compute unit hold for the counting kernel as for the other
-    (256 lanes each, of 256 compute units)."""
+    """The caller's workgroups per compute unit (four waves each, of 256 compute units) hold for
+    counting launches as for others; those run on the records."""
     a, b, c, d = _launches(scene_host, oracle, tmp_path, 4, "trace:4000000,2,8,1", "trace:4000000,0,8,1",
                            "trace:4000000,2,8,0", "trace:100,2,8,1")
-    assert (a["layout"], a["blocks"]) == (1, 512) and b["blocks"] == 4096
-    assert (c["layout"], c["blocks"]) == (0, 4 * 512) and d["blocks"] == 1
+    assert (a["pairs"], a["blocks"]) == (1, 2048) and b["blocks"] == 32768
+    assert (c["pairs"], c["blocks"]) == (0, 2048) and d["blocks"] == 25
 
 
 def test_spill_area_is_bounded(scene_host, oracle, tmp_path):
@@ -301,7 +301,6 @@ def test_fixed_spill_area_of_deep_trees(scene_host, oracle, tmp_path, ring, rays
         d = tmp_path / str(n)
         d.mkdir()
         got, = _launches(scene_host, oracle, d, n, f"fixed:{32 << 20}", f"trace:{rays},0,{ring},0")
-        assert got["layout"] == 0
         if n in (20, 73) and rays > 4097:
             assert got["pairs"] == (n == 73)
     d = tmp_path / "refused"
