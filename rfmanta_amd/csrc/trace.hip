@@ -7,7 +7,8 @@
 //   lane tests its own ray, and everything about the packet (rays still looking, rays that
 //   hit, firstActive/lastActive, child order) is kept as wave-uniform masks. The
 //   interval-arithmetic frustum test (DynBVH.cc:682-721) runs on wave-reduced ray bounds.
-//   Bound by vector issue, so what is uniform stays in scalar registers (vector loads of
+//   A wave visits one record at a time and waits for its scalar loads (vector instructions
+//   take 45% of their slots), and what is uniform stays in scalar registers (vector loads of
 //   the records, vector masks and a stack in LDS took 1.16 times as long: 801 against
 //   706 us for 2.07M camera rays in packets of 64 over a 1M-triangle heightfield). Testing
 //   both children at their parent, so that the farther one need not be pushed, was slower
