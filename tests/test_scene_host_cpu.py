@@ -292,19 +292,20 @@ def test_refill_is_the_callers(scene_host, oracle, tmp_path):
     assert [g["refill"] for g in got] == [1, 16, 32, 63, 64, 64, 40]
 
 
-@pytest.mark.parametrize("ring", [0, 8, 16, 32])
-@pytest.mark.parametrize("rays", [1, 64, 4097, 4000000])
-def test_fixed_spill_area_of_deep_trees(scene_host, oracle, tmp_path, ring, rays):
+def test_fixed_spill_area_of_deep_trees(scene_host, oracle, tmp_path):
     """Every launch fits the area (scene_host.cpp checks it), with the wide nodes while four
     waves per compute unit do, then on the records, up to the depth that is refused."""
+    sets = [(rays, ring) for rays in (1, 64, 4097, 4000000) for ring in (0, 8, 16, 32)]
     for n in (20, 50, 60, 73):
         d = tmp_path / str(n)
         d.mkdir()
-        got, = _launches(scene_host, oracle, d, n, f"fixed:{32 << 20}", f"trace:{rays},0,{ring},0")
-        if n in (20, 73) and rays > 4097:
-            assert got["pairs"] == (n == 73)
-    d = tmp_path / "refused"
-    d.mkdir()
-    if ring in (0, 8) and rays > 4097:
+        got = _launches(scene_host, oracle, d, n, f"fixed:{32 << 20}",
+                        *[f"trace:{rays},0,{ring},0" for rays, ring in sets])
+        assert len(got) == len(sets)
+        if n in (20, 73):
+            assert all(g["pairs"] == (n == 73) for g in got[-4:])
+    for ring in (0, 8):
+        d = tmp_path / f"refused {ring}"
+        d.mkdir()
         with pytest.raises(AssertionError, match="of stack spill for 256 workgroups"):
-            _launches(scene_host, oracle, d, 75, f"fixed:{32 << 20}", f"trace:{rays},0,{ring},0")
+            _launches(scene_host, oracle, d, 75, f"fixed:{32 << 20}", f"trace:4000000,0,{ring},0")
