@@ -461,10 +461,9 @@ int trace_impl(const mh_scene* cs, const mh_rays* rays, const mh_hits* hits, int
     const int S = own == 8 || own == 16 || own == 32 ? own
                   : waves <= kFewWaves * cus         ? kFewWavesRing
                                                      : kWideRing;
-    // Entries of a spill column: the wide nodes' stack, or the records' one entry a level (and
-    // the ring, which makes room for three at a time, spills two early).
+    // Entries of a spill column: the wide nodes' stack, or the records' one entry a level.
     const int64_t wide_need = std::max<int64_t>(0, (int64_t)s->stack_bound(MH_LAYOUT_PAIR) - S);
-    const int64_t pairs_need = std::max<int64_t>(0, (int64_t)s->depth + 2 - S);
+    const int64_t pairs_need = std::max<int64_t>(0, (int64_t)s->stack_bound(MH_LAYOUT_REF) - S);
     cfg.pairs = cfg.counters != nullptr;  // (the tests counted are those of the records' boxes)
     int64_t need = cfg.pairs ? pairs_need : wide_need;
     int64_t blocks = std::min(waves, 4 * cus * bpc);

@@ -6,24 +6,28 @@
 // and the direction's signs (isLeftCheaper for any hit, DynBVH.cc:386-398), and enters a
 // leaf if its slab test and those of the inner records above it pass with the minT of that
 // moment. Boxes nest and every step of the slab test is monotone (products that are not
-// numbers aside, see leaf_entered), so a leaf whose own test passes passes it all the way
-// up: which leaves are entered depends on the leaf boxes
-// alone, and inner boxes may be tested with any arithmetic that never rejects what the
-// reference accepts. So here an inner test is one fused multiply-add a plane, widened by
-// more than all rounding errors (WideRay), two tree levels are tested at a time, and the
-// exact test of a leaf is run only for leaves that gave a hit: when a later hit replaces it
-// or the ray ends, with the minT of the hit's acceptance (a leaf that passes with that one
-// passes with the larger one of its visit). While every such leaf passes, minT is the
-// reference's at every leaf, and the leaves visited here are its leaves and others that
-// accepted nothing. Should one fail, which takes a hit within rounding of its leaf's box,
-// the ray is traced again by the reference's own steps (wide_redo). Nothing is assumed of
-// where triangles lie in their boxes: a grazing ray's computed distance may lie before the
-// box, and a loaded tree's boxes may be those of another pose. (Leaving out the test of a
-// hit replaced by one that is clearly nearer gained up to 0.8%: 1,593 against 1,606 us for
-// 12 uneven batches in a 300,000-triangle soup, nothing on a heightfield.) Rays outside the
-// bounds below take wide_redo from the start. Trees whose boxes do not nest are traversed on
-// their 32-byte records, the two children of a record a step, every box tested exactly
-// (wide_pair_step).
+// numbers aside, see leaf_entered), so a leaf whose own test passes passes it all the way up:
+// which leaves are entered depends on the leaf boxes alone, and inner boxes may be tested with
+// any arithmetic that never rejects what the reference accepts. So here an inner test is one
+// fused multiply-add a plane, widened by more than all rounding errors (WideRay), two tree
+// levels are tested at a time, and the exact test of a leaf is run only for leaves that gave a
+// hit: when a later hit replaces it or the ray ends, with the minT of the hit's acceptance (a
+// leaf that passes with that one passes with the larger one of its visit). While every such
+// leaf passes, minT is the reference's at every leaf, and the leaves visited here are its
+// leaves and others that accepted nothing. Should one fail, which takes a hit within rounding
+// of its leaf's box, the ray is traced again, as are rays outside the bounds below. Nothing is
+// assumed of where triangles lie in their boxes: a grazing ray's computed distance may lie
+// before the box, and a loaded tree's boxes may be those of another pose. (Leaving out the
+// test of a hit replaced by one that is clearly nearer gained up to 0.8%: 1,593 against 1,606
+// us for 12 uneven batches in a 300,000-triangle soup, nothing on a heightfield.)
+//
+// Rays that are traced again, and trees whose boxes do not nest, are traversed on the 32-byte
+// records, the two children of a record a step, every box tested exactly (wide_pair_step;
+// k_wide_lanes, whose lanes are at different rays, runs the reference's own steps in one loop
+// instead, wide_redo). A whole wave may need it: of vertical rays from a heightfield's
+// vertices, which lie on box planes, every one with positive zero components hits a leaf that
+// the reference does not enter (500,000: 149 us, 172 with wide_redo, 47 on binary nodes alone,
+// which visit no such leaf; 61 from between the vertices).
 //
 // How the wave works. A node visit costs about 110 vector instructions and a triangle test
 // about 95, and each waits about 850 cycles for its record (L2 and MALL; a 10,000-triangle
@@ -109,14 +113,15 @@ struct WideLane {
 };
 constexpr unsigned kAnyOrder = 24;
 
-// Whether the ray passes the reference's slab test of the leaf that holds object slot `slot`.
-// Along an axis whose reciprocal may have been cut (wide_setup) the origin has to lie between
-// the leaf's planes: then the cut reciprocal changes no near distance and brings the far one
-// closer, so a box that passes passes uncut as well. (No reciprocal is formed again for that:
-// 1M vertical rays over a 1M-triangle heightfield took 98 us with one, 92 without.) False,
-// though the reference's test may pass, for an origin on or beyond such a plane: products
-// that are not numbers drop out of the reference's test there, and a box around one that
-// passes need not pass.
+// Whether the ray passes the reference's slab test of the leaf that holds object slot `slot`,
+// or false where that test and those of the boxes around the leaf may differ:
+//   - along a component so small that its reciprocal may have been cut (wide_setup), the
+//     origin has to lie between the leaf's planes, or on the near one: then the cut reciprocal
+//     changes no near distance and brings the far one closer, so a box that passes passes uncut
+//     as well (without forming the reciprocal again);
+//   - across a zero component the leaf must not be flat in the origin's plane: products that
+//     are not numbers drop out of the reference's test there, and a box around such a leaf
+//     need not pass.
 __device__ __forceinline__ bool leaf_entered(const DevScene& sc, const WideLane& L, int slot,
                                              float minT) {
   int rec = sc.leaf_at[slot];
@@ -128,12 +133,16 @@ __device__ __forceinline__ bool leaf_entered(const DevScene& sc, const WideLane&
   const float dmin = fminf(fminf(fabsf(r.d[0]), fabsf(r.d[1])), fabsf(r.d[2]));
   const float dmax = fmaxf(fmaxf(fabsf(r.d[0]), fabsf(r.d[1])), fabsf(r.d[2]));
   if (dmin * 0x1p39f < dmax) {
-    bool between = true;
+    bool same = true;
 #pragma unroll
-    for (int k = 0; k < 3; ++k)
-      between &= (fabsf(r.d[k]) * 0x1p39f >= dmax) |
-                 ((nd.box.lo[k] < r.o[k]) & (r.o[k] < nd.box.hi[k]));
-    if (!between) return false;
+    for (int k = 0; k < 3; ++k) {
+      const float o = r.o[k], lo = nd.box.lo[k], hi = nd.box.hi[k];
+      const bool zero = r.d[k] == 0.f, neg = r.inv[k] < 0.f;
+      const bool between = neg ? (lo < o) & (o <= hi) : (lo <= o) & (o < hi);
+      same &= (fabsf(r.d[k]) * 0x1p39f >= dmax) | (zero ? (lo != o) | (hi != o) : between);
+      r.inv[k] = zero ? __builtin_copysignf(__builtin_inff(), r.inv[k]) : r.inv[k];
+    }
+    if (!same) return false;
   }
   float tn;
   return slab(nd.box.lo[0], nd.box.hi[0], nd.box.lo[1], nd.box.hi[1], nd.box.lo[2], nd.box.hi[2],
@@ -153,10 +162,8 @@ __device__ __forceinline__ unsigned long long wide_box(float nx, float fx, float
 }
 
 // Per-lane stack, its newest S entries in LDS ([entry][lane], no bank conflicts), older ones
-// in the thread's spill column. sp and base count in steps of U bytes. A push makes room for
-// three entries whatever it keeps, so a column holds up to n - S of the wide nodes' at most n
-// entries (three a node), and up to n + 2 - S of n that come one at a time (wide_pair_step,
-// wide_redo: a tree of depth n; a column made for the wide nodes is longer than that).
+// in the thread's spill column, which holds n - S for a stack of at most n (three a wide node;
+// one a level on the records). sp and base count in steps of U bytes.
 template <int S, int BLOCK>
 struct WideStack {
   static_assert((S & (S - 1)) == 0 && S > 4, "ring size is a power of two");
@@ -179,7 +186,7 @@ struct WideStack {
   }
   __device__ __forceinline__ void reset() { sp = base = 0; }
   // Up to three entries, the deepest first; each is written, and kept for the lanes of its
-  // mask.
+  // mask. Room is made for three whatever is kept.
   __device__ __forceinline__ void push3(unsigned long long ma, int ra, float ta,
                                         unsigned long long mb, int rb, float tb,
                                         unsigned long long mc, int rc, float tc) {
@@ -195,6 +202,17 @@ struct WideStack {
     sp += lane_bit(mb) ? U : 0;
     *at(sp) = stack_entry(rc, tc);
     sp += lane_bit(mc) ? U : 0;
+  }
+  // One entry.
+  __device__ __forceinline__ void push1(unsigned long long m, int r, float t) {
+    if (wave_mask(sp - base > RM)) {
+      if (sp - base > RM) {
+        *spilled(base) = *at(base);
+        base += U;
+      }
+    }
+    *at(sp) = stack_entry(r, t);
+    sp += lane_bit(m) ? U : 0;
   }
   // The newest entry of the lanes that have one (`have`); the caller takes it off.
   __device__ __forceinline__ unsigned long long top(bool have) {
@@ -323,7 +341,7 @@ __device__ __forceinline__ void wide_pair_step(const DevScene& sc, WideLane& L,
   const int r0 = pair_ref(L, __float_as_int(B.z), __float_as_int(B.w)),
             r1 = pair_ref(L, __float_as_int(D.z), __float_as_int(D.w));
   const bool f = lane_bit(F);
-  st.push3(H0 & H1, f ? r0 : r1, f ? t0 : t1, 0, 0, 0.f, 0, 0, 0.f);
+  st.push1(H0 & H1, f ? r0 : r1, f ? t0 : t1);
   L.cur = lane_bit(H0 & H1) ? (f ? r1 : r0) : (lane_bit(H0) ? r0 : (lane_bit(H1) ? r1 : kPop));
 }
 
@@ -379,7 +397,7 @@ __device__ __forceinline__ void wide_redo(const DevScene& sc, const GRays& rays,
       } else {
         if (COUNT) L.nbox += 2;
         const int front = any ? ((nd.bits & 1) ? 0 : 1) : (((r.dpos >> (nd.axis & 3)) & 1) ? 0 : 1);
-        st.push3(0, 0, 0.f, 0, 0, 0.f, ~0ull, nd.child + 1 - front, 0.f);
+        st.push1(~0ull, nd.child + 1 - front, 0.f);
         cur = nd.child + front;
         continue;
       }
@@ -389,6 +407,18 @@ __device__ __forceinline__ void wide_redo(const DevScene& sc, const GRays& rays,
     st.sp -= st.U;
   }
   L.h = h;
+}
+
+// Starts ray L.r on the records.
+__device__ __forceinline__ void pair_start(const DevScene& sc, WideLane& L) {
+#pragma unroll
+  for (int k = 0; k < 3; ++k) L.w.inv[k] = L.r.inv[k];
+  const RefNode& nd = sc.refs[0];
+  float tn;
+  const bool in = slab(nd.box.lo[0], nd.box.hi[0], nd.box.lo[1], nd.box.hi[1], nd.box.lo[2],
+                       nd.box.hi[2], L.r, L.h.minT, tn);
+  L.bad = false;
+  L.cur = in ? pair_ref(L, nd.child, (nd.children << 16) | (nd.bits << 8) | nd.axis) : kIdle;
 }
 
 // Starts ray i of `rays` in an idle lane (Index: 32 bits where the views were moved to the
@@ -405,14 +435,7 @@ __device__ __forceinline__ void wide_start(const DevScene& sc, float reach, cons
   L.nbox = 1;  // the root's
   L.ntri = 0;
   if (irregular == 1) {
-#pragma unroll
-    for (int k = 0; k < 3; ++k) L.w.inv[k] = L.r.inv[k];
-    const RefNode& nd = sc.refs[0];
-    float tn;
-    const bool in = slab(nd.box.lo[0], nd.box.hi[0], nd.box.lo[1], nd.box.hi[1], nd.box.lo[2],
-                         nd.box.hi[2], L.r, L.h.minT, tn);
-    L.bad = false;
-    L.cur = in ? pair_ref(L, nd.child, (nd.children << 16) | (nd.bits << 8) | nd.axis) : kIdle;
+    pair_start(sc, L);
     return;
   }
   const bool ok = (irregular == 0) & wide_setup(reach, L.r, L.h.minT, L.w);
@@ -420,12 +443,16 @@ __device__ __forceinline__ void wide_start(const DevScene& sc, float reach, cons
   L.cur = ok ? sc.root_ref : kIdle;
 }
 
+// Whether the leaf of the ray's hit has yet to show that the reference enters it, and does not.
+__device__ __forceinline__ bool last_leaf_missed(const DevScene& sc, const WideLane& L) {
+  return !L.bad && L.h.best >= 0 && !leaf_entered(sc, L, L.h.best, L.enter);
+}
+
 // Stores the hit of a lane that has come to the end of ray i.
 template <int PRIM, bool COUNT, int S, int BLOCK, class Index>
 __device__ __forceinline__ void wide_finish(const DevScene& sc, const GRays& rays,
-                                            const GHits& hits, Index i, int irregular,
-                                            WideLane& L, WideStack<S, BLOCK>& st) {
-  if (irregular == 0 && !L.bad && L.h.best >= 0) L.bad = !leaf_entered(sc, L, L.h.best, L.enter);
+                                            const GHits& hits, Index i, WideLane& L,
+                                            WideStack<S, BLOCK>& st) {
   if (L.bad) wide_redo<PRIM, COUNT, S, BLOCK>(sc, rays, i, L, st);
   const bool hit = L.h.best >= 0;
   store_hit(hits, i, hit ? sc.obj_ids[L.h.best] : -1, (L.ord == kAnyOrder && hit) ? kEps : L.h.minT, L.h.u,
@@ -539,18 +566,26 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5, 8))) v
                                L, st);
         }
       }
-      if (!COUNT && irregular == 0)
+      if (!COUNT && irregular == 0) {
         while (wave_mask(L.cur != kIdle))
           wide_step<PRIM, false, COUNT, S, BLOCK>(a.sc, L, a.weight, st);
-      else
-        while (wave_mask(L.cur != kIdle))
-          wide_step<PRIM, true, COUNT, S, BLOCK>(a.sc, L, a.weight, st);
+        if (live) L.bad |= last_leaf_missed(a.sc, L);
+        if (wave_mask(live && L.bad)) {  // again, on the records
+          const BatchDev* E = TABLE ? args_again().table->batches + bi : &args_again().one;
+          const GRays rays = moved(global_view(E->rays), pos - first);
+          if (live && L.bad) {
+            wide_start<S, BLOCK>(a.sc, reach, rays, (unsigned)lane, L.ord == kAnyOrder, 1, L, st);
+          }
+        }
+      }
+      while (wave_mask(L.cur != kIdle))
+        wide_step<PRIM, true, COUNT, S, BLOCK>(a.sc, L, a.weight, st);
       if (live) {
         const WideArgs& again = args_again();
         const BatchDev* E = TABLE ? again.table->batches + bi : &again.one;
         wide_finish<PRIM, COUNT, S, BLOCK>(again.sc, moved(global_view(E->rays), pos - first),
                                            moved(global_view(E->hits), pos - first),
-                                           (unsigned)lane, irregular, L, st);
+                                           (unsigned)lane, L, st);
         if (COUNT) {
           nbox += L.nbox;
           ntri += L.ntri;
@@ -637,7 +672,8 @@ __device__ __forceinline__ void wide_lanes(const WideArgs& a, unsigned long long
     }
     if (take_rays) {
       by_batch(lane_bit(idle) && li >= 0, [&](const GRays& rays, const GHits& hits, uint32_t) {
-        wide_finish<PRIM, false, S, BLOCK>(sc, rays, hits, li, irregular, L, st);
+        if (!PAIRS && irregular == 0) L.bad |= last_leaf_missed(sc, L);
+        wide_finish<PRIM, false, S, BLOCK>(sc, rays, hits, li, L, st);
       });
       if (lane_bit(idle)) li = -1;
       if (!more) break;  // every lane is idle

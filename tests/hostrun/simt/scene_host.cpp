@@ -197,7 +197,7 @@ int main(int argc, char** argv) {
                     : mh_trace(s, &rays, &hits, n, 0, &o, nullptr), op);
       const mh::LaunchCfg& c = g_launch;
       const int64_t stack =
-          (c.pairs ? (int64_t)s->depth + 2 : (int64_t)s->stack_bound(MH_LAYOUT_PAIR)) - c.stack_lds;
+          (int64_t)s->stack_bound(c.pairs ? MH_LAYOUT_REF : MH_LAYOUT_PAIR) - c.stack_lds;
       need(c.blocks > 0 && c.spill_stride == (int64_t)c.blocks * 64, "spill columns", c.blocks);
       const size_t area = stack <= 0 ? 0 : g_fixed ? g_fixed : s->spill[nullptr]->bytes;
       if (stack > 0) need((size_t)stack * c.spill_stride * 8 <= area, "spill area", stack);

@@ -164,6 +164,29 @@ def test_axis_parallel_rays_without_end(oracle, mesh, axis):
         _check(oracle, s, v, i, nodes, ids, rays, mesh)
 
 
+@pytest.mark.parametrize("axis", [0, 1, 2])
+def test_rays_through_vertices(oracle, axis):
+    """Axis-parallel rays from the planes of their leaves' boxes, the other components zeros of
+    both signs or tiny, so that whole waves hit leaves that the reference does not enter."""
+    v, i = scenes.heightfield(33, 29, seed=4)
+    v = np.ascontiguousarray(np.roll(v, axis - 1, axis=1))
+    nodes, ids, _ = oracle.build_bvh(v, i)
+    small = [0.0, -0.0, 6e-17, -6e-17, 1e-30, -1e-13]
+    n, m = len(v), len(small)
+    rays = {k: np.zeros(2 * m * n, np.float32) for k in api.RAY_FIELDS}
+    for k, c in enumerate("xyz"):
+        rays["o" + c][:] = np.tile(v[:, k], 2 * m)
+        rays["d" + c][:] = np.repeat(np.array([small, small[1:] + small[:1]], np.float32).ravel(), n)
+    sign = np.repeat([1.0, -1.0], m * n).astype(np.float32)
+    rays["d" + "xyz"[axis]][:] = sign
+    rays["o" + "xyz"[axis]][:] = -2 * sign
+    rays["tmax"][:] = 1e19
+    with api.Scene(v, i) as s:
+        s.load_dynbvh(ids, nodes)
+        _check(oracle, s, v, i, nodes, ids, rays, axis)
+        _check_frames(oracle, s, v, i, nodes, ids, rays, axis)
+
+
 def test_origin_in_the_plane_of_a_flat_leaf(oracle):
     """Rays without an x component in the plane of a leaf's flat box, which passes the
     reference's slab test while its parent's fails (a loaded tree whose leaf holds its
